@@ -200,6 +200,17 @@ struct Mat {
 
 void pcg_release_workspace(Mat* A);
 
+// Whether the CSR kernels split the block's tiles by entries
+// (CsrLongStream) instead of rows (CsrTileStream, whose stage holds 2,044
+// entries of a 256-row tile; a larger tile is summed row by row from
+// global memory).  The line lies just below the average at which a tile
+// fills the stage (7.98), above the 7-point stencils, whose gathers of one
+// diagonal by 64 neighbouring rows are contiguous: measured FP64, one
+// product, split by rows / by entries: 100^3 7-point 21.7 / 25.4 us, 256^3
+// 328 / 382 us; 1,000,003 mesh rows of 6.1 entries 43.3 / 41.4 us, of 11.1
+// (split by rows: unstaged) 256 / 70 us.
+inline bool csr_long_rows(const Mat& A) { return (double)A.nnz > 7.5 * (double)A.n; }
+
 }  // namespace cel
 
 // the opaque handle of the C ABI

@@ -277,27 +277,23 @@ __device__ __forceinline__ const float* jad_vals<float>(const MatView& A) { retu
 // after the local sum ((0 + local) + halo...).  With xrow, x[row] is
 // loaded too (before the next tile's loads).  next() contains
 // __syncthreads() for CSR: every thread of the block calls it.
-template <typename VT, typename AT, int FMT, bool HALO>
+template <typename VT, typename AT, int FMT, bool HALO, bool LONG>
 struct TileWalk {
-    CsrTileStream<VT> cs;
+    using Stage = typename CsrStreamOf<VT, LONG>::Stage;
+    typename CsrStreamOf<VT, LONG>::Stream cs;
 
     // Contains __syncthreads() for CSR: every thread of the block calls it.
-    __device__ __forceinline__ void start(const MatView& A, long long t0, long long t1,
-                                          CsrStage<VT>& sm)
+    __device__ __forceinline__ void start(const MatView& A, long long t0, long long t1, Stage& sm)
     {
         if constexpr (FMT == CEL_FMT_CSR) {
-            if (t0 < t1) {  // uniform across the block
-                cs.start(A.n, (int)t0, t0 + 1 < t1 ? (int)t0 + 1 : -1, A.xadj, A.cols,
-                         csr_vals<VT>(A), sm);
-                cs.stage(sm);
-                __syncthreads();
-            }
+            if (t0 < t1)  // uniform across the block
+                cs.open(A.n, (int)t0, t0 + 1 < t1 ? (int)t0 + 1 : -1, A.xadj, A.cols,
+                        csr_vals<VT>(A), sm);
         }
     }
 
     __device__ __forceinline__ AT next(const MatView& A, long long t, long long t1,
-                                       const VT* __restrict__ x, CsrStage<VT>& sm, int& row,
-                                       VT* xrow)
+                                       const VT* __restrict__ x, Stage& sm, int& row, VT* xrow)
     {
         const int r0 = (int)t * kTileRows;
         AT s;
@@ -307,11 +303,7 @@ struct TileWalk {
             row = r0 + threadIdx.x;
             s = cs.template rows<AT>(A.n, (int)t, nxt, aft, A.xadj, A.cols, csr_vals<VT>(A), x, sm,
                                      row, xrow);
-            __syncthreads();  // every row of the tile is summed
-            if (nxt >= 0) {   // uniform across the block
-                cs.stage(sm);
-                __syncthreads();
-            }
+            cs.advance(nxt, sm);
             // CSR: r = 0; r = r + tmp.  COO: the entries were added to 0 one
             // by one (the same bits but for the sign of a zero sum)
             s = A.coo ? s : AT(0) + s;
@@ -344,7 +336,7 @@ struct TileWalk {
 // float): r rounded to FP32, z = jac32 * r32 (p = z at the start or on a
 // restart), e = 0 at the start, the norm taken in FP64 before rounding.
 // The next K1 folds the partials into the token.
-template <typename OUT_T, int FMT, bool HALO, bool REPLACE>
+template <typename OUT_T, int FMT, bool HALO, bool REPLACE, bool LONG>
 __global__ __launch_bounds__(kBlock) void k_residual(MatView A, const double* __restrict__ x,
                                                      const double* __restrict__ b,
                                                      const double* __restrict__ jac,
@@ -362,7 +354,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(MatView A, const double* __
             return;
         }
     }
-    __shared__ CsrStage<double> sm;
+    __shared__ typename CsrStreamOf<double, LONG>::Stage sm;
     __shared__ double red[3 * kWaves];
     const int lb = logical_block();
     const int G = gridDim.x;
@@ -371,7 +363,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(MatView A, const double* __
     unit_range(ntiles, G, lb, t0, t1);
     const bool restart = REPLACE && P.ru_restart;
     double arz = 0.0, arr = 0.0, abb = 0.0;
-    TileWalk<double, double, FMT, HALO> walk;
+    TileWalk<double, double, FMT, HALO, LONG> walk;
     walk.start(A, t0, t1, sm);
     for (long long t = t0; t < t1; ++t) {
         int row;
@@ -422,7 +414,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(MatView A, const double* __
 // K1: v = A p, per-block partial of v.p.  Folds pending set-up or
 // replacement partials into the token first (every block, same order) and
 // decides whether the iteration runs.
-template <typename VT, int FMT, bool HALO>
+template <typename VT, int FMT, bool HALO, bool LONG>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(VT) == 4 ? 5 : 4, 8))) void k_pcg_spmv(MatView A, const VT* __restrict__ p,
                                                      VT* __restrict__ v, double* __restrict__ part,
                                                      const double* __restrict__ rpart, int Gr,
@@ -465,7 +457,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         write_ctrl(cout, c);
         return;
     }
-    __shared__ CsrStage<VT> sm;
+    __shared__ typename CsrStreamOf<VT, LONG>::Stage sm;
     const int lb = logical_block();
     const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
     double acc = 0.0;
@@ -479,7 +471,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         // record and read count 0.  Each loaded value is used once in the
         // step after it, in place: a copy of a register still being loaded
         // would wait for every load issued before it.
-        CsrTileStream<VT> cs;
+        typename CsrStreamOf<VT, LONG>::Stream cs;
         const VT* vals = csr_vals<VT>(A);
         const long long tfirst = group_tile(0, ntiles);
         const auto rrec = tile_rsrc(HALO ? A.hrec : nullptr, HALO ? A.hnq * 16 : 0);
@@ -492,13 +484,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         // summed, and its wavefront's first compact halo index
         int hf = 0, hq = 0;
         if (tfirst >= 0) {  // uniform across the block
-            cs.start(A.n, (int)tfirst, (int)group_tile(1, ntiles), A.xadj, A.cols, vals, sm);
             if constexpr (HALO) {
                 hf = A.hflag[fidx(tfirst)];
                 hq = A.hwq[fidx(tfirst) >> 6];
             }
-            cs.stage(sm);
-            __syncthreads();
+            cs.open(A.n, (int)tfirst, (int)group_tile(1, ntiles), A.xadj, A.cols, vals, sm);
         }
         long long k = 0;
         for (long long t = tfirst; t >= 0; t = group_tile(++k, ntiles)) {
@@ -526,11 +516,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
                                         A.ghost)
                          : sh;
             }
-            __syncthreads();  // the tile's LDS stage is consumed
-            if (nxt >= 0) {
-                cs.stage(sm);
-                __syncthreads();
-            }
+            cs.advance(nxt, sm);
             if (row < A.n) {
                 v[row] = s;
                 double prod = double(s) * double(pr);
@@ -1026,6 +1012,52 @@ static int k1_cap(int G1, bool mixed)
     return G1;
 }
 
+// The K1 of a form, and the grid the FP64 K1s of the CSR and DIA forms
+// share (so that their partials, and the solves, stay bitwise equal).
+template <typename VT>
+using K1Fn = void (*)(MatView, const VT*, VT*, double*, const double*, int, const Ctrl*, Ctrl*, Prm);
+
+template <typename VT>
+static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr)
+{
+    if (fmt == CEL_FMT_JAD) return k_pcg_spmv<VT, CEL_FMT_JAD, false, false>;
+    if constexpr (sizeof(VT) == 8) {  // halo blocks: FP64 only
+        if (halo && fmt == CEL_FMT_DIA) return k_pcg_spmv<VT, CEL_FMT_DIA, true, false>;
+        if (halo) return lr ? k_pcg_spmv<VT, CEL_FMT_CSR, true, true> : k_pcg_spmv<VT, CEL_FMT_CSR, true, false>;
+    }
+    if (fmt == CEL_FMT_DIA) return k_pcg_spmv<VT, CEL_FMT_DIA, false, false>;
+    return lr ? k_pcg_spmv<VT, CEL_FMT_CSR, false, true> : k_pcg_spmv<VT, CEL_FMT_CSR, false, false>;
+}
+
+static int k1_grid_f64(long long ntiles)
+{
+    int g = 1 << 30;
+    for (const bool halo : {false, true}) {
+        for (const bool lr : {false, true})
+            g = std::min(g, resident_grid((const void*)k1_kernel<double>(CEL_FMT_CSR, halo, lr), ntiles));
+        g = std::min(g, resident_grid((const void*)k1_kernel<double>(CEL_FMT_DIA, halo, false), ntiles));
+    }
+    return g;
+}
+
+// The residual kernel of a solve (the set-up, or REPLACE: the mixed form's
+// FP64 replacement) in the CSR or JAD form.
+template <typename OUT_T>
+using ResFn = void (*)(MatView, const double*, const double*, const double*, const float*, OUT_T*,
+                       OUT_T*, float*, double*, const Ctrl*, Ctrl*, Prm);
+
+template <typename OUT_T, bool REPLACE>
+static ResFn<OUT_T> res_kernel(int fmt, bool halo, bool lr)
+{
+    if (fmt == CEL_FMT_JAD) return k_residual<OUT_T, CEL_FMT_JAD, false, REPLACE, false>;
+    if constexpr (sizeof(OUT_T) == 8)
+        if (halo)
+            return lr ? k_residual<OUT_T, CEL_FMT_CSR, true, REPLACE, true>
+                      : k_residual<OUT_T, CEL_FMT_CSR, true, REPLACE, false>;
+    return lr ? k_residual<OUT_T, CEL_FMT_CSR, false, REPLACE, true>
+              : k_residual<OUT_T, CEL_FMT_CSR, false, REPLACE, false>;
+}
+
 // The allocation-free entry point's device memory: a file-scope array
 // (one copy per GPU, resolved to a device address once per device), laid
 // out as r, p, v (kNoAllocMaxRows doubles each), the three partial-sum
@@ -1081,12 +1113,7 @@ int pcg_spmv_dot(Mat& A, int fmt, const double* x, const double* ghost, double* 
     if (dot) *dot = 0.0;
     if (n == 0) return CEL_OK;
     const int ntiles = (n + kTileRows - 1) / kTileRows;
-    const int G1 = k1_cap(common_grid({(const void*)k_pcg_spmv<double, CEL_FMT_CSR, false>,
-                                       (const void*)k_pcg_spmv<double, CEL_FMT_CSR, true>,
-                                       (const void*)k_pcg_spmv<double, CEL_FMT_DIA, false>,
-                                       (const void*)k_pcg_spmv<double, CEL_FMT_DIA, true>},
-                                      ntiles),
-                          false);
+    const int G1 = k1_cap(k1_grid_f64(ntiles), false);
     Workspace& W = ws_of(A);
     CEL_TRY(W.part1.reserve((size_t)G1));
     CEL_TRY(W.ctrl.reserve(5));
@@ -1132,18 +1159,8 @@ int pcg_spmv_dot(Mat& A, int fmt, const double* x, const double* ghost, double* 
                                W.ctrl.p);
     }
     const Prm P{};
-    if (fmt == CEL_FMT_CSR && halo)
-        hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_CSR, true>), dim3(G1), dim3(kBlock), 0, s, V, x, y,
-                           W.part1.p, nullptr, 0, W.ctrl.p, W.ctrl.p + 1, P);
-    else if (fmt == CEL_FMT_CSR)
-        hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_CSR, false>), dim3(G1), dim3(kBlock), 0, s, V, x, y,
-                           W.part1.p, nullptr, 0, W.ctrl.p, W.ctrl.p + 1, P);
-    else if (halo)
-        hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_DIA, true>), dim3(G1), dim3(kBlock), 0, s, V, x, y,
-                           W.part1.p, nullptr, 0, W.ctrl.p, W.ctrl.p + 1, P);
-    else
-        hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_DIA, false>), dim3(G1), dim3(kBlock), 0, s, V, x, y,
-                           W.part1.p, nullptr, 0, W.ctrl.p, W.ctrl.p + 1, P);
+    hipLaunchKernelGGL(k1_kernel<double>(fmt, halo, csr_long_rows(A)), dim3(G1), dim3(kBlock), 0, s, V,
+                       x, y, W.part1.p, nullptr, 0, W.ctrl.p, W.ctrl.p + 1, P);
     CEL_HIP(hipGetLastError());
     std::vector<double> part((size_t)G1);
     CEL_HIP(hipMemcpyAsync(part.data(), W.part1.p, sizeof(double) * G1, hipMemcpyDeviceToHost, s));
@@ -1216,29 +1233,20 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     // the DIA K1 runs on the CSR K1's grid (the same rows per block, so the
     // same partial sums); the residual kernels of a DIA solve use the CSR form
     const int rfmt = fmt == CEL_FMT_DIA ? CEL_FMT_CSR : fmt;
+    const bool lr = csr_long_rows(A);
     if (!mixed) {
-        if (fmt == CEL_FMT_DIA || fmt == CEL_FMT_CSR) {
-            G1 = common_grid({(const void*)k_pcg_spmv<double, CEL_FMT_CSR, false>,
-                              (const void*)k_pcg_spmv<double, CEL_FMT_CSR, true>,
-                              (const void*)k_pcg_spmv<double, CEL_FMT_DIA, false>,
-                              (const void*)k_pcg_spmv<double, CEL_FMT_DIA, true>}, ntiles);
-            Gr = common_grid({(const void*)k_residual<double, CEL_FMT_CSR, false, false>,
-                              (const void*)k_residual<double, CEL_FMT_CSR, true, false>}, ntiles);
-        } else {
-            G1 = common_grid({(const void*)k_pcg_spmv<double, CEL_FMT_JAD, false>}, ntiles);
-            Gr = common_grid({(const void*)k_residual<double, CEL_FMT_JAD, false, false>}, ntiles);
-        }
+        if (fmt == CEL_FMT_JAD) G1 = resident_grid((const void*)k1_kernel<double>(fmt, false, false), ntiles);
+        else G1 = k1_grid_f64(ntiles);
+        Gr = common_grid({(const void*)res_kernel<double, false>(rfmt, false, lr),
+                          (const void*)res_kernel<double, false>(rfmt, rfmt == CEL_FMT_CSR, lr)}, ntiles);
     } else {
-        if (fmt == CEL_FMT_DIA || fmt == CEL_FMT_CSR) {
-            G1 = common_grid({(const void*)k_pcg_spmv<float, CEL_FMT_CSR, false>,
-                              (const void*)k_pcg_spmv<float, CEL_FMT_DIA, false>}, ntiles);
-            Gr = common_grid({(const void*)k_residual<float, CEL_FMT_CSR, false, false>,
-                              (const void*)k_residual<float, CEL_FMT_CSR, false, true>}, ntiles);
-        } else {
-            G1 = common_grid({(const void*)k_pcg_spmv<float, CEL_FMT_JAD, false>}, ntiles);
-            Gr = common_grid({(const void*)k_residual<float, CEL_FMT_JAD, false, false>,
-                              (const void*)k_residual<float, CEL_FMT_JAD, false, true>}, ntiles);
-        }
+        G1 = fmt == CEL_FMT_JAD
+                 ? resident_grid((const void*)k1_kernel<float>(fmt, false, false), ntiles)
+                 : common_grid({(const void*)k1_kernel<float>(CEL_FMT_CSR, false, false),
+                                (const void*)k1_kernel<float>(CEL_FMT_CSR, false, true),
+                                (const void*)k1_kernel<float>(CEL_FMT_DIA, false, false)}, ntiles);
+        Gr = common_grid({(const void*)res_kernel<float, false>(rfmt, false, lr),
+                          (const void*)res_kernel<float, true>(rfmt, false, lr)}, ntiles);
     }
     G1 = k1_cap(G1, mixed);
     {
@@ -1442,27 +1450,12 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
 
     // r0, p0 and their partials; the first K1 folds them in.  The set-up
     // reads and writes token slot 0 (only block 0 writes, after its read).
-#define RES_ARGS(OT, R, P_)                                                                \
-    V, dx, db, jac64, jac32, (OT*)(R), (OT*)(P_), w.e32, w.rpart, C0, C0, P
-    if (!mixed) {
-        if (rfmt == CEL_FMT_CSR && halo)
-            hipLaunchKernelGGL((k_residual<double, CEL_FMT_CSR, true, false>), dim3(Gr), dim3(kBlock), 0, s,
-                               RES_ARGS(double, w.r, w.p));
-        else if (rfmt == CEL_FMT_CSR)
-            hipLaunchKernelGGL((k_residual<double, CEL_FMT_CSR, false, false>), dim3(Gr), dim3(kBlock), 0,
-                               s, RES_ARGS(double, w.r, w.p));
-        else
-            hipLaunchKernelGGL((k_residual<double, CEL_FMT_JAD, false, false>), dim3(Gr), dim3(kBlock), 0,
-                               s, RES_ARGS(double, w.r, w.p));
-    } else {
-        if (rfmt == CEL_FMT_CSR)
-            hipLaunchKernelGGL((k_residual<float, CEL_FMT_CSR, false, false>), dim3(Gr), dim3(kBlock), 0, s,
-                               RES_ARGS(float, w.r32, w.p32));
-        else
-            hipLaunchKernelGGL((k_residual<float, CEL_FMT_JAD, false, false>), dim3(Gr), dim3(kBlock), 0, s,
-                               RES_ARGS(float, w.r32, w.p32));
-    }
-#undef RES_ARGS
+    if (!mixed)
+        hipLaunchKernelGGL((res_kernel<double, false>(rfmt, halo, lr)), dim3(Gr), dim3(kBlock), 0, s, V, dx,
+                           db, jac64, jac32, w.r, w.p, w.e32, w.rpart, C0, C0, P);
+    else
+        hipLaunchKernelGGL((res_kernel<float, false>(rfmt, false, lr)), dim3(Gr), dim3(kBlock), 0, s, V, dx,
+                           db, jac64, jac32, w.r32, w.p32, w.e32, w.rpart, C0, C0, P);
     CEL_HIP(hipGetLastError());
     if (!noalloc) CEL_HIP(hipEventRecord(e1, s));
 
@@ -1496,49 +1489,23 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             CEL_HIP(hipEventRecord(ea, s));
         }
         if (!mixed) {
-            if (halo && fmt == CEL_FMT_DIA)
-                hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_DIA, true>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p, w.v, w.part1, w.rpart, Gr, C0, C1, P);
-            else if (halo)
-                hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_CSR, true>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p, w.v, w.part1, w.rpart, Gr, C0, C1, P);
-            else if (fmt == CEL_FMT_CSR)
-                hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_CSR, false>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p, w.v, w.part1, w.rpart, Gr, C0, C1, P);
-            else if (fmt == CEL_FMT_DIA)
-                hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_DIA, false>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p, w.v, w.part1, w.rpart, Gr, C0, C1, P);
-            else
-                hipLaunchKernelGGL((k_pcg_spmv<double, CEL_FMT_JAD, false>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p, w.v, w.part1, w.rpart, Gr, C0, C1, P);
+            hipLaunchKernelGGL(k1_kernel<double>(fmt, halo, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
+                               w.part1, w.rpart, Gr, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL((k_pcg_update_r<double>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
                                jac64, w.part2, w.part1, G1, C1, C2);
             hipLaunchKernelGGL((k_pcg_update_xp<double, double, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll,
                                dx, w.p, w.r, jac64, nullptr, w.part2, Gv, C2, C0, P);
         } else {
-            if (fmt == CEL_FMT_CSR)
-                hipLaunchKernelGGL((k_pcg_spmv<float, CEL_FMT_CSR, false>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p32, w.v32, w.part1, w.rpart, Gr, C0, C1, P);
-            else if (fmt == CEL_FMT_DIA)
-                hipLaunchKernelGGL((k_pcg_spmv<float, CEL_FMT_DIA, false>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p32, w.v32, w.part1, w.rpart, Gr, C0, C1, P);
-            else
-                hipLaunchKernelGGL((k_pcg_spmv<float, CEL_FMT_JAD, false>), dim3(G1), dim3(kBlock), 0, s, V,
-                                   w.p32, w.v32, w.part1, w.rpart, Gr, C0, C1, P);
+            hipLaunchKernelGGL(k1_kernel<float>(fmt, false, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
+                               w.part1, w.rpart, Gr, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL((k_pcg_update_r<float>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
                                jac32, w.part2, w.part1, G1, C1, C2);
             hipLaunchKernelGGL((k_pcg_update_xp<float, float, true>), dim3(Gv), dim3(kBlock), 0, s, n_ll,
                                w.e32, w.p32, w.r32, jac32, dx, w.part2, Gv, C2, C3, P);
-            if (rfmt == CEL_FMT_CSR)
-                hipLaunchKernelGGL((k_residual<float, CEL_FMT_CSR, false, true>), dim3(Gr), dim3(kBlock), 0, s,
-                                   V, dx, db, jac64, jac32, w.r32, w.p32, w.e32, w.rpart, C3,
-                                   C0, P);
-            else
-                hipLaunchKernelGGL((k_residual<float, CEL_FMT_JAD, false, true>), dim3(Gr), dim3(kBlock), 0, s,
-                                   V, dx, db, jac64, jac32, w.r32, w.p32, w.e32, w.rpart, C3,
-                                   C0, P);
+            hipLaunchKernelGGL((res_kernel<float, true>(rfmt, false, lr)), dim3(Gr), dim3(kBlock), 0, s, V, dx,
+                               db, jac64, jac32, w.r32, w.p32, w.e32, w.rpart, C3, C0, P);
         }
         CEL_HIP(hipGetLastError());
         return CEL_OK;

@@ -12,7 +12,7 @@ namespace cel {
 // assume, cel_sp_mat_module.f90:430-456), so a row's run of entries is
 // added to y one by one, in entry order, with no atomics: the row sum
 // starts from y(row) itself (INIT) or from 0 when y is overwritten.
-template <typename VT, bool INIT>
+template <typename VT, bool INIT, bool LONG>
 __global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int* __restrict__ xadj,
                                                      const int* __restrict__ cols,
                                                      const VT* __restrict__ vals,
@@ -21,14 +21,11 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int* __restric
                                                      const int* __restrict__ skip)
 {
     if (skip && *skip) return;  // uniform across the grid
-    __shared__ CsrStage<VT> sm;
-    CsrTileStream<VT> ts;
+    __shared__ typename CsrStreamOf<VT, LONG>::Stage sm;
+    typename CsrStreamOf<VT, LONG>::Stream ts;
     const int tfirst = (int)group_tile(0, ntiles);
-    if (tfirst >= 0) {  // uniform across the block
-        ts.start(n, tfirst, (int)group_tile(1, ntiles), xadj, cols, vals, sm);
-        ts.stage(sm);
-        __syncthreads();
-    }
+    if (tfirst >= 0)  // uniform across the block
+        ts.open(n, tfirst, (int)group_tile(1, ntiles), xadj, cols, vals, sm);
     int step = 0;
     for (int t = tfirst; t >= 0; t = (int)group_tile(++step, ntiles)) {
         const int row = t * kTileRows + threadIdx.x;
@@ -37,11 +34,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int* __restric
         VT init = VT(0);
         if constexpr (INIT) init = y[row < n ? row : 0];
         VT s = ts.template rows<VT>(n, t, nxt, aft, xadj, cols, vals, x, sm, row, nullptr, init);
-        __syncthreads();
-        if (nxt >= 0) {
-            ts.stage(sm);
-            __syncthreads();
-        }
+        ts.advance(nxt, sm);
         if (row < n) y[row] = coo ? s : accumulate ? y[row] + s : VT(0) + s;
     }
 }
@@ -50,7 +43,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int* __restric
 // cel_internal.hpp): block b walks the 256-row tiles of its row chunk
 // [b*chunk, b*chunk + chunk) with the same tile stream as k_csr_spmv (same
 // row sums), each thread its rows in ascending order.
-template <int FUSE>
+template <int FUSE, bool LONG>
 __global__ __launch_bounds__(kBlock) void k_csr_spmv_fused(int n, long long chunk,
                                                            const int* __restrict__ xadj,
                                                            const int* __restrict__ cols,
@@ -62,29 +55,22 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv_fused(int n, long long chun
                                                            const int* __restrict__ skip)
 {
     if (skip && *skip) return;  // uniform across the grid
-    __shared__ CsrStage<double> sm;
+    __shared__ typename CsrStreamOf<double, LONG>::Stage sm;
     __shared__ double red[kWaves];
     const long long c0 = (long long)blockIdx.x * chunk;
     const long long c1 = c0 + chunk < n ? c0 + chunk : n;
     const int t0 = (int)(c0 / kTileRows);  // chunk is a multiple of the tile
     const int t1 = c0 < c1 ? (int)((c1 + kTileRows - 1) / kTileRows) : t0;
-    CsrTileStream<double> ts;
-    if (t0 < t1) {  // uniform across the block
-        ts.start(n, t0, t0 + 1 < t1 ? t0 + 1 : -1, xadj, cols, vals, sm);
-        ts.stage(sm);
-        __syncthreads();
-    }
+    typename CsrStreamOf<double, LONG>::Stream ts;
+    if (t0 < t1)  // uniform across the block
+        ts.open(n, t0, t0 + 1 < t1 ? t0 + 1 : -1, xadj, cols, vals, sm);
     double acc = 0.0;
     for (int t = t0; t < t1; ++t) {
         const int row = t * kTileRows + threadIdx.x;
         const int nxt = t + 1 < t1 ? t + 1 : -1;
         const int aft = t + 2 < t1 ? t + 2 : -1;
         double s = ts.template rows<double>(n, t, nxt, aft, xadj, cols, vals, x, sm, row, nullptr);
-        __syncthreads();
-        if (nxt >= 0) {
-            ts.stage(sm);
-            __syncthreads();
-        }
+        ts.advance(nxt, sm);
         if (row < n) acc = acc + fuse_row<FUSE>(0.0 + s, row, aux, y);
     }
     const double bs = block_sum(acc, red);
@@ -124,22 +110,28 @@ static int spmv_no_columns(const Mat& A, T* y, int accumulate)
     return CEL_OK;
 }
 
+template <typename VT, bool INIT, bool LONG>
+static int launch_csr_tiles_of(const Mat& A, const VT* vals, const VT* x, VT* y, int accumulate,
+                               int coo, const int* skip)
+{
+    const int ntiles = (A.n + kTileRows - 1) / kTileRows;
+    const int G = resident_grid((const void*)k_csr_spmv<VT, INIT, LONG>, ntiles);
+    hipLaunchKernelGGL((k_csr_spmv<VT, INIT, LONG>), dim3(G), dim3(kBlock), 0, rt().stream, A.n,
+                       A.xadj.p, A.cols.p, vals, x, y, accumulate, coo, ntiles, skip);
+    CEL_HIP(hipGetLastError());
+    return CEL_OK;
+}
+
 template <typename VT>
 static int launch_csr_tiles(const Mat& A, const VT* vals, const VT* x, VT* y, int accumulate,
                             int coo, const int* skip)
 {
-    const int ntiles = (A.n + kTileRows - 1) / kTileRows;
-    if (coo && accumulate) {
-        const int G = resident_grid((const void*)k_csr_spmv<VT, true>, ntiles);
-        hipLaunchKernelGGL((k_csr_spmv<VT, true>), dim3(G), dim3(kBlock), 0, rt().stream, A.n,
-                           A.xadj.p, A.cols.p, vals, x, y, accumulate, coo, ntiles, skip);
-    } else {
-        const int G = resident_grid((const void*)k_csr_spmv<VT, false>, ntiles);
-        hipLaunchKernelGGL((k_csr_spmv<VT, false>), dim3(G), dim3(kBlock), 0, rt().stream, A.n,
-                           A.xadj.p, A.cols.p, vals, x, y, accumulate, coo, ntiles, skip);
-    }
-    CEL_HIP(hipGetLastError());
-    return CEL_OK;
+    const bool init = coo && accumulate;
+    if (csr_long_rows(A))
+        return init ? launch_csr_tiles_of<VT, true, true>(A, vals, x, y, accumulate, coo, skip)
+                    : launch_csr_tiles_of<VT, false, true>(A, vals, x, y, accumulate, coo, skip);
+    return init ? launch_csr_tiles_of<VT, true, false>(A, vals, x, y, accumulate, coo, skip)
+                : launch_csr_tiles_of<VT, false, false>(A, vals, x, y, accumulate, coo, skip);
 }
 
 int launch_csr_spmv(const Mat& A, const double* x, double* y, int accumulate, const int* skip,
@@ -157,14 +149,16 @@ int launch_csr_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const 
         return fail(CEL_ERR_ARG, "fused product: a square block with rows");
     if (chunk <= 0 || chunk % kTileRows != 0 || (long long)G * chunk < A.n)
         return fail(CEL_ERR_ARG, "fused product: chunks must be whole tiles covering every row");
-    if (fuse == kFuseDot)
-        hipLaunchKernelGGL(k_csr_spmv_fused<kFuseDot>, dim3(G), dim3(kBlock), 0, rt().stream, A.n,
-                           chunk, A.xadj.p, A.cols.p, A.vals.p, x, y, aux, part, skip);
+    void (*k)(int, long long, const int*, const int*, const double*, const double*, double*,
+              const double*, double*, const int*);
+    const bool lr = csr_long_rows(A);
+    if (fuse == kFuseDot) k = lr ? k_csr_spmv_fused<kFuseDot, true> : k_csr_spmv_fused<kFuseDot, false>;
     else if (fuse == kFuseResid)
-        hipLaunchKernelGGL(k_csr_spmv_fused<kFuseResid>, dim3(G), dim3(kBlock), 0, rt().stream, A.n,
-                           chunk, A.xadj.p, A.cols.p, A.vals.p, x, y, aux, part, skip);
+        k = lr ? k_csr_spmv_fused<kFuseResid, true> : k_csr_spmv_fused<kFuseResid, false>;
     else
         return fail(CEL_ERR_ARG, "fused product: unknown epilogue");
+    hipLaunchKernelGGL(k, dim3(G), dim3(kBlock), 0, rt().stream, A.n, chunk, A.xadj.p, A.cols.p,
+                       A.vals.p, x, y, aux, part, skip);
     CEL_HIP(hipGetLastError());
     return CEL_OK;
 }
