@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
             const int aft = t + 2 < t1 ? t + 2 : -1;
             const int row = t * kTileRows + threadIdx.x;
             double pr = 0.0;
-            double sum = cs.template rows<double>(S.n, t, nxt, aft, S.xadj, S.cols, S.vals, ps, sm,
+            double sum = cs.template rows<double>(S.n, t, nxt, aft, S.xadj, S.cols, S.vals, XPlain<double>{ps}, sm,
                                                   row, &pr);
             __syncthreads();
             if (nxt >= 0) {

@@ -96,7 +96,7 @@ k_dia_spmv(int n, Offsets O, const VT* __restrict__ dv, const uint32_t* __restri
         for (int k = 0; k < R; ++k) r[k] = (int)(T * R * kBlock) + threadIdx.x + k * kBlock;
         if (r[0] >= n) continue;
         VT s[R];
-        dia_rows<VT, R, GD>(n, O.nd, O.off, dv, mask8, mask, r, x, s);
+        dia_rows<VT, R, GD>(n, O.nd, O.off, dv, mask8, mask, r, XPlain<VT>{x}, s);
 #pragma unroll
         for (int k = 0; k < R; ++k)
             if (r[k] < n) y[r[k]] = accumulate ? y[r[k]] + s[k] : s[k];
@@ -158,7 +158,7 @@ k_dia_spmv_fused(int n, long long chunk, Offsets O, const double* __restrict__ d
         }
         if (r[0] >= n) continue;  // no barrier in this loop
         double s[R];
-        dia_rows<double, R, GD>(n, O.nd, O.off, dv, mask8, mask, r, x, s);
+        dia_rows<double, R, GD>(n, O.nd, O.off, dv, mask8, mask, r, XPlain<double>{x}, s);
 #pragma unroll
         for (int k = 0; k < R; ++k)
             if (r[k] < n) acc = acc + fuse_row<FUSE>(s[k], r[k], aux, y);

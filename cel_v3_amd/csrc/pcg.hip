@@ -301,7 +301,7 @@ struct TileWalk {
             const int nxt = (t + 1 < t1) ? (int)(t + 1) : -1;
             const int aft = (t + 2 < t1) ? (int)(t + 2) : -1;
             row = r0 + threadIdx.x;
-            s = cs.template rows<AT>(A.n, (int)t, nxt, aft, A.xadj, A.cols, csr_vals<VT>(A), x, sm,
+            s = cs.template rows<AT>(A.n, (int)t, nxt, aft, A.xadj, A.cols, csr_vals<VT>(A), XPlain<VT>{x}, sm,
                                      row, xrow);
             cs.advance(nxt, sm);
             // CSR: r = 0; r = r + tmp.  COO: the entries were added to 0 one
@@ -330,63 +330,58 @@ struct TileWalk {
     }
 };
 
-// ------------------------------------------------------------------ residual kernels
+// ------------------------------------------------------------------ residual
 // r = b - A x with the FP64 operator; per-block partials: r.z, r.r, b.b.
 // FP64 form: r and p = z = jac*r stored in FP64.  Mixed form (OUT_T =
 // float): r rounded to FP32, z = jac32 * r32 (p = z at the start or on a
 // restart), e = 0 at the start, the norm taken in FP64 before rounding.
 // The next K1 folds the partials into the token.
+template <typename OUT_T>
+struct ResArgs {
+    const double *x, *b, *jac;
+    const float* jac32;
+    OUT_T *r, *p;
+    float* e;
+    double* part;
+    int G;  // blocks of the partials
+};
+
+// Block lb of a.G: its contiguous tiles and its partials.
 template <typename OUT_T, int FMT, bool HALO, bool REPLACE, bool LONG>
-__global__ __launch_bounds__(kBlock) void k_residual(MatView A, const double* __restrict__ x,
-                                                     const double* __restrict__ b,
-                                                     const double* __restrict__ jac,
-                                                     const float* __restrict__ jac32,
-                                                     OUT_T* __restrict__ r, OUT_T* __restrict__ p,
-                                                     float* __restrict__ e,
-                                                     double* __restrict__ part,
-                                                     const Ctrl* __restrict__ cin,
-                                                     Ctrl* __restrict__ cout, Prm P)
+__device__ __forceinline__ void residual_block(const MatView& A, const ResArgs<OUT_T>& a, int lb,
+                                               bool restart,
+                                               typename CsrStreamOf<double, LONG>::Stage& sm,
+                                               double* red /* 3*kWaves */)
 {
-    Ctrl c = read_ctrl(cin);
-    if (REPLACE) {
-        if (!c.run || !c.ru) {
-            write_ctrl(cout, c);
-            return;
-        }
-    }
-    __shared__ typename CsrStreamOf<double, LONG>::Stage sm;
-    __shared__ double red[3 * kWaves];
-    const int lb = logical_block();
-    const int G = gridDim.x;
+    const int G = a.G;
     const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
     long long t0, t1;
     unit_range(ntiles, G, lb, t0, t1);
-    const bool restart = REPLACE && P.ru_restart;
     double arz = 0.0, arr = 0.0, abb = 0.0;
     TileWalk<double, double, FMT, HALO, LONG> walk;
     walk.start(A, t0, t1, sm);
     for (long long t = t0; t < t1; ++t) {
         int row;
-        double s = walk.next(A, t, t1, x, sm, row, nullptr);
+        double s = walk.next(A, t, t1, a.x, sm, row, nullptr);
         if (row < A.n) {
-            const double bi = b[row];
+            const double bi = a.b[row];
             const double ri = bi - s;  // r = 0; r = r + A x; r = b - r
             double bb = bi * bi;  // a non-finite b makes this sum non-finite
             abb = abb + bb;
             double rr = ri * ri;
             arr = arr + rr;
             if constexpr (sizeof(OUT_T) == 8) {
-                const double zi = ri * jac[row];
-                r[row] = ri;
-                p[row] = zi;
+                const double zi = ri * a.jac[row];
+                a.r[row] = ri;
+                a.p[row] = zi;
                 double rz = ri * zi;
                 arz = arz + rz;
             } else {
                 const float rf = (float)ri;
-                const float zf = rf * jac32[row];
-                r[row] = rf;
-                if (!REPLACE || restart) p[row] = zf;
-                if (!REPLACE) e[row] = 0.0f;
+                const float zf = rf * a.jac32[row];
+                a.r[row] = rf;
+                if (!REPLACE || restart) a.p[row] = zf;
+                if (!REPLACE) a.e[row] = 0.0f;
                 double rz = (double)rf * (double)zf;
                 arz = arz + rz;
             }
@@ -395,13 +390,46 @@ __global__ __launch_bounds__(kBlock) void k_residual(MatView A, const double* __
     block_sum2(arz, arr, red);
     const double sbb = block_sum(abb, red + 2 * kWaves);
     if (threadIdx.x == 0) {
-        part[lb] = arz;
-        part[G + lb] = arr;
-        part[2 * G + lb] = sbb;
+        a.part[lb] = arz;
+        a.part[G + lb] = arr;
+        a.part[2 * G + lb] = sbb;
     }
-    c.reduce = REPLACE ? kReduceReplace : kReduceSetup;
+}
+
+// Set-up of a solve: r0, p0, partials.
+template <typename OUT_T, int FMT, bool HALO, bool LONG>
+__global__ __launch_bounds__(kBlock) void k_residual(MatView A, ResArgs<OUT_T> a,
+                                                     const Ctrl* __restrict__ cin,
+                                                     Ctrl* __restrict__ cout)
+{
+    Ctrl c = read_ctrl(cin);
+    __shared__ typename CsrStreamOf<double, LONG>::Stage sm;
+    __shared__ double red[3 * kWaves];
+    residual_block<OUT_T, FMT, HALO, false, LONG>(A, a, logical_block(), false, sm, red);
+    c.reduce = kReduceSetup;
     c.ru = 0;
     write_ctrl(cout, c);
+}
+
+// Mixed form, requested replacement (token's ru): the FP64 residual in place
+// of the product of a K1 launch.  The K1's blocks share the a.G blocks of
+// the partials (the set-up's grid, so the sums are grouped alike).  A
+// launch of its own per iteration, almost always with nothing to do, cost
+// 1 us at 32^3 (mixed 15.2 against 14.4 us per iteration) to 7 us on larger
+// grids (600k-row mesh solve 9.13 against 8.80 ms).
+template <int FMT, bool LONG>
+__device__ __forceinline__ void replace_residual(const MatView& A, const ResArgs<float>& a, Ctrl& c,
+                                                 const Prm& P,
+                                                 typename CsrStreamOf<double, LONG>::Stage& sm,
+                                                 double* red)
+{
+    for (int vb = blockIdx.x; vb < a.G; vb += gridDim.x) {
+        const int lb = a.G % kXcds ? vb : (vb % kXcds) * (a.G / kXcds) + vb / kXcds;
+        residual_block<float, FMT, false, true, LONG>(A, a, lb, P.ru_restart, sm, red);
+        __syncthreads();  // the stage is free again
+    }
+    c.reduce = kReduceReplace;
+    c.ru = 0;
 }
 
 // The CSR, DIA and JAD K1s walk their tiles in group_tile's order
@@ -411,56 +439,104 @@ __global__ __launch_bounds__(kBlock) void k_residual(MatView A, const double* __
 // tiles, and its solves agree with the others to rounding.  (Groups of 4
 // tiles measured: FP64 DIA solve 1% faster, mixed DIA 1% slower.)
 
-// K1: v = A p, per-block partial of v.p.  Folds pending set-up or
-// replacement partials into the token first (every block, same order) and
-// decides whether the iteration runs.
-template <typename VT, int FMT, bool HALO, bool LONG>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(VT) == 4 ? 5 : 4, 8))) void k_pcg_spmv(MatView A, const VT* __restrict__ p,
-                                                     VT* __restrict__ v, double* __restrict__ part,
-                                                     const double* __restrict__ rpart, int Gr,
-                                                     const Ctrl* __restrict__ cin,
-                                                     Ctrl* __restrict__ cout, Prm P)
+// Folds pending set-up or replacement partials into the token (every block,
+// same order) and decides whether the iteration runs.
+__device__ __forceinline__ void fold_pending(Ctrl& c, const double* __restrict__ rpart, int Gr,
+                                             const Prm& P, double* red, double* bcast)
 {
-    __shared__ double red[kWaves];
-    __shared__ double bcast;
-    Ctrl c = read_ctrl(cin);
-    if (c.reduce != kReduceNone) {
-        const double rz = all_sum(rpart, Gr, red, &bcast);
-        const double rr = all_sum(rpart + Gr, Gr, red, &bcast);
-        const double rn = sqrt(rr);
-        if (c.reduce == kReduceSetup) {
-            const double bb = all_sum(rpart + 2 * Gr, Gr, red, &bcast);
-            c.bnorm = sqrt(bb);
-            c.norm0 = rn;
-            c.eps = eps_from(P, c.bnorm, rn);
-            c.iter = 0;
-            c.outer = 0;
-            if (!isfinite(bb) && c.status == 0) c.status = CEL_ERR_NONFINITE;
-            if (blockIdx.x == 0 && threadIdx.x == 0 && P.hist_cap > 0) P.hist[0] = rn;
-        } else {
-            c.outer = c.outer + 1;
-            // attainable accuracy: two cycles in a row that fail to halve the
-            // FP64 residual end the solve (not converged)
-            c.stall = (rn > 0.5 * c.rnorm_ref) ? c.stall + 1 : 0;
-        }
-        c.since = 0;
-        c.alpha = rz;
-        c.norm2 = rn;
-        c.rnorm_ref = rn;
-        c.reduce = kReduceNone;
-        c.run = (c.status == 0 && c.iter < P.iter_max && alpha_ok(P, c.alpha) &&
-                 c.norm2 > c.eps && c.stall < 2)
-                    ? 1
-                    : 0;
+    const double rz = all_sum(rpart, Gr, red, bcast);
+    const double rr = all_sum(rpart + Gr, Gr, red, bcast);
+    const double rn = sqrt(rr);
+    if (c.reduce == kReduceSetup) {
+        const double bb = all_sum(rpart + 2 * Gr, Gr, red, bcast);
+        c.bnorm = sqrt(bb);
+        c.norm0 = rn;
+        c.eps = eps_from(P, c.bnorm, rn);
+        c.iter = 0;
+        c.outer = 0;
+        if (!isfinite(bb) && c.status == 0) c.status = CEL_ERR_NONFINITE;
+        if (blockIdx.x == 0 && threadIdx.x == 0 && P.hist_cap > 0) P.hist[0] = rn;
+    } else {
+        c.outer = c.outer + 1;
+        // attainable accuracy: two cycles in a row that fail to halve the
+        // FP64 residual end the solve (not converged)
+        c.stall = (rn > 0.5 * c.rnorm_ref) ? c.stall + 1 : 0;
     }
-    if (!c.run) {
-        write_ctrl(cout, c);
-        return;
+    c.since = 0;
+    c.alpha = rz;
+    c.norm2 = rn;
+    c.rnorm_ref = rn;
+    c.reduce = kReduceNone;
+    c.run = (c.status == 0 && c.iter < P.iter_max && alpha_ok(P, c.alpha) &&
+             c.norm2 > c.eps && c.stall < 2)
+                ? 1
+                : 0;
+}
+
+// The scalars after r.z and r.r of an iteration: beta, alpha = r.z, norm2,
+// k++, history, loop decision (FP64) or replacement request (mixed).
+template <bool MIXED>
+__device__ __forceinline__ void next_scalars(Ctrl& c, double rz, double rr, const Prm& P)
+{
+    c.beta = rz / c.alpha;
+    c.alpha = rz;
+    c.norm2 = sqrt(rr);
+    c.iter = c.iter + 1;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && c.iter < P.hist_cap) P.hist[c.iter] = c.norm2;
+    if (!MIXED) {
+        c.run = (c.iter < P.iter_max && alpha_ok(P, c.alpha) && c.norm2 > c.eps) ? 1 : 0;
+    } else {
+        // replace the FP32 residual by the FP64 one when it has dropped by
+        // ru_delta since the last replacement, looks converged, the budget
+        // is spent, or the FP32 recurrence has stopped tracking the FP64
+        // residual (grown past it, or a cycle far longer than expected);
+        // the stop decision is taken on the FP64 norm
+        c.since = c.since + 1;
+        const bool drop = c.norm2 < P.ru_delta * c.rnorm_ref;
+        const bool astray = c.norm2 > 2.0 * c.rnorm_ref || c.since >= P.ru_max_inner;
+        c.ru = (drop || astray || c.norm2 <= c.eps || c.iter >= P.iter_max ||
+                !alpha_ok(P, c.alpha) || !isfinite(c.norm2))
+                   ? 1
+                   : 0;
     }
-    __shared__ typename CsrStreamOf<VT, LONG>::Stage sm;
-    const int lb = logical_block();
+}
+
+// What the tile walk of a K1 does with the rows besides the product: nothing,
+// or (k_pcg_step) p_new and x += sigma p of the thread's rows.
+template <typename VT>
+struct StepRows {
+    VT* pout;
+    VT* x;
+    VT sigma;
+    bool upd;  // x is updated (uniform; false right after a set-up or replacement)
+};
+
+// v = A d over the block's tiles, d the vector of the accessor X; returns the
+// thread's part of v.d.  STEP: X is XDirection, and d and the updated x of
+// every row are stored as well.  (Taking a step's scalars behind the first
+// tile's gathers instead of before them measured slower, 32^3 12.7 against
+// 12.3 us per iteration.)
+template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, typename X>
+__device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __restrict__ v,
+                                           typename CsrStreamOf<VT, LONG>::Stage& sm,
+                                           const StepRows<VT>& st)
+{
     const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
     double acc = 0.0;
+    // one finished row: its value, and in a step its direction and x
+    auto finish = [&](int row, VT s, const typename X::Raw& raw, VT xo) {
+        const VT d = x.value(raw);
+        v[row] = s;
+        if constexpr (STEP) {
+            st.pout[row] = d;
+            if (st.upd) {
+                const VT t = st.sigma * raw.p;
+                st.x[row] = xo + t;
+            }
+        }
+        double prod = double(s) * double(d);
+        acc = acc + prod;
+    };
     if constexpr (FMT == CEL_FMT_CSR) {
         // halo rows (HALO): a row's halo record (count and products, in
         // block order) is added after its local sum.  Its flag loads one
@@ -495,10 +571,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
             const int nxt = (int)group_tile(k + 1, ntiles);
             const int aft = (int)group_tile(k + 2, ntiles);
             const int row = (int)t * kTileRows + threadIdx.x;
-            VT pr = VT(0);
+            typename X::Raw pr{};
+            VT xo = VT(0);
             HaloRec hw{};
             int hc = 0;
             auto recs = [&]() {
+                if constexpr (STEP) xo = st.x[row < A.n ? row : 0];
                 if constexpr (HALO) {
                     hc = hf;
                     hw = halo_rec_load(rrec, hq, hc);
@@ -506,7 +584,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
                     hq = A.hwq[fidx(nxt) >> 6];
                 }
             };
-            VT s = cs.template rows<VT>(A.n, (int)t, nxt, aft, A.xadj, A.cols, vals, p, sm, row,
+            VT s = cs.template rows<VT>(A.n, (int)t, nxt, aft, A.xadj, A.cols, vals, x, sm, row,
                                         &pr, VT(0), recs);
             s = A.coo ? s : VT(0) + s;
             if constexpr (HALO) {
@@ -517,11 +595,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
                          : sh;
             }
             cs.advance(nxt, sm);
-            if (row < A.n) {
-                v[row] = s;
-                double prod = double(s) * double(pr);
-                acc = acc + prod;
-            }
+            if (row < A.n) finish(row, s, pr, xo);
         }
     } else if constexpr (FMT == CEL_FMT_DIA) {
         // all tiles of a group per step, one row of each per thread; the
@@ -573,14 +647,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
                 r[k] = t < ntiles ? (int)t * kTileRows + threadIdx.x : A.n;
             }
             if (r[0] < A.n) {
-                VT s[R], pr[R];
-                // p[row] comes from the loads of the diagonal with offset 0
+                VT s[R], xo[R];
+                typename X::Raw pr[R];
+                if constexpr (STEP) {
+#pragma unroll
+                    for (int k = 0; k < R; ++k) xo[k] = st.x[r[k] < A.n ? r[k] : r[0]];
+                }
+                // x[row] comes from the loads of the diagonal with offset 0
                 dia_rows<VT, R, (R >= 4 ? 4 : 8)>(A.n, A.nd, A.doff, dia_vals<VT>(A), A.dmask8,
-                                                   A.dmask, r, p, s, pr, A.dzero);
+                                                   A.dmask, r, x, s, pr, A.dzero);
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
                     if (r[k] < A.n) {
-                        const VT pk = A.dzero >= 0 ? pr[k] : p[r[k]];
+                        const typename X::Raw pk = A.dzero >= 0 ? pr[k] : x.load(r[k]);
                         VT sk = VT(0) + s[k];
                         if constexpr (HALO) {
                             bool over = false;
@@ -595,9 +674,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
                                 sk = s0;
                             }
                         }
-                        v[r[k]] = sk;
-                        double prod = double(sk) * double(pk);
-                        acc = acc + prod;
+                        finish(r[k], sk, pk, STEP ? xo[k] : VT(0));
                     }
                 }
             }
@@ -610,8 +687,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         // JAD in the permuted row order: the CSR K1's tile-pair order, one
         // row per thread and tile, the next tile's row loaded while this
         // one's gathers are in flight
-        JadStream<VT> js;
-        js.init(A.n, A.mmax, A.jnnz, A.jbegin, A.jcols, jad_vals<VT>(A), p);
+        JadStream<VT, X> js;
+        js.init(A.n, A.mmax, A.jnnz, A.jbegin, A.jcols, jad_vals<VT>(A), x);
         long long k = 0;
         long long t = group_tile(0, ntiles);
         if (t >= 0) js.fetch((int)t * kTileRows + threadIdx.x);
@@ -619,18 +696,129 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
             const long long tn = group_tile(k + 1, ntiles);
             const int row = (int)t * kTileRows + threadIdx.x;
             const int rn = tn >= 0 ? (int)tn * kTileRows + threadIdx.x : A.n;
-            VT pr;
-            VT s = js.template row<VT>(row, rn, A.mmax, A.jbegin, A.jcols, jad_vals<VT>(A), p, pr);
-            if (row < A.n) {
-                // the reference's JAD product overwrites v (y(perm(k)) = tmp(k))
-                v[row] = s;
-                double prod = double(s) * double(pr);
-                acc = acc + prod;
-            }
+            typename X::Raw pr;
+            VT xo = VT(0);
+            if constexpr (STEP) xo = st.x[row < A.n ? row : 0];
+            VT s = js.template row<VT>(row, rn, A.mmax, A.jbegin, A.jcols, jad_vals<VT>(A), x, pr);
+            // the reference's JAD product overwrites v (y(perm(k)) = tmp(k))
+            if (row < A.n) finish(row, s, pr, xo);
         }
     }
+    return acc;
+}
+
+// LDS of a K1: its tile stage; in the mixed form the FP64 stage of a
+// replacement residual takes the same place.
+template <typename VT, bool LONG>
+union K1Stage {
+    typename CsrStreamOf<VT, LONG>::Stage tile;
+    typename CsrStreamOf<double, LONG>::Stage res;
+};
+
+// K1: v = A p, per-block partial of v.p.  Mixed: a requested replacement
+// residual takes the place of the product (K2 and K3 then do nothing, and
+// the next K1 folds its partials).  LONG of a DIA K1: its residual's.
+template <typename VT, int FMT, bool HALO, bool LONG>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pcg_spmv(MatView A, const VT* __restrict__ p,
+                                                     VT* __restrict__ v, double* __restrict__ part,
+                                                     ResArgs<VT> R,
+                                                     const Ctrl* __restrict__ cin,
+                                                     Ctrl* __restrict__ cout, Prm P)
+{
+    constexpr bool MIXED = sizeof(VT) == 4;
+    __shared__ K1Stage<VT, LONG> sm;
+    __shared__ double red[3 * kWaves];
+    __shared__ double bcast;
+    Ctrl c = read_ctrl(cin);
+    if (c.reduce != kReduceNone) fold_pending(c, R.part, R.G, P, red, &bcast);
+    if (!c.run) {
+        write_ctrl(cout, c);
+        return;
+    }
+    if constexpr (MIXED) {
+        if (c.ru) {  // uniform
+            replace_residual<FMT == CEL_FMT_DIA ? CEL_FMT_CSR : FMT, LONG>(A, R, c, P, sm.res, red);
+            write_ctrl(cout, c);
+            return;
+        }
+    }
+    const double acc = k1_tiles<VT, FMT, HALO, LONG, false>(A, XPlain<VT>{p}, v, sm.tile, StepRows<VT>{});
     const double bs = block_sum(acc, red);
-    if (threadIdx.x == 0) part[lb] = bs;
+    if (threadIdx.x == 0) part[logical_block()] = bs;
+    write_ctrl(cout, c);
+}
+
+// K3 and the next iteration's K1 in one launch, for small systems (rule at
+// step_rows): beta and the loop decision from K2's partials, x += sigma p,
+// p_new = beta p + z, v = A p_new and the partials of v.p_new.  A block
+// needs p_new of its neighbours' rows as well, so every gather reads p and
+// z and forms p_new itself (the same roundings as K3), and p_new goes to a
+// second buffer.  The rows, blocks and orders are the K1's, so the solve is
+// bit for bit the three-kernel one.  An iteration that stops or requests
+// the FP64 residual (mixed) only updates the vectors; the request's flush
+// (x64 += e, e = 0) is K3's, and the next launch forms the residual.  What
+// it saves is a launch and K3's second look at p; what it costs is a second
+// gather per entry.
+template <typename VT, int FMT, bool LONG>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(VT) == 4 ? 4 : 2, 8))) void k_pcg_step(
+    MatView A, const VT* __restrict__ p, const VT* __restrict__ z, VT* __restrict__ pout,
+    VT* __restrict__ x, double* __restrict__ x64, VT* __restrict__ v, double* __restrict__ part,
+    ResArgs<VT> R, const double* __restrict__ part2, int G2, const Ctrl* __restrict__ cin,
+    Ctrl* __restrict__ cout, Prm P)
+{
+    constexpr bool MIXED = sizeof(VT) == 4;
+    __shared__ K1Stage<VT, LONG> sm;
+    __shared__ double red[3 * kWaves];
+    __shared__ double bcast[2];
+    Ctrl c = read_ctrl(cin);
+    if (!c.run) {
+        write_ctrl(cout, c);
+        return;
+    }
+    if constexpr (MIXED) {
+        if (c.ru) {  // uniform; the direction moves on to the next slot's buffer
+            replace_residual<FMT == CEL_FMT_DIA ? CEL_FMT_CSR : FMT, LONG>(A, R, c, P, sm.res, red);
+            if (!P.ru_restart)
+                for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < A.n;
+                     i += (long long)gridDim.x * kBlock)
+                    pout[i] = p[i];
+            write_ctrl(cout, c);
+            return;
+        }
+    }
+    const bool pending = c.reduce != kReduceNone;
+    if (pending) {
+        fold_pending(c, R.part, R.G, P, red, bcast);
+    } else {
+        double rz, rr;
+        all_sum2(part2, part2 + G2, G2, red, bcast, rz, rr);
+        next_scalars<MIXED>(c, rz, rr, P);
+    }
+    const VT sigma = VT(c.sigma), beta = VT(c.beta);
+    if (!c.run || (MIXED && c.ru)) {  // uniform: no product
+        const bool flush = MIXED && c.ru;
+        if (!pending)
+            for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < A.n;
+                 i += (long long)gridDim.x * kBlock) {
+                const VT pi = p[i];
+                const VT t = sigma * pi;
+                VT xi = x[i] + t;
+                if (flush) {
+                    const double tt = (double)xi;
+                    x64[i] = x64[i] + tt;
+                    xi = VT(0);
+                }
+                x[i] = xi;
+                const VT bp = beta * pi;
+                pout[i] = bp + z[i];
+            }
+        write_ctrl(cout, c);
+        return;
+    }
+    const double acc = k1_tiles<VT, FMT, false, LONG, true>(
+        A, XDirection<VT>{p, z, beta, pending}, v, sm.tile, StepRows<VT>{pout, x, sigma, !pending});
+    const double bs = block_sum(acc, red);
+    if (threadIdx.x == 0) part[logical_block()] = bs;
     write_ctrl(cout, c);
 }
 
@@ -681,11 +869,12 @@ template <typename VT>
 constexpr int kVecUnrollOf = sizeof(VT) == 4 ? 4 : 2;
 
 // K2: sigma = alpha / sum(v.p) ; r = r + (-sigma) v ; z = jac*r ;
-// per-block partials of r.z and r.r.
-template <typename VT>
+// per-block partials of r.z and r.r.  ZOUT: z is stored too (for k_pcg_step).
+template <typename VT, bool ZOUT>
 __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __restrict__ r,
                                                          const VT* __restrict__ v,
                                                          const VT* __restrict__ jac,
+                                                         VT* __restrict__ z,
                                                          double* __restrict__ part,
                                                          const double* __restrict__ vpart, int G1,
                                                          const Ctrl* __restrict__ cin,
@@ -694,10 +883,21 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
     __shared__ double red[2 * kWaves];
     __shared__ double bcast;
     Ctrl c = read_ctrl(cin);
-    if (!c.run) {
+    // a slot without a product: a replacement was requested (ru) or its
+    // residual is pending (reduce)
+    if (!c.run || c.ru || c.reduce != kReduceNone) {
         write_ctrl(cout, c);
         return;
     }
+    using V = typename Vec<VT>::T;
+    constexpr int W = Vec<VT>::W;
+    const int lb = logical_block();
+    const int G = gridDim.x;
+    const long long unit = (long long)kBlock * W;
+    long long u0, u1;
+    unit_range((n + unit - 1) / unit, G, lb, u0, u1);
+    const long long lo = u0 * unit, hi = min(u1 * unit, n);
+    long long i = lo + (long long)threadIdx.x * W;
     const double vp = all_sum(vpart, G1, red, &bcast);
     const double sigma = c.alpha / vp;
     if (!(vp > 0.0) || !isfinite(sigma)) {
@@ -707,18 +907,9 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
         return;
     }
     c.sigma = sigma;
-    using V = typename Vec<VT>::T;
-    constexpr int W = Vec<VT>::W;
-    const int lb = logical_block();
-    const int G = gridDim.x;
-    const long long unit = (long long)kBlock * W;
-    long long u0, u1;
-    unit_range((n + unit - 1) / unit, G, lb, u0, u1);
-    const long long lo = u0 * unit, hi = min(u1 * unit, n);
     const VT ms = VT(-sigma);
     double arz = 0.0, arr = 0.0;
     constexpr int kVecUnroll = kVecUnrollOf<VT>;
-    long long i = lo + (long long)threadIdx.x * W;
     // kVecUnroll units per step while they are whole vectors (all their
     // loads in flight together), added to the partials in unit order
     for (; i + (kVecUnroll - 1) * unit + W <= hi; i += kVecUnroll * unit) {
@@ -737,37 +928,42 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
                 VT ri = lane<VT>(rv[u], k) + t;
                 set_lane<VT>(rv[u], k, ri);
                 VT zi = ri * lane<VT>(jv[u], k);
+                if constexpr (ZOUT) set_lane<VT>(jv[u], k, zi);
                 double rz = double(ri) * double(zi);
                 arz = arz + rz;
                 double rr = double(ri) * double(ri);
                 arr = arr + rr;
             }
             *reinterpret_cast<V*>(r + i + u * unit) = rv[u];
+            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i + u * unit) = jv[u];
         }
     }
     for (; i < hi; i += unit) {
         if (i + W <= n) {
             const V vv = *reinterpret_cast<const V*>(v + i);
             V rv = *reinterpret_cast<const V*>(r + i);
-            const V jv = *reinterpret_cast<const V*>(jac + i);
+            V jv = *reinterpret_cast<const V*>(jac + i);
 #pragma unroll
             for (int k = 0; k < W; ++k) {
                 VT t = ms * lane<VT>(vv, k);
                 VT ri = lane<VT>(rv, k) + t;
                 set_lane<VT>(rv, k, ri);
                 VT zi = ri * lane<VT>(jv, k);
+                if constexpr (ZOUT) set_lane<VT>(jv, k, zi);
                 double rz = double(ri) * double(zi);
                 arz = arz + rz;
                 double rr = double(ri) * double(ri);
                 arr = arr + rr;
             }
             *reinterpret_cast<V*>(r + i) = rv;
+            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i) = jv;
         } else {
             for (long long j = i; j < hi; ++j) {
                 VT t = ms * v[j];
                 VT ri = r[j] + t;
                 r[j] = ri;
                 VT zi = ri * jac[j];
+                if constexpr (ZOUT) z[j] = zi;
                 double rz = double(ri) * double(zi);
                 arz = arz + rz;
                 double rr = double(ri) * double(ri);
@@ -799,36 +995,16 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
     __shared__ double red[2 * kWaves];
     __shared__ double bcast[2];
     Ctrl c = read_ctrl(cin);
-    if (!c.run) {
+    if (!c.run || c.reduce != kReduceNone) {
         write_ctrl(cout, c);
         return;
     }
     double rz, rr;
     all_sum2(rpart, rpart + G2, G2, red, bcast, rz, rr);  // r.z and r.r in one pass
-    const double beta_d = rz / c.alpha;
-    const VT sigma = VT(c.sigma), beta = VT(beta_d);
+    const VT sigma = VT(c.sigma);
     // scalars of the next iteration (they do not depend on the vectors)
-    c.beta = beta_d;
-    c.alpha = rz;
-    c.norm2 = sqrt(rr);
-    c.iter = c.iter + 1;
-    if (blockIdx.x == 0 && threadIdx.x == 0 && c.iter < P.hist_cap) P.hist[c.iter] = c.norm2;
-    if (!MIXED) {
-        c.run = (c.iter < P.iter_max && alpha_ok(P, c.alpha) && c.norm2 > c.eps) ? 1 : 0;
-    } else {
-        // replace the FP32 residual by the FP64 one when it has dropped by
-        // ru_delta since the last replacement, looks converged, the budget
-        // is spent, or the FP32 recurrence has stopped tracking the FP64
-        // residual (grown past it, or a cycle far longer than expected);
-        // the stop decision is taken on the FP64 norm
-        c.since = c.since + 1;
-        const bool drop = c.norm2 < P.ru_delta * c.rnorm_ref;
-        const bool astray = c.norm2 > 2.0 * c.rnorm_ref || c.since >= P.ru_max_inner;
-        c.ru = (drop || astray || c.norm2 <= c.eps || c.iter >= P.iter_max ||
-                !alpha_ok(P, c.alpha) || !isfinite(c.norm2))
-                   ? 1
-                   : 0;
-    }
+    next_scalars<MIXED>(c, rz, rr, P);
+    const VT beta = VT(c.beta);
     // mixed, replacement iteration: the FP32 correction is folded into the
     // FP64 solution here (x64 = x64 + e, e = 0) instead of in a kernel of
     // its own; same arithmetic
@@ -947,6 +1123,9 @@ __global__ __launch_bounds__(kBlock) void k_ru_flush(long long n, double* __rest
 struct Workspace {
     DevBuf<double> r, p, v, x, b, part1, part2, rpart, ghost, sendbuf, hist;
     DevBuf<float> r32, p32, v32, e32;
+    // two-kernel iterations: the second direction buffer and z = jac*r
+    DevBuf<double> p2, z;
+    DevBuf<float> p2_32, z32;
     // JAD solves: b, x and the Jacobi vector in the permuted row order
     DevBuf<double> bp, xp, jacp;
     // halo solves: per-row halo records {count, p1, p2, p3}
@@ -1015,7 +1194,7 @@ static int k1_cap(int G1, bool mixed)
 // The K1 of a form, and the grid the FP64 K1s of the CSR and DIA forms
 // share (so that their partials, and the solves, stay bitwise equal).
 template <typename VT>
-using K1Fn = void (*)(MatView, const VT*, VT*, double*, const double*, int, const Ctrl*, Ctrl*, Prm);
+using K1Fn = void (*)(MatView, const VT*, VT*, double*, ResArgs<VT>, const Ctrl*, Ctrl*, Prm);
 
 template <typename VT>
 static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr)
@@ -1024,8 +1203,10 @@ static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr)
     if constexpr (sizeof(VT) == 8) {  // halo blocks: FP64 only
         if (halo && fmt == CEL_FMT_DIA) return k_pcg_spmv<VT, CEL_FMT_DIA, true, false>;
         if (halo) return lr ? k_pcg_spmv<VT, CEL_FMT_CSR, true, true> : k_pcg_spmv<VT, CEL_FMT_CSR, true, false>;
+        if (fmt == CEL_FMT_DIA) return k_pcg_spmv<VT, CEL_FMT_DIA, false, false>;
+    } else if (fmt == CEL_FMT_DIA) {
+        return lr ? k_pcg_spmv<VT, CEL_FMT_DIA, false, true> : k_pcg_spmv<VT, CEL_FMT_DIA, false, false>;
     }
-    if (fmt == CEL_FMT_DIA) return k_pcg_spmv<VT, CEL_FMT_DIA, false, false>;
     return lr ? k_pcg_spmv<VT, CEL_FMT_CSR, false, true> : k_pcg_spmv<VT, CEL_FMT_CSR, false, false>;
 }
 
@@ -1040,22 +1221,47 @@ static int k1_grid_f64(long long ntiles)
     return g;
 }
 
-// The residual kernel of a solve (the set-up, or REPLACE: the mixed form's
-// FP64 replacement) in the CSR or JAD form.
-template <typename OUT_T>
-using ResFn = void (*)(MatView, const double*, const double*, const double*, const float*, OUT_T*,
-                       OUT_T*, float*, double*, const Ctrl*, Ctrl*, Prm);
+template <typename VT>
+using StepFn = void (*)(MatView, const VT*, const VT*, VT*, VT*, double*, VT*, double*, ResArgs<VT>,
+                        const double*, int, const Ctrl*, Ctrl*, Prm);
 
-template <typename OUT_T, bool REPLACE>
+template <typename VT>
+static StepFn<VT> step_kernel(int fmt, bool lr)
+{
+    if (fmt == CEL_FMT_JAD) return k_pcg_step<VT, CEL_FMT_JAD, false>;
+    if constexpr (sizeof(VT) == 8) {
+        if (fmt == CEL_FMT_DIA) return k_pcg_step<VT, CEL_FMT_DIA, false>;
+    } else if (fmt == CEL_FMT_DIA) {
+        return lr ? k_pcg_step<VT, CEL_FMT_DIA, true> : k_pcg_step<VT, CEL_FMT_DIA, false>;
+    }
+    return lr ? k_pcg_step<VT, CEL_FMT_CSR, true> : k_pcg_step<VT, CEL_FMT_CSR, false>;
+}
+
+// Whether a solve iterates with two kernels (k_pcg_step, K2) instead of
+// three: small systems, whose iteration is launches and latency rather than
+// bytes.  Measured per iteration on variable-coefficient 7-point cubes, two
+// against three kernels, CSR: FP64 32^3 12.3 / 13.6 us, 64^3 17.4 / 18.6,
+// 80^3 28.7 / 29.3, 100^3 43.0 / 39.8; mixed 32^3 12.6 / 14.4, 80^3 22.9 /
+// 24.6, 100^3 32.7 / 33.6, 128^3 48.8 / 49.1 (DIA and JAD alike).  Long rows
+// pay for the second gather at any size (30,011 mesh rows of 11 entries 19.3
+// / 18.7 us, 200,003 rows 36.5 / 29.3 us).
+static bool step_form(const Mat& A, int fmt, bool mixed)
+{
+    return A.n <= (mixed ? 1200000 : 300000) && !csr_long_rows(A) && !(fmt == CEL_FMT_JAD && A.jad_mmax > kGather);
+}
+
+// The set-up kernel of a solve in the CSR or JAD form.
+template <typename OUT_T>
+using ResFn = void (*)(MatView, ResArgs<OUT_T>, const Ctrl*, Ctrl*);
+
+template <typename OUT_T>
 static ResFn<OUT_T> res_kernel(int fmt, bool halo, bool lr)
 {
-    if (fmt == CEL_FMT_JAD) return k_residual<OUT_T, CEL_FMT_JAD, false, REPLACE, false>;
+    if (fmt == CEL_FMT_JAD) return k_residual<OUT_T, CEL_FMT_JAD, false, false>;
     if constexpr (sizeof(OUT_T) == 8)
         if (halo)
-            return lr ? k_residual<OUT_T, CEL_FMT_CSR, true, REPLACE, true>
-                      : k_residual<OUT_T, CEL_FMT_CSR, true, REPLACE, false>;
-    return lr ? k_residual<OUT_T, CEL_FMT_CSR, false, REPLACE, true>
-              : k_residual<OUT_T, CEL_FMT_CSR, false, REPLACE, false>;
+            return lr ? k_residual<OUT_T, CEL_FMT_CSR, true, true> : k_residual<OUT_T, CEL_FMT_CSR, true, false>;
+    return lr ? k_residual<OUT_T, CEL_FMT_CSR, false, true> : k_residual<OUT_T, CEL_FMT_CSR, false, false>;
 }
 
 // The allocation-free entry point's device memory: a file-scope array
@@ -1160,7 +1366,7 @@ int pcg_spmv_dot(Mat& A, int fmt, const double* x, const double* ghost, double* 
     }
     const Prm P{};
     hipLaunchKernelGGL(k1_kernel<double>(fmt, halo, csr_long_rows(A)), dim3(G1), dim3(kBlock), 0, s, V,
-                       x, y, W.part1.p, nullptr, 0, W.ctrl.p, W.ctrl.p + 1, P);
+                       x, y, W.part1.p, ResArgs<double>{}, W.ctrl.p, W.ctrl.p + 1, P);
     CEL_HIP(hipGetLastError());
     std::vector<double> part((size_t)G1);
     CEL_HIP(hipMemcpyAsync(part.data(), W.part1.p, sizeof(double) * G1, hipMemcpyDeviceToHost, s));
@@ -1237,16 +1443,16 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     if (!mixed) {
         if (fmt == CEL_FMT_JAD) G1 = resident_grid((const void*)k1_kernel<double>(fmt, false, false), ntiles);
         else G1 = k1_grid_f64(ntiles);
-        Gr = common_grid({(const void*)res_kernel<double, false>(rfmt, false, lr),
-                          (const void*)res_kernel<double, false>(rfmt, rfmt == CEL_FMT_CSR, lr)}, ntiles);
+        Gr = common_grid({(const void*)res_kernel<double>(rfmt, false, lr),
+                          (const void*)res_kernel<double>(rfmt, rfmt == CEL_FMT_CSR, lr)}, ntiles);
     } else {
         G1 = fmt == CEL_FMT_JAD
                  ? resident_grid((const void*)k1_kernel<float>(fmt, false, false), ntiles)
                  : common_grid({(const void*)k1_kernel<float>(CEL_FMT_CSR, false, false),
                                 (const void*)k1_kernel<float>(CEL_FMT_CSR, false, true),
-                                (const void*)k1_kernel<float>(CEL_FMT_DIA, false, false)}, ntiles);
-        Gr = common_grid({(const void*)res_kernel<float, false>(rfmt, false, lr),
-                          (const void*)res_kernel<float, true>(rfmt, false, lr)}, ntiles);
+                                (const void*)k1_kernel<float>(CEL_FMT_DIA, false, false),
+                                (const void*)k1_kernel<float>(CEL_FMT_DIA, false, true)}, ntiles);
+        Gr = resident_grid((const void*)res_kernel<float>(rfmt, false, lr), ntiles);
     }
     G1 = k1_cap(G1, mixed);
     {
@@ -1317,6 +1523,25 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         w.v32 = W.v32.p;
         w.e32 = W.e32.p;
     }
+    // two kernels per iteration on small systems; the halo blocks need a
+    // stored direction before the product, profiling a product of its own
+    const bool step = !noalloc && !halo && !prm.profile && step_form(A, fmt, mixed);
+    double *pbuf[2] = {w.p, nullptr}, *zbuf = nullptr;
+    float *pbuf32[2] = {w.p32, nullptr}, *zbuf32 = nullptr;
+    if (step) {
+        Workspace& W = *Wp;
+        if (mixed) {
+            CEL_TRY(W.p2_32.alloc(nn));
+            CEL_TRY(W.z32.alloc(nn));
+            pbuf32[1] = W.p2_32.p;
+            zbuf32 = W.z32.p;
+        } else {
+            CEL_TRY(W.p2.alloc(nn));
+            CEL_TRY(W.z.alloc(nn));
+            pbuf[1] = W.p2.p;
+            zbuf = W.z.p;
+        }
+    }
     const double* db = b;
     double* dx = x;
     if (prm.memspace == CEL_MEM_HOST) {
@@ -1369,7 +1594,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     // last call's contents; everything else is written before it is read)
     CEL_HIP(hipMemcpyAsync(w.ctrl, &c0, sizeof(Ctrl), hipMemcpyHostToDevice, s));
     // token slots: 0 -> K1 -> 1 -> K2 -> 2 -> K3 -> 0 (FP64);
-    // mixed: K3 -> 3 -> replacement residual -> 0 (K3 folds e into x64)
+    // (two-kernel form: 0 -> step -> 1 -> K2 -> 0)
     Ctrl* C0 = w.ctrl;
     Ctrl* C1 = w.ctrl + 1;
     Ctrl* C2 = w.ctrl + 2;
@@ -1450,12 +1675,12 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
 
     // r0, p0 and their partials; the first K1 folds them in.  The set-up
     // reads and writes token slot 0 (only block 0 writes, after its read).
+    const ResArgs<double> R64{dx, db, jac64, nullptr, w.r, w.p, nullptr, w.rpart, Gr};
+    const ResArgs<float> R32{dx, db, nullptr, jac32, w.r32, w.p32, w.e32, w.rpart, Gr};
     if (!mixed)
-        hipLaunchKernelGGL((res_kernel<double, false>(rfmt, halo, lr)), dim3(Gr), dim3(kBlock), 0, s, V, dx,
-                           db, jac64, jac32, w.r, w.p, w.e32, w.rpart, C0, C0, P);
+        hipLaunchKernelGGL(res_kernel<double>(rfmt, halo, lr), dim3(Gr), dim3(kBlock), 0, s, V, R64, C0, C0);
     else
-        hipLaunchKernelGGL((res_kernel<float, false>(rfmt, false, lr)), dim3(Gr), dim3(kBlock), 0, s, V, dx,
-                           db, jac64, jac32, w.r32, w.p32, w.e32, w.rpart, C0, C0, P);
+        hipLaunchKernelGGL(res_kernel<float>(rfmt, false, lr), dim3(Gr), dim3(kBlock), 0, s, V, R32, C0, C0);
     CEL_HIP(hipGetLastError());
     if (!noalloc) CEL_HIP(hipEventRecord(e1, s));
 
@@ -1472,7 +1697,31 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     };
 
     const long long n_ll = n;
-    auto enqueue_iter = [&](bool profile) -> int {
+    // One slot of the two-kernel form: the step finishes the iteration before
+    // (its vectors and scalars) and forms the next product, K2 updates r.
+    // The direction alternates between two buffers by slot.
+    auto enqueue_step = [&](long long slot) -> int {
+        const int in = (int)(slot & 1), out = in ^ 1;
+        if (!mixed) {
+            hipLaunchKernelGGL(step_kernel<double>(fmt, lr), dim3(G1), dim3(kBlock), 0, s, V,
+                               (const double*)pbuf[in], (const double*)zbuf, pbuf[out], dx, (double*)nullptr, w.v,
+                               w.part1, R64, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
+            hipLaunchKernelGGL((k_pcg_update_r<double, true>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
+                               jac64, zbuf, w.part2, w.part1, G1, C1, C0);
+        } else {
+            ResArgs<float> R = R32;
+            R.p = pbuf32[out];  // a restart's direction
+            hipLaunchKernelGGL(step_kernel<float>(fmt, lr), dim3(G1), dim3(kBlock), 0, s, V,
+                               (const float*)pbuf32[in], (const float*)zbuf32, pbuf32[out], w.e32, dx, w.v32,
+                               w.part1, R, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
+            hipLaunchKernelGGL((k_pcg_update_r<float, true>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
+                               jac32, zbuf32, w.part2, w.part1, G1, C1, C0);
+        }
+        CEL_HIP(hipGetLastError());
+        return CEL_OK;
+    };
+    auto enqueue_iter = [&](bool profile, long long slot) -> int {
+        if (step) return enqueue_step(slot);
         hipEvent_t ea = nullptr, eb = nullptr;
         if (halo) {
             CEL_TRY(launch_face_pack(A, w.p, Wp->sendbuf.p));
@@ -1490,22 +1739,20 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         }
         if (!mixed) {
             hipLaunchKernelGGL(k1_kernel<double>(fmt, halo, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
-                               w.part1, w.rpart, Gr, C0, C1, P);
+                               w.part1, R64, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
-            hipLaunchKernelGGL((k_pcg_update_r<double>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
-                               jac64, w.part2, w.part1, G1, C1, C2);
+            hipLaunchKernelGGL((k_pcg_update_r<double, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
+                               jac64, (double*)nullptr, w.part2, w.part1, G1, C1, C2);
             hipLaunchKernelGGL((k_pcg_update_xp<double, double, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll,
                                dx, w.p, w.r, jac64, nullptr, w.part2, Gv, C2, C0, P);
         } else {
             hipLaunchKernelGGL(k1_kernel<float>(fmt, false, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
-                               w.part1, w.rpart, Gr, C0, C1, P);
+                               w.part1, R32, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
-            hipLaunchKernelGGL((k_pcg_update_r<float>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
-                               jac32, w.part2, w.part1, G1, C1, C2);
+            hipLaunchKernelGGL((k_pcg_update_r<float, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
+                               jac32, (float*)nullptr, w.part2, w.part1, G1, C1, C2);
             hipLaunchKernelGGL((k_pcg_update_xp<float, float, true>), dim3(Gv), dim3(kBlock), 0, s, n_ll,
-                               w.e32, w.p32, w.r32, jac32, dx, w.part2, Gv, C2, C3, P);
-            hipLaunchKernelGGL((res_kernel<float, true>(rfmt, false, lr)), dim3(Gr), dim3(kBlock), 0, s, V, dx,
-                               db, jac64, jac32, w.r32, w.p32, w.e32, w.rpart, C3, C0, P);
+                               w.e32, w.p32, w.r32, jac32, dx, w.part2, Gv, C2, C0, P);
         }
         CEL_HIP(hipGetLastError());
         return CEL_OK;
@@ -1525,9 +1772,12 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         CEL_TRY(R.event(cev[1], hipEventDisableTiming));
     }
 
-    const bool use_graph = prm.use_graph && !prm.profile && !noalloc;
+    // (a captured chunk of the two-kernel form starts at an even slot)
+    const bool use_graph = prm.use_graph && !prm.profile && !noalloc && !(step && (chunk & 1));
     int status = CEL_OK;
-    const long long budget = (long long)prm.iter_max + 1;
+    // mixed: a replacement takes a slot, or two (the request of the two-kernel
+    // form), and there is at most one per iteration
+    const long long budget = (long long)(mixed ? (step ? 3 : 2) : 1) * ((long long)prm.iter_max + 1);
     long long enqueued = 0;
     int k = 0;
     while (enqueued < budget) {
@@ -1536,7 +1786,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             if (!R.exec) {
                 CEL_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
                 for (int i = 0; i < c; ++i) {
-                    int rc = enqueue_iter(false);
+                    int rc = enqueue_iter(false, i);
                     if (rc < 0) {
                         (void)hipStreamEndCapture(s, &R.graph);
                         return rc;
@@ -1548,7 +1798,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             CEL_HIP(hipGraphLaunch(R.exec, s));
         } else {
             for (int i = 0; i < c; ++i) {
-                status = enqueue_iter(prm.profile != 0 && !noalloc);
+                status = enqueue_iter(prm.profile != 0 && !noalloc, enqueued + i);
                 if (status < 0) break;
             }
             if (status < 0) break;

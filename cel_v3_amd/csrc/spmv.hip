@@ -33,7 +33,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int* __restric
         const int aft = (int)group_tile(step + 2, ntiles);
         VT init = VT(0);
         if constexpr (INIT) init = y[row < n ? row : 0];
-        VT s = ts.template rows<VT>(n, t, nxt, aft, xadj, cols, vals, x, sm, row, nullptr, init);
+        VT s = ts.template rows<VT>(n, t, nxt, aft, xadj, cols, vals, XPlain<VT>{x}, sm, row, nullptr, init);
         ts.advance(nxt, sm);
         if (row < n) y[row] = coo ? s : accumulate ? y[row] + s : VT(0) + s;
     }
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv_fused(int n, long long chun
         const int row = t * kTileRows + threadIdx.x;
         const int nxt = t + 1 < t1 ? t + 1 : -1;
         const int aft = t + 2 < t1 ? t + 2 : -1;
-        double s = ts.template rows<double>(n, t, nxt, aft, xadj, cols, vals, x, sm, row, nullptr);
+        double s = ts.template rows<double>(n, t, nxt, aft, xadj, cols, vals, XPlain<double>{x}, sm, row, nullptr);
         ts.advance(nxt, sm);
         if (row < n) acc = acc + fuse_row<FUSE>(0.0 + s, row, aux, y);
     }

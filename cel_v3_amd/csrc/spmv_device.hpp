@@ -84,15 +84,15 @@ struct CsrStage {
 // stage.  Kept lean on purpose -- its registers would count against the
 // occupancy of the common path.  LDS or global a/c (NT: non-temporal
 // global loads).
-template <typename AT, typename VT, bool NT>
+template <typename AT, typename VT, bool NT, typename X>
 __device__ __forceinline__ AT row_sum_from(AT sum, const VT* a, const int* c, int start, int len,
-                                           const VT* __restrict__ x)
+                                           const X& x)
 {
 #pragma unroll 1
     for (int j = start; j < len; ++j) {
         const int col = NT ? ld_stream(c + j) : c[j];
         const VT av = NT ? ld_stream(a + j) : a[j];
-        AT prod = AT(av) * AT(x[col]);
+        AT prod = AT(av) * AT(x.value(x.load(col)));
         sum = sum + prod;
     }
     return sum;
@@ -139,6 +139,57 @@ __device__ __forceinline__ float buf_load<float>(__amdgpu_buffer_rsrc_t r, int v
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
 }
 
+// The vector a product gathers, as an accessor: load() issues the loads of
+// an entry, value() combines them once they are in (a kernel issues many
+// loads before it uses the first).  buf() is the same vector through buffer
+// resources; an offset outside them reads 0.
+template <typename VT>
+struct XPlain {
+    using Raw = VT;
+    struct Buf {
+        __amdgpu_buffer_rsrc_t r;
+    };
+    const VT* x;
+    __device__ __forceinline__ Raw load(int i) const { return x[i]; }
+    __device__ __forceinline__ VT value(Raw r) const { return r; }
+    __device__ __forceinline__ Buf buf(unsigned bytes) const
+    {
+        return Buf{tile_rsrc(x, (int)bytes)};
+    }
+    __device__ __forceinline__ Raw load(const Buf& b, int off) const { return buf_load<VT>(b.r, off); }
+};
+
+// beta p + z: the search direction of the next iteration, formed where it
+// is gathered (each product rounded before its add, as the update kernel
+// rounds them).  keep: the direction is p itself.
+template <typename VT>
+struct XDirection {
+    struct Raw {
+        VT p, z;
+    };
+    struct Buf {
+        __amdgpu_buffer_rsrc_t p, z;
+    };
+    const VT *p, *z;
+    VT beta;
+    bool keep;
+    __device__ __forceinline__ Raw load(int i) const { return Raw{p[i], z[i]}; }
+    __device__ __forceinline__ VT value(const Raw& r) const
+    {
+        const VT bp = beta * r.p;
+        const VT d = bp + r.z;
+        return keep ? r.p : d;
+    }
+    __device__ __forceinline__ Buf buf(unsigned bytes) const
+    {
+        return Buf{tile_rsrc(p, (int)bytes), tile_rsrc(z, (int)bytes)};
+    }
+    __device__ __forceinline__ Raw load(const Buf& b, int off) const
+    {
+        return Raw{buf_load<VT>(b.p, off), buf_load<VT>(b.z, off)};
+    }
+};
+
 // DIA row sums of R rows r[0..R) (r[k] >= n: not used; r[0] < n) of a block
 // stored per diagonal (vals[d*n + i]; offsets ascending; bit d of the row
 // mask marks an entry): each row's entries in ascending offset (= CSR
@@ -152,10 +203,10 @@ __device__ __forceinline__ float buf_load<float>(__amdgpu_buffer_rsrc_t r, int v
 // diagonal with offset 0 (index dzero >= 0, present in the caller's
 // layout), taken after the products' wait, so it costs no load and no
 // round trip of its own.
-template <typename VT, int R, int GD>
+template <typename VT, int R, int GD, typename X>
 __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const VT* vals,
                                          const uint8_t* m8, const uint32_t* m32, const int (&r)[R],
-                                         const VT* __restrict__ x, VT (&s)[R], VT* xr = nullptr,
+                                         const X& x, VT (&s)[R], typename X::Raw* xr = nullptr,
                                          int dzero = -1)
 {
     constexpr int B = (int)sizeof(VT);
@@ -167,9 +218,10 @@ __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const V
         m[k] = m8 ? (unsigned)m8[rc[k]] : m32[rc[k]];  // m8: uniform
         s[k] = VT(0);
     }
-    const auto rx = tile_rsrc(x, n * B);
+    const auto rx = x.buf((unsigned)n * (unsigned)B);
     for (int d0 = 0; d0 < nd; d0 += GD) {
-        VT v[GD][R], xv[GD][R];
+        VT v[GD][R];
+        typename X::Raw xv[GD][R];
 #pragma unroll
         for (int g = 0; g < GD; ++g) {
             const int d = d0 + g;
@@ -182,7 +234,7 @@ __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const V
                     // an absent entry's column may lie outside [0, n): its
                     // byte offset wraps modulo 2^32 (unsigned, defined) and
                     // the load returns 0 or a value the mask discards
-                    xv[g][k] = buf_load<VT>(rx, (int)((unsigned)(rc[k] + o) * (unsigned)B));
+                    xv[g][k] = x.load(rx, (int)((unsigned)(rc[k] + o) * (unsigned)B));
                 }
             }
         }
@@ -192,7 +244,7 @@ __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const V
             if (d < nd) {
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
-                    const VT prod = v[g][k] * xv[g][k];
+                    const VT prod = v[g][k] * x.value(xv[g][k]);
                     s[k] = ((m[k] >> d) & 1u) ? s[k] + prod : s[k];
                 }
                 if (xr && d == dzero) {
@@ -360,12 +412,12 @@ struct CsrTileStream {
     // is not null) are issued first (see above).  The fetched registers are
     // consumed by the caller's stage() in the same iteration, never carried
     // across it.
-    template <typename AT, typename Extra = NoLoads>
+    template <typename AT, typename X, typename Extra = NoLoads>
     __device__ __forceinline__ AT rows(int n, int t, int next, int after,
                                        const int* __restrict__ xadj, const int* __restrict__ cols,
-                                       const VT* __restrict__ vals, const VT* __restrict__ x,
-                                       const CsrStage<VT>& sm, int row, VT* xrow, AT init = AT(0),
-                                       Extra&& extra = Extra{})
+                                       const VT* __restrict__ vals, const X& x,
+                                       const CsrStage<VT>& sm, int row, typename X::Raw* xrow,
+                                       AT init = AT(0), Extra&& extra = Extra{})
     {
         const int b0 = e0, l = lo - e0, len = hi - lo;
         const bool staged = cnt <= kStageMax;  // uniform across the block
@@ -377,14 +429,14 @@ struct CsrTileStream {
         // different loads in flight, so the waits below (for the next
         // tile's entry range, for the gathers) would have to cover every
         // load issued, the next tile's included.
-        VT xv[kGather];
+        typename X::Raw xv[kGather];
 #pragma unroll
         for (int i = 0; i < kGather; ++i) {
             const int ci = sm.col[min(l + i, kStageCap - 1)];
-            xv[i] = x[i < len ? ci : 0];
+            xv[i] = x.load(i < len ? ci : 0);
         }
-        VT xr = VT(0);
-        if (xrow) xr = x[row < n ? row : 0];
+        typename X::Raw xr{};
+        if (xrow) xr = x.load(row < n ? row : 0);
         // the caller's loads for this step: behind the gathers (waiting for
         // those does not wait for these), ahead of the next tile's entries
         // (whose wait, for the stage, covers these)
@@ -400,7 +452,7 @@ struct CsrTileStream {
 #pragma unroll
         for (int i = 0; i < kGather; ++i) {
             const VT a = sm.val[min(l + i, kStageCap - 1)];
-            AT prod = AT(a) * AT(xv[i]);
+            AT prod = AT(a) * AT(x.value(xv[i]));
             AT tt = sum + prod;
             sum = i < len ? tt : sum;
         }
@@ -519,21 +571,21 @@ struct CsrLongStream {
 
     // As CsrTileStream::rows(); it synchronises (every thread of the block
     // calls it) and leaves the stage free.
-    template <typename AT, typename Extra = NoLoads>
+    template <typename AT, typename X, typename Extra = NoLoads>
     __device__ __forceinline__ AT rows(int n, int t, int next, int after,
                                        const int* __restrict__ xadj, const int* __restrict__ cols,
-                                       const VT* __restrict__ vals, const VT* __restrict__ x,
-                                       CsrLongStage<VT>& sm, int row, VT* xrow, AT init = AT(0),
-                                       Extra&& extra = Extra{})
+                                       const VT* __restrict__ vals, const X& x,
+                                       CsrLongStage<VT>& sm, int row, typename X::Raw* xrow,
+                                       AT init = AT(0), Extra&& extra = Extra{})
     {
         AT sum = init;
         bool first = true, more;  // uniform across the block
         do {
-            VT xv[kPer];
+            typename X::Raw xv[kPer];
 #pragma unroll
-            for (int i = 0; i < kPer; ++i) xv[i] = x[c[i]];
+            for (int i = 0; i < kPer; ++i) xv[i] = x.load(c[i]);
             if (first) {
-                if (xrow) *xrow = x[row < n ? row : 0];
+                if (xrow) *xrow = x.load(row < n ? row : 0);
                 extra();
             }
             first = false;
@@ -558,7 +610,7 @@ struct CsrLongStream {
             for (int i = 0; i < kPer / 4; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const VT prod = v[i * 4 + j] * xv[i * 4 + j];
+                    const VT prod = v[i * 4 + j] * x.value(xv[i * 4 + j]);
                     sm.prod[slot(4 * (int)threadIdx.x + 4 * kBlock * i + j)] = prod;
                 }
             __syncthreads();
@@ -652,17 +704,18 @@ __device__ __forceinline__ AT jad_row(int k, int mmax, const int* __restrict__ b
 // Diagonals past kGather are summed after the first kGather, in order,
 // from global memory.  jad_nnz * sizeof(VT) and n * sizeof(VT) must stay
 // below 2^32 - 16 (unsigned 32-bit byte offsets).
-template <typename VT>
+template <typename VT, typename X = XPlain<VT>>
 struct JadStream {
     int bg[kGather];  // starts of diagonals 0..kGather-1 (clamped)
     int ln[kGather];  // their lengths (0 past the last diagonal)
     int c[kGather];   // the fetched row's columns and values
     VT a[kGather];
-    __amdgpu_buffer_rsrc_t rc, rv, rx;
+    __amdgpu_buffer_rsrc_t rc, rv;
+    typename X::Buf rx;
 
     __device__ __forceinline__ void init(int n, int mmax, long long nnz,
                                          const int* __restrict__ begin, const int* cols,
-                                         const VT* vals, const VT* x)
+                                         const VT* vals, const X& x)
     {
         constexpr unsigned B = sizeof(VT);
         const int nd = min(mmax, kGather);
@@ -676,8 +729,7 @@ struct JadStream {
                                                (int)((unsigned)nnz * 4u), 0x00020000);
         rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<VT*>(vals), (short)0,
                                                (int)((unsigned)nnz * B), 0x00020000);
-        rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<VT*>(x), (short)0,
-                                               (int)((unsigned)n * B), 0x00020000);
+        rx = x.buf((unsigned)n * B);
     }
 
     // every load is issued (entries a row lacks read from outside the
@@ -701,13 +753,13 @@ struct JadStream {
     template <typename AT>
     __device__ __forceinline__ AT row(int k, int kn, int mmax, const int* __restrict__ begin,
                                       const int* __restrict__ cols, const VT* __restrict__ vals,
-                                      const VT* __restrict__ x, VT& xr)
+                                      const X& x, typename X::Raw& xr)
     {
         constexpr unsigned B = sizeof(VT);
-        VT xv[kGather];
+        typename X::Raw xv[kGather];
 #pragma unroll
-        for (int i = 0; i < kGather; ++i) xv[i] = buf_load<VT>(rx, (int)((unsigned)c[i] * B));
-        xr = buf_load<VT>(rx, (int)((unsigned)k * B));
+        for (int i = 0; i < kGather; ++i) xv[i] = x.load(rx, (int)((unsigned)c[i] * B));
+        xr = x.load(rx, (int)((unsigned)k * B));
         VT ac[kGather];
 #pragma unroll
         for (int i = 0; i < kGather; ++i) ac[i] = a[i];
@@ -717,7 +769,7 @@ struct JadStream {
         AT sum = AT(0);
 #pragma unroll
         for (int i = 0; i < kGather; ++i) {
-            AT prod = AT(ac[i]) * AT(xv[i]);
+            AT prod = AT(ac[i]) * AT(x.value(xv[i]));
             AT tt = sum + prod;
             sum = k < ln[i] ? tt : sum;
         }
@@ -725,7 +777,7 @@ struct JadStream {
             for (int d = kGather; d < mmax; ++d) {
                 const int b = begin[d];
                 if (k >= begin[d + 1] - b) break;
-                AT prod = AT(ld_stream(vals + b + k)) * AT(x[ld_stream(cols + b + k)]);
+                AT prod = AT(ld_stream(vals + b + k)) * AT(x.value(x.load(ld_stream(cols + b + k))));
                 sum = sum + prod;
             }
         }
