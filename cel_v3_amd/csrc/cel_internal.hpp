@@ -252,6 +252,13 @@ int launch_csr_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const 
 int launch_dia_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const double* x,
                           double* y, const double* aux, double* part, const int* skip);
 int dia_prepare_f32(Mat& A);
+// The distinct offsets col - row of the local block, ascending, at most
+// `most` (<= 32) of them: *nd = most + 1 when there are more.  *ascending:
+// every row's columns strictly ascend (known only when *nd <= most).
+int dia_offsets(const Mat& A, int most, int* nd, int* off, bool* ascending);
+// Diagonal-major values (v64, or v32 rounded to FP32) and row masks on at
+// most 8 diagonals; slots without an entry are left as they are.
+int dia_fill(const Mat& A, int nd, const int* off, double* v64, float* v32, uint8_t* mask8);
 // Sets bit `bit` (= dia_nd) of the DIA row masks on the rows with halo
 // entries and clears it elsewhere; fails when the masks have no spare bit.
 int launch_halo_spmv(const Mat& A, const double* ghost, double* y);
