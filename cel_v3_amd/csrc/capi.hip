@@ -19,6 +19,7 @@ int pcg_noalloc_setup(int device);
 static thread_local std::string g_err;
 
 void set_error(const std::string& msg) { g_err = msg; }
+const std::string& last_error() { return g_err; }
 int fail(int code, const std::string& msg)
 {
     set_error(msg);
@@ -384,6 +385,7 @@ extern "C" int cel_gpu_mat_set_jacobi(cel_gpu_mat* A, int row_scaled)
     Mat& M = A->m;
     if (!M.has_diag) CEL_TRY(launch_extract_diag(M));
     M.has_diag = true;
+    M.derived.release();  // its row forms hold the Jacobi values
     CEL_TRY(launch_set_jacobi(M, row_scaled));
     M.has_jac = true;
     M.jac_row_scaled = row_scaled != 0;
@@ -399,6 +401,7 @@ extern "C" int cel_gpu_mat_scale_diagonal(cel_gpu_mat* A)
     CEL_TRY(launch_scale_rows(M));
     M.is_scaled = true;
     // derived copies are stale now
+    M.derived.release();
     M.vals32.release();
     M.jad_mode = -1;
     M.jad_vals32.release();

@@ -16,6 +16,7 @@ namespace cel {
 
 // ---------------------------------------------------------------- errors
 void set_error(const std::string& msg);
+const std::string& last_error();
 int fail(int code, const std::string& msg);
 
 #define CEL_HIP(call)                                                              \
@@ -138,6 +139,40 @@ struct HaloBlock {
     std::vector<int> h_recv_perm;  // ascending local column ids (1-based)
 };
 
+// Derived forms of a block for long solves (rowclass.hip).
+constexpr int kMaxClass = 256;   // row forms a byte tells apart
+constexpr int kClassDiag = 8;    // diagonals of a row form
+constexpr int kDerivedRows = 800000;
+
+// Table of the row forms, by class: values by diagonal, presence mask,
+// Jacobi value (device pointers).
+struct RowClasses {
+    double *val64, *jac64;
+    float *val32, *jac32;
+    uint32_t* mask;
+};
+
+struct Derived {
+    enum { kNone = 0, kClasses, kDiagonals };
+    int kind = kNone;  // kClasses once the classes are built
+    bool tried = false, tried32 = false, tried64 = false;
+    int nd = 0;        // diagonals (0: more than kClassDiag, or unsorted rows)
+    int off[32] = {};  // ascending
+    DevBuf<uint8_t> cls;      // per row: its class
+    DevBuf<double> tab64;     // val64, then jac64
+    DevBuf<float> tab32;
+    DevBuf<uint32_t> tabm;
+    DevBuf<double> vals;      // diagonal storage of a CSR solve, as Mat::dia_vals
+    DevBuf<float> vals32;
+    DevBuf<uint8_t> mask8;
+    RowClasses classes() const
+    {
+        return RowClasses{tab64.p, tab64.p + kMaxClass * kClassDiag, tab32.p, tab32.p + kMaxClass * kClassDiag,
+                          tabm.p};
+    }
+    void release();
+};
+
 struct Mat {
     int n = 0;          // local rows
     int ncols = 0;      // local columns (== n for a square local block)
@@ -173,6 +208,8 @@ struct Mat {
     DevBuf<uint32_t> dia_mask;      // presence bits per row (more than 8 diagonals)
     DevBuf<uint8_t> dia_mask8;      // the same in one byte (at most 8 diagonals)
     std::vector<int> h_jad_begin;  // host copy (0-based starts, mmax+1)
+
+    Derived derived;
 
     // halo (distributed block split of one rank)
     std::vector<HaloBlock> halo;
@@ -252,6 +289,9 @@ int launch_csr_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const 
 int launch_dia_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const double* x,
                           double* y, const double* aux, double* part, const int* skip);
 int dia_prepare_f32(Mat& A);
+// The derived form (Derived::k*) a PCG solve of at most iter_max iterations
+// runs on, built on the first call that wants it; never an error.
+int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max);
 // The distinct offsets col - row of the local block, ascending, at most
 // `most` (<= 32) of them: *nd = most + 1 when there are more.  *ascending:
 // every row's columns strictly ascend (known only when *nd <= most).

@@ -216,6 +216,10 @@ struct MatView {
     int nd;
     int dzero;               // index of the diagonal with offset 0, or -1
     int doff[32];
+    // row classes (rowclass.hip), with the diagonals above
+    const uint8_t* cls;
+    RowClasses ctab;
+    const int* walk;  // by K1 block: the walk it takes (null: its own)
     // halo (FP64 only)
     const int *hrow_tile, *hrows, *hrowq, *hptr, *hcols;
     const double* hvals;
@@ -263,6 +267,32 @@ __device__ __forceinline__ const double* dia_vals<double>(const MatView& A) { re
 template <>
 __device__ __forceinline__ const float* dia_vals<float>(const MatView& A) { return A.dvals32; }
 
+// A solve's matrix as row classes: a form of its own beside CEL_FMT_*.
+constexpr int kFmtClass = 64;
+
+template <typename VT>
+__device__ __forceinline__ void load_classes(const MatView& A, ClassTab<VT>& t);
+template <>
+__device__ __forceinline__ void load_classes<double>(const MatView& A, ClassTab<double>& t)
+{
+    t.load(A.ctab.val64, A.ctab.mask);
+}
+template <>
+__device__ __forceinline__ void load_classes<float>(const MatView& A, ClassTab<float>& t)
+{
+    t.load(A.ctab.val32, A.ctab.mask);
+}
+
+// The LDS a form's tile walk uses.
+template <typename VT, int FMT, bool LONG>
+struct StageOf {
+    using T = typename CsrStreamOf<VT, LONG>::Stage;
+};
+template <typename VT, bool LONG>
+struct StageOf<VT, kFmtClass, LONG> {
+    using T = ClassTab<VT>;
+};
+
 template <typename VT>
 __device__ __forceinline__ const VT* jad_vals(const MatView& A);
 template <>
@@ -279,7 +309,7 @@ __device__ __forceinline__ const float* jad_vals<float>(const MatView& A) { retu
 // __syncthreads() for CSR: every thread of the block calls it.
 template <typename VT, typename AT, int FMT, bool HALO, bool LONG>
 struct TileWalk {
-    using Stage = typename CsrStreamOf<VT, LONG>::Stage;
+    using Stage = typename StageOf<VT, FMT, LONG>::T;
     typename CsrStreamOf<VT, LONG>::Stream cs;
 
     // Contains __syncthreads() for CSR: every thread of the block calls it.
@@ -290,6 +320,7 @@ struct TileWalk {
                 cs.open(A.n, (int)t0, t0 + 1 < t1 ? (int)t0 + 1 : -1, A.xadj, A.cols,
                         csr_vals<VT>(A), sm);
         }
+        if constexpr (FMT == kFmtClass) load_classes<VT>(A, sm);
     }
 
     __device__ __forceinline__ AT next(const MatView& A, long long t, long long t1,
@@ -311,6 +342,15 @@ struct TileWalk {
                 if (row < A.n)
                     s = halo_row<AT>(row, (int)t, s, A.hrow_tile, A.hrows, A.hptr, A.hcols,
                                      A.hvals, A.ghost);
+            }
+        } else if constexpr (FMT == kFmtClass) {
+            row = r0 + threadIdx.x;
+            s = AT(0);
+            if (row < A.n) {
+                const int r[1] = {row};
+                VT sum[1];
+                class_rows<VT, 1>(A.n, A.nd, A.doff, A.cls, sm, r, XPlain<VT>{x}, sum);
+                s = AT(0) + sum[0];
             }
         } else {
             // JAD solves keep their vectors in the permuted row order, with
@@ -349,8 +389,7 @@ struct ResArgs {
 // Block lb of a.G: its contiguous tiles and its partials.
 template <typename OUT_T, int FMT, bool HALO, bool REPLACE, bool LONG>
 __device__ __forceinline__ void residual_block(const MatView& A, const ResArgs<OUT_T>& a, int lb,
-                                               bool restart,
-                                               typename CsrStreamOf<double, LONG>::Stage& sm,
+                                               bool restart, typename StageOf<double, FMT, LONG>::T& sm,
                                                double* red /* 3*kWaves */)
 {
     const int G = a.G;
@@ -403,7 +442,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(MatView A, ResArgs<OUT_T> a
                                                      Ctrl* __restrict__ cout)
 {
     Ctrl c = read_ctrl(cin);
-    __shared__ typename CsrStreamOf<double, LONG>::Stage sm;
+    __shared__ typename StageOf<double, FMT, LONG>::T sm;
     __shared__ double red[3 * kWaves];
     residual_block<OUT_T, FMT, HALO, false, LONG>(A, a, logical_block(), false, sm, red);
     c.reduce = kReduceSetup;
@@ -419,8 +458,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(MatView A, ResArgs<OUT_T> a
 // grids (600k-row mesh solve 9.13 against 8.80 ms).
 template <int FMT, bool LONG>
 __device__ __forceinline__ void replace_residual(const MatView& A, const ResArgs<float>& a, Ctrl& c,
-                                                 const Prm& P,
-                                                 typename CsrStreamOf<double, LONG>::Stage& sm,
+                                                 const Prm& P, typename StageOf<double, FMT, LONG>::T& sm,
                                                  double* red)
 {
     for (int vb = blockIdx.x; vb < a.G; vb += gridDim.x) {
@@ -501,6 +539,12 @@ __device__ __forceinline__ void next_scalars(Ctrl& c, double rz, double rr, cons
     }
 }
 
+// Tile groups a row-class K1 sums per step.  Measured on the 256^3 Poisson
+// block, time per iteration with 1 / 2 / 3 groups: mixed 163 / 158 / 158 us,
+// FP64 371 / 352 / 346; 100^3 mixed 24.7 / 24.3 / 25.7, FP64 30.2 / 30.0 /
+// 33.4.
+constexpr int kClassGroups = 2;
+
 // What the tile walk of a K1 does with the rows besides the product: nothing,
 // or (k_pcg_step) p_new and x += sigma p of the thread's rows.
 template <typename VT>
@@ -518,11 +562,12 @@ struct StepRows {
 // 12.3 us per iteration.)
 template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, typename X>
 __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __restrict__ v,
-                                           typename CsrStreamOf<VT, LONG>::Stage& sm,
-                                           const StepRows<VT>& st)
+                                           typename StageOf<VT, FMT, LONG>::T& sm,
+                                           const StepRows<VT>& st, int walk = 0)
 {
     const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
     double acc = 0.0;
+    static_assert(!(STEP && FMT == kFmtClass), "large systems only");
     // one finished row: its value, and in a step its direction and x
     auto finish = [&](int row, VT s, const typename X::Raw& raw, VT xo) {
         const VT d = x.value(raw);
@@ -596,6 +641,31 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
             }
             cs.advance(nxt, sm);
             if (row < A.n) finish(row, s, pr, xo);
+        }
+    } else if constexpr (FMT == kFmtClass) {
+        // a row is one byte and its gathers, so a step is one round trip to
+        // the caches whatever it holds: kClassGroups groups of tiles per step
+        load_classes<VT>(A, sm);
+        constexpr int NG = kClassGroups, R = kTileGroup * NG;
+        const long long ngroups = (ntiles + kTileGroup - 1) / kTileGroup, G = gridDim.x;
+        for (long long q = walk; q < ngroups; q += NG * G) {
+            int r[R];
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const long long t = kTileGroup * (q + (k / kTileGroup) * G) + k % kTileGroup;
+                r[k] = t < ntiles ? (int)t * kTileRows + threadIdx.x : A.n;
+            }
+            if (r[0] < A.n) {
+                VT s[R];
+                typename X::Raw pr[R];
+                class_rows<VT, R>(A.n, A.nd, A.doff, A.cls, sm, r, x, s, pr, A.dzero);
+#pragma unroll
+                for (int k = 0; k < R; ++k)
+                    if (r[k] < A.n) {
+                        const typename X::Raw pk = A.dzero >= 0 ? pr[k] : x.load(r[k]);
+                        finish(r[k], VT(0) + s[k], pk, VT(0));
+                    }
+            }
         }
     } else if constexpr (FMT == CEL_FMT_DIA) {
         // all tiles of a group per step, one row of each per thread; the
@@ -709,10 +779,10 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
 
 // LDS of a K1: its tile stage; in the mixed form the FP64 stage of a
 // replacement residual takes the same place.
-template <typename VT, bool LONG>
+template <typename VT, int FMT, bool LONG>
 union K1Stage {
-    typename CsrStreamOf<VT, LONG>::Stage tile;
-    typename CsrStreamOf<double, LONG>::Stage res;
+    typename StageOf<VT, FMT, LONG>::T tile;
+    typename StageOf<double, FMT, LONG>::T res;
 };
 
 // K1: v = A p, per-block partial of v.p.  Mixed: a requested replacement
@@ -726,7 +796,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                                                      Ctrl* __restrict__ cout, Prm P)
 {
     constexpr bool MIXED = sizeof(VT) == 4;
-    __shared__ K1Stage<VT, LONG> sm;
+    __shared__ K1Stage<VT, FMT, LONG> sm;
     __shared__ double red[3 * kWaves];
     __shared__ double bcast;
     Ctrl c = read_ctrl(cin);
@@ -742,9 +812,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             return;
         }
     }
-    const double acc = k1_tiles<VT, FMT, HALO, LONG, false>(A, XPlain<VT>{p}, v, sm.tile, StepRows<VT>{});
+    // the walk (first group, and the partial's slot) of this block: by classes
+    // it may be another block's
+    int walk = blockIdx.x, slot = logical_block();
+    if constexpr (FMT == kFmtClass) {
+        if (A.walk) {
+            walk = A.walk[blockIdx.x];
+            slot = gridDim.x % kXcds ? walk : (walk % kXcds) * (gridDim.x / kXcds) + walk / kXcds;
+        }
+    }
+    const double acc = k1_tiles<VT, FMT, HALO, LONG, false>(A, XPlain<VT>{p}, v, sm.tile, StepRows<VT>{}, walk);
     const double bs = block_sum(acc, red);
-    if (threadIdx.x == 0) part[logical_block()] = bs;
+    if (threadIdx.x == 0) part[slot] = bs;
     write_ctrl(cout, c);
 }
 
@@ -767,7 +846,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     Ctrl* __restrict__ cout, Prm P)
 {
     constexpr bool MIXED = sizeof(VT) == 4;
-    __shared__ K1Stage<VT, LONG> sm;
+    __shared__ K1Stage<VT, FMT, LONG> sm;
     __shared__ double red[3 * kWaves];
     __shared__ double bcast[2];
     Ctrl c = read_ctrl(cin);
@@ -860,6 +939,45 @@ __device__ __forceinline__ void set_lane(typename Vec<VT>::T& a, int k, VT v)
     }
 }
 
+// The Jacobi values of W consecutive elements: from the vector, or (CLS)
+// from the rows' classes and their table in LDS.
+template <typename VT, bool CLS>
+struct JacOf {
+    using Raw = typename Vec<VT>::T;
+    const VT* jac;
+    __device__ __forceinline__ Raw load(long long i) const { return *reinterpret_cast<const Raw*>(jac + i); }
+    __device__ __forceinline__ VT value(const Raw& r, int k) const { return lane<VT>(r, k); }
+    __device__ __forceinline__ VT at(long long i) const { return jac[i]; }
+};
+template <typename VT>
+struct JacOf<VT, true> {
+    using Raw = unsigned;  // W class bytes
+    const uint8_t* cls;
+    const VT* tab;
+    __device__ __forceinline__ Raw load(long long i) const
+    {
+        if constexpr (Vec<VT>::W == 2) return *reinterpret_cast<const uint16_t*>(cls + i);
+        else return *reinterpret_cast<const uint32_t*>(cls + i);
+    }
+    __device__ __forceinline__ VT value(Raw r, int k) const { return tab[(r >> (8 * k)) & 255u]; }
+    __device__ __forceinline__ VT at(long long i) const { return tab[cls[i]]; }
+};
+
+// (CLS) the table to LDS; every thread of the block; it synchronises
+template <typename VT, bool CLS>
+__device__ __forceinline__ JacOf<VT, CLS> jac_of(const VT* __restrict__ jac, const uint8_t* __restrict__ cls,
+                                                 VT* lds)
+{
+    if constexpr (CLS) {
+        lds[threadIdx.x] = jac[threadIdx.x];  // kMaxClass == kBlock
+        __syncthreads();
+        return JacOf<VT, true>{cls, lds};
+    } else {
+        return JacOf<VT, false>{jac};
+    }
+}
+static_assert(kMaxClass == kBlock, "one table entry per thread");
+
 // Whole 16-byte units per thread and loop step in the vector kernels (all
 // their loads in flight together).  Measured on the 256^3 solves (two
 // interleaved repetitions, one box): FP32 4 (mixed CSR 304-305 ms against
@@ -870,10 +988,11 @@ constexpr int kVecUnrollOf = sizeof(VT) == 4 ? 4 : 2;
 
 // K2: sigma = alpha / sum(v.p) ; r = r + (-sigma) v ; z = jac*r ;
 // per-block partials of r.z and r.r.  ZOUT: z is stored too (for k_pcg_step).
-template <typename VT, bool ZOUT>
+template <typename VT, bool ZOUT, bool CLS>
 __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __restrict__ r,
                                                          const VT* __restrict__ v,
                                                          const VT* __restrict__ jac,
+                                                         const uint8_t* __restrict__ cls,
                                                          VT* __restrict__ z,
                                                          double* __restrict__ part,
                                                          const double* __restrict__ vpart, int G1,
@@ -907,18 +1026,21 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
         return;
     }
     c.sigma = sigma;
+    __shared__ VT jlds[CLS ? kMaxClass : 1];
+    const auto J = jac_of<VT, CLS>(jac, cls, jlds);
     const VT ms = VT(-sigma);
     double arz = 0.0, arr = 0.0;
     constexpr int kVecUnroll = kVecUnrollOf<VT>;
     // kVecUnroll units per step while they are whole vectors (all their
     // loads in flight together), added to the partials in unit order
     for (; i + (kVecUnroll - 1) * unit + W <= hi; i += kVecUnroll * unit) {
-        V vv[kVecUnroll], rv[kVecUnroll], jv[kVecUnroll];
+        V vv[kVecUnroll], rv[kVecUnroll], zv[kVecUnroll];
+        typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
 #pragma unroll
         for (int u = 0; u < kVecUnroll; ++u) {
             vv[u] = *reinterpret_cast<const V*>(v + i + u * unit);
             rv[u] = *reinterpret_cast<const V*>(r + i + u * unit);
-            jv[u] = *reinterpret_cast<const V*>(jac + i + u * unit);
+            jv[u] = J.load(i + u * unit);
         }
 #pragma unroll
         for (int u = 0; u < kVecUnroll; ++u) {
@@ -927,42 +1049,43 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
                 VT t = ms * lane<VT>(vv[u], k);
                 VT ri = lane<VT>(rv[u], k) + t;
                 set_lane<VT>(rv[u], k, ri);
-                VT zi = ri * lane<VT>(jv[u], k);
-                if constexpr (ZOUT) set_lane<VT>(jv[u], k, zi);
+                VT zi = ri * J.value(jv[u], k);
+                if constexpr (ZOUT) set_lane<VT>(zv[u], k, zi);
                 double rz = double(ri) * double(zi);
                 arz = arz + rz;
                 double rr = double(ri) * double(ri);
                 arr = arr + rr;
             }
             *reinterpret_cast<V*>(r + i + u * unit) = rv[u];
-            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i + u * unit) = jv[u];
+            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i + u * unit) = zv[u];
         }
     }
     for (; i < hi; i += unit) {
         if (i + W <= n) {
             const V vv = *reinterpret_cast<const V*>(v + i);
             V rv = *reinterpret_cast<const V*>(r + i);
-            V jv = *reinterpret_cast<const V*>(jac + i);
+            const auto jv = J.load(i);
+            V zv{};
 #pragma unroll
             for (int k = 0; k < W; ++k) {
                 VT t = ms * lane<VT>(vv, k);
                 VT ri = lane<VT>(rv, k) + t;
                 set_lane<VT>(rv, k, ri);
-                VT zi = ri * lane<VT>(jv, k);
-                if constexpr (ZOUT) set_lane<VT>(jv, k, zi);
+                VT zi = ri * J.value(jv, k);
+                if constexpr (ZOUT) set_lane<VT>(zv, k, zi);
                 double rz = double(ri) * double(zi);
                 arz = arz + rz;
                 double rr = double(ri) * double(ri);
                 arr = arr + rr;
             }
             *reinterpret_cast<V*>(r + i) = rv;
-            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i) = jv;
+            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i) = zv;
         } else {
             for (long long j = i; j < hi; ++j) {
                 VT t = ms * v[j];
                 VT ri = r[j] + t;
                 r[j] = ri;
-                VT zi = ri * jac[j];
+                VT zi = ri * J.at(j);
                 if constexpr (ZOUT) z[j] = zi;
                 double rz = double(ri) * double(zi);
                 arz = arz + rz;
@@ -982,11 +1105,12 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
 // K3: beta = sum(r.z)/alpha ; x = x + sigma p ; p = beta p + jac*r ;
 // alpha = r.z, norm2, k++, history, loop decision (FP64) or replacement
 // request (mixed).
-template <typename VT, typename XT, bool MIXED>
+template <typename VT, typename XT, bool MIXED, bool CLS>
 __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __restrict__ x,
                                                           VT* __restrict__ p,
                                                           const VT* __restrict__ r,
                                                           const VT* __restrict__ jac,
+                                                          const uint8_t* __restrict__ cls,
                                                           double* __restrict__ x64,
                                                           const double* __restrict__ rpart, int G2,
                                                           const Ctrl* __restrict__ cin,
@@ -1009,6 +1133,8 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
     // FP64 solution here (x64 = x64 + e, e = 0) instead of in a kernel of
     // its own; same arithmetic
     const bool flush = MIXED && c.ru;
+    __shared__ VT jlds[CLS ? kMaxClass : 1];
+    const auto J = jac_of<VT, CLS>(jac, cls, jlds);
     using V = typename Vec<VT>::T;
     constexpr int W = Vec<VT>::W;
     const int lb = logical_block();
@@ -1020,13 +1146,14 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
     long long i = lo + (long long)threadIdx.x * W;
     // kVecUnroll units per step while they are whole vectors
     for (; i + (kVecUnroll - 1) * unit + W <= hi; i += kVecUnroll * unit) {
-        V pv[kVecUnroll], rv[kVecUnroll], jv[kVecUnroll];
+        V pv[kVecUnroll], rv[kVecUnroll];
+        typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
         XT xs[kVecUnroll][W];
 #pragma unroll
         for (int u = 0; u < kVecUnroll; ++u) {
             pv[u] = *reinterpret_cast<const V*>(p + i + u * unit);
             rv[u] = *reinterpret_cast<const V*>(r + i + u * unit);
-            jv[u] = *reinterpret_cast<const V*>(jac + i + u * unit);
+            jv[u] = J.load(i + u * unit);
 #pragma unroll
             for (int k = 0; k < W; ++k) xs[u][k] = x[i + u * unit + k];
         }
@@ -1037,7 +1164,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
                 const VT pi = lane<VT>(pv[u], k);
                 XT t = XT(sigma * pi);
                 xs[u][k] = xs[u][k] + t;
-                VT zi = lane<VT>(rv[u], k) * lane<VT>(jv[u], k);
+                VT zi = lane<VT>(rv[u], k) * J.value(jv[u], k);
                 VT bp = beta * pi;
                 set_lane<VT>(pv[u], k, bp + zi);
             }
@@ -1058,7 +1185,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
         if (i + W <= n) {
             V pv = *reinterpret_cast<const V*>(p + i);
             const V rv = *reinterpret_cast<const V*>(r + i);
-            const V jv = *reinterpret_cast<const V*>(jac + i);
+            const auto jv = J.load(i);
             XT xs[W];
 #pragma unroll
             for (int k = 0; k < W; ++k) xs[k] = x[i + k];
@@ -1067,7 +1194,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
                 const VT pi = lane<VT>(pv, k);
                 XT t = XT(sigma * pi);
                 xs[k] = xs[k] + t;
-                VT zi = lane<VT>(rv, k) * lane<VT>(jv, k);
+                VT zi = lane<VT>(rv, k) * J.value(jv, k);
                 VT bp = beta * pi;
                 set_lane<VT>(pv, k, bp + zi);
             }
@@ -1093,7 +1220,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
                     xj = XT(0);
                 }
                 x[j] = xj;
-                VT zi = r[j] * jac[j];
+                VT zi = r[j] * J.at(j);
                 VT bp = beta * pi;
                 p[j] = bp + zi;
             }
@@ -1128,6 +1255,7 @@ struct Workspace {
     DevBuf<float> p2_32, z32;
     // JAD solves: b, x and the Jacobi vector in the permuted row order
     DevBuf<double> bp, xp, jacp;
+    DevBuf<int> walk;  // row-class solves: the K1 blocks' walks
     // halo solves: per-row halo records {count, p1, p2, p3}
     DevBuf<double> hrec;
     DevBuf<float> jacp32;
@@ -1200,6 +1328,7 @@ template <typename VT>
 static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr)
 {
     if (fmt == CEL_FMT_JAD) return k_pcg_spmv<VT, CEL_FMT_JAD, false, false>;
+    if (fmt == kFmtClass) return k_pcg_spmv<VT, kFmtClass, false, false>;
     if constexpr (sizeof(VT) == 8) {  // halo blocks: FP64 only
         if (halo && fmt == CEL_FMT_DIA) return k_pcg_spmv<VT, CEL_FMT_DIA, true, false>;
         if (halo) return lr ? k_pcg_spmv<VT, CEL_FMT_CSR, true, true> : k_pcg_spmv<VT, CEL_FMT_CSR, true, false>;
@@ -1258,6 +1387,7 @@ template <typename OUT_T>
 static ResFn<OUT_T> res_kernel(int fmt, bool halo, bool lr)
 {
     if (fmt == CEL_FMT_JAD) return k_residual<OUT_T, CEL_FMT_JAD, false, false>;
+    if (fmt == kFmtClass) return k_residual<OUT_T, kFmtClass, false, false>;
     if constexpr (sizeof(OUT_T) == 8)
         if (halo)
             return lr ? k_residual<OUT_T, CEL_FMT_CSR, true, true> : k_residual<OUT_T, CEL_FMT_CSR, true, false>;
@@ -1377,6 +1507,33 @@ int pcg_spmv_dot(Mat& A, int fmt, const double* x, const double* ghost, double* 
     return CEL_OK;
 }
 
+// The walks of a row-class K1's blocks: the walks whose groups start in the
+// same eighth of the matrix's period (its farthest diagonal) go to one XCD,
+// so the rows a tile gathers from the planes beside it, and all but the
+// outermost of its own plane's neighbours, are in that XCD's L2.  Each block
+// keeps its walk's slot, so the partials are the same.  Measured per
+// iteration: mixed 100^3 27.0 -> 24.3 us, 200^3 82.0 -> 80.2; FP64 256^3
+// 357 -> 351.
+static int class_walk(const Mat& A, Workspace& W, int G, const int** walk)
+{
+    *walk = nullptr;
+    const Derived& D = A.derived;
+    const int far = std::max(std::abs(D.off[0]), std::abs(D.off[D.nd - 1]));
+    const int period = std::max(1, (far + kTileGroup * kTileRows / 2) / (kTileGroup * kTileRows));
+    if (G % kXcds || period < 2 * kXcds) return CEL_OK;
+    std::vector<int> order(G), w(G);
+    for (int b = 0; b < G; ++b) order[b] = b;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+        return (long long)(a % period) * kXcds / period < (long long)(b % period) * kXcds / period;
+    });
+    for (int h = 0; h < G; ++h) w[h] = order[(h % kXcds) * (G / kXcds) + h / kXcds];
+    CEL_TRY(W.walk.reserve(G));
+    CEL_HIP(hipMemcpyAsync(W.walk.p, w.data(), sizeof(int) * G, hipMemcpyHostToDevice, rt().stream));
+    CEL_HIP(hipStreamSynchronize(rt().stream));
+    *walk = W.walk.p;
+    return CEL_OK;
+}
+
 int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel_pcg_stats& stats,
               double* hist, bool noalloc)
 {
@@ -1462,6 +1619,13 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         if (Gv >= kXcds) Gv = Gv / kXcds * kXcds;
     }
 
+    // the form the K1s run on, and its residual's: the caller's, or a derived
+    // one with the same bits (its grids are the caller's form's)
+    int use = Derived::kNone;
+    if (!noalloc && !halo && !coo && fmt != CEL_FMT_JAD) use = derived_prepare(A, fmt, mixed, prm.iter_max);
+    const int kfmt = use == Derived::kClasses ? kFmtClass : use == Derived::kDiagonals ? CEL_FMT_DIA : fmt;
+    const int kres = use == Derived::kClasses ? kFmtClass : rfmt;
+
     if (noalloc && ((size_t)G1 > kNoAllocMaxGrid || (size_t)Gr > kNoAllocMaxGrid ||
                     (size_t)Gv > kNoAllocMaxGrid))
         return fail(CEL_ERR_ARG, "the allocation-free solve holds at most " +
@@ -1469,10 +1633,10 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
 
     // matrix data for the mixed inner operator (once per matrix)
     if (mixed) {
-        if (fmt == CEL_FMT_DIA) CEL_TRY(dia_prepare_f32(A));
+        if (fmt == CEL_FMT_DIA && kfmt == CEL_FMT_DIA) CEL_TRY(dia_prepare_f32(A));
         // the DIA K1 reads dia_vals32 and the residual kernels the FP64 CSR
         // values, so only a CSR solve needs the FP32 CSR copy
-        if (fmt == CEL_FMT_CSR && !A.vals32.p) {
+        if (kfmt == CEL_FMT_CSR && !A.vals32.p) {
             CEL_TRY(A.vals32.alloc(A.nnz > 0 ? A.nnz : 1));
             CEL_TRY(launch_to_f32(A.vals.p, A.vals32.p, A.nnz));
         }
@@ -1525,7 +1689,8 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     }
     // two kernels per iteration on small systems; the halo blocks need a
     // stored direction before the product, profiling a product of its own
-    const bool step = !noalloc && !halo && !prm.profile && step_form(A, fmt, mixed);
+    const bool step = !noalloc && !halo && !prm.profile && use == Derived::kNone &&
+                      step_form(A, fmt, mixed);
     double *pbuf[2] = {w.p, nullptr}, *zbuf = nullptr;
     float *pbuf32[2] = {w.p32, nullptr}, *zbuf32 = nullptr;
     if (step) {
@@ -1619,10 +1784,23 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     V.dmask = A.dia_mask.p;
     V.dmask8 = A.dia_mask8.p;
     V.nd = A.dia_nd;
+    const int* doff = A.dia_off;
+    if (use != Derived::kNone) {
+        const Derived& D = A.derived;
+        V.nd = D.nd;
+        doff = D.off;
+        V.cls = D.cls.p;
+        V.ctab = D.classes();
+        V.dvals = D.vals.p;
+        V.dvals32 = D.vals32.p;
+        V.dmask = nullptr;
+        V.dmask8 = D.mask8.p;
+    }
+    if (use == Derived::kClasses) CEL_TRY(class_walk(A, *Wp, G1, &V.walk));
     V.dzero = -1;
-    for (int d = 0; d < A.dia_nd; ++d) {
-        V.doff[d] = A.dia_off[d];
-        if (A.dia_off[d] == 0) V.dzero = d;
+    for (int d = 0; d < V.nd; ++d) {
+        V.doff[d] = doff[d];
+        if (doff[d] == 0) V.dzero = d;
     }
     if (halo) {
         V.hrow_tile = Wp->hrow_tile.p;
@@ -1678,9 +1856,9 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     const ResArgs<double> R64{dx, db, jac64, nullptr, w.r, w.p, nullptr, w.rpart, Gr};
     const ResArgs<float> R32{dx, db, nullptr, jac32, w.r32, w.p32, w.e32, w.rpart, Gr};
     if (!mixed)
-        hipLaunchKernelGGL(res_kernel<double>(rfmt, halo, lr), dim3(Gr), dim3(kBlock), 0, s, V, R64, C0, C0);
+        hipLaunchKernelGGL(res_kernel<double>(kres, halo, lr), dim3(Gr), dim3(kBlock), 0, s, V, R64, C0, C0);
     else
-        hipLaunchKernelGGL(res_kernel<float>(rfmt, false, lr), dim3(Gr), dim3(kBlock), 0, s, V, R32, C0, C0);
+        hipLaunchKernelGGL(res_kernel<float>(kres, false, lr), dim3(Gr), dim3(kBlock), 0, s, V, R32, C0, C0);
     CEL_HIP(hipGetLastError());
     if (!noalloc) CEL_HIP(hipEventRecord(e1, s));
 
@@ -1697,6 +1875,11 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     };
 
     const long long n_ll = n;
+    // the vector kernels' Jacobi values: the vector, or the classes' table
+    const bool bycls = use == Derived::kClasses;
+    const double* vjac64 = bycls ? V.ctab.jac64 : jac64;
+    const float* vjac32 = bycls ? V.ctab.jac32 : jac32;
+    const uint8_t *vcls = bycls ? V.cls : nullptr, *nocls = nullptr;
     // One slot of the two-kernel form: the step finishes the iteration before
     // (its vectors and scalars) and forms the next product, K2 updates r.
     // The direction alternates between two buffers by slot.
@@ -1706,16 +1889,16 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             hipLaunchKernelGGL(step_kernel<double>(fmt, lr), dim3(G1), dim3(kBlock), 0, s, V,
                                (const double*)pbuf[in], (const double*)zbuf, pbuf[out], dx, (double*)nullptr, w.v,
                                w.part1, R64, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
-            hipLaunchKernelGGL((k_pcg_update_r<double, true>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
-                               jac64, zbuf, w.part2, w.part1, G1, C1, C0);
+            hipLaunchKernelGGL((k_pcg_update_r<double, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
+                               jac64, nocls, zbuf, w.part2, w.part1, G1, C1, C0);
         } else {
             ResArgs<float> R = R32;
             R.p = pbuf32[out];  // a restart's direction
             hipLaunchKernelGGL(step_kernel<float>(fmt, lr), dim3(G1), dim3(kBlock), 0, s, V,
                                (const float*)pbuf32[in], (const float*)zbuf32, pbuf32[out], w.e32, dx, w.v32,
                                w.part1, R, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
-            hipLaunchKernelGGL((k_pcg_update_r<float, true>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
-                               jac32, zbuf32, w.part2, w.part1, G1, C1, C0);
+            hipLaunchKernelGGL((k_pcg_update_r<float, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
+                               jac32, nocls, zbuf32, w.part2, w.part1, G1, C1, C0);
         }
         CEL_HIP(hipGetLastError());
         return CEL_OK;
@@ -1738,21 +1921,23 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             CEL_HIP(hipEventRecord(ea, s));
         }
         if (!mixed) {
-            hipLaunchKernelGGL(k1_kernel<double>(fmt, halo, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
+            hipLaunchKernelGGL(k1_kernel<double>(kfmt, halo, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
                                w.part1, R64, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
-            hipLaunchKernelGGL((k_pcg_update_r<double, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
-                               jac64, (double*)nullptr, w.part2, w.part1, G1, C1, C2);
-            hipLaunchKernelGGL((k_pcg_update_xp<double, double, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll,
-                               dx, w.p, w.r, jac64, nullptr, w.part2, Gv, C2, C0, P);
+            hipLaunchKernelGGL((bycls ? k_pcg_update_r<double, false, true> : k_pcg_update_r<double, false, false>),
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v, vjac64, vcls, (double*)nullptr, w.part2, w.part1, G1, C1, C2);
+            hipLaunchKernelGGL((bycls ? k_pcg_update_xp<double, double, false, true>
+                                      : k_pcg_update_xp<double, double, false, false>),
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, dx, w.p, w.r, vjac64, vcls, nullptr, w.part2, Gv, C2, C0, P);
         } else {
-            hipLaunchKernelGGL(k1_kernel<float>(fmt, false, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
+            hipLaunchKernelGGL(k1_kernel<float>(kfmt, false, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
                                w.part1, R32, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
-            hipLaunchKernelGGL((k_pcg_update_r<float, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
-                               jac32, (float*)nullptr, w.part2, w.part1, G1, C1, C2);
-            hipLaunchKernelGGL((k_pcg_update_xp<float, float, true>), dim3(Gv), dim3(kBlock), 0, s, n_ll,
-                               w.e32, w.p32, w.r32, jac32, dx, w.part2, Gv, C2, C0, P);
+            hipLaunchKernelGGL((bycls ? k_pcg_update_r<float, false, true> : k_pcg_update_r<float, false, false>),
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32, vjac32, vcls, (float*)nullptr, w.part2, w.part1, G1, C1, C2);
+            hipLaunchKernelGGL((bycls ? k_pcg_update_xp<float, float, true, true>
+                                      : k_pcg_update_xp<float, float, true, false>),
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.e32, w.p32, w.r32, vjac32, vcls, dx, w.part2, Gv, C2, C0, P);
         }
         CEL_HIP(hipGetLastError());
         return CEL_OK;
@@ -1871,13 +2056,16 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     stats.spmv_ms = spmv_ms;
     stats.spmv_launches = spmv_n;
     const int prec = mixed ? CEL_PREC_MIXED : CEL_PREC_FP64;
+    const double vb = mixed ? 4.0 : 8.0;
     stats.spmv_bytes = spmv_bytes(A, fmt, prec);
     if (jadp) stats.spmv_bytes -= 4.0 * n;  // the permuted-order K1 reads no permutation
+    // a derived form: a class or mask byte per row, the diagonals' values, p and v
+    if (use != Derived::kNone) stats.spmv_bytes = (1.0 + (bycls ? 2.0 : 2.0 + V.nd) * vb) * n;
     {
-        const double vb = mixed ? 4.0 : 8.0;
         // K1 matrix + p gather + v write ; K2 r,v,jac read + r write ;
         // K3 p,r,jac,x read + p,x write
-        stats.iter_bytes = stats.spmv_bytes + vb * n * 4.0 + vb * n * 6.0 +
+        // (by classes: a byte for the Jacobi value in each)
+        stats.iter_bytes = stats.spmv_bytes + vb * n * 4.0 + vb * n * 6.0 - (bycls ? 2.0 * (vb - 1.0) * n : 0.0) +
                            (halo ? 20.0 * A.send_total + 12.0 * A.ghost_len : 0.0);
     }
     if (out.status != 0) {

@@ -1,0 +1,366 @@
+// rowclass.hip -- derived forms of a block's CSR arrays for long solves (no
+// reference counterpart).
+//
+// A solve reads its matrix hundreds of times, and the matrices of structured
+// grids repeat themselves: the rows of a constant-coefficient stencil on a
+// box differ only by which neighbours exist (27 kinds of row for 7 points),
+// piecewise constant coefficients add one kind per material boundary.  A
+// block whose entries lie on at most 8 diagonals and whose rows take at
+// most 256 different forms (offsets, value bits, Jacobi value) is kept as
+// one byte per row and a table of the forms: the product then reads 1 byte
+// per row instead of 84 (FP64 CSR) or 57 (DIA), and the vector kernels take
+// the Jacobi value from the table too.  A block on at most 8 diagonals with
+// more forms than that (variable coefficients) is kept in diagonal storage,
+// as cel_gpu_mat_to_dia builds it, for solves that asked for CSR.
+//
+// Both forms visit a row's entries in the CSR column order with the same
+// values, so the sums are the CSR sums bit for bit.  The table is verified
+// entry by entry against the matrix (the 64-bit keys only find candidates).
+// They are built on the first long solve of a matrix (rule at
+// derived_prepare), belong to the handle, and are dropped when the values,
+// the Jacobi vector or the scaling change.  A matrix they do not fit costs
+// one pass that stops early; without memory for them the solve runs on the
+// CSR arrays.
+#include <algorithm>
+
+#include "cel_internal.hpp"
+#include "device_common.hpp"
+#include "spmv_device.hpp"
+
+namespace cel {
+namespace {
+
+constexpr int kKeySlots = 1024;  // open addressing, at most 256 keys
+constexpr int kProbes = 32;
+constexpr int kNear = 512;       // keys a block remembers (direct mapped)
+
+struct KeyTable {
+    unsigned long long key[kKeySlots];  // 0: free
+    int cls[kKeySlots];
+    int row[kMaxClass];                 // a row of each class
+    int count;
+    int over;  // more than kMaxClass classes, or a row that has no form
+    int bad;   // a row that differs from its class (keys collided)
+};
+
+struct Offs {
+    int nd;
+    int off[kClassDiag];
+};
+
+__device__ __forceinline__ unsigned long long mix(unsigned long long h)
+{
+    h ^= h >> 30;
+    h *= 0xbf58476d1ce4e5b9ull;
+    h ^= h >> 27;
+    h *= 0x94d049bb133111ebull;
+    return h ^ (h >> 31);
+}
+
+// A row's entries by diagonal, and its key (never 0).
+struct RowForm {
+    unsigned mask;
+    double v[kClassDiag];
+    unsigned long long key;
+};
+
+// false: the row has more entries than diagonals (a repeated column)
+__device__ __forceinline__ bool row_form(long long i, const int* __restrict__ xadj,
+                                         const int* __restrict__ cols,
+                                         const double* __restrict__ vals, double jac, const Offs& O,
+                                         RowForm& f)
+{
+    const int lo = xadj[i], len = xadj[i + 1] - lo;
+    f.mask = 0;
+#pragma unroll
+    for (int d = 0; d < kClassDiag; ++d) f.v[d] = 0.0;
+    if (len > O.nd) return false;
+    int c[kClassDiag];
+    double a[kClassDiag];
+#pragma unroll
+    for (int k = 0; k < kClassDiag; ++k) {
+        c[k] = k < len ? cols[lo + k] - (int)i : 0;
+        a[k] = k < len ? vals[lo + k] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < kClassDiag; ++k)
+#pragma unroll
+        for (int d = 0; d < kClassDiag; ++d)
+            if (k < len && d < O.nd && c[k] == O.off[d]) {
+                f.mask |= 1u << d;
+                f.v[d] = a[k];
+            }
+    unsigned long long h = mix(f.mask + 0x9e3779b97f4a7c15ull);
+#pragma unroll
+    for (int d = 0; d < kClassDiag; ++d)
+        h = mix(h + __builtin_bit_cast(unsigned long long, f.v[d]) + (unsigned long long)d);
+    h = mix(h + __builtin_bit_cast(unsigned long long, jac));
+    f.key = h ? h : 1;
+    return true;
+}
+
+__global__ void __launch_bounds__(kBlock) k_keys_clear(KeyTable* T)
+{
+    for (int i = threadIdx.x; i < kKeySlots; i += kBlock) {
+        T->key[i] = 0;
+        T->cls[i] = -1;
+    }
+    if (threadIdx.x == 0) T->count = T->over = T->bad = 0;
+}
+
+// Classes of the rows: one thread per row puts its key into the table
+// unless the block has met it before.  Bound by one read of the matrix; it
+// stops as soon as there are too many classes.
+__global__ void __launch_bounds__(kBlock)
+k_class_scan(int n, const int* __restrict__ xadj, const int* __restrict__ cols,
+             const double* __restrict__ vals, const double* __restrict__ jac, Offs O, KeyTable* T)
+{
+    __shared__ unsigned long long near_key[kNear];
+    __shared__ int stop;
+    for (int i = threadIdx.x; i < kNear; i += kBlock) near_key[i] = 0;
+    __syncthreads();
+    for (long long i0 = (long long)blockIdx.x * kBlock; i0 < n; i0 += (long long)gridDim.x * kBlock) {
+        const long long i = i0 + threadIdx.x;
+        if (i < n) {
+            RowForm f;
+            if (!row_form(i, xadj, cols, vals, jac[i], O, f)) {
+                atomicOr(&T->over, 1);
+            } else {
+                const int at = (int)(f.key % kNear);
+                if (near_key[at] != f.key && !*(volatile int*)&T->over) {
+                    bool found = false;
+                    int s = (int)(f.key >> 32) & (kKeySlots - 1);
+                    for (int k = 0; k < kProbes && !found; ++k, s = (s + 1) & (kKeySlots - 1)) {
+                        // (a plain look first: atomics of every row on the same
+                        // few keys took 11 ms on the 256^3 block)
+                        unsigned long long old = T->key[s];
+                        if (old == 0) old = atomicCAS(&T->key[s], 0ull, f.key);
+                        if (old == 0) {
+                            const int id = atomicAdd(&T->count, 1);
+                            if (id < kMaxClass) {
+                                T->row[id] = (int)i;
+                                T->cls[s] = id;
+                            } else {
+                                atomicOr(&T->over, 1);
+                            }
+                        }
+                        found = old == 0 || old == f.key;
+                    }
+                    if (!found) atomicOr(&T->over, 1);
+                    near_key[at] = f.key;
+                }
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) stop = *(volatile int*)&T->over;
+        __syncthreads();
+        if (stop) break;  // uniform
+    }
+}
+
+// The table of the forms: thread c writes class c.
+__global__ void __launch_bounds__(kBlock)
+k_class_table(int count, const KeyTable* __restrict__ T, const int* __restrict__ xadj,
+              const int* __restrict__ cols, const double* __restrict__ vals,
+              const double* __restrict__ jac, const float* __restrict__ jac32, Offs O,
+              RowClasses out)
+{
+    const int c = threadIdx.x;
+    RowForm f;
+    f.mask = 0;
+    double j64 = 0.0;
+    float j32 = 0.0f;
+#pragma unroll
+    for (int d = 0; d < kClassDiag; ++d) f.v[d] = 0.0;
+    if (c < count) {
+        const int i = T->row[c];
+        j64 = jac[i];
+        j32 = jac32[i];
+        (void)row_form(i, xadj, cols, vals, j64, O, f);
+    }
+#pragma unroll
+    for (int d = 0; d < kClassDiag; ++d) {
+        out.val64[c * kClassDiag + d] = f.v[d];
+        out.val32[c * kClassDiag + d] = (float)f.v[d];
+    }
+    out.mask[c] = f.mask;
+    out.jac64[c] = j64;
+    out.jac32[c] = j32;
+}
+
+// Every row's class, checked against the table bit for bit.
+__global__ void __launch_bounds__(kBlock)
+k_class_assign(int n, const int* __restrict__ xadj, const int* __restrict__ cols,
+               const double* __restrict__ vals, const double* __restrict__ jac,
+               const float* __restrict__ jac32, Offs O, KeyTable* T, RowClasses tab,
+               uint8_t* __restrict__ cls)
+{
+    __shared__ unsigned long long near_key[kNear];
+    __shared__ int near_cls[kNear];
+    for (int i = threadIdx.x; i < kNear; i += kBlock) near_key[i] = 0;
+    __syncthreads();
+    int any = 0;
+    for (long long i0 = (long long)blockIdx.x * kBlock; i0 < n; i0 += (long long)gridDim.x * kBlock) {
+        const long long i = i0 + threadIdx.x;
+        int id = -1;
+        RowForm f;
+        f.key = 0;
+        const double j = i < n ? jac[i] : 0.0;
+        if (i < n && row_form(i, xadj, cols, vals, j, O, f)) {
+            const int at = (int)(f.key % kNear);
+            if (near_key[at] == f.key) {
+                id = near_cls[at];
+            } else {
+                int s = (int)(f.key >> 32) & (kKeySlots - 1);
+                for (int k = 0; k < kProbes; ++k, s = (s + 1) & (kKeySlots - 1)) {
+                    if (T->key[s] != f.key) continue;
+                    id = T->cls[s];
+                    break;
+                }
+            }
+        }
+        __syncthreads();  // every lookup of the block is done
+        if (id >= 0) {  // the threads of one slot write whole pairs one after another, checked below
+            const int at = (int)(f.key % kNear);
+            near_key[at] = f.key;
+        }
+        __syncthreads();
+        if (id >= 0 && near_key[(int)(f.key % kNear)] == f.key) near_cls[(int)(f.key % kNear)] = id;
+        __syncthreads();
+        if (i >= n) continue;
+        bool same = id >= 0;
+        if (same) {
+            same = tab.mask[id] == f.mask &&
+                   __builtin_bit_cast(unsigned long long, tab.jac64[id]) == __builtin_bit_cast(unsigned long long, j) &&
+                   __builtin_bit_cast(unsigned, tab.jac32[id]) == __builtin_bit_cast(unsigned, jac32[i]);
+#pragma unroll
+            for (int d = 0; d < kClassDiag; ++d)
+                same = same && __builtin_bit_cast(unsigned long long, tab.val64[id * kClassDiag + d]) ==
+                                   __builtin_bit_cast(unsigned long long, f.v[d]);
+        }
+        if (!same) any = 1;
+        cls[i] = (uint8_t)(same ? id : 0);
+    }
+    if (any) atomicOr(&T->bad, 1);
+}
+
+int grid_of(long long n)
+{
+    const long long g = (n + kBlock - 1) / kBlock, cap = (long long)rt().num_cus * 16;
+    return (int)(g < 1 ? 1 : g > cap ? cap : g);
+}
+
+// The classes of A's rows into A.derived; *ok = false: the rows do not fit.
+int build_classes(Mat& A, const Offs& O, bool* ok)
+{
+    *ok = false;
+    Derived& D = A.derived;
+    hipStream_t st = rt().stream;
+    DevBuf<KeyTable> T;
+    CEL_TRY(T.alloc(1));
+    hipLaunchKernelGGL(k_keys_clear, dim3(1), dim3(kBlock), 0, st, T.p);
+    hipLaunchKernelGGL(k_class_scan, dim3(grid_of(A.n)), dim3(kBlock), 0, st, A.n, A.xadj.p, A.cols.p, A.vals.p,
+                       A.jac.p, O, T.p);
+    CEL_HIP(hipGetLastError());
+    int h[3];
+    CEL_HIP(hipMemcpyAsync(h, &T.p->count, sizeof(h), hipMemcpyDeviceToHost, st));
+    CEL_HIP(hipStreamSynchronize(st));
+    if (h[1] || h[0] > kMaxClass) return CEL_OK;
+    CEL_TRY(D.cls.alloc((size_t)A.n));
+    CEL_TRY(D.tab64.alloc((size_t)kMaxClass * (kClassDiag + 1)));
+    CEL_TRY(D.tab32.alloc((size_t)kMaxClass * (kClassDiag + 1)));
+    CEL_TRY(D.tabm.alloc(kMaxClass));
+    const RowClasses tab = D.classes();
+    hipLaunchKernelGGL(k_class_table, dim3(1), dim3(kBlock), 0, st, h[0], T.p, A.xadj.p, A.cols.p, A.vals.p,
+                       A.jac.p, A.jac32.p, O, tab);
+    hipLaunchKernelGGL(k_class_assign, dim3(grid_of(A.n)), dim3(kBlock), 0, st, A.n, A.xadj.p, A.cols.p, A.vals.p,
+                       A.jac.p, A.jac32.p, O, T.p, tab, D.cls.p);
+    CEL_HIP(hipGetLastError());
+    CEL_HIP(hipMemcpyAsync(h, &T.p->count, sizeof(h), hipMemcpyDeviceToHost, st));
+    CEL_HIP(hipStreamSynchronize(st));
+    *ok = !h[2];
+    return CEL_OK;
+}
+
+}  // namespace
+
+void Derived::release()
+{
+    kind = kNone;
+    tried = tried32 = tried64 = false;
+    nd = 0;
+    cls.release();
+    tab64.release();
+    tab32.release();
+    tabm.release();
+    vals.release();
+    vals32.release();
+    mask8.release();
+}
+
+// Which derived form a solve of A (CSR or DIA form, no halo blocks) runs on;
+// builds it on the first call that wants it.  Never fails: what cannot be
+// built is not used.
+int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max)
+{
+    Derived& D = A.derived;
+    // Smaller solves live in the caches and their iterations are launches;
+    // few iterations do not pay for the passes over the matrix.  Measured per
+    // iteration, CSR arrays / classes / diagonal storage: 64^3 FP64 17.2 /
+    // 17.0 / 17.1 us; 80^3 29.1 / 25.4 / 27.8, mixed 22.9 / 22.0 / 21.4;
+    // 100^3 39.6 / 30.0 / 36.4, mixed 31.8 / 24.3 / 28.4; 256^3 618 / 350 /
+    // 507, mixed 358 / 158 / 232.  Building takes 0.4 ms (100^3) to 1.3 ms
+    // (256^3), as much as 40 to 10 iterations save; a solve of such a block
+    // to 1e-10 takes 300 to 800.
+    if (A.n < kDerivedRows || (iter_max < 32 && !D.tried) || !A.jac.p || !A.jac32.p) return Derived::kNone;
+    const std::string err = last_error();
+    int rc = CEL_OK;
+    if (!D.tried) {
+        D.tried = true;
+        bool asc = false;
+        int nd = 0;
+        if (A.ncols == A.n && A.nnz > 0 && (long long)A.n * 8 < (1LL << 31))
+            rc = dia_offsets(A, kClassDiag, &nd, D.off, &asc);
+        if (rc == CEL_OK && asc && nd <= kClassDiag) {
+            D.nd = nd;
+            Offs O{};
+            O.nd = nd;
+            for (int d = 0; d < nd; ++d) O.off[d] = D.off[d];
+            bool ok = false;
+            rc = build_classes(A, O, &ok);
+            if (rc == CEL_OK && ok) D.kind = Derived::kClasses;
+        }
+        if (D.kind == Derived::kNone) {
+            D.cls.release();
+            D.tab64.release();
+            D.tab32.release();
+            D.tabm.release();
+        }
+    }
+    int use = D.kind;
+    if (use == Derived::kNone && fmt == CEL_FMT_CSR && D.nd > 0 && (long long)D.nd * A.n <= 2LL * A.nnz) {
+        // diagonal storage in the precision of the solve; the matrix's own
+        // DIA form, where the caller has built one, is the same
+        bool& tried = mixed ? D.tried32 : D.tried64;
+        const size_t cnt = (size_t)D.nd * (size_t)A.n;
+        if (!tried) {
+            tried = true;
+            rc = D.mask8.p ? CEL_OK : D.mask8.alloc((size_t)A.n);
+            if (rc == CEL_OK) rc = mixed ? D.vals32.alloc(cnt) : D.vals.alloc(cnt);
+            if (rc == CEL_OK)
+                rc = dia_fill(A, D.nd, D.off, mixed ? nullptr : D.vals.p, mixed ? D.vals32.p : nullptr, D.mask8.p);
+            if (rc != CEL_OK) {
+                if (mixed) D.vals32.release();
+                else D.vals.release();
+            }
+        }
+        if (D.mask8.p && (mixed ? (const void*)D.vals32.p : (const void*)D.vals.p)) use = Derived::kDiagonals;
+    }
+    if (rc != CEL_OK) {  // no memory: no error of the solve
+        set_error(err);
+        (void)hipGetLastError();
+    }
+    return use;
+}
+
+}  // namespace cel

@@ -256,6 +256,64 @@ __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const V
     }
 }
 
+// Row sums of a block kept as row classes (rowclass.hip): one byte per row
+// and, in LDS, the classes' values by diagonal and presence masks.  Rows,
+// order and x loads as dia_rows; the values come from the table, so a row
+// costs its byte and its gathers.
+template <typename VT>
+struct ClassTab {
+    VT val[kMaxClass * kClassDiag];
+    uint32_t mask[kMaxClass];
+    // every thread of the block; it synchronises
+    __device__ __forceinline__ void load(const VT* __restrict__ v, const uint32_t* __restrict__ m)
+    {
+        for (int i = threadIdx.x; i < kMaxClass * kClassDiag; i += kBlock) val[i] = v[i];
+        for (int i = threadIdx.x; i < kMaxClass; i += kBlock) mask[i] = m[i];
+        __syncthreads();
+    }
+};
+
+template <typename VT, int R, typename X>
+__device__ __forceinline__ void class_rows(int n, int nd, const int* doff, const uint8_t* __restrict__ cls,
+                                           const ClassTab<VT>& tab, const int (&r)[R], const X& x,
+                                           VT (&s)[R], typename X::Raw* xr = nullptr, int dzero = -1)
+{
+    constexpr int B = (int)sizeof(VT);
+    int rc[R], c[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        rc[k] = r[k] < n ? r[k] : r[0];
+        c[k] = cls[rc[k]];
+        s[k] = VT(0);
+    }
+    const auto rx = x.buf((unsigned)n * (unsigned)B);
+    typename X::Raw xv[kClassDiag][R];
+#pragma unroll
+    for (int d = 0; d < kClassDiag; ++d)
+        if (d < nd) {
+            const int o = doff[d];
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+                xv[d][k] = x.load(rx, (int)((unsigned)(rc[k] + o) * (unsigned)B));
+        }
+    unsigned m[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) m[k] = tab.mask[c[k]];
+#pragma unroll
+    for (int d = 0; d < kClassDiag; ++d)
+        if (d < nd) {
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const VT prod = tab.val[c[k] * kClassDiag + d] * x.value(xv[d][k]);
+                s[k] = ((m[k] >> d) & 1u) ? s[k] + prod : s[k];
+            }
+            if (xr && d == dzero) {
+#pragma unroll
+                for (int k = 0; k < R; ++k) xr[k] = xv[d][k];
+            }
+        }
+}
+
 struct NoLoads {
     __device__ __forceinline__ void operator()() const {}
 };
