@@ -19,20 +19,25 @@
 // loops do.
 //
 // Everything stays on the device; the host only enqueues.  The scalars (the
-// Hessenberg columns, rotations, gamma, back-substitution coefficients,
-// residual norms, counters and stop flags) live in one state record in HBM.
-// Each vector kernel writes per-block partial sums over fixed contiguous
-// chunks; the next kernel sums them in a fixed order (every block that needs
-// the value, or a one-block kernel that updates the state), so the result
-// depends on n only, never on timing.  In the CSR and DIA forms the products
-// w = A z_j and r = b - A x form the partials of v_1 . w and r . r
-// themselves, over the same chunks and in the same order as the separate
-// dot kernels the JAD form runs after its product, so all three forms give
-// the same bits.  The small Hessenberg algebra
-// (rotations, convergence test, back substitution) runs in one thread of a
-// one-block kernel, in the reference's order.  Partials alternate between
-// two buffers, so no kernel writes the partials it reads, and every state
-// field a kernel writes is one that no other block of that kernel reads.
+// Hessenberg columns, rotations, gamma, residual norms, counters and stop
+// flags) live in one state record in HBM.  Each vector kernel writes
+// per-block partial sums over fixed contiguous chunks; the next kernel sums
+// them in a fixed order, in every block, so the result depends on n only,
+// never on timing.  In the CSR and DIA forms the products w = A z_j and r =
+// b - A x form the partials of v_1 . w and r . r themselves, over the same
+// chunks and in the same order as the separate dot kernels the JAD form runs
+// after its product, so all three forms give the same bits.
+//
+// The small algebra has no launch of its own: the kernel that needs a norm
+// (the one that forms v_j+1, or the cycle's x update) sums its partials and
+// rotates the column in every block, in the reference's order, and block 0
+// records the result.  Every state field a kernel writes is one that no
+// other block of that kernel reads (raw and rotated columns, and gamma before
+// and after its rotation, are kept apart), and the convergence flag names
+// its column, so a block that starts late does not mistake it for an
+// earlier one.  Partials alternate between two buffers.  On small systems the
+// product that follows forms v_j and z_j itself (k_col); a cycle of
+// GMRES(3) is then 11 launches, 14 otherwise.
 //
 // One outer iteration (its residual and m+1 cycles) is captured once as a
 // hipGraph and replayed up to iter_max+1 times; after a replay the host
@@ -47,6 +52,7 @@
 
 #include "cel_internal.hpp"
 #include "device_common.hpp"
+#include "spmv_device.hpp"
 
 namespace cel {
 namespace {
@@ -54,33 +60,45 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kMaxRestart = 32;
 constexpr int kM1 = kMaxRestart + 2;  // 1-based index range of the small arrays
+constexpr int kNoColumn = 1 << 20;    // halt without a converged column
+constexpr int kWide = 1024;           // threads of the kernels of small systems
+constexpr int kWideRows = 2048;       // rows of a chunk there
 
 struct GmState {
-    double H[kM1 * kM1];  // H(i, j) = H[i * kM1 + j], 1-based, rotated in place
-    double cs[kM1], sn[kM1], gam[kM1], alp[kM1];
-    double residuum, local_residuum, norm0, eps;
+    double H[kM1 * kM1];  // h(i, j) = H[i * kM1 + j], 1-based, as the Gram-Schmidt passes leave it
+    double R[kM1 * kM1];  // the rotated columns
+    double cs[kM1], sn[kM1];
+    double gin[kM1], gam[kM1];  // gamma(j) as column j finds it, and after its rotation
+    double residuum, norm0, eps;
     int iter, cycles, ncols;  // outer iterations, cycles, Arnoldi columns run
-    int conv_col;             // column at which the current cycle converged (0: none)
-    int nalp;                 // coefficients in alp for the pending x update
-    int halt;                 // converged or stopped: later columns and cycles do nothing
+    int halt;                 // the column that converged (0: none): later columns and cycles do nothing
     int stop;                 // nothing runs any more
     int status;               // 0 or CEL_ERR_NONFINITE
+    int pad[2];
 };
 
-__device__ __forceinline__ double& Hij(GmState* st, int i, int j) { return st->H[i * kM1 + j]; }
-
-// Per-block partial of a sum, written to part[blockIdx].
-__device__ __forceinline__ void put_partial(double acc, double* __restrict__ part, double* red)
+// Sum over the first 256 threads of the block in block_sum's order; valid in
+// thread 0.
+__device__ __forceinline__ double sum256(double v, double* red)
 {
-    const double s = block_sum(acc, red);  // valid in thread 0
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
+    v = wave_sum(v);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0 && wave < kWaves) red[wave] = v;
+    __syncthreads();
+    double s = 0.0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < kWaves; ++w) s = s + red[w];
+    return s;
 }
 
 // Sum of the G partials in a fixed order, returned to every thread.
 __device__ __forceinline__ double fold(const double* __restrict__ part, int G, double* red,
                                        double* bcast)
 {
-    const double s = sum_partials(part, G, red);
+    double s = 0.0;
+    if (threadIdx.x < kBlock)
+        for (int i = threadIdx.x; i < G; i += kBlock) s = s + part[i];
+    s = sum256(s, red);
     if (threadIdx.x == 0) *bcast = s;
     __syncthreads();
     const double v = *bcast;
@@ -88,10 +106,33 @@ __device__ __forceinline__ double fold(const double* __restrict__ part, int G, d
     return v;
 }
 
-#define CHUNK_LOOP(i)                                                        \
+// The terms f(i) of the block's chunk [c0, c1) summed into its partial: 256
+// threads take rows 256 apart in ascending order, then block_sum's order.  A
+// block of more threads evaluates the rows side by side and adds them from
+// LDS in that same order.
+template <int T, typename F>
+__device__ __forceinline__ void chunk_partial(long long c0, long long c1, F&& f, double* __restrict__ part,
+                                              double* red, double* terms /* chunk, T > 256 only */)
+{
+    double acc = 0.0;
+    if constexpr (T == kBlock) {
+        for (long long i = c0 + threadIdx.x; i < c1; i += T) acc = acc + f(i);
+    } else {
+        for (long long i = c0 + threadIdx.x; i < c1; i += T) terms[i - c0] = f(i);
+        __syncthreads();
+        if (threadIdx.x < kBlock)
+            for (int i = threadIdx.x; i < (int)(c1 - c0); i += kBlock) acc = acc + terms[i];
+    }
+    const double s = sum256(acc, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+#define CHUNK_BOUNDS                                                         \
     const long long c0 = (long long)blockIdx.x * chunk;                      \
-    const long long c1 = c0 + chunk < n ? c0 + chunk : n;                    \
-    for (long long i = c0 + threadIdx.x; i < c1; i += kThreads)
+    const long long c1 = c0 + chunk < n ? c0 + chunk : n;
+#define CHUNK_LOOP(i)                                                        \
+    CHUNK_BOUNDS                                                             \
+    for (long long i = c0 + threadIdx.x; i < c1; i += blockDim.x)
 
 __global__ void __launch_bounds__(kThreads)
 k_fill(long long n, long long chunk, double* __restrict__ x, double v)
@@ -116,71 +157,70 @@ k_resid(long long n, long long chunk, const double* __restrict__ b, double* __re
 {
     __shared__ double red[kWaves];
     if (st->stop) return;
-    double acc = 0.0;
-    CHUNK_LOOP(i) {
+    CHUNK_BOUNDS
+    chunk_partial<kThreads>(c0, c1, [&](long long i) {
         const double ri = b[i] - r[i];
         r[i] = ri;
         const double p = ri * ri;
-        acc = acc + p;
-    }
-    put_partial(acc, part, red);
+        return p;
+    }, part, red, nullptr);
 }
 
-// Start of an outer iteration (one block): iter += 1 ; residuum = ||r||
-// (the first one is norm0) ; a non-finite residual ends the solve.
-__global__ void __launch_bounds__(kThreads)
-k_outer_start(const double* __restrict__ part, int G, GmState* st)
+// After the closing residual of a cycle (CYCLE) or the first one of an outer
+// iteration: residuum = ||r|| from its partials; returns it, or a negative
+// number where nothing more runs.  A cycle that converged ends the solve.
+// Every thread of the block; block 0 records.
+__device__ __forceinline__ double residual_done(bool cycle, const double* __restrict__ part, int G,
+                                                GmState* st, double* red, double* bcast)
 {
-    __shared__ double red[kWaves];
-    __shared__ double bcast;
-    if (st->stop) return;
-    const double s = fold(part, G, red, &bcast);
-    if (threadIdx.x == 0) {
-        const double res = sqrt(s);
-        st->iter = st->iter + 1;
-        if (st->iter == 1) st->norm0 = res;
+    const int halt = st->halt;
+    const double res = sqrt(fold(part, G, red, bcast));
+    const bool end = cycle ? halt != 0 : !isfinite(res);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
         st->residuum = res;
-        st->local_residuum = res;
-        if (!isfinite(res)) {
-            st->status = CEL_ERR_NONFINITE;
-            st->halt = 1;
-            st->stop = 1;
+        if (cycle) {
+            st->cycles = st->cycles + 1;
+        } else {
+            st->iter = st->iter + 1;
+            if (st->iter == 1) st->norm0 = res;
+            if (end) {
+                st->status = CEL_ERR_NONFINITE;
+                st->halt = kNoColumn;
+            }
         }
+        if (end) st->stop = 1;
     }
+    return end ? -1.0 : res;
 }
 
-// End of a cycle (one block): residuum = ||r|| ; cycles += 1 ; a cycle that
-// converged ends the solve here.
+// End of the last cycle of an outer iteration (one block).
 __global__ void __launch_bounds__(kThreads)
 k_cycle_end(const double* __restrict__ part, int G, GmState* st)
 {
     __shared__ double red[kWaves];
     __shared__ double bcast;
     if (st->stop) return;
-    const double s = fold(part, G, red, &bcast);
-    if (threadIdx.x == 0) {
-        const double res = sqrt(s);
-        st->residuum = res;
-        st->local_residuum = res;
-        st->cycles = st->cycles + 1;
-        if (st->conv_col) st->stop = 1;
-    }
+    (void)residual_done(true, part, G, st, red, &bcast);
 }
 
 // v1 = r * (1/beta) ; z1 = v1 * jac ; gamma1 = beta
 __global__ void __launch_bounds__(kThreads)
-k_scale_jac(long long n, long long chunk, const double* __restrict__ r,
-            const double* __restrict__ jac, double* __restrict__ v, double* __restrict__ z,
-            GmState* st)
+k_scale_jac(long long n, long long chunk, int cycle, const double* __restrict__ part, int G,
+            const double* __restrict__ r, const double* __restrict__ jac, double* __restrict__ v,
+            double* __restrict__ z, GmState* st)
 {
-    if (st->halt) return;
-    const double tmp = 1.0 / st->local_residuum;
+    __shared__ double red[kWaves];
+    __shared__ double bcast;
+    if (st->stop) return;
+    const double beta = residual_done(cycle, part, G, st, red, &bcast);
+    if (beta < 0.0) return;  // uniform
+    const double tmp = 1.0 / beta;
     CHUNK_LOOP(i) {
         const double vi = r[i] * tmp;
         v[i] = vi;
         z[i] = vi * jac[i];
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->gam[1] = st->residuum;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->gin[1] = beta;
 }
 
 // partial a . b
@@ -190,118 +230,139 @@ k_dot(long long n, long long chunk, const double* __restrict__ a, const double* 
 {
     __shared__ double red[kWaves];
     if (st->halt) return;
-    double acc = 0.0;
-    CHUNK_LOOP(i) {
+    CHUNK_BOUNDS
+    chunk_partial<kThreads>(c0, c1, [&](long long i) {
         const double p = a[i] * b[i];
-        acc = acc + p;
-    }
-    put_partial(acc, part, red);
+        return p;
+    }, part, red, nullptr);
 }
 
 // h_ii,jj = sum(prev partials) ; w = w - h vi ; partial (next ? next . w : w . w)
-__global__ void __launch_bounds__(kThreads)
+template <int T>
+__global__ void __launch_bounds__(T)
 k_mgs(long long n, long long chunk, int ii, int jj, const double* __restrict__ prev, int G,
       const double* __restrict__ vi, double* __restrict__ w, const double* __restrict__ next,
       double* __restrict__ part, GmState* st)
 {
     __shared__ double red[kWaves];
     __shared__ double bcast;
+    __shared__ double terms[T == kThreads ? 1 : kWideRows];
     if (st->halt) return;
     const double h = fold(prev, G, red, &bcast);
-    if (blockIdx.x == 0 && threadIdx.x == 0) Hij(st, ii, jj) = h;
-    double acc = 0.0;
-    CHUNK_LOOP(i) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->H[ii * kM1 + jj] = h;
+    CHUNK_BOUNDS
+    chunk_partial<T>(c0, c1, [&](long long i) {
         const double t = h * vi[i];
         const double wi = w[i] - t;
         w[i] = wi;
         const double p = (next ? next[i] : wi) * wi;
-        acc = acc + p;
-    }
-    put_partial(acc, part, red);
+        return p;
+    }, part, red, terms);
 }
 
-// Back substitution on the first k columns (cel_gmresalg_module.f90:760-772
-// order), one thread.
-__device__ void back_substitute(GmState* st, int k)
+// What a block knows after a column (LDS).
+struct Column {
+    double h[kM1], cs[kM1], sn[kM1], gam[kM1], alp[kM1];
+    double R[kMaxRestart * (kMaxRestart + 1) / 2];  // the rotated columns before it, packed
+    int k;  // coefficients of the x update in alp (0: none)
+};
+
+// After the last Gram-Schmidt pass of column jj: h_jj+1,jj = sqrt(sum of its
+// partials) ; the column's rotations as the reference writes them ; new
+// rotation ; gamma ; convergence test ; the back-substitution coefficients
+// (cel_gmresalg_module.f90:760-772 order) when the column converged or is
+// the cycle's last.  Every thread of the block; the algebra runs in one
+// thread over LDS, block 0 records it.
+__device__ __forceinline__ void column_done(int jj, int m, const double* __restrict__ part, int G,
+                                            GmState* st, Column& c, double* red, double* bcast)
 {
-    for (int ii = k; ii >= 1; --ii) {
-        double a = 0.0;
-        for (int kk = ii + 1; kk <= k; ++kk) {
-            const double t = Hij(st, ii, kk) * st->alp[kk];
-            a = a + t;
-        }
-        const double inv = 1.0 / Hij(st, ii, ii);
-        st->alp[ii] = inv * (st->gam[ii] - a);
+    const int tid = threadIdx.x;
+    if (tid <= jj && tid > 0) c.h[tid] = st->H[tid * kM1 + jj];
+    if (tid < jj && tid > 0) {
+        c.cs[tid] = st->cs[tid];
+        c.sn[tid] = st->sn[tid];
+        c.gam[tid] = st->gam[tid];
     }
-    st->nalp = k;
+    if (tid == 0) c.gam[jj] = st->gin[jj];
+    for (int q = tid; q < jj * (jj - 1) / 2; q += blockDim.x) {
+        int k = 1, at = q;  // entry (i, k), i <= k < jj
+        while (at >= k) at -= k++;
+        c.R[q] = st->R[(at + 1) * kM1 + k];
+    }
+    const double s = fold(part, G, red, bcast);  // (synchronises)
+    if (tid == 0) {
+        c.h[jj + 1] = sqrt(s);
+        for (int ii = 1; ii <= jj - 1; ++ii) {  // both statements assign h(ii,jj) (:722-727)
+            double a = c.h[ii] * c.cs[ii];
+            double d = c.h[ii + 1] * c.sn[ii];
+            c.h[ii] = a + d;
+            a = -c.h[ii] * c.sn[ii];
+            d = c.h[ii + 1] * c.cs[ii];
+            c.h[ii] = a + d;
+        }
+        const double a = c.h[jj] * c.h[jj];
+        const double d = c.h[jj + 1] * c.h[jj + 1];
+        const double betta = sqrt(a + d);
+        const double sn = c.h[jj + 1] / betta, cs = c.h[jj] / betta;
+        const double gnext = -sn * c.gam[jj];
+        c.h[jj] = betta;
+        c.gam[jj] = cs * c.gam[jj];
+        const bool conv = fabs(gnext) <= st->eps;
+        c.k = conv || jj == m ? jj : 0;
+        for (int ii = c.k; ii >= 1; --ii) {
+            double sum = 0.0;
+            for (int kk = ii + 1; kk <= c.k; ++kk) {
+                const double hik = kk == jj ? c.h[ii] : c.R[kk * (kk - 1) / 2 + ii - 1];
+                const double t = hik * c.alp[kk];
+                sum = sum + t;
+            }
+            const double hii = ii == jj ? betta : c.R[ii * (ii - 1) / 2 + ii - 1];
+            const double inv = 1.0 / hii;
+            c.alp[ii] = inv * (c.gam[ii] - sum);
+        }
+        if (blockIdx.x == 0) {
+            for (int ii = 1; ii <= jj; ++ii) st->R[ii * kM1 + jj] = c.h[ii];
+            st->cs[jj] = cs;
+            st->sn[jj] = sn;
+            st->gin[jj + 1] = gnext;
+            st->gam[jj] = c.gam[jj];
+            st->ncols = st->ncols + 1;
+            if (conv) st->halt = jj;
+        }
+    }
+    __syncthreads();
 }
 
-// One block: h_jj+1,jj = sqrt(sum of the last partials) ; the column's
-// rotations as the reference writes them ; new rotation ; gamma ;
-// convergence test ; the back-substitution coefficients when the column
-// converged or is the cycle's last.
+// x = x + a_1 z_1 + ... + a_k z_k, added in that order
+__device__ __forceinline__ double x_updated(double xi, const Column& c, const double* __restrict__ Z,
+                                            long long n, long long i)
+{
+    for (int j = 0; j < c.k; ++j) {
+        const double t = c.alp[j + 1] * Z[(long long)j * n + i];
+        xi = xi + t;
+    }
+    return xi;
+}
+
+// After column jj: with coefficients (the column converged or is the
+// cycle's last) the x update; else v_jj+1 = w / h_jj+1,jj and z_jj+1 =
+// v_jj+1 * jac.
 __global__ void __launch_bounds__(kThreads)
-k_givens(int jj, int m, const double* __restrict__ part, int G, GmState* st)
+k_next(long long n, long long chunk, int jj, int m, const double* __restrict__ part, int G,
+       const double* __restrict__ w, const double* __restrict__ jac, double* __restrict__ V,
+       double* __restrict__ Z, double* __restrict__ x, GmState* st)
 {
     __shared__ double red[kWaves];
     __shared__ double bcast;
-    if (st->halt) return;
-    const double s = fold(part, G, red, &bcast);
-    if (threadIdx.x != 0) return;
-    Hij(st, jj + 1, jj) = sqrt(s);
-    for (int ii = 1; ii <= jj - 1; ++ii) {  // both statements assign h(ii,jj) (:722-727)
-        double a = Hij(st, ii, jj) * st->cs[ii];
-        double c = Hij(st, ii + 1, jj) * st->sn[ii];
-        Hij(st, ii, jj) = a + c;
-        a = -Hij(st, ii, jj) * st->sn[ii];
-        c = Hij(st, ii + 1, jj) * st->cs[ii];
-        Hij(st, ii, jj) = a + c;
-    }
-    {
-        const double a = Hij(st, jj, jj) * Hij(st, jj, jj);
-        const double c = Hij(st, jj + 1, jj) * Hij(st, jj + 1, jj);
-        const double betta = sqrt(a + c);
-        st->sn[jj] = Hij(st, jj + 1, jj) / betta;
-        st->cs[jj] = Hij(st, jj, jj) / betta;
-        Hij(st, jj, jj) = betta;
-        st->gam[jj + 1] = -st->sn[jj] * st->gam[jj];
-        st->gam[jj] = st->cs[jj] * st->gam[jj];
-    }
-    st->ncols = st->ncols + 1;
-    st->nalp = 0;
-    if (fabs(st->gam[jj + 1]) <= st->eps) {
-        back_substitute(st, jj);
-        st->conv_col = jj;
-        st->halt = 1;
-    } else if (jj == m) {
-        back_substitute(st, m);
-    }
-}
-
-// After column jj: with coefficients pending (the column converged or is the
-// cycle's last) x = x + a_1 z_1 + ... + a_k z_k, added in that order; else
-// v_jj+1 = w / h_jj+1,jj and z_jj+1 = v_jj+1 * jac.
-__global__ void __launch_bounds__(kThreads)
-k_next(long long n, long long chunk, int jj, int m, const double* __restrict__ w,
-       const double* __restrict__ jac, double* __restrict__ V, double* __restrict__ Z,
-       double* __restrict__ x, const GmState* __restrict__ st)
-{
-    if (st->stop) return;
-    if (st->halt && st->conv_col != jj) return;  // converged at an earlier column
-    const int k = st->nalp;
-    if (k > 0) {
-        CHUNK_LOOP(i) {
-            double xi = x[i];
-            for (int j = 0; j < k; ++j) {
-                const double t = st->alp[j + 1] * Z[(long long)j * n + i];
-                xi = xi + t;
-            }
-            x[i] = xi;
-        }
+    __shared__ Column c;
+    // (a flag of this column is this launch's own)
+    if (st->stop || (st->halt && st->halt != jj)) return;
+    column_done(jj, m, part, G, st, c, red, &bcast);
+    if (c.k > 0) {
+        CHUNK_LOOP(i) x[i] = x_updated(x[i], c, Z, n, i);
         return;
     }
-    if (jj == m) return;
-    const double h = st->H[(jj + 1) * kM1 + jj];
+    const double h = c.h[jj + 1];
     double* v = V + (long long)jj * n;  // v_jj+1
     double* z = Z + (long long)jj * n;  // z_jj+1
     CHUNK_LOOP(i) {
@@ -309,6 +370,195 @@ k_next(long long n, long long chunk, int jj, int m, const double* __restrict__ w
         v[i] = vi;
         z[i] = vi * jac[i];
     }
+}
+
+// ------------------------------------------------------------------ small systems
+// w / h for many w: y = 1/h and two residual corrections, which give the
+// correctly rounded quotient (Markstein's theorem: the first correction is
+// within an ulp, the second rounds it; checked against w / h on 2.6e8 pairs)
+// away from the ends of the exponent range, where w / h itself is taken.
+struct Quotient {
+    double h, y;
+    bool mid;
+    __device__ explicit Quotient(double d) : h(d), y(1.0 / d), mid(fabs(d) > 1e-100 && fabs(d) < 1e100) {}
+    __device__ __forceinline__ double operator()(double w) const
+    {
+        const double q0 = w * y;
+        const double q1 = __builtin_fma(__builtin_fma(-h, q0, w), y, q0);
+        const double q2 = __builtin_fma(__builtin_fma(-h, q1, w), y, q1);
+        const double a = fabs(w);
+        return mid && a > 1e-150 && a < 1e150 ? q2 : w / h;
+    }
+};
+
+// z_j where a product gathers it: (r * (1/beta)) * jac for the first column
+// of a cycle, (w / h) * jac for the others.
+template <bool FIRST>
+struct XKrylov {
+    struct Raw {
+        double a, j;
+    };
+    struct Buf {
+        __amdgpu_buffer_rsrc_t a, j;
+    };
+    const double *a, *jac;
+    double s;  // 1/beta
+    Quotient q;
+    __device__ __forceinline__ Raw load(int i) const { return Raw{a[i], jac[i]}; }
+    __device__ __forceinline__ double v(const Raw& r) const
+    {
+        if constexpr (FIRST) return r.a * s;
+        else return q(r.a);
+    }
+    __device__ __forceinline__ double value(const Raw& r) const { return v(r) * r.j; }
+    __device__ __forceinline__ Buf buf(unsigned bytes) const
+    {
+        return Buf{tile_rsrc(a, (int)bytes), tile_rsrc(jac, (int)bytes)};
+    }
+    __device__ __forceinline__ Raw load(const Buf& b, int off) const
+    {
+        return Raw{buf_load<double>(b.a, off), buf_load<double>(b.j, off)};
+    }
+};
+
+struct GmMat {
+    int n;
+    const int *xadj, *cols;
+    const double *vals, *dvals;
+    const uint32_t* mask;
+    const uint8_t* mask8;
+    int nd, off[32];
+};
+
+// Row sums of rows r[0..2) (r[k] >= n: not used) in CSR column order.
+template <int FMT, typename X>
+__device__ __forceinline__ void two_rows(const GmMat& A, const int (&r)[2], const X& x, double (&s)[2])
+{
+    if constexpr (FMT == CEL_FMT_DIA) {
+        if (r[0] < A.n) dia_rows<double, 2, 4>(A.n, A.nd, A.off, A.dvals, A.mask8, A.mask, r, x, s);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            s[k] = 0.0;
+            const int lo = r[k] < A.n ? A.xadj[r[k]] : 0, hi = r[k] < A.n ? A.xadj[r[k] + 1] : 0;
+            for (int j0 = lo; j0 < hi; j0 += kGather) {
+                typename X::Raw xv[kGather];
+                double a[kGather];
+#pragma unroll
+                for (int i = 0; i < kGather; ++i) {
+                    const bool on = j0 + i < hi;
+                    const int c = A.cols[on ? j0 + i : lo];
+                    a[i] = A.vals[on ? j0 + i : lo];
+                    xv[i] = x.load(c);
+                }
+#pragma unroll
+                for (int i = 0; i < kGather; ++i) {
+                    const double t = a[i] * x.value(xv[i]);
+                    const double u = s[k] + t;
+                    s[k] = j0 + i < hi ? u : s[k];
+                }
+            }
+        }
+    }
+}
+
+// Column j of a small system's cycle in one launch: the scalars that end the
+// column before it (FIRST: the residual), v_j and z_j, w_j = A z_j and the
+// partials of v_1 . w_j.  Every gather forms z_j itself from r or the last
+// w and jac, so no launch stands between a norm and the product; w
+// alternates between two buffers.  With coefficients after the column
+// before it (it converged), the x update instead.  One block of 1,024
+// threads per chunk, two rows each.
+template <int FMT, bool FIRST>
+__global__ void __launch_bounds__(kWide)
+k_col(GmMat A, long long chunk, int j, int m, int cycle, const double* __restrict__ prev, int G,
+      const double* __restrict__ src, const double* __restrict__ jac, double* __restrict__ V,
+      double* __restrict__ Z, double* __restrict__ w, double* __restrict__ x,
+      double* __restrict__ part, GmState* st)
+{
+    __shared__ double red[kWaves];
+    __shared__ double bcast;
+    __shared__ double terms[kWideRows];
+    __shared__ Column c;
+    const long long n = A.n;
+    double beta = 1.0;
+    if (st->stop) return;
+    if constexpr (FIRST) {
+        beta = residual_done(cycle, prev, G, st, red, &bcast);
+        if (beta < 0.0) return;  // uniform
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->gin[1] = beta;
+    } else {
+        if (st->halt && st->halt != j - 1) return;
+        column_done(j - 1, m, prev, G, st, c, red, &bcast);
+        if (c.k > 0) {
+            CHUNK_LOOP(i) x[i] = x_updated(x[i], c, Z, n, i);
+            return;
+        }
+    }
+    const XKrylov<FIRST> X{src, jac, 1.0 / beta, Quotient(FIRST ? 1.0 : c.h[j])};
+    double* v = V + (long long)(j - 1) * n;
+    double* z = Z + (long long)(j - 1) * n;
+    CHUNK_BOUNDS
+    int r[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const long long i = c0 + threadIdx.x + (long long)k * kWide;
+        r[k] = i < c1 ? (int)i : A.n;
+    }
+    double s[2] = {0.0, 0.0};
+    two_rows<FMT>(A, r, X, s);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        if (r[k] < A.n) {
+            const auto raw = X.load(r[k]);
+            const double vi = X.v(raw), wi = 0.0 + s[k];
+            v[r[k]] = vi;
+            z[r[k]] = vi * raw.j;
+            w[r[k]] = wi;
+            const double p = (FIRST ? vi : V[r[k]]) * wi;
+            terms[r[k] - c0] = p;
+        }
+    __syncthreads();
+    double acc = 0.0;
+    if (threadIdx.x < kBlock)
+        for (int i = threadIdx.x; i < (int)(c1 - c0); i += kBlock) acc = acc + terms[i];
+    const double t = sum256(acc, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = t;
+}
+
+// r = b - A x and the partials of r . r
+template <int FMT>
+__global__ void __launch_bounds__(kWide)
+k_resid_small(GmMat A, long long chunk, const double* __restrict__ x, const double* __restrict__ b,
+              double* __restrict__ rr, double* __restrict__ part, const GmState* __restrict__ st)
+{
+    __shared__ double red[kWaves];
+    __shared__ double terms[kWideRows];
+    if (st->stop) return;
+    const long long n = A.n;
+    CHUNK_BOUNDS
+    int r[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const long long i = c0 + threadIdx.x + (long long)k * kWide;
+        r[k] = i < c1 ? (int)i : A.n;
+    }
+    double s[2] = {0.0, 0.0};
+    two_rows<FMT>(A, r, XPlain<double>{x}, s);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        if (r[k] < A.n) {
+            const double ri = b[r[k]] - (0.0 + s[k]);
+            rr[r[k]] = ri;
+            const double p = ri * ri;
+            terms[r[k] - c0] = p;
+        }
+    __syncthreads();
+    double acc = 0.0;
+    if (threadIdx.x < kBlock)
+        for (int i = threadIdx.x; i < (int)(c1 - c0); i += kBlock) acc = acc + terms[i];
+    const double t = sum256(acc, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
 struct Gmres {
@@ -327,6 +577,28 @@ struct Gmres {
         G = (int)(g < 1 ? 1 : g > 1024 ? 1024 : g);
         chunk = ((n + G - 1) / G + kThreads - 1) / kThreads * kThreads;
         if (chunk < kThreads) chunk = kThreads;
+    }
+    // Whether a column is one launch (k_col) plus its Gram-Schmidt passes.
+    // Measured per cycle of GMRES(3), 7-point cubes, k_col / separate
+    // launches: 16^3 DIA 76.0 / 83.2 us, CSR 88.8 / 105; 48^3 84.8 / 92.1, 101
+    // / 119; 80^3 112 / 129, 121 / 155; 100^3 183 / 175, 196 / 198; 128^3 338 /
+    // 283, 420 / 328 (the second gathered array and the quotients cost more
+    // than the launches).  Long rows gather too much at any size (30,011 mesh
+    // rows of 11 entries 185 / 169).
+    bool small() const { return format != CEL_FMT_JAD && n <= 600000 && !csr_long_rows(A); }
+    GmMat mat() const
+    {
+        GmMat M{};
+        M.n = A.n;
+        M.xadj = A.xadj.p;
+        M.cols = A.cols.p;
+        M.vals = A.vals.p;
+        M.dvals = A.dia_vals.p;
+        M.mask = A.dia_mask.p;
+        M.mask8 = A.dia_mask8.p;
+        M.nd = A.dia_nd;
+        for (int d = 0; d < A.dia_nd; ++d) M.off[d] = A.dia_off[d];
+        return M;
     }
     // w = A z with the partials of v1 . w (skipped once halt is set)
     int spmv_dot(const double* z, double* w, const double* v1, double* part, GmState* gs)
@@ -402,27 +674,62 @@ int gmres_solve(Mat& A, const double* b_in, double* x_out, const cel_gmres_param
     auto vv = [&](int k) { return V.p + (size_t)(k - 1) * n; };  // v_k, 1-based
     auto zz = [&](int k) { return Z.p + (size_t)(k - 1) * n; };
 
+    const bool small = S.small();
+    DevBuf<double> w2;
+    if (small) CEL_TRY(w2.alloc(n));
+    const GmMat GM = S.mat();
+    const bool dia = prm.format == CEL_FMT_DIA;
+    // the same on a small system: k_col in place of k_scale_jac / k_next and
+    // the product
+    auto enqueue_small = [&]() -> int {
+        auto resid = [&]() {
+            if (dia) k_resid_small<CEL_FMT_DIA><<<G, kWide, 0, st>>>(GM, ck, x, b, r.p, partA.p, gs);
+            else k_resid_small<CEL_FMT_CSR><<<G, kWide, 0, st>>>(GM, ck, x, b, r.p, partA.p, gs);
+        };
+        auto col = [&](auto kernel, int j, int cycle, const double* prev, const double* src, double* out, double* part) {
+            kernel<<<G, kWide, 0, st>>>(GM, ck, j, m, cycle, prev, G, src, A.jac.p, V.p, Z.p, out, x, part, gs);
+        };
+        resid();
+        for (int c = 0; c <= m; ++c) {
+            double *cur = partA.p, *nxt = partB.p, *wi = w.p, *wo = w2.p;
+            for (int jj = 1; jj <= m; ++jj) {
+                if (jj == 1) col(dia ? k_col<CEL_FMT_DIA, true> : k_col<CEL_FMT_CSR, true>, jj, c > 0, cur, r.p, wo, nxt);
+                else col(dia ? k_col<CEL_FMT_DIA, false> : k_col<CEL_FMT_CSR, false>, jj, 0, cur, wi, wo, nxt);
+                std::swap(cur, nxt);
+                std::swap(wi, wo);
+                for (int ii = 1; ii <= jj; ++ii) {
+                    const double* next = ii < jj ? vv(ii + 1) : nullptr;
+                    k_mgs<kWide><<<G, kWide, 0, st>>>(n, ck, ii, jj, cur, G, vv(ii), wi, next, nxt, gs);
+                    std::swap(cur, nxt);
+                }
+            }
+            k_next<<<G, kThreads, 0, st>>>(n, ck, m, m, cur, G, wi, A.jac.p, V.p, Z.p, x, gs);
+            resid();
+        }
+        k_cycle_end<<<1, kThreads, 0, st>>>(partA.p, G, gs);
+        CEL_HIP(hipGetLastError());
+        return CEL_OK;
+    };
     // one outer iteration: r = b - A x, then up to m+1 cycles
     auto enqueue_outer = [&]() -> int {
+        if (small) return enqueue_small();
         CEL_TRY(S.spmv_resid(x, r.p, b, partA.p, gs));
-        k_outer_start<<<1, kThreads, 0, st>>>(partA.p, G, gs);
         for (int c = 0; c <= m; ++c) {
-            k_scale_jac<<<G, kThreads, 0, st>>>(n, ck, r.p, A.jac.p, vv(1), zz(1), gs);
+            k_scale_jac<<<G, kThreads, 0, st>>>(n, ck, c > 0, partA.p, G, r.p, A.jac.p, vv(1), zz(1), gs);
             for (int jj = 1; jj <= m; ++jj) {
-                double* cur = partA.p;
-                double* nxt = partB.p;
+                double* cur = partB.p;
+                double* nxt = partA.p;
                 CEL_TRY(S.spmv_dot(zz(jj), w.p, vv(1), cur, gs));
                 for (int ii = 1; ii <= jj; ++ii) {
                     const double* next = ii < jj ? vv(ii + 1) : nullptr;
-                    k_mgs<<<G, kThreads, 0, st>>>(n, ck, ii, jj, cur, G, vv(ii), w.p, next, nxt, gs);
+                    k_mgs<kThreads><<<G, kThreads, 0, st>>>(n, ck, ii, jj, cur, G, vv(ii), w.p, next, nxt, gs);
                     std::swap(cur, nxt);
                 }
-                k_givens<<<1, kThreads, 0, st>>>(jj, m, cur, G, gs);
-                k_next<<<G, kThreads, 0, st>>>(n, ck, jj, m, w.p, A.jac.p, V.p, Z.p, x, gs);
+                k_next<<<G, kThreads, 0, st>>>(n, ck, jj, m, cur, G, w.p, A.jac.p, V.p, Z.p, x, gs);
             }
             CEL_TRY(S.spmv_resid(x, r.p, b, partA.p, gs));
-            k_cycle_end<<<1, kThreads, 0, st>>>(partA.p, G, gs);
         }
+        k_cycle_end<<<1, kThreads, 0, st>>>(partA.p, G, gs);
         CEL_HIP(hipGetLastError());
         return CEL_OK;
     };
@@ -482,7 +789,7 @@ int gmres_solve(Mat& A, const double* b_in, double* x_out, const cel_gmres_param
         stats.status = out.status;
         return fail(out.status, "the residual is not finite");
     }
-    stats.status = out.conv_col ? CEL_OK : CEL_NOT_CONVERGED;
+    stats.status = out.halt ? CEL_OK : CEL_NOT_CONVERGED;
     return stats.status;
 }
 
