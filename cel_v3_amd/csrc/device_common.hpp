@@ -9,7 +9,7 @@
 //  * Reductions are deterministic: a fixed per-thread order, a fixed
 //    butterfly inside the wavefront, a fixed order across waves, one partial
 //    per logical block; the consuming kernel sums the partials in
-//    logical-block order (sum_partials), in every block that needs them.
+//    logical-block order (strided_sum), in every block that needs them.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -36,11 +36,66 @@ __device__ __forceinline__ T ld_stream(const T* p)
     return __builtin_nontemporal_load(p);
 }
 
+// Lane exchanges of the butterfly sums, in registers: halves of the wave and
+// of its 32-lane halves through the swap instructions, the rest through
+// DPP.  (Through LDS, as __shfl_xor does it, a wave sum took 490 cycles; so
+// it takes 190, and every kernel of a solver iteration has two to four of
+// them in its chain.)
+__device__ __forceinline__ double lanes_f64(unsigned lo, unsigned hi)
+{
+    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+
+// v[l] + v[l ^ 32] and v[l] + v[l ^ 16]
+__device__ __forceinline__ double add_xor32(double v)
+{
+    const auto u = __builtin_bit_cast(unsigned long long, v);
+    const auto a = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+    return lanes_f64(a[0], b[0]) + lanes_f64(a[1], b[1]);
+}
+__device__ __forceinline__ double add_xor16(double v)
+{
+    const auto u = __builtin_bit_cast(unsigned long long, v);
+    const auto a = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+    return lanes_f64(a[0], b[0]) + lanes_f64(a[1], b[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double v)
+{
+    const auto u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (unsigned)u, CTRL, 0xf, 0xf, false);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (unsigned)(u >> 32), CTRL, 0xf, 0xf, false);
+    return v + lanes_f64(lo, hi);
+}
+// v[l] + v[l ^ 8]: rows of 16 lanes rotated by 8
+__device__ __forceinline__ double add_xor8(double v) { return add_dpp<0x128>(v); }
+// v[l] + v[l ^ 4] of values that repeat with period 8: rows rotated by 4
+__device__ __forceinline__ double add_xor4_of8(double v) { return add_dpp<0x124>(v); }
+// v[l] + v[l ^ 2] and v[l] + v[l ^ 1]: quad permutations
+__device__ __forceinline__ double add_xor2(double v) { return add_dpp<0x4E>(v); }
+__device__ __forceinline__ double add_xor1(double v) { return add_dpp<0xB1>(v); }
+
+// Sum of the wave's lanes in every lane: the butterfly over lane distances
+// 32, 16, 8, 4, 2, 1.
 __device__ __forceinline__ double wave_sum(double v)
 {
+    return add_xor1(add_xor2(add_xor4_of8(add_xor8(add_xor16(add_xor32(v))))));
+}
+
+// Sum over the block in every thread, in block_sum's order.  smem must not be
+// written again before the block's next barrier.
+__device__ __forceinline__ double block_sum_all(double v, double* smem /* kWaves */)
+{
+    v = wave_sum(v);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) smem[wave] = v;
+    __syncthreads();
+    double s = 0.0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = v + __shfl_xor(v, off, 64);
-    return v;
+    for (int w = 0; w < kWaves; ++w) s = s + smem[w];
+    return s;
 }
 
 // Sum over the block; valid in thread 0.  Order: butterfly in each wave,
@@ -82,15 +137,15 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* smem /*
     __syncthreads();
 }
 
-// Sum of G partials in logical-block order by the whole block: thread t
-// sums t, t+256, ... sequentially, then block_sum.  Valid in thread 0.
-// Every block of the consuming kernel reads the same partials, so they are
-// plain (cached) loads: after the first block on an XCD the rest hit its L2.
-__device__ __forceinline__ double sum_partials(const double* partials, int G, double* smem)
+// The calling thread's part of a fold of G partials: t, t + 256, ...
+// in order; block_sum_all of the parts is the fold.  Every block of the
+// consuming kernel reads the same partials, so they are plain (cached)
+// loads: after the first block on an XCD the rest hit its L2.
+__device__ __forceinline__ double strided_sum(const double* __restrict__ partials, int G)
 {
     double s = 0.0;
     for (int i = threadIdx.x; i < G; i += kBlock) s = s + partials[i];
-    return block_sum(s, smem);
+    return s;
 }
 
 }  // namespace cel

@@ -77,8 +77,8 @@ struct GmState {
     int pad[2];
 };
 
-// Sum over the first 256 threads of the block in block_sum's order; valid in
-// thread 0.
+// Sum over the first 256 threads of the block in block_sum's order, in every
+// thread; red as block_sum_all.
 __device__ __forceinline__ double sum256(double v, double* red)
 {
     v = wave_sum(v);
@@ -86,24 +86,16 @@ __device__ __forceinline__ double sum256(double v, double* red)
     if (lane == 0 && wave < kWaves) red[wave] = v;
     __syncthreads();
     double s = 0.0;
-    if (threadIdx.x == 0)
-        for (int w = 0; w < kWaves; ++w) s = s + red[w];
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s = s + red[w];
     return s;
 }
 
-// Sum of the G partials in a fixed order, returned to every thread.
-__device__ __forceinline__ double fold(const double* __restrict__ part, int G, double* red,
-                                       double* bcast)
+// The calling thread's part of a fold of the G partials; sum256 of the parts
+// is their sum in a fixed order.
+__device__ __forceinline__ double fold_part(const double* __restrict__ part, int G)
 {
-    double s = 0.0;
-    if (threadIdx.x < kBlock)
-        for (int i = threadIdx.x; i < G; i += kBlock) s = s + part[i];
-    s = sum256(s, red);
-    if (threadIdx.x == 0) *bcast = s;
-    __syncthreads();
-    const double v = *bcast;
-    __syncthreads();
-    return v;
+    return threadIdx.x < kBlock ? strided_sum(part, G) : 0.0;
 }
 
 // The terms f(i) of the block's chunk [c0, c1) summed into its partial: 256
@@ -170,11 +162,10 @@ k_resid(long long n, long long chunk, const double* __restrict__ b, double* __re
 // iteration: residuum = ||r|| from its partials; returns it, or a negative
 // number where nothing more runs.  A cycle that converged ends the solve.
 // Every thread of the block; block 0 records.
-__device__ __forceinline__ double residual_done(bool cycle, const double* __restrict__ part, int G,
-                                                GmState* st, double* red, double* bcast)
+__device__ __forceinline__ double residual_done(bool cycle, double folded, GmState* st, double* red)
 {
     const int halt = st->halt;
-    const double res = sqrt(fold(part, G, red, bcast));
+    const double res = sqrt(sum256(folded, red));
     const bool end = cycle ? halt != 0 : !isfinite(res);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st->residuum = res;
@@ -198,9 +189,9 @@ __global__ void __launch_bounds__(kThreads)
 k_cycle_end(const double* __restrict__ part, int G, GmState* st)
 {
     __shared__ double red[kWaves];
-    __shared__ double bcast;
+    const double f = fold_part(part, G);
     if (st->stop) return;
-    (void)residual_done(true, part, G, st, red, &bcast);
+    (void)residual_done(true, f, st, red);
 }
 
 // v1 = r * (1/beta) ; z1 = v1 * jac ; gamma1 = beta
@@ -210,9 +201,9 @@ k_scale_jac(long long n, long long chunk, int cycle, const double* __restrict__ 
             double* __restrict__ z, GmState* st)
 {
     __shared__ double red[kWaves];
-    __shared__ double bcast;
+    const double f = fold_part(part, G);  // (the loads do not wait for the flag)
     if (st->stop) return;
-    const double beta = residual_done(cycle, part, G, st, red, &bcast);
+    const double beta = residual_done(cycle, f, st, red);
     if (beta < 0.0) return;  // uniform
     const double tmp = 1.0 / beta;
     CHUNK_LOOP(i) {
@@ -244,11 +235,11 @@ k_mgs(long long n, long long chunk, int ii, int jj, const double* __restrict__ p
       const double* __restrict__ vi, double* __restrict__ w, const double* __restrict__ next,
       double* __restrict__ part, GmState* st)
 {
-    __shared__ double red[kWaves];
-    __shared__ double bcast;
+    __shared__ double red[2 * kWaves];
     __shared__ double terms[T == kThreads ? 1 : kWideRows];
+    const double f = fold_part(prev, G);
     if (st->halt) return;
-    const double h = fold(prev, G, red, &bcast);
+    const double h = sum256(f, red + kWaves);
     if (blockIdx.x == 0 && threadIdx.x == 0) st->H[ii * kM1 + jj] = h;
     CHUNK_BOUNDS
     chunk_partial<T>(c0, c1, [&](long long i) {
@@ -273,8 +264,8 @@ struct Column {
 // (cel_gmresalg_module.f90:760-772 order) when the column converged or is
 // the cycle's last.  Every thread of the block; the algebra runs in one
 // thread over LDS, block 0 records it.
-__device__ __forceinline__ void column_done(int jj, int m, const double* __restrict__ part, int G,
-                                            GmState* st, Column& c, double* red, double* bcast)
+__device__ __forceinline__ void column_done(int jj, int m, double folded, GmState* st, Column& c,
+                                            double* red)
 {
     const int tid = threadIdx.x;
     if (tid <= jj && tid > 0) c.h[tid] = st->H[tid * kM1 + jj];
@@ -289,7 +280,7 @@ __device__ __forceinline__ void column_done(int jj, int m, const double* __restr
         while (at >= k) at -= k++;
         c.R[q] = st->R[(at + 1) * kM1 + k];
     }
-    const double s = fold(part, G, red, bcast);  // (synchronises)
+    const double s = sum256(folded, red);  // (synchronises)
     if (tid == 0) {
         c.h[jj + 1] = sqrt(s);
         for (int ii = 1; ii <= jj - 1; ++ii) {  // both statements assign h(ii,jj) (:722-727)
@@ -353,11 +344,11 @@ k_next(long long n, long long chunk, int jj, int m, const double* __restrict__ p
        double* __restrict__ Z, double* __restrict__ x, GmState* st)
 {
     __shared__ double red[kWaves];
-    __shared__ double bcast;
     __shared__ Column c;
+    const double f = fold_part(part, G);
     // (a flag of this column is this launch's own)
     if (st->stop || (st->halt && st->halt != jj)) return;
-    column_done(jj, m, part, G, st, c, red, &bcast);
+    column_done(jj, m, f, st, c, red);
     if (c.k > 0) {
         CHUNK_LOOP(i) x[i] = x_updated(x[i], c, Z, n, i);
         return;
@@ -476,20 +467,20 @@ k_col(GmMat A, long long chunk, int j, int m, int cycle, const double* __restric
       double* __restrict__ Z, double* __restrict__ w, double* __restrict__ x,
       double* __restrict__ part, GmState* st)
 {
-    __shared__ double red[kWaves];
-    __shared__ double bcast;
+    __shared__ double red[2 * kWaves];
     __shared__ double terms[kWideRows];
     __shared__ Column c;
     const long long n = A.n;
     double beta = 1.0;
+    const double f = fold_part(prev, G);
     if (st->stop) return;
     if constexpr (FIRST) {
-        beta = residual_done(cycle, prev, G, st, red, &bcast);
+        beta = residual_done(cycle, f, st, red + kWaves);
         if (beta < 0.0) return;  // uniform
         if (blockIdx.x == 0 && threadIdx.x == 0) st->gin[1] = beta;
     } else {
         if (st->halt && st->halt != j - 1) return;
-        column_done(j - 1, m, prev, G, st, c, red, &bcast);
+        column_done(j - 1, m, f, st, c, red + kWaves);
         if (c.k > 0) {
             CHUNK_LOOP(i) x[i] = x_updated(x[i], c, Z, n, i);
             return;

@@ -130,37 +130,29 @@ __device__ __forceinline__ void write_ctrl(Ctrl* __restrict__ dst, const Ctrl& c
 }
 
 // Sum of G partials in fixed order, returned to every thread of the block.
-__device__ __forceinline__ double all_sum(const double* __restrict__ part, int G, double* red,
-                                          double* bcast)
+// red: as block_sum_all.
+__device__ __forceinline__ double all_sum(const double* __restrict__ part, int G, double* red)
 {
-    const double s = sum_partials(part, G, red);
-    if (threadIdx.x == 0) *bcast = s;
-    __syncthreads();
-    const double v = *bcast;
-    __syncthreads();
-    return v;
+    return block_sum_all(strided_sum(part, G), red);
 }
 
-// Two folds at once, each in all_sum's order (thread-strided sums, then the
-// block tree of block_sum): one pass over both partial arrays.
-__device__ __forceinline__ void all_sum2(const double* __restrict__ pa, const double* __restrict__ pb,
-                                         int G, double* red /* 2*kWaves */, double* bcast /* 2 */,
-                                         double& a, double& b)
+// Two folds at once, each in all_sum's order, from the threads' parts.
+__device__ __forceinline__ void all_sum2(double sa, double sb, double* red /* 2*kWaves */, double& a, double& b)
 {
-    double sa = 0.0, sb = 0.0;
-    for (int i = threadIdx.x; i < G; i += kBlock) {
-        sa = sa + pa[i];
-        sb = sb + pb[i];
-    }
-    block_sum2(sa, sb, red);
-    if (threadIdx.x == 0) {
-        bcast[0] = sa;
-        bcast[1] = sb;
+    sa = wave_sum(sa);
+    sb = wave_sum(sb);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) {
+        red[wave] = sa;
+        red[kWaves + wave] = sb;
     }
     __syncthreads();
-    a = bcast[0];
-    b = bcast[1];
-    __syncthreads();
+    a = b = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        a = a + red[w];
+        b = b + red[kWaves + w];
+    }
 }
 
 // Balanced contiguous ranges: logical block lb of G owns units [u0, u1).
@@ -480,13 +472,14 @@ __device__ __forceinline__ void replace_residual(const MatView& A, const ResArgs
 // Folds pending set-up or replacement partials into the token (every block,
 // same order) and decides whether the iteration runs.
 __device__ __forceinline__ void fold_pending(Ctrl& c, const double* __restrict__ rpart, int Gr,
-                                             const Prm& P, double* red, double* bcast)
+                                             const Prm& P, double* red /* 2*kWaves */)
 {
-    const double rz = all_sum(rpart, Gr, red, bcast);
-    const double rr = all_sum(rpart + Gr, Gr, red, bcast);
+    double rz, rr;
+    all_sum2(strided_sum(rpart, Gr), strided_sum(rpart + Gr, Gr), red, rz, rr);
     const double rn = sqrt(rr);
+    __syncthreads();
     if (c.reduce == kReduceSetup) {
-        const double bb = all_sum(rpart + 2 * Gr, Gr, red, bcast);
+        const double bb = all_sum(rpart + 2 * Gr, Gr, red);
         c.bnorm = sqrt(bb);
         c.norm0 = rn;
         c.eps = eps_from(P, c.bnorm, rn);
@@ -798,9 +791,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     constexpr bool MIXED = sizeof(VT) == 4;
     __shared__ K1Stage<VT, FMT, LONG> sm;
     __shared__ double red[3 * kWaves];
-    __shared__ double bcast;
+    __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
-    if (c.reduce != kReduceNone) fold_pending(c, R.part, R.G, P, red, &bcast);
+    if (c.reduce != kReduceNone) fold_pending(c, R.part, R.G, P, fred);
     if (!c.run) {
         write_ctrl(cout, c);
         return;
@@ -848,8 +841,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     constexpr bool MIXED = sizeof(VT) == 4;
     __shared__ K1Stage<VT, FMT, LONG> sm;
     __shared__ double red[3 * kWaves];
-    __shared__ double bcast[2];
+    __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
+    // the partials' loads do not wait for the token
+    const double sz = strided_sum(part2, G2), sr = strided_sum(part2 + G2, G2);
     if (!c.run) {
         write_ctrl(cout, c);
         return;
@@ -867,10 +862,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     }
     const bool pending = c.reduce != kReduceNone;
     if (pending) {
-        fold_pending(c, R.part, R.G, P, red, bcast);
+        fold_pending(c, R.part, R.G, P, fred);
     } else {
         double rz, rr;
-        all_sum2(part2, part2 + G2, G2, red, bcast, rz, rr);
+        all_sum2(sz, sr, fred, rz, rr);
         next_scalars<MIXED>(c, rz, rr, P);
     }
     const VT sigma = VT(c.sigma), beta = VT(c.beta);
@@ -1000,8 +995,9 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
                                                          Ctrl* __restrict__ cout)
 {
     __shared__ double red[2 * kWaves];
-    __shared__ double bcast;
+    __shared__ double fred[kWaves];
     Ctrl c = read_ctrl(cin);
+    const double sv = strided_sum(vpart, G1);  // (its loads do not wait for the token)
     // a slot without a product: a replacement was requested (ru) or its
     // residual is pending (reduce)
     if (!c.run || c.ru || c.reduce != kReduceNone) {
@@ -1017,7 +1013,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
     unit_range((n + unit - 1) / unit, G, lb, u0, u1);
     const long long lo = u0 * unit, hi = min(u1 * unit, n);
     long long i = lo + (long long)threadIdx.x * W;
-    const double vp = all_sum(vpart, G1, red, &bcast);
+    const double vp = block_sum_all(sv, fred);
     const double sigma = c.alpha / vp;
     if (!(vp > 0.0) || !isfinite(sigma)) {
         c.status = CEL_ERR_BREAKDOWN;
@@ -1117,14 +1113,14 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
                                                           Ctrl* __restrict__ cout, Prm P)
 {
     __shared__ double red[2 * kWaves];
-    __shared__ double bcast[2];
     Ctrl c = read_ctrl(cin);
+    const double sz = strided_sum(rpart, G2), sr = strided_sum(rpart + G2, G2);
     if (!c.run || c.reduce != kReduceNone) {
         write_ctrl(cout, c);
         return;
     }
     double rz, rr;
-    all_sum2(rpart, rpart + G2, G2, red, bcast, rz, rr);  // r.z and r.r in one pass
+    all_sum2(sz, sr, red, rz, rr);
     const VT sigma = VT(c.sigma);
     // scalars of the next iteration (they do not depend on the vectors)
     next_scalars<MIXED>(c, rz, rr, P);
