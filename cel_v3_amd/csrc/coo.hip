@@ -171,14 +171,19 @@ k_starts(long long nnz, const int* __restrict__ head, const int* __restrict__ ih
     }
 }
 
-// Groups of at most kSmall entries, one thread each: the rank of entry j is
-// #{k : col_k < col_j} + #{k < j : col_k == col_j}, i.e. the stable order by
-// column, and entry j goes to slot rank.  A workgroup takes 256 consecutive
-// groups; when their entries fit (kTileCap) they are loaded into LDS and
-// written back with coalesced accesses, otherwise each thread works on its
-// group in global memory.  Longer groups are left in place here and listed
-// for k_group_medium (order of the list is free: groups are independent).
+// Groups of at most kSmall entries: the rank of entry j is #{k : col_k <
+// col_j} + #{k < j : col_k == col_j}, i.e. the stable order by column, and
+// entry j goes to slot rank.  A workgroup takes 256 consecutive groups; when
+// their entries fit (kTileCap) the columns go to LDS, with each entry's
+// group beside it, and every thread ranks up to 8 entries, which it holds in
+// registers (neighbouring lanes compare within the same group, so their LDS
+// reads coincide; a thread per group with the entries staged in and out
+// of 66 KB of LDS took 331 us for the 14.6M entries of a 128^3 block, 118 us
+// so).  Otherwise each thread works on its group in global memory.  Longer
+// groups are left in place here and listed for k_group_medium (order of the
+// list is free: groups are independent).
 constexpr int kTileCap = 2048;
+constexpr int kPerThread = kTileCap / kThreads;
 
 __global__ void __launch_bounds__(kThreads)
 k_group_small(int G, const int* __restrict__ starts, const uint32_t* __restrict__ rk,
@@ -187,8 +192,8 @@ k_group_small(int G, const int* __restrict__ starts, const uint32_t* __restrict_
               int* __restrict__ maxlen)
 {
     __shared__ int st[kThreads + 1];
-    __shared__ uint32_t in_rk[kTileCap], out_rk[kTileCap];
-    __shared__ Pay in_pay[kTileCap], out_pay[kTileCap];
+    __shared__ uint32_t col[kTileCap];
+    __shared__ uint32_t grp[kTileCap];  // first entry of the group | entries << 16
     const int tid = threadIdx.x;
     for (long long g0 = (long long)blockIdx.x * kThreads; g0 < G; g0 += (long long)gridDim.x * kThreads) {
         const int ng = (int)min((long long)kThreads, G - g0);
@@ -207,36 +212,41 @@ k_group_small(int G, const int* __restrict__ starts, const uint32_t* __restrict_
             }
         }
         if (E <= kTileCap) {
-            const uint32_t* p32 = reinterpret_cast<const uint32_t*>(pay + base);
-            uint32_t* l32 = reinterpret_cast<uint32_t*>(in_pay);
-            for (int i = tid; i < 3 * E; i += kThreads) l32[i] = p32[i];
-            for (int i = tid; i < E; i += kThreads) in_rk[i] = rk[base + i];
-            __syncthreads();
-            if (tid < ng) {
-                if (L <= kSmall) {
-                    for (int j = 0; j < L; ++j) {
-                        const uint32_t cj = in_pay[s + j].col;
-                        int r = 0;
-                        for (int k = 0; k < L; ++k) {
-                            const uint32_t ck = in_pay[s + k].col;
-                            r += ck < cj || (ck == cj && k < j);
-                        }
-                        out_pay[s + r] = in_pay[s + j];
-                        out_rk[s + r] = in_rk[s + j];
-                    }
-                } else {  // k_group_medium rewrites this group later
-                    for (int j = 0; j < L; ++j) {
-                        out_pay[s + j] = in_pay[s + j];
-                        out_rk[s + j] = in_rk[s + j];
-                    }
+            Pay q[kPerThread];
+            uint32_t row[kPerThread];
+#pragma unroll
+            for (int k = 0; k < kPerThread; ++k) {
+                const int i = tid + k * kThreads;
+                if (i < E) {
+                    q[k] = pay[base + i];
+                    row[k] = rk[base + i];
                 }
             }
+            // a longer group's entries keep their places (k_group_medium
+            // rewrites it later): groups of one entry each
+            for (int j = 0; j < L; ++j)
+                grp[s + j] = L <= kSmall ? (uint32_t)s | ((uint32_t)L << 16) : (uint32_t)(s + j) | (1u << 16);
+#pragma unroll
+            for (int k = 0; k < kPerThread; ++k) {
+                const int i = tid + k * kThreads;
+                if (i < E) col[i] = q[k].col;
+            }
             __syncthreads();
-            for (int i = tid; i < E; i += kThreads) {
-                const Pay q = out_pay[i];
-                rows[base + i] = (int)out_rk[i] + rbase;
-                cols[base + i] = (int)q.col + cbase;
-                vals[base + i] = pay_val(q);
+#pragma unroll
+            for (int k = 0; k < kPerThread; ++k) {
+                const int i = tid + k * kThreads;
+                if (i < E) {
+                    const int gs = (int)(grp[i] & 0xffffu), gl = (int)(grp[i] >> 16);
+                    const uint32_t ci = q[k].col;
+                    int r = gs;
+                    for (int e = gs; e < gs + gl; ++e) {
+                        const uint32_t ce = col[e];
+                        r += ce < ci || (ce == ci && e < i);
+                    }
+                    rows[base + r] = (int)row[k] + rbase;
+                    cols[base + r] = (int)ci + cbase;
+                    vals[base + r] = pay_val(q[k]);
+                }
             }
         } else if (tid < ng && L <= kSmall) {
             const int gs = base + s;
@@ -336,25 +346,33 @@ k_rows_monotone(long long nnz, const int* __restrict__ rows, int* __restrict__ b
 }
 
 // cel_sp_mat_to_csr: counts per row, then a scan.  cnt has nrows+1 slots;
-// rows outside [0, nrows) are counted nowhere (flagged by k_rows_in_range).
+// rows outside [0, nrows) are counted nowhere and flagged.  A wavefront's
+// runs of equal rows are counted by one atomic each: entries mostly come
+// row-sorted, and one atomic per entry on neighbouring counters took 0.50 ms
+// for the 14.6M entries of a 128^3 block (and a pass of its own for the
+// range check) against 30 us so.
 __global__ void __launch_bounds__(kThreads)
 k_row_count(long long nnz, const int* __restrict__ rows, int rbase, int nrows,
-            int* __restrict__ cnt)
+            int* __restrict__ cnt, int* __restrict__ bad)
 {
-    CEL_GRID_STRIDE(p, nnz) {
-        long long r = (long long)rows[p] - rbase;
-        if (r >= 0 && r < nrows) atomicAdd(&cnt[r + 1], 1);
-    }
-}
-
-__global__ void __launch_bounds__(kThreads)
-k_rows_in_range(long long nnz, const int* __restrict__ rows, int rbase, int nrows,
-                int* __restrict__ bad)
-{
+    const int lane = threadIdx.x & 63;
     int any = 0;
-    CEL_GRID_STRIDE(p, nnz) {
-        long long r = (long long)rows[p] - rbase;
-        any |= r < 0 || r >= nrows;
+    for (long long p0 = (long long)blockIdx.x * kThreads; p0 < nnz; p0 += (long long)gridDim.x * kThreads) {
+        const long long p = p0 + threadIdx.x;
+        long long r = p < nnz ? (long long)rows[p] - rbase : -1;
+        if (r < 0 || r >= nrows) {
+            any |= p < nnz;
+            r = -1;
+        }
+        const int ri = (int)r;
+        const int before = __shfl_up(ri, 1, 64);
+        const bool head = lane == 0 || ri != before;
+        const unsigned long long heads = __ballot(head);
+        if (head && ri >= 0) {
+            const unsigned long long later = lane < 63 ? heads >> (lane + 1) : 0ull;
+            const int len = later ? __ffsll((long long)later) : 64 - lane;
+            atomicAdd(&cnt[ri + 1], len);
+        }
     }
     if (any) atomicOr(bad, 1);
 }
@@ -562,8 +580,7 @@ int row_offsets_device(int nrows, long long nnz, const int* rows, int rbase, int
     k_fill_int<<<grid_for(nrows + 1LL), kThreads, 0, st>>>(nrows + 1LL, cnt, 0);
     k_fill_int<<<1, 1, 0, st>>>(1, cnt, out_base);  // xadj[0] = out_base carries through the scan
     if (nnz > 0) {
-        k_rows_in_range<<<grid_for(nnz), kThreads, 0, st>>>(nnz, rows, rbase, nrows, flag);
-        k_row_count<<<grid_for(nnz), kThreads, 0, st>>>(nnz, rows, rbase, nrows, cnt);
+        k_row_count<<<grid_for(nnz), kThreads, 0, st>>>(nnz, rows, rbase, nrows, cnt, flag);
     }
     CEL_HIP(hipGetLastError());
     int bad = 0;

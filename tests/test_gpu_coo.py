@@ -272,3 +272,27 @@ def test_dense_short_rows_overflow_the_lds_tile(gpu):
     r1, c1, v1 = O.coo_sort_rowcol(rows, cols, vals)
     _, r, c, v = gpu.coo_sort(n, rows, cols, vals, ncols=50, mode=gpu.SORT_ROW_COL)
     _check_same((r, c, v), (r1, c1, v1))
+
+
+@pytest.mark.parametrize("lens", [[2048], [8] * 256, [8] * 255 + [9], [1] * 300, [32] * 64 + [33] * 3, [31, 0, 5] * 90,
+                                  [0] * 70 + [40, 1, 1] * 10 + [7] * 300], ids=lambda v: f"{len(v)}x{v[0]}")
+def test_group_tiles_and_row_runs(gpu, lens):
+    """The (row, column) order at the edges of the 2,048-entry tiles and of the
+    32-entry groups, with repeated columns, and row counts over runs that
+    cross wavefronts, sorted and shuffled."""
+    rng = np.random.default_rng(61)
+    n = len(lens)
+    rows = np.repeat(np.arange(1, n + 1), lens)
+    cols = rng.integers(1, 60, rows.size)
+    vals = rng.normal(size=rows.size)
+    order = rng.permutation(rows.size)
+    r, c, v = rows[order], cols[order], vals[order]
+    rc, sr, sc, sv = gpu.coo_sort(n, r, c, v, ncols=60, mode=gpu.SORT_ROW_COL)
+    ref = np.lexsort((np.arange(r.size), c, r))
+    assert rc == 0
+    np.testing.assert_array_equal(sr, r[ref])
+    np.testing.assert_array_equal(sc, c[ref])
+    np.testing.assert_array_equal(sv, v[ref])
+    xadj = 1 + np.concatenate([[0], np.cumsum(lens)])
+    np.testing.assert_array_equal(gpu.coo_row_offsets(n, sr), xadj)
+    np.testing.assert_array_equal(gpu.coo_row_offsets(n, r), xadj)
