@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -30,6 +31,96 @@ Runtime& rt()
 {
     static Runtime r;
     return r;
+}
+
+namespace {
+struct Pool {
+    std::mutex mu;
+    std::map<int, std::multimap<size_t, void*>> free;  // by device: size -> block
+    size_t held = 0;
+};
+Pool& pool()
+{
+    static Pool* p = new Pool;  // outlives every buffer with static storage
+    return *p;
+}
+// with the lock held; the calling thread's device is `device`
+void pool_drop(Pool& P, int device)
+{
+    const auto d = P.free.find(device);
+    if (d == P.free.end()) return;
+    for (auto& b : d->second) {
+        P.held -= b.first;
+        (void)hipFree(b.second);
+    }
+    d->second.clear();
+}
+}  // namespace
+
+void* pool_alloc(size_t bytes, size_t* got, int* device)
+{
+    Pool& P = pool();
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    *device = dev;
+    // whole 2 MB pieces for large blocks, so that near sizes share them
+    const size_t unit = bytes >= (size_t(1) << 20) ? size_t(2) << 20 : 512;
+    const size_t want = (bytes + unit - 1) / unit * unit;
+    *got = want;
+    void* p = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(P.mu);
+        const auto d = P.free.find(dev);
+        if (d != P.free.end()) {
+            const auto it = d->second.lower_bound(want);
+            if (it != d->second.end() && it->first <= want + want / 4) {
+                p = it->second;
+                *got = it->first;
+                P.held -= it->first;
+                d->second.erase(it);
+            }
+        }
+    }
+    if (p) {
+        if (rt().stream) (void)hipStreamSynchronize(rt().stream);
+        return p;
+    }
+    if (hipMalloc(&p, want) == hipSuccess) return p;
+    (void)hipGetLastError();
+    {
+        std::lock_guard<std::mutex> lock(P.mu);
+        pool_drop(P, dev);
+    }
+    if (hipMalloc(&p, want) == hipSuccess) return p;
+    return nullptr;
+}
+
+void pool_free(void* p, size_t bytes, int device)
+{
+    Pool& P = pool();
+    try {
+        std::lock_guard<std::mutex> lock(P.mu);
+        if (bytes <= kPoolBytes / 2 && P.held + bytes <= kPoolBytes && rt().ready) {
+            P.free[device].emplace(bytes, p);
+            P.held += bytes;
+            return;
+        }
+    } catch (...) {  // no host memory for the list
+    }
+    (void)hipFree(p);
+}
+
+void pool_release()
+{
+    Pool& P = pool();
+    std::lock_guard<std::mutex> lock(P.mu);
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    for (auto& d : P.free) {
+        (void)hipSetDevice(d.first);
+        pool_drop(P, d.first);
+    }
+    (void)hipSetDevice(dev);
 }
 
 int resident_grid(const void* kernel, long long work_items)
@@ -84,6 +175,7 @@ extern "C" int cel_gpu_finalize(void)
     if (!R.ready) return CEL_OK;
     (void)hipStreamSynchronize(R.stream);
     coo_release_workspace();
+    pool_release();
     (void)hipStreamDestroy(R.stream);
     R.stream = nullptr;
     R.ready = false;

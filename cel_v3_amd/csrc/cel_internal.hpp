@@ -47,11 +47,25 @@ int ensure_init();
 // persistent grid never exceeds this, so no block waits for a second wave.
 int resident_grid(const void* kernel, long long work_items);
 
+// Device memory of the library's buffers.  A freed block is kept for the next
+// buffer of about its size instead of going back to the driver, whose
+// allocations and (synchronising) frees of large blocks cost 0.1-0.2 ms
+// each.  Kept blocks are bounded (kPoolBytes in all), go back when an
+// allocation fails and with cel_gpu_finalize.  A reused block may still be
+// read by work on the library's stream, so that is waited for before it is
+// handed out; the lists are per device and locked.
+constexpr size_t kPoolBytes = size_t(2) << 30;
+void* pool_alloc(size_t bytes, size_t* got, int* device);  // null: no memory
+void pool_free(void* p, size_t bytes, int device);
+void pool_release();
+
 // Device buffer owned by the library.
 template <typename T>
 struct DevBuf {
     T* p = nullptr;
     size_t n = 0;
+    size_t bytes = 0;  // of the block
+    int device = -1;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
@@ -60,8 +74,8 @@ struct DevBuf {
         if (count == n && p) return CEL_OK;
         release();
         if (count == 0) return CEL_OK;
-        if (hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T)) != hipSuccess) {
-            p = nullptr;
+        p = static_cast<T*>(pool_alloc(count * sizeof(T), &bytes, &device));
+        if (!p) {
             return fail(CEL_ERR_OOM, "hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed");
         }
         n = count;
@@ -74,7 +88,7 @@ struct DevBuf {
         return alloc(count);
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) pool_free(p, bytes, device);
         p = nullptr;
         n = 0;
     }
@@ -297,7 +311,7 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max);
 // every row's columns strictly ascend (known only when *nd <= most).
 int dia_offsets(const Mat& A, int most, int* nd, int* off, bool* ascending);
 // Diagonal-major values (v64, or v32 rounded to FP32) and row masks on at
-// most 8 diagonals; slots without an entry are left as they are.
+// most 8 diagonals; slots without an entry hold 0.
 int dia_fill(const Mat& A, int nd, const int* off, double* v64, float* v32, uint8_t* mask8);
 // Sets bit `bit` (= dia_nd) of the DIA row masks on the rows with halo
 // entries and clears it elsewhere; fails when the masks have no spare bit.
