@@ -36,6 +36,7 @@
 #include <chrono>
 #include <cmath>
 #include <initializer_list>
+#include <thread>
 #include <vector>
 
 #include "cel_internal.hpp"
@@ -54,6 +55,8 @@ struct Ctrl {
     int outer;   // mixed: replacements done
     int since;   // mixed: iterations since the last replacement
     int stall;   // mixed: consecutive replacements that did not halve the FP64 residual
+    int slots;   // finished slots (launch groups of one iteration or replacement)
+    int pad;
 };
 
 // Constant solver parameters.
@@ -104,6 +107,8 @@ __device__ __forceinline__ Ctrl read_ctrl(const Ctrl* __restrict__ p)
     c.outer = p->outer;
     c.since = p->since;
     c.stall = p->stall;
+    c.slots = p->slots;
+    c.pad = 0;
     return c;
 }
 
@@ -126,7 +131,27 @@ __device__ __forceinline__ void write_ctrl(Ctrl* __restrict__ dst, const Ctrl& c
         dst->outer = c.outer;
         dst->since = c.since;
         dst->stall = c.stall;
+        dst->slots = c.slots;
+        dst->pad = c.pad;
     }
+}
+
+// End of a slot, in its last kernel: the token, and the host's progress
+// word (may be null): slots finished, or -1 once the solve has stopped.
+__device__ __forceinline__ void end_slot(Ctrl* __restrict__ dst, Ctrl& c, int* progress)
+{
+    c.slots = c.slots + 1;
+    write_ctrl(dst, c);
+    if (progress && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(progress, c.run ? c.slots : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A fresh token.
+__global__ void k_token(Ctrl* c)
+{
+    Ctrl t{};
+    t.run = 1;
+    write_ctrl(c, t);
 }
 
 // Sum of G partials in fixed order, returned to every thread of the block.
@@ -992,16 +1017,21 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
                                                          double* __restrict__ part,
                                                          const double* __restrict__ vpart, int G1,
                                                          const Ctrl* __restrict__ cin,
-                                                         Ctrl* __restrict__ cout)
+                                                         Ctrl* __restrict__ cout, int* progress)
 {
     __shared__ double red[2 * kWaves];
     __shared__ double fred[kWaves];
     Ctrl c = read_ctrl(cin);
+    // (in the two-kernel form K2 ends the slot)
+    auto done = [&]() {
+        if constexpr (ZOUT) end_slot(cout, c, progress);
+        else write_ctrl(cout, c);
+    };
     const double sv = strided_sum(vpart, G1);  // (its loads do not wait for the token)
     // a slot without a product: a replacement was requested (ru) or its
     // residual is pending (reduce)
     if (!c.run || c.ru || c.reduce != kReduceNone) {
-        write_ctrl(cout, c);
+        done();
         return;
     }
     using V = typename Vec<VT>::T;
@@ -1018,7 +1048,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
     if (!(vp > 0.0) || !isfinite(sigma)) {
         c.status = CEL_ERR_BREAKDOWN;
         c.run = 0;
-        write_ctrl(cout, c);
+        done();
         return;
     }
     c.sigma = sigma;
@@ -1095,7 +1125,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
         part[lb] = arz;
         part[G + lb] = arr;
     }
-    write_ctrl(cout, c);
+    done();
 }
 
 // K3: beta = sum(r.z)/alpha ; x = x + sigma p ; p = beta p + jac*r ;
@@ -1110,13 +1140,13 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
                                                           double* __restrict__ x64,
                                                           const double* __restrict__ rpart, int G2,
                                                           const Ctrl* __restrict__ cin,
-                                                          Ctrl* __restrict__ cout, Prm P)
+                                                          Ctrl* __restrict__ cout, Prm P, int* progress)
 {
     __shared__ double red[2 * kWaves];
     Ctrl c = read_ctrl(cin);
     const double sz = strided_sum(rpart, G2), sr = strided_sum(rpart + G2, G2);
     if (!c.run || c.reduce != kReduceNone) {
-        write_ctrl(cout, c);
+        end_slot(cout, c, progress);
         return;
     }
     double rz, rr;
@@ -1222,7 +1252,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
             }
         }
     }
-    write_ctrl(cout, c);
+    end_slot(cout, c, progress);
 }
 
 // Mixed form, replacement step 1: x64 = x64 + e32 ; e32 = 0.
@@ -1257,7 +1287,53 @@ struct Workspace {
     DevBuf<float> jacp32;
     DevBuf<Ctrl> ctrl;
     DevBuf<int> hrow_tile;
+    // pinned: the progress word the kernels write and the final token
+    struct Host {
+        int progress;
+        int pad[31];
+        Ctrl ctrl;
+    };
+    Host* host = nullptr;
+    int host_alloc()
+    {
+        if (host) return CEL_OK;
+        void* q = nullptr;
+        if (hipHostMalloc(&q, sizeof(Host), hipHostMallocCoherent) != hipSuccess)
+            return fail(CEL_ERR_OOM, "hipHostMalloc failed");
+        host = static_cast<Host*>(q);
+        return CEL_OK;
+    }
+    ~Workspace()
+    {
+        if (host) (void)hipHostFree(host);
+    }
 };
+
+// Waits until the solve's kernels have finished `upto` slots (1), or stopped
+// (0), or there is an error (< 0).  The word is in host memory, so looking
+// at it costs the stream nothing.
+static int wait_progress(hipStream_t s, const volatile int* progress, long long upto)
+{
+    auto last = std::chrono::steady_clock::now();
+    for (;;) {
+        for (int k = 0; k < 512; ++k) {
+            const int v = *progress;
+            if (v < 0) return 0;
+            if (v >= upto) return 1;
+            __builtin_ia32_pause();
+        }
+        const auto now = std::chrono::steady_clock::now();
+        if (now - last < std::chrono::milliseconds(1)) continue;
+        last = now;
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) {
+            std::this_thread::yield();
+            continue;
+        }
+        if (e != hipSuccess) return fail(CEL_ERR_HIP, std::string("the solve's kernels: ") + hipGetErrorString(e));
+        return *progress < 0 ? 0 : 1;  // everything enqueued has run
+    }
+}
 
 static Workspace& ws_of(Mat& A)
 {
@@ -1749,11 +1825,15 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     P.ru_max_inner = 1000;
     P.hist = hist_cap ? Wp->hist.p : nullptr;
     P.hist_cap = hist_cap;
-    Ctrl c0{};
-    c0.run = 1;
     // every solve starts from a fresh token (the scratch array keeps the
     // last call's contents; everything else is written before it is read)
-    CEL_HIP(hipMemcpyAsync(w.ctrl, &c0, sizeof(Ctrl), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_token, dim3(1), dim3(64), 0, s, w.ctrl);
+    int* progress = nullptr;
+    if (!noalloc) {
+        CEL_TRY(Wp->host_alloc());
+        Wp->host->progress = 0;
+        progress = &Wp->host->progress;
+    }
     // token slots: 0 -> K1 -> 1 -> K2 -> 2 -> K3 -> 0 (FP64);
     // (two-kernel form: 0 -> step -> 1 -> K2 -> 0)
     Ctrl* C0 = w.ctrl;
@@ -1886,7 +1966,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
                                (const double*)pbuf[in], (const double*)zbuf, pbuf[out], dx, (double*)nullptr, w.v,
                                w.part1, R64, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
             hipLaunchKernelGGL((k_pcg_update_r<double, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
-                               jac64, nocls, zbuf, w.part2, w.part1, G1, C1, C0);
+                               jac64, nocls, zbuf, w.part2, w.part1, G1, C1, C0, progress);
         } else {
             ResArgs<float> R = R32;
             R.p = pbuf32[out];  // a restart's direction
@@ -1894,7 +1974,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
                                (const float*)pbuf32[in], (const float*)zbuf32, pbuf32[out], w.e32, dx, w.v32,
                                w.part1, R, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
             hipLaunchKernelGGL((k_pcg_update_r<float, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
-                               jac32, nocls, zbuf32, w.part2, w.part1, G1, C1, C0);
+                               jac32, nocls, zbuf32, w.part2, w.part1, G1, C1, C0, progress);
         }
         CEL_HIP(hipGetLastError());
         return CEL_OK;
@@ -1921,37 +2001,37 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
                                w.part1, R64, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL((bycls ? k_pcg_update_r<double, false, true> : k_pcg_update_r<double, false, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v, vjac64, vcls, (double*)nullptr, w.part2, w.part1, G1, C1, C2);
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v, vjac64, vcls, (double*)nullptr, w.part2, w.part1, G1, C1, C2,
+                               (int*)nullptr);
             hipLaunchKernelGGL((bycls ? k_pcg_update_xp<double, double, false, true>
                                       : k_pcg_update_xp<double, double, false, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, dx, w.p, w.r, vjac64, vcls, nullptr, w.part2, Gv, C2, C0, P);
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, dx, w.p, w.r, vjac64, vcls, nullptr, w.part2, Gv, C2, C0, P, progress);
         } else {
             hipLaunchKernelGGL(k1_kernel<float>(kfmt, false, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
                                w.part1, R32, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL((bycls ? k_pcg_update_r<float, false, true> : k_pcg_update_r<float, false, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32, vjac32, vcls, (float*)nullptr, w.part2, w.part1, G1, C1, C2);
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32, vjac32, vcls, (float*)nullptr, w.part2, w.part1, G1, C1, C2,
+                               (int*)nullptr);
             hipLaunchKernelGGL((bycls ? k_pcg_update_xp<float, float, true, true>
                                       : k_pcg_update_xp<float, float, true, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.e32, w.p32, w.r32, vjac32, vcls, dx, w.part2, Gv, C2, C0, P);
+                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.e32, w.p32, w.r32, vjac32, vcls, dx, w.part2, Gv, C2, C0, P, progress);
         }
         CEL_HIP(hipGetLastError());
         return CEL_OK;
     };
 
-    // iteration loop: chunks of `chunk` iterations, one chunk in flight
-    // ahead of the host's check of the token.  The loop needs at most
-    // iter_max iterations plus one K1 that folds in the final partials.
+    // iteration loop.  The loop needs at most iter_max iterations plus one
+    // K1 that folds in the final partials.  The host runs a few slots ahead
+    // of the progress word, so few launches find the solve stopped (a flag
+    // copied back every 16 iterations, one chunk late, left 17 to 47 of them
+    // and a copy a chunk: 1.78 against 1.51 ms for a 32^3 solve of 104
+    // iterations); replayed graphs go chunk by chunk, one chunk ahead.  The
+    // allocation-free solve, which has no host memory, reads the token after
+    // every chunk.
     const int chunk = prm.check_every > 0 ? prm.check_every : 16;
-    int* hrun = nullptr;
-    int hrun_sync = 1;  // the allocation-free solve reads the flag synchronously
-    hipEvent_t cev[2] = {nullptr, nullptr};
-    if (!noalloc) {
-        CEL_TRY(R.host_alloc(hrun, 2));
-        hrun[0] = hrun[1] = 1;
-        CEL_TRY(R.event(cev[0], hipEventDisableTiming));
-        CEL_TRY(R.event(cev[1], hipEventDisableTiming));
-    }
+    const long long ahead = std::min(std::max(chunk, 2), 8);
+    int hrun_sync = 1;
 
     // (a captured chunk of the two-kernel form starts at an even slot)
     const bool use_graph = prm.use_graph && !prm.profile && !noalloc && !(step && (chunk & 1));
@@ -1960,9 +2040,8 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     // form), and there is at most one per iteration
     const long long budget = (long long)(mixed ? (step ? 3 : 2) : 1) * ((long long)prm.iter_max + 1);
     long long enqueued = 0;
-    int k = 0;
     while (enqueued < budget) {
-        const int c = (int)std::min<long long>(chunk, budget - enqueued);
+        const int c = (int)std::min<long long>(use_graph || noalloc ? chunk : 1, budget - enqueued);
         if (use_graph && c == chunk) {
             if (!R.exec) {
                 CEL_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -1989,16 +2068,11 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             CEL_HIP(hipMemcpyAsync(&hrun_sync, &C0->run, sizeof(int), hipMemcpyDeviceToHost, s));
             CEL_HIP(hipStreamSynchronize(s));
             if (!hrun_sync) break;
-            ++k;
             continue;
         }
-        CEL_HIP(hipMemcpyAsync(&hrun[k & 1], &C0->run, sizeof(int), hipMemcpyDeviceToHost, s));
-        CEL_HIP(hipEventRecord(cev[k & 1], s));
-        if (k > 0) {
-            CEL_HIP(hipEventSynchronize(cev[(k - 1) & 1]));
-            if (!hrun[(k - 1) & 1]) break;
-        }
-        ++k;
+        status = wait_progress(s, progress, enqueued - (use_graph ? chunk : ahead));
+        if (status <= 0) break;
+        status = CEL_OK;
     }
     if (mixed) {
         // a budget that ran out mid-way leaves a correction in e: fold it in
@@ -2010,11 +2084,17 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         CEL_HIP(hipGetLastError());
     }
     if (!noalloc) CEL_HIP(hipEventRecord(e2, s));
-    CEL_HIP(hipStreamSynchronize(s));
-    if (status < 0) return status;
-
     Ctrl out;
-    CEL_HIP(hipMemcpy(&out, C0, sizeof(Ctrl), hipMemcpyDeviceToHost));
+    if (noalloc) {
+        CEL_HIP(hipStreamSynchronize(s));
+        if (status < 0) return status;
+        CEL_HIP(hipMemcpy(&out, C0, sizeof(Ctrl), hipMemcpyDeviceToHost));
+    } else {
+        CEL_HIP(hipMemcpyAsync(&Wp->host->ctrl, C0, sizeof(Ctrl), hipMemcpyDeviceToHost, s));
+        CEL_HIP(hipStreamSynchronize(s));
+        if (status < 0) return status;
+        out = Wp->host->ctrl;
+    }
     float ms_setup = 0, ms_all = 0;
     if (!noalloc) {
         CEL_HIP(hipEventElapsedTime(&ms_setup, e0, e1));

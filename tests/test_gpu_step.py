@@ -50,7 +50,7 @@ def test_two_kernel_iterations_are_the_three_kernel_ones(gpu, shape, mixed):
                            for extra in (dict(), dict(use_graph=1), dict(use_graph=1, check_every=5)))
                 continue
             assert three["iters"] <= kw["iter_max"]
-            for extra in (dict(), dict(use_graph=1), dict(use_graph=1, check_every=5)):
+            for extra in (dict(), dict(check_every=1), dict(use_graph=1), dict(use_graph=1, check_every=5)):
                 two = solve(gpu, M, b, **kw, **extra)
                 assert (two["status"], two["iters"], two["outer_iters"]) == \
                     (three["status"], three["iters"], three["outer_iters"])
