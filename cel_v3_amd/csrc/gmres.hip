@@ -426,7 +426,7 @@ template <int FMT, typename X>
 __device__ __forceinline__ void two_rows(const GmMat& A, const int (&r)[2], const X& x, double (&s)[2])
 {
     if constexpr (FMT == CEL_FMT_DIA) {
-        if (r[0] < A.n) dia_rows<double, 2, 4>(A.n, A.nd, A.off, A.dvals, A.mask8, A.mask, r, x, s);
+        if (r[0] < A.n) dia_rows<double, 2, 4, true>(A.n, A.nd, A.off, A.dvals, A.mask8, A.mask, r, x, s);
     } else {
 #pragma unroll
         for (int k = 0; k < 2; ++k) {

@@ -577,8 +577,8 @@ struct StepRows {
 // thread's part of v.d.  STEP: X is XDirection, and d and the updated x of
 // every row are stored as well.  (Taking a step's scalars behind the first
 // tile's gathers instead of before them measured slower, 32^3 12.7 against
-// 12.3 us per iteration.)
-template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, typename X>
+// 12.3 us per iteration.)  KEEP: keep_matrix().
+template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, bool KEEP, typename X>
 __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __restrict__ v,
                                            typename StageOf<VT, FMT, LONG>::T& sm,
                                            const StepRows<VT>& st, int walk = 0)
@@ -610,7 +610,7 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
         // record and read count 0.  Each loaded value is used once in the
         // step after it, in place: a copy of a register still being loaded
         // would wait for every load issued before it.
-        typename CsrStreamOf<VT, LONG>::Stream cs;
+        typename CsrStreamOf<VT, LONG, KEEP>::Stream cs;
         const VT* vals = csr_vals<VT>(A);
         const long long tfirst = group_tile(0, ntiles);
         const auto rrec = tile_rsrc(HALO ? A.hrec : nullptr, HALO ? A.hnq * 16 : 0);
@@ -742,8 +742,8 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
                     for (int k = 0; k < R; ++k) xo[k] = st.x[r[k] < A.n ? r[k] : r[0]];
                 }
                 // x[row] comes from the loads of the diagonal with offset 0
-                dia_rows<VT, R, (R >= 4 ? 4 : 8)>(A.n, A.nd, A.doff, dia_vals<VT>(A), A.dmask8,
-                                                   A.dmask, r, x, s, pr, A.dzero);
+                dia_rows<VT, R, (R >= 4 ? 4 : 8), KEEP>(A.n, A.nd, A.doff, dia_vals<VT>(A), A.dmask8,
+                                                        A.dmask, r, x, s, pr, A.dzero);
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
                     if (r[k] < A.n) {
@@ -775,7 +775,7 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
         // JAD in the permuted row order: the CSR K1's tile-pair order, one
         // row per thread and tile, the next tile's row loaded while this
         // one's gathers are in flight
-        JadStream<VT, X> js;
+        JadStream<VT, X, KEEP> js;
         js.init(A.n, A.mmax, A.jnnz, A.jbegin, A.jcols, jad_vals<VT>(A), x);
         long long k = 0;
         long long t = group_tile(0, ntiles);
@@ -806,7 +806,7 @@ union K1Stage {
 // K1: v = A p, per-block partial of v.p.  Mixed: a requested replacement
 // residual takes the place of the product (K2 and K3 then do nothing, and
 // the next K1 folds its partials).  LONG of a DIA K1: its residual's.
-template <typename VT, int FMT, bool HALO, bool LONG>
+template <typename VT, int FMT, bool HALO, bool LONG, bool KEEP = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pcg_spmv(MatView A, const VT* __restrict__ p,
                                                      VT* __restrict__ v, double* __restrict__ part,
                                                      ResArgs<VT> R,
@@ -839,14 +839,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             slot = gridDim.x % kXcds ? walk : (walk % kXcds) * (gridDim.x / kXcds) + walk / kXcds;
         }
     }
-    const double acc = k1_tiles<VT, FMT, HALO, LONG, false>(A, XPlain<VT>{p}, v, sm.tile, StepRows<VT>{}, walk);
+    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, sm.tile, StepRows<VT>{}, walk);
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[slot] = bs;
     write_ctrl(cout, c);
 }
 
 // K3 and the next iteration's K1 in one launch, for small systems (rule at
-// step_rows): beta and the loop decision from K2's partials, x += sigma p,
+// step_form): beta and the loop decision from K2's partials, x += sigma p,
 // p_new = beta p + z, v = A p_new and the partials of v.p_new.  A block
 // needs p_new of its neighbours' rows as well, so every gather reads p and
 // z and forms p_new itself (the same roundings as K3), and p_new goes to a
@@ -856,7 +856,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 // (x64 += e, e = 0) is K3's, and the next launch forms the residual.  What
 // it saves is a launch and K3's second look at p; what it costs is a second
 // gather per entry.
-template <typename VT, int FMT, bool LONG>
+template <typename VT, int FMT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(VT) == 4 ? 4 : 2, 8))) void k_pcg_step(
     MatView A, const VT* __restrict__ p, const VT* __restrict__ z, VT* __restrict__ pout,
     VT* __restrict__ x, double* __restrict__ x64, VT* __restrict__ v, double* __restrict__ part,
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     Ctrl* __restrict__ cout, Prm P)
 {
     constexpr bool MIXED = sizeof(VT) == 4;
-    __shared__ K1Stage<VT, FMT, LONG> sm;
+    __shared__ K1Stage<VT, FMT, false> sm;
     __shared__ double red[3 * kWaves];
     __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
@@ -876,7 +876,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     }
     if constexpr (MIXED) {
         if (c.ru) {  // uniform; the direction moves on to the next slot's buffer
-            replace_residual<FMT == CEL_FMT_DIA ? CEL_FMT_CSR : FMT, LONG>(A, R, c, P, sm.res, red);
+            replace_residual<FMT == CEL_FMT_DIA ? CEL_FMT_CSR : FMT, false>(A, R, c, P, sm.res, red);
             if (!P.ru_restart)
                 for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < A.n;
                      i += (long long)gridDim.x * kBlock)
@@ -914,7 +914,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         write_ctrl(cout, c);
         return;
     }
-    const double acc = k1_tiles<VT, FMT, false, LONG, true>(
+    const double acc = k1_tiles<VT, FMT, false, false, true, true>(
         A, XDirection<VT>{p, z, beta, pending}, v, sm.tile, StepRows<VT>{pout, x, sigma, !pending});
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[logical_block()] = bs;
@@ -1396,9 +1396,18 @@ static int k1_cap(int G1, bool mixed)
 template <typename VT>
 using K1Fn = void (*)(MatView, const VT*, VT*, double*, ResArgs<VT>, const Ctrl*, Ctrl*, Prm);
 
+// keep: the same kernel with ordinary loads of the matrix (keep_matrix); it
+// runs on the other one's grid.
 template <typename VT>
-static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr)
+static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr, bool keep = false)
 {
+    if (keep && !halo && fmt != kFmtClass) {
+        if (fmt == CEL_FMT_JAD) return k_pcg_spmv<VT, CEL_FMT_JAD, false, false, true>;
+        if constexpr (sizeof(VT) == 4)
+            if (fmt == CEL_FMT_DIA && lr) return k_pcg_spmv<VT, CEL_FMT_DIA, false, true, true>;
+        if (fmt == CEL_FMT_DIA) return k_pcg_spmv<VT, CEL_FMT_DIA, false, false, true>;
+        return lr ? k_pcg_spmv<VT, CEL_FMT_CSR, false, true, true> : k_pcg_spmv<VT, CEL_FMT_CSR, false, false, true>;
+    }
     if (fmt == CEL_FMT_JAD) return k_pcg_spmv<VT, CEL_FMT_JAD, false, false>;
     if (fmt == kFmtClass) return k_pcg_spmv<VT, kFmtClass, false, false>;
     if constexpr (sizeof(VT) == 8) {  // halo blocks: FP64 only
@@ -1409,6 +1418,30 @@ static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr)
         return lr ? k_pcg_spmv<VT, CEL_FMT_DIA, false, true> : k_pcg_spmv<VT, CEL_FMT_DIA, false, false>;
     }
     return lr ? k_pcg_spmv<VT, CEL_FMT_CSR, false, true> : k_pcg_spmv<VT, CEL_FMT_CSR, false, false>;
+}
+
+// Whether the K1s load the matrix (nd > 0: nd diagonals) so that it stays in
+// the infinity cache: what an iteration touches, matrix and vectors, is at
+// most kKeepBytes.  Above it the matrix would push out the vectors, which
+// are touched more than once an iteration, and come from HBM all the same.
+// Measured per iteration on 7-point cubes, marked as read once / kept, by
+// the bytes touched: CSR FP64 112^3 (185 MB) 51.3 / 46.9 us, 128^3 (277)
+// 71.5 / 65.8, 136^3 (332) 84.0 / 86.0, 144^3 (395) 96.6 / 101.9; DIA FP64
+// 128^3 (218) 65.3 / 58.2, 144^3 (311) 85.4 / 84.9, 152^3 (365) 99.1 / 103.9;
+// CSR mixed 144^3 (251) 62.9 / 58.7, 152^3 (295) 74.3 / 73.4, 160^3 (344)
+// 85.8 / 88.2; DIA mixed 160^3 (230) 63.5 / 62.3, 176^3 (305) 80.9 / 81.9;
+// JAD FP64 209,000 rows 17.0 / 15.7; 600,011 mesh rows mixed, whole solve
+// 8.20 / 7.39 ms.  (A product by itself is better off without: 1,000,003
+// mesh rows 99.0 / 102.3 us a call.)
+constexpr double kKeepBytes = 300e6;
+static bool keep_matrix(const Mat& A, int fmt, int nd, bool mixed)
+{
+    const double vb = mixed ? 4.0 : 8.0, n = A.n;
+    const double m = fmt == CEL_FMT_DIA   ? nd * vb * n
+                     : fmt == CEL_FMT_JAD ? (4.0 + vb) * (double)A.jad_nnz
+                                          : (4.0 + vb) * (double)A.nnz + 4.0 * n;
+    // the vectors: FP64 x, r, p, v, b, Jacobi; mixed r, p, v, e, Jacobi and x
+    return m + (mixed ? 28.0 : 48.0) * n <= kKeepBytes;
 }
 
 static int k1_grid_f64(long long ntiles)
@@ -1427,15 +1460,10 @@ using StepFn = void (*)(MatView, const VT*, const VT*, VT*, VT*, double*, VT*, d
                         const double*, int, const Ctrl*, Ctrl*, Prm);
 
 template <typename VT>
-static StepFn<VT> step_kernel(int fmt, bool lr)
+static StepFn<VT> step_kernel(int fmt)
 {
-    if (fmt == CEL_FMT_JAD) return k_pcg_step<VT, CEL_FMT_JAD, false>;
-    if constexpr (sizeof(VT) == 8) {
-        if (fmt == CEL_FMT_DIA) return k_pcg_step<VT, CEL_FMT_DIA, false>;
-    } else if (fmt == CEL_FMT_DIA) {
-        return lr ? k_pcg_step<VT, CEL_FMT_DIA, true> : k_pcg_step<VT, CEL_FMT_DIA, false>;
-    }
-    return lr ? k_pcg_step<VT, CEL_FMT_CSR, true> : k_pcg_step<VT, CEL_FMT_CSR, false>;
+    if (fmt == CEL_FMT_JAD) return k_pcg_step<VT, CEL_FMT_JAD>;
+    return fmt == CEL_FMT_DIA ? k_pcg_step<VT, CEL_FMT_DIA> : k_pcg_step<VT, CEL_FMT_CSR>;
 }
 
 // Whether a solve iterates with two kernels (k_pcg_step, K2) instead of
@@ -1872,6 +1900,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         V.dmask = nullptr;
         V.dmask8 = D.mask8.p;
     }
+    const bool keep = keep_matrix(A, kfmt, V.nd, mixed);
     if (use == Derived::kClasses) CEL_TRY(class_walk(A, *Wp, G1, &V.walk));
     V.dzero = -1;
     for (int d = 0; d < V.nd; ++d) {
@@ -1962,7 +1991,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     auto enqueue_step = [&](long long slot) -> int {
         const int in = (int)(slot & 1), out = in ^ 1;
         if (!mixed) {
-            hipLaunchKernelGGL(step_kernel<double>(fmt, lr), dim3(G1), dim3(kBlock), 0, s, V,
+            hipLaunchKernelGGL(step_kernel<double>(fmt), dim3(G1), dim3(kBlock), 0, s, V,
                                (const double*)pbuf[in], (const double*)zbuf, pbuf[out], dx, (double*)nullptr, w.v,
                                w.part1, R64, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
             hipLaunchKernelGGL((k_pcg_update_r<double, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
@@ -1970,7 +1999,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         } else {
             ResArgs<float> R = R32;
             R.p = pbuf32[out];  // a restart's direction
-            hipLaunchKernelGGL(step_kernel<float>(fmt, lr), dim3(G1), dim3(kBlock), 0, s, V,
+            hipLaunchKernelGGL(step_kernel<float>(fmt), dim3(G1), dim3(kBlock), 0, s, V,
                                (const float*)pbuf32[in], (const float*)zbuf32, pbuf32[out], w.e32, dx, w.v32,
                                w.part1, R, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
             hipLaunchKernelGGL((k_pcg_update_r<float, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
@@ -1997,7 +2026,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             CEL_HIP(hipEventRecord(ea, s));
         }
         if (!mixed) {
-            hipLaunchKernelGGL(k1_kernel<double>(kfmt, halo, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
+            hipLaunchKernelGGL(k1_kernel<double>(kfmt, halo, lr, keep), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
                                w.part1, R64, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL((bycls ? k_pcg_update_r<double, false, true> : k_pcg_update_r<double, false, false>),
@@ -2007,7 +2036,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
                                       : k_pcg_update_xp<double, double, false, false>),
                                dim3(Gv), dim3(kBlock), 0, s, n_ll, dx, w.p, w.r, vjac64, vcls, nullptr, w.part2, Gv, C2, C0, P, progress);
         } else {
-            hipLaunchKernelGGL(k1_kernel<float>(kfmt, false, lr), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
+            hipLaunchKernelGGL(k1_kernel<float>(kfmt, false, lr, keep), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
                                w.part1, R32, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL((bycls ? k_pcg_update_r<float, false, true> : k_pcg_update_r<float, false, false>),

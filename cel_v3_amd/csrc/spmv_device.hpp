@@ -106,23 +106,22 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* base, in
                                              0x00020000);
 }
 
-// Non-temporal buffer load (aux bit 1 = nt on gfx950).
-template <typename T>
-__device__ __forceinline__ T buf_load_nt(__amdgpu_buffer_rsrc_t r, int voff, int soff);
-template <>
-__device__ __forceinline__ double buf_load_nt<double>(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+// Cache hint of the loads that stream a matrix (aux operand of a buffer
+// load, bit 1 = non-temporal on gfx950).  KEEP: an ordinary load, for solves
+// that find the matrix in the 256 MB infinity cache in the next iteration;
+// otherwise the entries are marked as read once, so that they do not push
+// the vectors out of the caches (rule: pcg.hip, keep_matrix).
+template <bool KEEP>
+constexpr int kStreamAux = KEEP ? 0 : 2;
+
+// Buffer load of a matrix stream.
+template <typename T, bool KEEP>
+__device__ __forceinline__ T buf_load_stream(__amdgpu_buffer_rsrc_t r, int voff, int soff)
 {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 2));
-}
-template <>
-__device__ __forceinline__ float buf_load_nt<float>(__amdgpu_buffer_rsrc_t r, int voff, int soff)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 2));
-}
-template <>
-__device__ __forceinline__ int buf_load_nt<int>(__amdgpu_buffer_rsrc_t r, int voff, int soff)
-{
-    return (int)__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 2);
+    if constexpr (sizeof(T) == 8)
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, kStreamAux<KEEP>));
+    else
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kStreamAux<KEEP>));
 }
 
 // Cached buffer load; an offset outside the resource returns 0.
@@ -195,7 +194,7 @@ struct XDirection {
 // mask marks an entry): each row's entries in ascending offset (= CSR
 // column) order, absent ones skipped, so the sums are the CSR row sums bit
 // for bit.  A group of GD diagonals of all R rows is loaded before any of
-// their products is added; values through non-temporal buffer loads (one
+// their products is added; values through streaming buffer loads (one
 // resource per diagonal), x through one buffer resource, so the x of an
 // absent boundary entry reads 0 from outside the resource instead of
 // needing a clamp.  n * sizeof(VT) must stay below 2^31 (32-bit byte
@@ -203,7 +202,7 @@ struct XDirection {
 // diagonal with offset 0 (index dzero >= 0, present in the caller's
 // layout), taken after the products' wait, so it costs no load and no
 // round trip of its own.
-template <typename VT, int R, int GD, typename X>
+template <typename VT, int R, int GD, bool KEEP = false, typename X>
 __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const VT* vals,
                                          const uint8_t* m8, const uint32_t* m32, const int (&r)[R],
                                          const X& x, VT (&s)[R], typename X::Raw* xr = nullptr,
@@ -230,7 +229,7 @@ __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const V
                 const int o = doff[d];
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
-                    v[g][k] = buf_load_nt<VT>(rv, rc[k] * B, 0);
+                    v[g][k] = buf_load_stream<VT, KEEP>(rv, rc[k] * B, 0);
                     // an absent entry's column may lie outside [0, n): its
                     // byte offset wraps modulo 2^32 (unsigned, defined) and
                     // the load returns 0 or a value the mask discards
@@ -334,7 +333,7 @@ struct NoLoads {
 // as its entries, the tile's loads had to wait for the gathers issued before
 // them, which put one L2 round trip and one HBM round trip in series on
 // every step.)
-template <typename VT>
+template <typename VT, bool KEEP = false>
 struct CsrTileStream {
     static constexpr int EV = 16 / (int)sizeof(VT);  // values per 16-byte load
     VT v[kPer];
@@ -380,7 +379,7 @@ struct CsrTileStream {
         const auto rc = tile_rsrc(cols + (e0 - sc), m > 0 ? (m + sc) * (int)sizeof(int) : 0);
 #pragma unroll
         for (int i = 0; i < kPer / EV; ++i) {
-            const auto w = __builtin_amdgcn_raw_buffer_load_b128(rv, 16 * tid, 16 * kBlock * i, 2);
+            const auto w = __builtin_amdgcn_raw_buffer_load_b128(rv, 16 * tid, 16 * kBlock * i, kStreamAux<KEEP>);
 #pragma unroll
             for (int j = 0; j < EV; ++j) {
                 if constexpr (sizeof(VT) == 8) {
@@ -395,7 +394,7 @@ struct CsrTileStream {
         }
 #pragma unroll
         for (int i = 0; i < kPer / 4; ++i) {
-            const auto w = __builtin_amdgcn_raw_buffer_load_b128(rc, 16 * tid, 16 * kBlock * i, 2);
+            const auto w = __builtin_amdgcn_raw_buffer_load_b128(rc, 16 * tid, 16 * kBlock * i, kStreamAux<KEEP>);
 #pragma unroll
             for (int j = 0; j < 4; ++j) c[i * 4 + j] = (int)w[j];
         }
@@ -548,7 +547,7 @@ struct CsrLongStage {
     VT prod[kStageCap + kStageCap / 16];
 };
 
-template <typename VT>
+template <typename VT, bool KEEP = false>
 struct CsrLongStream {
     static constexpr int EV = 16 / (int)sizeof(VT);  // values per 16-byte load
     VT v[kPer];    // the fetched segment
@@ -579,7 +578,7 @@ struct CsrLongStream {
         const int tid = threadIdx.x;
 #pragma unroll
         for (int i = 0; i < kPer / 4; ++i) {
-            const auto w = __builtin_amdgcn_raw_buffer_load_b128(rc, 16 * tid, 16 * kBlock * i, 2);
+            const auto w = __builtin_amdgcn_raw_buffer_load_b128(rc, 16 * tid, 16 * kBlock * i, kStreamAux<KEEP>);
 #pragma unroll
             for (int j = 0; j < 4; ++j) cc[i * 4 + j] = (int)w[j];
         }
@@ -587,7 +586,7 @@ struct CsrLongStream {
         for (int i = 0; i < kPer / EV; ++i) {
             constexpr int P = 4 / EV;  // 16-byte loads per 4 entries
             const auto w = __builtin_amdgcn_raw_buffer_load_b128(
-                rv, 16 * P * tid + 16 * (i % P), 16 * P * kBlock * (i / P), 2);
+                rv, 16 * P * tid + 16 * (i % P), 16 * P * kBlock * (i / P), kStreamAux<KEEP>);
 #pragma unroll
             for (int j = 0; j < EV; ++j) {
                 if constexpr (sizeof(VT) == 8) {
@@ -701,14 +700,14 @@ struct CsrLongStream {
 };
 
 // The tile stream of a CSR kernel and its LDS stage.
-template <typename VT, bool LONG>
+template <typename VT, bool LONG, bool KEEP = false>
 struct CsrStreamOf {
-    using Stream = CsrTileStream<VT>;
+    using Stream = CsrTileStream<VT, KEEP>;
     using Stage = CsrStage<VT>;
 };
-template <typename VT>
-struct CsrStreamOf<VT, true> {
-    using Stream = CsrLongStream<VT>;
+template <typename VT, bool KEEP>
+struct CsrStreamOf<VT, true, KEEP> {
+    using Stream = CsrLongStream<VT, KEEP>;
     using Stage = CsrLongStage<VT>;
 };
 
@@ -762,7 +761,7 @@ __device__ __forceinline__ AT jad_row(int k, int mmax, const int* __restrict__ b
 // Diagonals past kGather are summed after the first kGather, in order,
 // from global memory.  jad_nnz * sizeof(VT) and n * sizeof(VT) must stay
 // below 2^32 - 16 (unsigned 32-bit byte offsets).
-template <typename VT, typename X = XPlain<VT>>
+template <typename VT, typename X = XPlain<VT>, bool KEEP = false>
 struct JadStream {
     int bg[kGather];  // starts of diagonals 0..kGather-1 (clamped)
     int ln[kGather];  // their lengths (0 past the last diagonal)
@@ -800,8 +799,8 @@ struct JadStream {
         for (int i = 0; i < kGather; ++i) {
             const unsigned e = (unsigned)(bg[i] + k);
             const bool on = k < ln[i];
-            c[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rc, on ? e * 4u : 0xFFFFFFFFu, 0, 2);
-            a[i] = buf_load_nt<VT>(rv, (int)(on ? e * B : 0xFFFFFFFFu), 0);
+            c[i] = buf_load_stream<int, KEEP>(rc, (int)(on ? e * 4u : 0xFFFFFFFFu), 0);
+            a[i] = buf_load_stream<VT, KEEP>(rv, (int)(on ? e * B : 0xFFFFFFFFu), 0);
         }
     }
 
