@@ -36,6 +36,16 @@ __device__ __forceinline__ T ld_stream(const T* p)
     return __builtin_nontemporal_load(p);
 }
 
+// A 16-byte load; NT: of data that is not wanted in the caches any more.
+template <bool NT, typename V>
+__device__ __forceinline__ V ld_vec(const void* p)
+{
+    typedef unsigned int U4 __attribute__((ext_vector_type(4)));
+    static_assert(sizeof(V) == 16, "one 16-byte load");
+    if constexpr (NT) return __builtin_bit_cast(V, __builtin_nontemporal_load((const U4*)p));
+    else return *(const V*)p;
+}
+
 // Lane exchanges of the butterfly sums, in registers: halves of the wave and
 // of its 32-lane halves through the swap instructions, the rest through
 // DPP.  (Through LDS, as __shfl_xor does it, a wave sum took 490 cycles; so

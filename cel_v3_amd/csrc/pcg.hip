@@ -1006,9 +1006,31 @@ static_assert(kMaxClass == kBlock, "one table entry per thread");
 template <typename VT>
 constexpr int kVecUnrollOf = sizeof(VT) == 4 ? 4 : 2;
 
+// Which vectors K2 and K3 keep in the infinity cache, by the bytes of the
+// vectors an iteration touches (x, p, r, v, and the Jacobi vector or the
+// class bytes).  A vector that is marked as read once leaves its room to the
+// others: kStreamX: x, which only K3 touches; kStreamAll: also v and r where
+// they are read, so that what stays is what the next kernel reads (v from K1
+// to K2, r from K2 to K3, p from K3 to K1).  Measured per iteration with
+// none / x / all marked, Poisson cubes on row classes: FP64 192^3 (233 MB)
+// 125 / 127 / 130 us, 200^3 (264) 147.5 / 141 / 144, 216^3 (333) 181 / 175 /
+// 177, 232^3 (412) 236 / 214 / 214, 256^3 (554) 358 / 336 / 283, 320^3
+// (1081) 691 / 683 / 644; mixed 232^3 (212) 113 / 114 / 117, 256^3 (285)
+// 155 / 149 / 151, 288^3 (406) 231 / 213 / 209, 320^3 (557) 336 / 320 /
+// 284; variable coefficients FP64 176^3 (218) 146 / 147 / 149, 192^3 (283)
+// 189 / 186 / 188, 216^3 (403) 285 / 267 / 264, 256^3 (671) 521 / 494 / 459.
+enum StreamLevel { kStreamNone = 0, kStreamX = 1, kStreamAll = 2 };
+static int stream_level(long long n, bool mixed, bool cls)
+{
+    const double vb = mixed ? 4.0 : 8.0;
+    const double bytes = ((cls ? 4.0 : 5.0) * vb + (cls ? 1.0 : 0.0)) * (double)n;
+    return bytes > 380e6 ? kStreamAll : bytes > 240e6 ? kStreamX : kStreamNone;
+}
+
 // K2: sigma = alpha / sum(v.p) ; r = r + (-sigma) v ; z = jac*r ;
 // per-block partials of r.z and r.r.  ZOUT: z is stored too (for k_pcg_step).
-template <typename VT, bool ZOUT, bool CLS>
+// STREAM: stream_level (K2 knows none and all).
+template <typename VT, bool ZOUT, bool CLS, int STREAM = kStreamNone>
 __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __restrict__ r,
                                                          const VT* __restrict__ v,
                                                          const VT* __restrict__ jac,
@@ -1064,8 +1086,8 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
         typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
 #pragma unroll
         for (int u = 0; u < kVecUnroll; ++u) {
-            vv[u] = *reinterpret_cast<const V*>(v + i + u * unit);
-            rv[u] = *reinterpret_cast<const V*>(r + i + u * unit);
+            vv[u] = ld_vec<STREAM == kStreamAll, V>(v + i + u * unit);
+            rv[u] = ld_vec<STREAM == kStreamAll, V>(r + i + u * unit);
             jv[u] = J.load(i + u * unit);
         }
 #pragma unroll
@@ -1130,9 +1152,9 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
 
 // K3: beta = sum(r.z)/alpha ; x = x + sigma p ; p = beta p + jac*r ;
 // alpha = r.z, norm2, k++, history, loop decision (FP64) or replacement
-// request (mixed).
-template <typename VT, typename XT, bool MIXED, bool CLS>
-__global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __restrict__ x,
+// request (mixed).  STREAM: stream_level.
+template <typename VT, bool MIXED, bool CLS, int STREAM>
+__global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, VT* __restrict__ x,
                                                           VT* __restrict__ p,
                                                           const VT* __restrict__ r,
                                                           const VT* __restrict__ jac,
@@ -1174,21 +1196,23 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
     for (; i + (kVecUnroll - 1) * unit + W <= hi; i += kVecUnroll * unit) {
         V pv[kVecUnroll], rv[kVecUnroll];
         typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
-        XT xs[kVecUnroll][W];
+        VT xs[kVecUnroll][W];
 #pragma unroll
         for (int u = 0; u < kVecUnroll; ++u) {
             pv[u] = *reinterpret_cast<const V*>(p + i + u * unit);
-            rv[u] = *reinterpret_cast<const V*>(r + i + u * unit);
+            rv[u] = ld_vec<STREAM == kStreamAll, V>(r + i + u * unit);
             jv[u] = J.load(i + u * unit);
 #pragma unroll
-            for (int k = 0; k < W; ++k) xs[u][k] = x[i + u * unit + k];
+            for (int k = 0; k < W; ++k)
+                xs[u][k] = STREAM != kStreamNone ? __builtin_nontemporal_load(x + i + u * unit + k)
+                                                 : x[i + u * unit + k];
         }
 #pragma unroll
         for (int u = 0; u < kVecUnroll; ++u) {
 #pragma unroll
             for (int k = 0; k < W; ++k) {
                 const VT pi = lane<VT>(pv[u], k);
-                XT t = XT(sigma * pi);
+                VT t = VT(sigma * pi);
                 xs[u][k] = xs[u][k] + t;
                 VT zi = lane<VT>(rv[u], k) * J.value(jv[u], k);
                 VT bp = beta * pi;
@@ -1199,11 +1223,14 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
                 for (int k = 0; k < W; ++k) {
                     double t = (double)xs[u][k];
                     x64[i + u * unit + k] = x64[i + u * unit + k] + t;
-                    xs[u][k] = XT(0);
+                    xs[u][k] = VT(0);
                 }
             }
 #pragma unroll
-            for (int k = 0; k < W; ++k) x[i + u * unit + k] = xs[u][k];
+            for (int k = 0; k < W; ++k) {
+                if constexpr (STREAM != kStreamNone) __builtin_nontemporal_store(xs[u][k], x + i + u * unit + k);
+                else x[i + u * unit + k] = xs[u][k];
+            }
             *reinterpret_cast<V*>(p + i + u * unit) = pv[u];
         }
     }
@@ -1212,13 +1239,13 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
             V pv = *reinterpret_cast<const V*>(p + i);
             const V rv = *reinterpret_cast<const V*>(r + i);
             const auto jv = J.load(i);
-            XT xs[W];
+            VT xs[W];
 #pragma unroll
             for (int k = 0; k < W; ++k) xs[k] = x[i + k];
 #pragma unroll
             for (int k = 0; k < W; ++k) {
                 const VT pi = lane<VT>(pv, k);
-                XT t = XT(sigma * pi);
+                VT t = VT(sigma * pi);
                 xs[k] = xs[k] + t;
                 VT zi = lane<VT>(rv, k) * J.value(jv, k);
                 VT bp = beta * pi;
@@ -1229,7 +1256,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
                 for (int k = 0; k < W; ++k) {
                     double t = (double)xs[k];
                     x64[i + k] = x64[i + k] + t;
-                    xs[k] = XT(0);
+                    xs[k] = VT(0);
                 }
             }
 #pragma unroll
@@ -1238,12 +1265,12 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, XT* __res
         } else {
             for (long long j = i; j < hi; ++j) {
                 const VT pi = p[j];
-                XT t = XT(sigma * pi);
-                XT xj = x[j] + t;
+                VT t = VT(sigma * pi);
+                VT xj = x[j] + t;
                 if (flush) {
                     double tt = (double)xj;
                     x64[j] = x64[j] + tt;
-                    xj = XT(0);
+                    xj = VT(0);
                 }
                 x[j] = xj;
                 VT zi = r[j] * J.at(j);
@@ -1453,6 +1480,34 @@ static int k1_grid_f64(long long ntiles)
         g = std::min(g, resident_grid((const void*)k1_kernel<double>(CEL_FMT_DIA, halo, false), ntiles));
     }
     return g;
+}
+
+template <typename VT>
+using K2Fn = void (*)(long long, VT*, const VT*, const VT*, const uint8_t*, VT*, double*, const double*, int,
+                      const Ctrl*, Ctrl*, int*);
+template <typename VT>
+static K2Fn<VT> k2_kernel(bool cls, int stream)
+{
+    if (stream == kStreamAll)
+        return cls ? k_pcg_update_r<VT, false, true, kStreamAll> : k_pcg_update_r<VT, false, false, kStreamAll>;
+    return cls ? k_pcg_update_r<VT, false, true> : k_pcg_update_r<VT, false, false>;
+}
+
+template <typename VT>
+using K3Fn = void (*)(long long, VT*, VT*, const VT*, const VT*, const uint8_t*, double*, const double*, int,
+                      const Ctrl*, Ctrl*, Prm, int*);
+template <typename VT>
+static K3Fn<VT> k3_kernel(bool cls, int stream)
+{
+    constexpr bool M = sizeof(VT) == 4;
+    switch (stream) {
+    case kStreamAll:
+        return cls ? k_pcg_update_xp<VT, M, true, kStreamAll> : k_pcg_update_xp<VT, M, false, kStreamAll>;
+    case kStreamX:
+        return cls ? k_pcg_update_xp<VT, M, true, kStreamX> : k_pcg_update_xp<VT, M, false, kStreamX>;
+    default:
+        return cls ? k_pcg_update_xp<VT, M, true, kStreamNone> : k_pcg_update_xp<VT, M, false, kStreamNone>;
+    }
 }
 
 template <typename VT>
@@ -1985,6 +2040,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     const double* vjac64 = bycls ? V.ctab.jac64 : jac64;
     const float* vjac32 = bycls ? V.ctab.jac32 : jac32;
     const uint8_t *vcls = bycls ? V.cls : nullptr, *nocls = nullptr;
+    const int stream = stream_level(n, mixed, bycls);
     // One slot of the two-kernel form: the step finishes the iteration before
     // (its vectors and scalars) and forms the next product, K2 updates r.
     // The direction alternates between two buffers by slot.
@@ -2029,22 +2085,18 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             hipLaunchKernelGGL(k1_kernel<double>(kfmt, halo, lr, keep), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
                                w.part1, R64, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
-            hipLaunchKernelGGL((bycls ? k_pcg_update_r<double, false, true> : k_pcg_update_r<double, false, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v, vjac64, vcls, (double*)nullptr, w.part2, w.part1, G1, C1, C2,
-                               (int*)nullptr);
-            hipLaunchKernelGGL((bycls ? k_pcg_update_xp<double, double, false, true>
-                                      : k_pcg_update_xp<double, double, false, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, dx, w.p, w.r, vjac64, vcls, nullptr, w.part2, Gv, C2, C0, P, progress);
+            hipLaunchKernelGGL(k2_kernel<double>(bycls, stream), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v, vjac64,
+                               vcls, (double*)nullptr, w.part2, w.part1, G1, C1, C2, (int*)nullptr);
+            hipLaunchKernelGGL(k3_kernel<double>(bycls, stream), dim3(Gv), dim3(kBlock), 0, s, n_ll, dx, w.p, w.r,
+                               vjac64, vcls, nullptr, w.part2, Gv, C2, C0, P, progress);
         } else {
             hipLaunchKernelGGL(k1_kernel<float>(kfmt, false, lr, keep), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
                                w.part1, R32, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
-            hipLaunchKernelGGL((bycls ? k_pcg_update_r<float, false, true> : k_pcg_update_r<float, false, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32, vjac32, vcls, (float*)nullptr, w.part2, w.part1, G1, C1, C2,
-                               (int*)nullptr);
-            hipLaunchKernelGGL((bycls ? k_pcg_update_xp<float, float, true, true>
-                                      : k_pcg_update_xp<float, float, true, false>),
-                               dim3(Gv), dim3(kBlock), 0, s, n_ll, w.e32, w.p32, w.r32, vjac32, vcls, dx, w.part2, Gv, C2, C0, P, progress);
+            hipLaunchKernelGGL(k2_kernel<float>(bycls, stream), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,
+                               vjac32, vcls, (float*)nullptr, w.part2, w.part1, G1, C1, C2, (int*)nullptr);
+            hipLaunchKernelGGL(k3_kernel<float>(bycls, stream), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.e32, w.p32,
+                               w.r32, vjac32, vcls, dx, w.part2, Gv, C2, C0, P, progress);
         }
         CEL_HIP(hipGetLastError());
         return CEL_OK;
