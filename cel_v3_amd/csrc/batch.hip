@@ -558,8 +558,24 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
     write_lanes(cout, S, b == S.b0, lc);
 }
 
+// Which vectors K2 and K3 keep in the infinity cache, by the bytes of x, p,
+// r, v and the Jacobi vectors of all systems (the lines of the single
+// solver, but for the second one: K1 stores v as read once here, and 404 MB
+// are still better off with x alone).  Measured per iteration with none / x
+// / all marked: 16 right-hand sides on 128^3 (1.1 GB) 677 / 671 / 632 us; 64
+// systems of 24^3..96^3 (0.6 GB) 445 / 429 / 411; 11 on 91^3 (0.4 GB) 289 /
+// 275 / 297; 8 systems of 60^3..90^3 (0.1 GB) 115.5 / 116.7 / 117.2.
+enum BStream { kBStreamNone = 0, kBStreamX = 1, kBStreamAll = 2 };
+
+template <bool NT>
+__device__ __forceinline__ double ld_elem(const double* p)
+{
+    return NT ? ld_stream(p) : *p;
+}
+
 // ---------------------------------------------------------------- K2
 // sigma = alpha / sum(v.p) ; r = r + (-sigma) v ; z = jac r ; partials r.z, r.r.
+template <int STREAM>
 __global__ __launch_bounds__(kBlock) void k_bupdate_r(const BSys* __restrict__ sys,
                                                       const BBlk* __restrict__ tbl,
                                                       double* __restrict__ r,
@@ -618,8 +634,8 @@ __global__ __launch_bounds__(kBlock) void k_bupdate_r(const BSys* __restrict__ s
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
                 const long long eu = e + u * kBlock;
-                vv[u] = v[S.voff + eu];
-                rv[u] = r[S.voff + eu];
+                vv[u] = ld_elem<STREAM == kBStreamAll>(v + S.voff + eu);
+                rv[u] = ld_elem<STREAM == kBStreamAll>(r + S.voff + eu);
                 jv[u] = S.jac[eu >> S.ksh];
             }
 #pragma unroll
@@ -658,6 +674,7 @@ __global__ __launch_bounds__(kBlock) void k_bupdate_r(const BSys* __restrict__ s
 // ---------------------------------------------------------------- K3
 // beta = sum(r.z)/alpha ; x = x + sigma p ; p = beta p + jac r ; norm, k++,
 // stop decision.
+template <int STREAM>
 __global__ __launch_bounds__(kBlock) void k_bupdate_xp(const BSys* __restrict__ sys,
                                                        const BBlk* __restrict__ tbl,
                                                        double* __restrict__ x,
@@ -704,15 +721,17 @@ __global__ __launch_bounds__(kBlock) void k_bupdate_xp(const BSys* __restrict__ 
             for (int u = 0; u < kUnroll; ++u) {
                 const long long eu = e + u * kBlock;
                 pv[u] = p[S.voff + eu];
-                xv[u] = x[S.voff + eu];
-                rv[u] = r[S.voff + eu];
+                xv[u] = ld_elem<STREAM != kBStreamNone>(x + S.voff + eu);
+                rv[u] = ld_elem<STREAM == kBStreamAll>(r + S.voff + eu);
                 jv[u] = S.jac[eu >> S.ksh];
             }
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
                 const size_t g = S.voff + e + u * kBlock;
                 double t = sigma * pv[u];
-                x[g] = xv[u] + t;
+                const double xn = xv[u] + t;
+                if constexpr (STREAM != kBStreamNone) __builtin_nontemporal_store(xn, x + g);
+                else x[g] = xn;
                 const double zi = rv[u] * jv[u];
                 double bp = beta * pv[u];
                 p[g] = bp + zi;
@@ -807,8 +826,10 @@ static int grid_max()
 {
     int g = resident_grid((const void*)k_bspmv, 1 << 30);
     g = std::min(g, resident_grid((const void*)k_bresidual, 1 << 30));
-    g = std::min(g, resident_grid((const void*)k_bupdate_r, 1 << 30));
-    g = std::min(g, resident_grid((const void*)k_bupdate_xp, 1 << 30));
+    for (const void* k : {(const void*)k_bupdate_r<kBStreamNone>, (const void*)k_bupdate_r<kBStreamAll>,
+                          (const void*)k_bupdate_xp<kBStreamNone>, (const void*)k_bupdate_xp<kBStreamX>,
+                          (const void*)k_bupdate_xp<kBStreamAll>})
+        g = std::min(g, resident_grid(k, 1 << 30));
     return g;
 }
 
@@ -945,12 +966,19 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
                        B.r.p, B.p.p, B.rpart.p, B.kpmax, G, C0);
     CEL_HIP(hipGetLastError());
 
+    double bytes = 32.0 * (double)B.elems;
+    for (const Mat* A : B.mats) bytes += 8.0 * (double)A->n;
+    const int stream = bytes > 450e6 ? kBStreamAll : bytes > 240e6 ? kBStreamX : kBStreamNone;
+    const auto k2 = stream == kBStreamAll ? k_bupdate_r<kBStreamAll> : k_bupdate_r<kBStreamNone>;
+    const auto k3 = stream == kBStreamAll ? k_bupdate_xp<kBStreamAll>
+                    : stream == kBStreamX ? k_bupdate_xp<kBStreamX>
+                                          : k_bupdate_xp<kBStreamNone>;
     auto enqueue_iter = [&]() -> int {
         hipLaunchKernelGGL(k_bspmv, dim3(G), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl.p, B.p.p, B.v.p,
                            B.part1.p, B.rpart.p, B.kpmax, G, C0, C1, P);
-        hipLaunchKernelGGL(k_bupdate_r, dim3(G2), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl2.p, B.r.p,
+        hipLaunchKernelGGL(k2, dim3(G2), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl2.p, B.r.p,
                            B.v.p, B.part2.p, B.part1.p, B.kpmax, G2, C1, C2);
-        hipLaunchKernelGGL(k_bupdate_xp, dim3(G2), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl2.p, B.x.p,
+        hipLaunchKernelGGL(k3, dim3(G2), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl2.p, B.x.p,
                            B.p.p, B.r.p, B.part2.p, B.kpmax, G2, C2, C0, P);
         CEL_HIP(hipGetLastError());
         return CEL_OK;
