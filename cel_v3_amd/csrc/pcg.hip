@@ -557,10 +557,8 @@ __device__ __forceinline__ void next_scalars(Ctrl& c, double rz, double rr, cons
     }
 }
 
-// Tile groups a row-class K1 sums per step.  Measured on the 256^3 Poisson
-// block, time per iteration with 1 / 2 / 3 groups: mixed 163 / 158 / 158 us,
-// FP64 371 / 352 / 346; 100^3 mixed 24.7 / 24.3 / 25.7, FP64 30.2 / 30.0 /
-// 33.4.
+// Tile groups a row-class K1 sums per step: with 2, four waves of FP32 lanes
+// have one 16-byte task each and those of FP64 two.
 constexpr int kClassGroups = 2;
 
 // What the tile walk of a K1 does with the rows besides the product: nothing,
@@ -573,6 +571,106 @@ struct StepRows {
     bool upd;  // x is updated (uniform; false right after a set-up or replacement)
 };
 
+// LDS of the wide walk: the rows' terms of v.d, two steps of them.
+struct WideStage {
+    double prod[2][kClassGroups * kTileGroup * kTileRows];
+};
+struct NoStage {};
+template <int FMT>
+struct WideStageOf {
+    using T = NoStage;
+};
+template <>
+struct WideStageOf<kFmtClass> {
+    using T = WideStage;
+};
+
+// k1_tiles of row classes: v = A d with E = 16 / sizeof(VT) consecutive rows
+// per lane.  What bounds a product of so few bytes per row (x, v and a byte)
+// is the work per row: one row per lane took 7 loads, 8 LDS reads and 90
+// instructions, 56.6 us on the 256^3 block in FP32 (151 MB); this one takes
+// 7/4 loads, 3 LDS reads and 45 instructions, 35.8 us (4.2 TB/s).  (Loading
+// the next step before the sums needs two sets of registers; in FP32 they
+// spill, 50 us.)  The rows of a step are those of the row-per-thread kernels
+// (kClassGroups groups of kTileGroup tiles) and their terms of v.d go
+// through LDS to the threads that add them there, so the partials are the
+// same bit for bit.  Waves that hold a row without all of its neighbours in
+// [0, n) (the ends of the matrix) take loads that are checked one by one
+// (edge).  Per iteration,
+// before and after: mixed 256^3 150.6 -> 130.2 us, 200^3 79.5 -> 68.5, 128^3
+// 30.5 -> 29.8, 100^3 23.7 -> 23.7; FP64 256^3 283 -> 244, 200^3 141 -> 120,
+// 128^3 47 -> 43, 100^3 28.7 -> 27.5.
+template <typename VT, int ND, typename SRC, typename EDGE>
+__device__ __forceinline__ double k1_wide(const MatView& A, const VT* __restrict__ x, VT* __restrict__ v,
+                                          const SRC& src, const EDGE& edge, WideStage& st, int walk)
+{
+    constexpr int E = WideOf<VT>::E, WR = 64 * E;               // rows of a wave
+    constexpr int NG = kClassGroups, GR = kTileGroup * kTileRows;  // groups per step, rows of a group
+    constexpr int WPG = GR / WR;                                // waves that cover a group
+    constexpr int U = NG * WPG / kWaves;                        // tasks of a wave per step
+    static_assert(NG * WPG % kWaves == 0 && GR % WR == 0, "whole tasks");
+    const long long ngroups = ((long long)A.n + GR - 1) / GR, G = gridDim.x;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int omin = min(0, A.doff[0]), omax = max(0, A.doff[A.nd - 1]);
+    double acc = 0.0;
+    int buf = 0;
+    for (long long q = walk; q < ngroups; q += NG * G, buf ^= 1) {
+        int row[U], at[U];
+        bool inside = true;  // uniform across the wave
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int task = u * kWaves + wave, g = task / WPG;
+            const long long w0 = (q + g * G) * GR + (task % WPG) * WR;
+            inside = inside && w0 + omin >= 0 && w0 + WR + omax <= A.n;
+            row[u] = w0 < A.n ? (int)w0 + lane * E : A.n;
+            at[u] = g * GR + (task % WPG) * WR + lane * E;
+        }
+        double* prod = st.prod[buf];
+        if (inside) {
+            WideRows<VT, ND, U, SRC> R;
+            R.load(row, A.doff, x, src);
+            typename WideOf<VT>::T xr[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) xr[u] = *reinterpret_cast<const typename WideOf<VT>::T*>(x + row[u]);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                typename WideOf<VT>::T vv;
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const VT s = R.sum(u, e, src);
+                    vv[e] = s;
+                    prod[at[u] + e] = double(s) * double(xr[u][e]);
+                }
+                *reinterpret_cast<typename WideOf<VT>::T*>(v + row[u]) = vv;
+            }
+        } else {
+#pragma unroll 1
+            for (int u = 0; u < U; ++u) {
+                int r[E];
+                VT s[E], pr[E];
+#pragma unroll
+                for (int e = 0; e < E; ++e) r[e] = min(row[u] + e, A.n);
+                if (r[0] < A.n) edge(r, s, pr);
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    double t = 0.0;
+                    if (r[e] < A.n) {
+                        const VT d = A.dzero >= 0 ? pr[e] : x[r[e]];
+                        const VT sk = VT(0) + s[e];
+                        v[r[e]] = sk;
+                        t = double(sk) * double(d);
+                    }
+                    prod[at[u] + e] = t;
+                }
+            }
+        }
+        __syncthreads();  // one per step: the next one writes the other half
+#pragma unroll
+        for (int k = 0; k < NG * kTileGroup; ++k) acc = acc + prod[k * kTileRows + threadIdx.x];
+    }
+    return acc;
+}
+
 // v = A d over the block's tiles, d the vector of the accessor X; returns the
 // thread's part of v.d.  STEP: X is XDirection, and d and the updated x of
 // every row are stored as well.  (Taking a step's scalars behind the first
@@ -581,6 +679,7 @@ struct StepRows {
 template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, bool KEEP, typename X>
 __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __restrict__ v,
                                            typename StageOf<VT, FMT, LONG>::T& sm,
+                                           typename WideStageOf<FMT>::T& wide,
                                            const StepRows<VT>& st, int walk = 0)
 {
     const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
@@ -661,30 +760,12 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
             if (row < A.n) finish(row, s, pr, xo);
         }
     } else if constexpr (FMT == kFmtClass) {
-        // a row is one byte and its gathers, so a step is one round trip to
-        // the caches whatever it holds: kClassGroups groups of tiles per step
-        load_classes<VT>(A, sm);
-        constexpr int NG = kClassGroups, R = kTileGroup * NG;
-        const long long ngroups = (ntiles + kTileGroup - 1) / kTileGroup, G = gridDim.x;
-        for (long long q = walk; q < ngroups; q += NG * G) {
-            int r[R];
-#pragma unroll
-            for (int k = 0; k < R; ++k) {
-                const long long t = kTileGroup * (q + (k / kTileGroup) * G) + k % kTileGroup;
-                r[k] = t < ntiles ? (int)t * kTileRows + threadIdx.x : A.n;
-            }
-            if (r[0] < A.n) {
-                VT s[R];
-                typename X::Raw pr[R];
-                class_rows<VT, R>(A.n, A.nd, A.doff, A.cls, sm, r, x, s, pr, A.dzero);
-#pragma unroll
-                for (int k = 0; k < R; ++k)
-                    if (r[k] < A.n) {
-                        const typename X::Raw pk = A.dzero >= 0 ? pr[k] : x.load(r[k]);
-                        finish(r[k], VT(0) + s[k], pk, VT(0));
-                    }
-            }
-        }
+        // (the table is in LDS: k_pcg_spmv loads it before it has the token)
+        const WideClasses<VT> src{A.cls, &sm};
+        auto edge = [&](const int (&r)[WideOf<VT>::E], VT (&s)[WideOf<VT>::E], VT (&pr)[WideOf<VT>::E]) {
+            class_rows<VT, WideOf<VT>::E>(A.n, A.nd, A.doff, A.cls, sm, r, x, s, pr, A.dzero);
+        };
+        acc = A.nd <= 7 ? k1_wide<VT, 7>(A, x.x, v, src, edge, wide, walk) : k1_wide<VT, 8>(A, x.x, v, src, edge, wide, walk);
     } else if constexpr (FMT == CEL_FMT_DIA) {
         // all tiles of a group per step, one row of each per thread; the
         // rows are added to the partial in tile order, as in the CSR K1.
@@ -803,11 +884,17 @@ union K1Stage {
     typename StageOf<double, FMT, LONG>::T res;
 };
 
+// Waves per SIMD the K1s are compiled for.  The FP64 wide walk holds two
+// tasks' loads in registers; the FP64 K1s run on 2 blocks per CU
+// (kK1BlocksPerCuF64), so it may take the registers of 2 waves.
+template <typename VT, int FMT>
+constexpr int k1_waves = sizeof(VT) == 8 && FMT == kFmtClass ? 2 : 4;
+
 // K1: v = A p, per-block partial of v.p.  Mixed: a requested replacement
 // residual takes the place of the product (K2 and K3 then do nothing, and
 // the next K1 folds its partials).  LONG of a DIA K1: its residual's.
 template <typename VT, int FMT, bool HALO, bool LONG, bool KEEP = false>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pcg_spmv(MatView A, const VT* __restrict__ p,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves<VT, FMT>, 8))) void k_pcg_spmv(MatView A, const VT* __restrict__ p,
                                                      VT* __restrict__ v, double* __restrict__ part,
                                                      ResArgs<VT> R,
                                                      const Ctrl* __restrict__ cin,
@@ -815,9 +902,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 {
     constexpr bool MIXED = sizeof(VT) == 4;
     __shared__ K1Stage<VT, FMT, LONG> sm;
+    __shared__ typename WideStageOf<FMT>::T wide;
     __shared__ double red[3 * kWaves];
     __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
+    if constexpr (FMT == kFmtClass) load_classes<VT>(A, sm.tile);
     if (c.reduce != kReduceNone) fold_pending(c, R.part, R.G, P, fred);
     if (!c.run) {
         write_ctrl(cout, c);
@@ -839,7 +928,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             slot = gridDim.x % kXcds ? walk : (walk % kXcds) * (gridDim.x / kXcds) + walk / kXcds;
         }
     }
-    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, sm.tile, StepRows<VT>{}, walk);
+    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, sm.tile, wide, StepRows<VT>{}, walk);
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[slot] = bs;
     write_ctrl(cout, c);
@@ -865,6 +954,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
 {
     constexpr bool MIXED = sizeof(VT) == 4;
     __shared__ K1Stage<VT, FMT, false> sm;
+    NoStage wide;
     __shared__ double red[3 * kWaves];
     __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
@@ -915,7 +1005,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         return;
     }
     const double acc = k1_tiles<VT, FMT, false, false, true, true>(
-        A, XDirection<VT>{p, z, beta, pending}, v, sm.tile, StepRows<VT>{pout, x, sigma, !pending});
+        A, XDirection<VT>{p, z, beta, pending}, v, sm.tile, wide, StepRows<VT>{pout, x, sigma, !pending});
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[logical_block()] = bs;
     write_ctrl(cout, c);

@@ -261,7 +261,7 @@ __device__ __forceinline__ void dia_rows(int n, int nd, const int* doff, const V
 // costs its byte and its gathers.
 template <typename VT>
 struct ClassTab {
-    VT val[kMaxClass * kClassDiag];
+    alignas(16) VT val[kMaxClass * kClassDiag];
     uint32_t mask[kMaxClass];
     // every thread of the block; it synchronises
     __device__ __forceinline__ void load(const VT* __restrict__ v, const uint32_t* __restrict__ m)
@@ -312,6 +312,99 @@ __device__ __forceinline__ void class_rows(int n, int nd, const int* doff, const
             }
         }
 }
+
+// A 16-byte access at an element's own alignment.
+template <typename VT>
+struct WideOf {
+    static constexpr int E = 16 / (int)sizeof(VT);
+    typedef VT T __attribute__((ext_vector_type(E), aligned(sizeof(VT))));
+};
+
+// The T at byte offset o of a uniform base: one offset register per lane
+// serves every base.
+template <typename T>
+__device__ __forceinline__ T ld_at(const void* base, unsigned o)
+{
+    return *reinterpret_cast<const T*>(static_cast<const char*>(base) + o);
+}
+
+// The rows of a wide step: where their matrix values come from.
+// Row classes: a byte per row, values and mask from the table in LDS.
+template <typename VT>
+struct WideClasses {
+    static constexpr int E = WideOf<VT>::E;
+    const uint8_t* cls;
+    const ClassTab<VT>* tab;
+    struct Raw {
+        unsigned c;
+    };
+    template <int ND>
+    __device__ __forceinline__ Raw load(int row) const
+    {
+        if constexpr (E == 4) return Raw{*reinterpret_cast<const uint32_t*>(cls + row)};
+        else return Raw{*reinterpret_cast<const uint16_t*>(cls + row)};
+    }
+    // values by diagonal and mask of row e of the lane
+    template <int ND>
+    __device__ __forceinline__ unsigned row(const Raw& r, int e, VT (&a)[ND]) const
+    {
+        const unsigned c = (r.c >> (8 * e)) & 255u;
+        typedef VT V __attribute__((ext_vector_type(E)));
+#pragma unroll
+        for (int d = 0; d < ND; d += E) {
+            const V w = *reinterpret_cast<const V*>(tab->val + c * kClassDiag + d);
+#pragma unroll
+            for (int k = 0; k < E; ++k)
+                if (d + k < ND) a[d + k] = w[k];
+        }
+        return tab->mask[c];
+    }
+};
+
+// Row sums of U x E rows per lane, E = 16 / sizeof(VT) consecutive ones, every
+// load of x 16 bytes: rows [row, row + E) with all of row + off[d], d < ND, in
+// range (off[d] = 0 for the diagonals past the matrix's).  Entries a row does
+// not have are and-ed to +0 before they are added, and the sums start from
+// +0 (so they never are -0): the CSR sums bit for bit.
+template <typename VT, int ND, int U, typename SRC>
+struct WideRows {
+    using W = WideOf<VT>;
+    static constexpr int E = W::E;
+    typename W::T xv[U][ND];
+    typename SRC::Raw raw[U];
+
+    __device__ __forceinline__ void load(const int (&row)[U], const int* off, const VT* __restrict__ x, const SRC& src)
+    {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            raw[u] = src.template load<ND>(row[u]);
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+                xv[u][d] = ld_at<typename W::T>(x + off[d], (unsigned)row[u] * (unsigned)sizeof(VT));
+        }
+    }
+    __device__ __forceinline__ VT sum(int u, int e, const SRC& src) const
+    {
+        VT a[ND];
+        const unsigned m = src.template row<ND>(raw[u], e, a);
+        VT s = VT(0);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            const VT prod = a[d] * xv[u][d][e];
+            // all ones: the row has the entry (the empty asm keeps the compiler
+            // from making it a compare and a select again)
+            int on = __builtin_amdgcn_sbfe((int)m, d, 1);
+            asm("" : "+v"(on));
+            if constexpr (sizeof(VT) == 4) {
+                s = s + __builtin_bit_cast(float, __builtin_bit_cast(int, prod) & on);
+            } else {
+                const auto b = __builtin_bit_cast(unsigned long long, prod);
+                s = s + lanes_f64((unsigned)b & (unsigned)on, (unsigned)(b >> 32) & (unsigned)on);
+            }
+        }
+        return s;
+    }
+};
 
 struct NoLoads {
     __device__ __forceinline__ void operator()() const {}
