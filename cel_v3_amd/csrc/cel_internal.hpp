@@ -172,6 +172,8 @@ struct Derived {
     bool tried = false, tried32 = false, tried64 = false;
     int nd = 0;        // diagonals (0: more than kClassDiag, or unsorted rows)
     int off[32] = {};  // ascending
+    enum { kOwnDia = 0, kVals, kVals32 };
+    signed char sym[3] = {-1, -1, -1};  // symmetric: Mat::dia_vals, vals, vals32 (-1: not looked at)
     DevBuf<uint8_t> cls;      // per row: its class
     DevBuf<double> tab64;     // val64, then jac64
     DevBuf<float> tab32;
@@ -305,7 +307,9 @@ int launch_dia_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const 
 int dia_prepare_f32(Mat& A);
 // The derived form (Derived::k*) a PCG solve of at most iter_max iterations
 // runs on, built on the first call that wants it; never an error.
-int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max);
+// *symmetric: the diagonal storage the solve runs on (its own or a derived
+// one) holds bit for bit the same value at (i, j) and (j, i).
+int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric);
 // The distinct offsets col - row of the local block, ascending, at most
 // `most` (<= 32) of them: *nd = most + 1 when there are more.  *ascending:
 // every row's columns strictly ascend (known only when *nd <= most).

@@ -233,10 +233,12 @@ struct MatView {
     int nd;
     int dzero;               // index of the diagonal with offset 0, or -1
     int doff[32];
+    int dwide;                    // the K1 walks the diagonals with several rows per lane
+    long long dbase[kClassDiag];  // then entry (i, d) is dvals[dbase[d] + i] (dia_bases)
     // row classes (rowclass.hip), with the diagonals above
     const uint8_t* cls;
     RowClasses ctab;
-    const int* walk;  // by K1 block: the walk it takes (null: its own)
+    const int* walk;  // by K1 block, wide walks: the walk it takes (null: its own)
     // halo (FP64 only)
     const int *hrow_tile, *hrows, *hrowq, *hptr, *hcols;
     const double* hvals;
@@ -308,6 +310,11 @@ struct StageOf {
 template <typename VT, bool LONG>
 struct StageOf<VT, kFmtClass, LONG> {
     using T = ClassTab<VT>;
+};
+struct NoStage {};
+template <typename VT, bool LONG>
+struct StageOf<VT, CEL_FMT_DIA, LONG> {
+    using T = NoStage;
 };
 
 template <typename VT>
@@ -557,9 +564,9 @@ __device__ __forceinline__ void next_scalars(Ctrl& c, double rz, double rr, cons
     }
 }
 
-// Tile groups a row-class K1 sums per step: with 2, four waves of FP32 lanes
-// have one 16-byte task each and those of FP64 two.
-constexpr int kClassGroups = 2;
+// Most tile groups a wide walk sums per step: with 2, the four waves have one
+// 16-byte task each in FP32 and two in FP64.
+constexpr int kWideGroups = 2;
 
 // What the tile walk of a K1 does with the rows besides the product: nothing,
 // or (k_pcg_step) p_new and x += sigma p of the thread's rows.
@@ -571,85 +578,107 @@ struct StepRows {
     bool upd;  // x is updated (uniform; false right after a set-up or replacement)
 };
 
-// LDS of the wide walk: the rows' terms of v.d, two steps of them.
+// LDS of a wide walk: the rows' terms of v.d, two steps of them.
 struct WideStage {
-    double prod[2][kClassGroups * kTileGroup * kTileRows];
+    double prod[2][kWideGroups * kTileGroup * kTileRows];
 };
-struct NoStage {};
-template <int FMT>
+template <int FMT, bool HALO, bool STEP>
+constexpr bool wide_form = FMT == kFmtClass || (FMT == CEL_FMT_DIA && !HALO && !STEP);
+template <bool WIDE>
 struct WideStageOf {
     using T = NoStage;
 };
 template <>
-struct WideStageOf<kFmtClass> {
+struct WideStageOf<true> {
     using T = WideStage;
 };
 
-// k1_tiles of row classes: v = A d with E = 16 / sizeof(VT) consecutive rows
-// per lane.  What bounds a product of so few bytes per row (x, v and a byte)
-// is the work per row: one row per lane took 7 loads, 8 LDS reads and 90
-// instructions, 56.6 us on the 256^3 block in FP32 (151 MB); this one takes
-// 7/4 loads, 3 LDS reads and 45 instructions, 35.8 us (4.2 TB/s).  (Loading
-// the next step before the sums needs two sets of registers; in FP32 they
-// spill, 50 us.)  The rows of a step are those of the row-per-thread kernels
-// (kClassGroups groups of kTileGroup tiles) and their terms of v.d go
-// through LDS to the threads that add them there, so the partials are the
-// same bit for bit.  Waves that hold a row without all of its neighbours in
-// [0, n) (the ends of the matrix) take loads that are checked one by one
-// (edge).  Per iteration,
-// before and after: mixed 256^3 150.6 -> 130.2 us, 200^3 79.5 -> 68.5, 128^3
-// 30.5 -> 29.8, 100^3 23.7 -> 23.7; FP64 256^3 283 -> 244, 200^3 141 -> 120,
-// 128^3 47 -> 43, 100^3 28.7 -> 27.5.
-template <typename VT, int ND, typename SRC, typename EDGE>
+// k1_tiles of row classes and of symmetric diagonal storage: v = A d with E =
+// 16 / sizeof(VT) consecutive rows per lane.  What bounds a product of so few
+// bytes per row (classes: x, v and a byte) is the work per row: one row per
+// lane took 7 loads, 8 LDS reads and 90 instructions, 56.6 us on the 256^3
+// block in FP32 (151 MB); this one takes 7/4 loads, 3 LDS reads and 45
+// instructions, 35.8 us (4.2 TB/s).  The rows of a step are those of the
+// row-per-thread kernels (NG groups of kTileGroup tiles) and their terms of
+// v.d go through LDS to the threads that add them there, so the partials are
+// the same bit for bit.  Waves that hold a row without all of its neighbours
+// in [0, n) (the ends of the matrix) take loads that are checked one by one
+// (edge).  AHEAD: the next step's loads are issued before the sums of this
+// one, into a second set of registers: for diagonals in FP64, whose loads are
+// memory's (200^3 192 us per iteration without, 181 with); by classes it
+// measured slower (FP64 100^3 27.8 against 28.9 us), in FP32 it spills (K1 of
+// 256^3 50 us).
+// Per iteration, before and after, classes: mixed 256^3 150.6 -> 130.2 us,
+// 200^3 79.5 -> 68.5, 128^3 30.5 -> 29.8, 100^3 23.7 -> 23.7; FP64 256^3 283
+// -> 244, 200^3 141 -> 120, 128^3 47 -> 43, 100^3 28.7 -> 27.5.  Symmetric
+// diagonals: FP64 256^3 454 -> 407, 200^3 208 -> 181, 128^3 58.3 -> 51.8,
+// 820,911 rows 29.5 -> 27.2; mixed 128^3 36.7 -> 33.0.
+template <typename VT, int ND, int NG, bool AHEAD, typename SRC, typename EDGE>
 __device__ __forceinline__ double k1_wide(const MatView& A, const VT* __restrict__ x, VT* __restrict__ v,
                                           const SRC& src, const EDGE& edge, WideStage& st, int walk)
 {
-    constexpr int E = WideOf<VT>::E, WR = 64 * E;               // rows of a wave
-    constexpr int NG = kClassGroups, GR = kTileGroup * kTileRows;  // groups per step, rows of a group
-    constexpr int WPG = GR / WR;                                // waves that cover a group
-    constexpr int U = NG * WPG / kWaves;                        // tasks of a wave per step
-    static_assert(NG * WPG % kWaves == 0 && GR % WR == 0, "whole tasks");
+    constexpr int E = WideOf<VT>::E, WR = 64 * E;        // rows of a wave's task
+    constexpr int GR = kTileGroup * kTileRows;           // rows of a group
+    constexpr int WPG = GR / WR, U = NG * WPG / kWaves;  // tasks of a group, and of a wave per step
+    static_assert(NG <= kWideGroups && NG * WPG % kWaves == 0 && GR % WR == 0, "whole tasks");
+    using V = typename WideOf<VT>::T;
     const long long ngroups = ((long long)A.n + GR - 1) / GR, G = gridDim.x;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int omin = min(0, A.doff[0]), omax = max(0, A.doff[A.nd - 1]);
-    double acc = 0.0;
-    int buf = 0;
-    for (long long q = walk; q < ngroups; q += NG * G, buf ^= 1) {
-        int row[U], at[U];
-        bool inside = true;  // uniform across the wave
+    // the first rows that have all neighbours, as a multiple of E: what a task
+    // loads that is summed row by row (loads under a branch would be waited
+    // for at its end)
+    const int safe = (-omin + E - 1) / E * E;
+    struct Step {
+        WideRows<VT, ND, U, SRC> R;
+        V xr[U];
+        int row[U];
+        bool inside;  // uniform across the wave
+    };
+    // the u-th task of the step at q: its first row, and the place of its terms
+    auto first_row = [&](long long q, int u) -> long long {
+        const int task = u * kWaves + wave;
+        return (q + task / WPG * G) * GR + task % WPG * WR;
+    };
+    auto place = [&](int u) { return (u * kWaves + wave) * WR + lane * E; };
+    auto fetch = [&](long long q, Step& T) {
+        T.inside = true;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int task = u * kWaves + wave, g = task / WPG;
-            const long long w0 = (q + g * G) * GR + (task % WPG) * WR;
-            inside = inside && w0 + omin >= 0 && w0 + WR + omax <= A.n;
-            row[u] = w0 < A.n ? (int)w0 + lane * E : A.n;
-            at[u] = g * GR + (task % WPG) * WR + lane * E;
+            const long long w0 = first_row(q, u);
+            T.inside = T.inside && w0 + omin >= 0 && w0 + WR + omax <= A.n;
         }
-        double* prod = st.prod[buf];
-        if (inside) {
-            WideRows<VT, ND, U, SRC> R;
-            R.load(row, A.doff, x, src);
-            typename WideOf<VT>::T xr[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) xr[u] = *reinterpret_cast<const typename WideOf<VT>::T*>(x + row[u]);
+        for (int u = 0; u < U; ++u) T.row[u] = (T.inside ? (int)first_row(q, u) : safe) + lane * E;
+        T.R.load(T.row, A.doff, x, src);
+#pragma unroll
+        for (int u = 0; u < U; ++u) T.xr[u] = ld_at<V>(x, (unsigned)T.row[u] * (unsigned)sizeof(VT));
+    };
+    double acc = 0.0;
+    int buf = 0;
+    auto sum = [&](long long q, const Step& T) {
+        double* prod = st.prod[buf];
+        buf ^= 1;
+        if (T.inside) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                typename WideOf<VT>::T vv;
+                V vv;
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
-                    const VT s = R.sum(u, e, src);
+                    const VT s = T.R.sum(u, e, src);
                     vv[e] = s;
-                    prod[at[u] + e] = double(s) * double(xr[u][e]);
+                    prod[place(u) + e] = double(s) * double(T.xr[u][e]);
                 }
-                *reinterpret_cast<typename WideOf<VT>::T*>(v + row[u]) = vv;
+                *reinterpret_cast<V*>(v + T.row[u]) = vv;
             }
         } else {
 #pragma unroll 1
             for (int u = 0; u < U; ++u) {
+                const long long r0 = first_row(q, u) + lane * E;
                 int r[E];
                 VT s[E], pr[E];
 #pragma unroll
-                for (int e = 0; e < E; ++e) r[e] = min(row[u] + e, A.n);
+                for (int e = 0; e < E; ++e) r[e] = (int)min(r0 + e, (long long)A.n);
                 if (r[0] < A.n) edge(r, s, pr);
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
@@ -660,13 +689,37 @@ __device__ __forceinline__ double k1_wide(const MatView& A, const VT* __restrict
                         v[r[e]] = sk;
                         t = double(sk) * double(d);
                     }
-                    prod[at[u] + e] = t;
+                    prod[place(u) + e] = t;
                 }
             }
         }
         __syncthreads();  // one per step: the next one writes the other half
 #pragma unroll
         for (int k = 0; k < NG * kTileGroup; ++k) acc = acc + prod[k * kTileRows + threadIdx.x];
+    };
+    if ((long long)safe + WR + omax > A.n) {  // no such rows (uniform across the grid)
+        Step T;
+        T.inside = false;
+        for (long long q = walk; q < ngroups; q += NG * G) sum(q, T);
+    } else if constexpr (!AHEAD) {
+        for (long long q = walk; q < ngroups; q += NG * G) {
+            Step T;
+            fetch(q, T);
+            sum(q, T);
+        }
+    } else {
+        // two sets of registers by turns: a copy would wait for the loads
+        Step T0, T1;
+        if (walk < ngroups) fetch(walk, T0);
+        for (long long q = walk; q < ngroups; q += 2 * NG * G) {
+            fetch(q + NG * G, T1);
+            __builtin_amdgcn_sched_barrier(0);
+            sum(q, T0);
+            if (q + NG * G >= ngroups) break;
+            fetch(q + 2 * NG * G, T0);
+            __builtin_amdgcn_sched_barrier(0);
+            sum(q + NG * G, T1);
+        }
     }
     return acc;
 }
@@ -679,7 +732,7 @@ __device__ __forceinline__ double k1_wide(const MatView& A, const VT* __restrict
 template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, bool KEEP, typename X>
 __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __restrict__ v,
                                            typename StageOf<VT, FMT, LONG>::T& sm,
-                                           typename WideStageOf<FMT>::T& wide,
+                                           typename WideStageOf<wide_form<FMT, HALO, STEP>>::T& wide,
                                            const StepRows<VT>& st, int walk = 0)
 {
     const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
@@ -765,8 +818,22 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
         auto edge = [&](const int (&r)[WideOf<VT>::E], VT (&s)[WideOf<VT>::E], VT (&pr)[WideOf<VT>::E]) {
             class_rows<VT, WideOf<VT>::E>(A.n, A.nd, A.doff, A.cls, sm, r, x, s, pr, A.dzero);
         };
-        acc = A.nd <= 7 ? k1_wide<VT, 7>(A, x.x, v, src, edge, wide, walk) : k1_wide<VT, 8>(A, x.x, v, src, edge, wide, walk);
+        acc = A.nd <= 7 ? k1_wide<VT, 7, 2, false>(A, x.x, v, src, edge, wide, walk)
+                        : k1_wide<VT, 8, 2, false>(A, x.x, v, src, edge, wide, walk);
     } else if constexpr (FMT == CEL_FMT_DIA) {
+        if constexpr (!HALO && !STEP) {
+            if (A.dwide) {  // uniform
+                const WideDiags<VT, KEEP> src{dia_vals<VT>(A), A.dbase, A.dmask8};
+                auto edge = [&](const int (&r)[WideOf<VT>::E], VT (&s)[WideOf<VT>::E], VT (&pr)[WideOf<VT>::E]) {
+                    dia_rows<VT, WideOf<VT>::E, (WideOf<VT>::E >= 4 ? 4 : 8), KEEP>(
+                        A.n, A.nd, A.doff, dia_vals<VT>(A), A.dmask8, nullptr, r, x, s, pr, A.dzero);
+                };
+                constexpr bool F64 = sizeof(VT) == 8;
+                constexpr int NG = F64 ? 1 : 2;
+                return A.nd <= 7 ? k1_wide<VT, 7, NG, F64>(A, x.x, v, src, edge, wide, walk)
+                                 : k1_wide<VT, 8, NG, F64>(A, x.x, v, src, edge, wide, walk);
+            }
+        }
         // all tiles of a group per step, one row of each per thread; the
         // rows are added to the partial in tile order, as in the CSR K1.
         // Halo rows (HALO): as in the CSR K1, a row's record is added after
@@ -876,19 +943,22 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
     return acc;
 }
 
-// LDS of a K1: its tile stage; in the mixed form the FP64 stage of a
-// replacement residual takes the same place.
-template <typename VT, int FMT, bool LONG>
+// LDS of a K1: its tile stage and that of a wide walk; in the mixed form the
+// FP64 stage of a replacement residual takes the same place.
+template <typename VT, int FMT, bool LONG, bool WIDE>
 union K1Stage {
-    typename StageOf<VT, FMT, LONG>::T tile;
-    typename StageOf<double, FMT, LONG>::T res;
+    struct {
+        typename StageOf<VT, FMT, LONG>::T tile;
+        typename WideStageOf<WIDE>::T wide;
+    };
+    typename StageOf<double, FMT == CEL_FMT_DIA ? CEL_FMT_CSR : FMT, LONG>::T res;
 };
 
-// Waves per SIMD the K1s are compiled for.  The FP64 wide walk holds two
-// tasks' loads in registers; the FP64 K1s run on 2 blocks per CU
+// Waves per SIMD the K1s are compiled for.  The FP64 wide walks hold the loads
+// of two tasks or steps in registers; the FP64 K1s run on 2 blocks per CU
 // (kK1BlocksPerCuF64), so it may take the registers of 2 waves.
 template <typename VT, int FMT>
-constexpr int k1_waves = sizeof(VT) == 8 && FMT == kFmtClass ? 2 : 4;
+constexpr int k1_waves = sizeof(VT) == 8 && (FMT == kFmtClass || FMT == CEL_FMT_DIA) ? 2 : 4;
 
 // K1: v = A p, per-block partial of v.p.  Mixed: a requested replacement
 // residual takes the place of the product (K2 and K3 then do nothing, and
@@ -901,8 +971,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves
                                                      Ctrl* __restrict__ cout, Prm P)
 {
     constexpr bool MIXED = sizeof(VT) == 4;
-    __shared__ K1Stage<VT, FMT, LONG> sm;
-    __shared__ typename WideStageOf<FMT>::T wide;
+    __shared__ K1Stage<VT, FMT, LONG, wide_form<FMT, HALO, false>> sm;
     __shared__ double red[3 * kWaves];
     __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
@@ -919,16 +988,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves
             return;
         }
     }
-    // the walk (first group, and the partial's slot) of this block: by classes
-    // it may be another block's
+    // the walk (first group, and the partial's slot) of this block: a wide one
+    // may be another block's
     int walk = blockIdx.x, slot = logical_block();
-    if constexpr (FMT == kFmtClass) {
+    if constexpr (wide_form<FMT, HALO, false>) {
         if (A.walk) {
             walk = A.walk[blockIdx.x];
             slot = gridDim.x % kXcds ? walk : (walk % kXcds) * (gridDim.x / kXcds) + walk / kXcds;
         }
     }
-    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, sm.tile, wide, StepRows<VT>{}, walk);
+    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, sm.tile, sm.wide, StepRows<VT>{}, walk);
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[slot] = bs;
     write_ctrl(cout, c);
@@ -953,8 +1022,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     Ctrl* __restrict__ cout, Prm P)
 {
     constexpr bool MIXED = sizeof(VT) == 4;
-    __shared__ K1Stage<VT, FMT, false> sm;
-    NoStage wide;
+    __shared__ K1Stage<VT, FMT, false, false> sm;
     __shared__ double red[3 * kWaves];
     __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
@@ -1005,7 +1073,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         return;
     }
     const double acc = k1_tiles<VT, FMT, false, false, true, true>(
-        A, XDirection<VT>{p, z, beta, pending}, v, sm.tile, wide, StepRows<VT>{pout, x, sigma, !pending});
+        A, XDirection<VT>{p, z, beta, pending}, v, sm.tile, sm.wide, StepRows<VT>{pout, x, sigma, !pending});
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[logical_block()] = bs;
     write_ctrl(cout, c);
@@ -1663,6 +1731,27 @@ int pcg_noalloc_setup(int device)
     return CEL_OK;
 }
 
+// Where the wide walk of a symmetric block finds the diagonals' values (V.nd
+// and V.doff are set): those below the main diagonal in the arrays above it,
+// as entry (i, i + o), o < 0, is entry (i + o, i) of the diagonal -o, so an
+// iteration reads 4 of 7 arrays.  Returns the number of arrays.
+static int dia_bases(MatView& V)
+{
+    int arrays = V.nd;
+    V.dwide = 1;
+    for (int d = 0; d < V.nd; ++d) {
+        V.dbase[d] = (long long)d * V.n;
+        if (V.doff[d] >= 0) continue;
+        for (int u = d + 1; u < V.nd; ++u)
+            if (V.doff[u] == -V.doff[d]) {
+                V.dbase[d] = (long long)u * V.n + V.doff[d];
+                --arrays;
+                break;
+            }
+    }
+    return arrays;
+}
+
 // Device pointers of one solve's work vectors, partial sums and token.
 struct WorkPtrs {
     double *r = nullptr, *p = nullptr, *v = nullptr, *part1 = nullptr, *part2 = nullptr,
@@ -1752,18 +1841,16 @@ int pcg_spmv_dot(Mat& A, int fmt, const double* x, const double* ghost, double* 
     return CEL_OK;
 }
 
-// The walks of a row-class K1's blocks: the walks whose groups start in the
+// The walks of a wide K1's blocks: the walks whose groups start in the
 // same eighth of the matrix's period (its farthest diagonal) go to one XCD,
 // so the rows a tile gathers from the planes beside it, and all but the
 // outermost of its own plane's neighbours, are in that XCD's L2.  Each block
 // keeps its walk's slot, so the partials are the same.  Measured per
 // iteration: mixed 100^3 27.0 -> 24.3 us, 200^3 82.0 -> 80.2; FP64 256^3
-// 357 -> 351.
-static int class_walk(const Mat& A, Workspace& W, int G, const int** walk)
+// 357 -> 351; symmetric diagonals FP64 200^3 198 -> 192.
+static int wide_walk(MatView& V, Workspace& W, int G)
 {
-    *walk = nullptr;
-    const Derived& D = A.derived;
-    const int far = std::max(std::abs(D.off[0]), std::abs(D.off[D.nd - 1]));
+    const int far = std::max(std::abs(V.doff[0]), std::abs(V.doff[V.nd - 1]));
     const int period = std::max(1, (far + kTileGroup * kTileRows / 2) / (kTileGroup * kTileRows));
     if (G % kXcds || period < 2 * kXcds) return CEL_OK;
     std::vector<int> order(G), w(G);
@@ -1775,7 +1862,7 @@ static int class_walk(const Mat& A, Workspace& W, int G, const int** walk)
     CEL_TRY(W.walk.reserve(G));
     CEL_HIP(hipMemcpyAsync(W.walk.p, w.data(), sizeof(int) * G, hipMemcpyHostToDevice, rt().stream));
     CEL_HIP(hipStreamSynchronize(rt().stream));
-    *walk = W.walk.p;
+    V.walk = W.walk.p;
     return CEL_OK;
 }
 
@@ -1867,7 +1954,9 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     // the form the K1s run on, and its residual's: the caller's, or a derived
     // one with the same bits (its grids are the caller's form's)
     int use = Derived::kNone;
-    if (!noalloc && !halo && !coo && fmt != CEL_FMT_JAD) use = derived_prepare(A, fmt, mixed, prm.iter_max);
+    bool symmetric = false;
+    if (!noalloc && !halo && !coo && fmt != CEL_FMT_JAD)
+        use = derived_prepare(A, fmt, mixed, prm.iter_max, &symmetric);
     const int kfmt = use == Derived::kClasses ? kFmtClass : use == Derived::kDiagonals ? CEL_FMT_DIA : fmt;
     const int kres = use == Derived::kClasses ? kFmtClass : rfmt;
 
@@ -2045,13 +2134,17 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         V.dmask = nullptr;
         V.dmask8 = D.mask8.p;
     }
-    const bool keep = keep_matrix(A, kfmt, V.nd, mixed);
-    if (use == Derived::kClasses) CEL_TRY(class_walk(A, *Wp, G1, &V.walk));
     V.dzero = -1;
     for (int d = 0; d < V.nd; ++d) {
         V.doff[d] = doff[d];
         if (doff[d] == 0) V.dzero = d;
     }
+    const bool sym = kfmt == CEL_FMT_DIA && symmetric;
+    const int arrays = sym ? dia_bases(V) : V.nd;
+    // (a symmetric block's values are read again a row, a line and a plane
+    // later: 256^3 FP64 427 us per iteration marked as read once, 425 kept)
+    const bool keep = sym || keep_matrix(A, kfmt, arrays, mixed);
+    if (use == Derived::kClasses || sym) CEL_TRY(wide_walk(V, *Wp, G1));
     if (halo) {
         V.hrow_tile = Wp->hrow_tile.p;
         V.hrows = A.halo_rows.p;
@@ -2307,7 +2400,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     stats.spmv_bytes = spmv_bytes(A, fmt, prec);
     if (jadp) stats.spmv_bytes -= 4.0 * n;  // the permuted-order K1 reads no permutation
     // a derived form: a class or mask byte per row, the diagonals' values, p and v
-    if (use != Derived::kNone) stats.spmv_bytes = (1.0 + (bycls ? 2.0 : 2.0 + V.nd) * vb) * n;
+    if (use != Derived::kNone || sym) stats.spmv_bytes = (1.0 + (bycls ? 2.0 : 2.0 + arrays) * vb) * n;
     {
         // K1 matrix + p gather + v write ; K2 r,v,jac read + r write ;
         // K3 p,r,jac,x read + p,x write

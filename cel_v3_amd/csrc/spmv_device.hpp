@@ -328,6 +328,14 @@ __device__ __forceinline__ T ld_at(const void* base, unsigned o)
     return *reinterpret_cast<const T*>(static_cast<const char*>(base) + o);
 }
 
+// The bytes of a lane's E rows (E = 2 or 4, p a multiple of E).
+template <int E>
+__device__ __forceinline__ unsigned ld_bytes(const uint8_t* p)
+{
+    if constexpr (E == 4) return *reinterpret_cast<const uint32_t*>(p);
+    else return *reinterpret_cast<const uint16_t*>(p);
+}
+
 // The rows of a wide step: where their matrix values come from.
 // Row classes: a byte per row, values and mask from the table in LDS.
 template <typename VT>
@@ -335,18 +343,18 @@ struct WideClasses {
     static constexpr int E = WideOf<VT>::E;
     const uint8_t* cls;
     const ClassTab<VT>* tab;
+    template <int ND>
     struct Raw {
         unsigned c;
     };
     template <int ND>
-    __device__ __forceinline__ Raw load(int row) const
+    __device__ __forceinline__ Raw<ND> load(int row) const
     {
-        if constexpr (E == 4) return Raw{*reinterpret_cast<const uint32_t*>(cls + row)};
-        else return Raw{*reinterpret_cast<const uint16_t*>(cls + row)};
+        return Raw<ND>{ld_bytes<E>(cls + row)};
     }
     // values by diagonal and mask of row e of the lane
     template <int ND>
-    __device__ __forceinline__ unsigned row(const Raw& r, int e, VT (&a)[ND]) const
+    __device__ __forceinline__ unsigned row(const Raw<ND>& r, int e, VT (&a)[ND]) const
     {
         const unsigned c = (r.c >> (8 * e)) & 255u;
         typedef VT V __attribute__((ext_vector_type(E)));
@@ -361,6 +369,41 @@ struct WideClasses {
     }
 };
 
+// Diagonal storage: entry (i, d) at vals[base[d] + i], a presence byte per row.
+template <typename VT, bool KEEP>
+struct WideDiags {
+    using W = WideOf<VT>;
+    static constexpr int E = W::E;
+    const VT* vals;
+    const long long* base;
+    const uint8_t* mask;
+    template <int ND>
+    struct Raw {
+        typename W::T a[ND];
+        unsigned m;
+    };
+    template <int ND>
+    __device__ __forceinline__ Raw<ND> load(int row) const
+    {
+        Raw<ND> r;
+        r.m = ld_bytes<E>(mask + row);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            const typename W::T* p = reinterpret_cast<const typename W::T*>(vals + base[d] + row);
+            if constexpr (KEEP) r.a[d] = *p;
+            else r.a[d] = __builtin_nontemporal_load(p);
+        }
+        return r;
+    }
+    template <int ND>
+    __device__ __forceinline__ unsigned row(const Raw<ND>& r, int e, VT (&a)[ND]) const
+    {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) a[d] = r.a[d][e];
+        return r.m >> (8 * e);
+    }
+};
+
 // Row sums of U x E rows per lane, E = 16 / sizeof(VT) consecutive ones, every
 // load of x 16 bytes: rows [row, row + E) with all of row + off[d], d < ND, in
 // range (off[d] = 0 for the diagonals past the matrix's).  Entries a row does
@@ -371,7 +414,7 @@ struct WideRows {
     using W = WideOf<VT>;
     static constexpr int E = W::E;
     typename W::T xv[U][ND];
-    typename SRC::Raw raw[U];
+    typename SRC::template Raw<ND> raw[U];
 
     __device__ __forceinline__ void load(const int (&row)[U], const int* off, const VT* __restrict__ x, const SRC& src)
     {
