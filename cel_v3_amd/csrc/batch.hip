@@ -78,13 +78,49 @@ struct BSys {
 struct BBlk {
     int sys;         // -1: idle
     int t0, t1;      // K1 tiles [t0, t1)
+    int slot;        // of their partials
     long long u0, u1;  // K2/K3 units of 256 elements [u0, u1)
+};
+
+// The form K1 reads a system's matrix in (rowclass.hip): its CSR arrays, row
+// classes or diagonal storage (entry (i, d) at vals[base[d] + i]).
+struct BForm {
+    enum { kCsr = 0, kClasses, kDiagonals };
+    int kind, nd;
+    int arrays;      // diagonals that are read
+    int omin, omax;  // least and greatest of 0 and the offsets
+    int off[kClassDiag];
+    long long base[kClassDiag];
+    const double* vals;     // [nd][n]; classes: the table's values
+    const uint8_t* rowb;    // per row: presence bits or class
+    const uint32_t* cmask;  // classes: presence bits
 };
 
 struct BPrm {
     double tol, small;
     int tol_mode, iter_max, alpha_stop, kpmax;
 };
+
+// A pointer that a kernel finds in memory, not in its arguments.  Through the
+// integer the compiler knows that it points to global memory; otherwise its
+// loads are flat ones, which wait for LDS as well and for each other (K1 by
+// diagonals of 4 systems of 1.15M rows: 105 us so, 61 us with global loads;
+// by CSR 107 -> 93, 16 right-hand sides on 128^3 648 -> 625 us per iteration).
+template <typename T>
+__device__ __forceinline__ T* as_global(T* p)
+{
+    return (T*)(__attribute__((address_space(1))) T*)(unsigned long long)p;
+}
+
+__device__ __forceinline__ BSys load_sys(const BSys* p)
+{
+    BSys S = *p;
+    S.xadj = as_global(S.xadj);
+    S.cols = as_global(S.cols);
+    S.vals = as_global(S.vals);
+    S.jac = as_global(S.jac);
+    return S;
+}
 
 enum { kBReduceNone = 0, kBReduceSetup = 1 };
 
@@ -242,7 +278,7 @@ __global__ __launch_bounds__(kBlock) void k_bresidual(const BSys* __restrict__ s
     const int b = blockIdx.x;  // hardware order: a block range has equal shares of every XCD
     const BBlk blk = tbl[b];
     if (blk.sys < 0) return;
-    const BSys S = sys[blk.sys];
+    const BSys S = load_sys(sys + blk.sys);
     const double* xs = x + S.voff;
     const int j = threadIdx.x & (S.kp - 1);
     double arz = 0.0, arr = 0.0, abb = 0.0;
@@ -268,9 +304,9 @@ __global__ __launch_bounds__(kBlock) void k_bresidual(const BSys* __restrict__ s
     const double s2 = lane_block_sum(arr, S.kp, red);
     const double s3 = lane_block_sum(abb, S.kp, red);
     if (threadIdx.x < S.kp) {
-        part[(size_t)b * kpmax + threadIdx.x] = s1;
-        part[((size_t)G + b) * kpmax + threadIdx.x] = s2;
-        part[((size_t)2 * G + b) * kpmax + threadIdx.x] = s3;
+        part[(size_t)blk.slot * kpmax + threadIdx.x] = s1;
+        part[((size_t)G + blk.slot) * kpmax + threadIdx.x] = s2;
+        part[((size_t)2 * G + blk.slot) * kpmax + threadIdx.x] = s3;
     }
     if (b == S.b0 && threadIdx.x < S.kp) {
         BCtrl c{};
@@ -280,9 +316,122 @@ __global__ __launch_bounds__(kBlock) void k_bresidual(const BSys* __restrict__ s
     }
 }
 
+// LDS of K1: a CSR chunk (diagonals of several right-hand sides: the chunk's
+// values by diagonal, and its rows' presence bits in place of the columns),
+// or the class table and two steps of a wide walk's terms.
+union BK1Stage {
+    CsrStage<double> csr;
+    struct {
+        ClassTab<double> tab;
+        double prod[2][2 * kTileRows];
+    };
+};
+
+// v = A p of tiles [t0, t1) by classes or diagonals, one right-hand side: two
+// consecutive rows per lane, 16-byte loads, two tiles per step; the rows'
+// terms of v.p go through LDS to the threads that add them in the CSR walk,
+// so the partials are the same bit for bit (pcg.hip, k1_wide).
+template <int ND, typename SRC, typename EDGE>
+__device__ __forceinline__ double b_wide(int n, const BForm& F, const double* __restrict__ x,
+                                         double* __restrict__ v, const SRC& src, const EDGE& edge,
+                                         double (*prod2)[2 * kTileRows], int t0, int t1)
+{
+    using V = WideOf<double>::T;
+    constexpr int E = 2, WR = 64 * E;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int omin = F.omin, omax = F.omax;
+    const long long hi = min((long long)t1 * kTileRows, (long long)n);
+    double acc = 0.0;
+    int buf = 0;
+    for (int t = t0; t < t1; t += 2, buf ^= 1) {
+        double* prod = prod2[buf];
+        const long long w0 = (long long)t * kTileRows + wave * WR;
+        const int at = wave * WR + lane * E;
+        if (w0 + omin >= 0 && w0 + WR <= hi && w0 + WR + omax <= n) {  // uniform across the wave
+            WideRows<double, ND, 1, SRC> R;
+            const int row[1] = {(int)w0 + lane * E};
+            R.load(row, F.off, x, src);
+            const V xr = ld_at<V>(x, (unsigned)row[0] * 8u);
+            V vv;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const double sum = R.sum(0, e, src);
+                vv[e] = sum;
+                prod[at + e] = sum * xr[e];
+            }
+            *reinterpret_cast<V*>(v + row[0]) = vv;
+        } else {
+            int r[E];
+            double sum[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const long long re = w0 + lane * E + e;
+                r[e] = re < hi ? (int)re : n;
+            }
+            if (r[0] < n) edge(r, sum);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                double d = 0.0;
+                if (r[e] < n) {
+                    v[r[e]] = sum[e];
+                    d = sum[e] * x[r[e]];
+                }
+                prod[at + e] = d;
+            }
+        }
+        __syncthreads();  // one per step: the next one writes the other half
+        acc = acc + prod[threadIdx.x];
+        acc = acc + prod[kTileRows + threadIdx.x];
+    }
+    return acc;
+}
+
+// One chunk of 256 rows, kp right-hand sides, two per thread, by classes (CLS,
+// the table in LDS) or diagonals (the chunk staged in LDS): the gathers of a
+// row depend on nothing that is loaded.  An entry that the row does not have
+// gathers the row's own x and is and-ed to +0.
+template <int ND, bool CLS>
+__device__ __forceinline__ void b_wide_rows(const BSys& S, const BForm& F, const uint8_t* rowb,
+                                            const BK1Stage& sm, int r0, int r1,
+                                            const double* __restrict__ pl, double* __restrict__ vl, double& acc,
+                                            double& acc1)
+{
+    const int kh = S.ksh - 1, R2 = kBlock >> kh, my = threadIdx.x >> kh;
+    for (int row = r0 + my; row < r1; row += R2) {
+        Dbl2 xv[ND];
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            const int c = row + F.off[d];
+            xv[d] = *(const Dbl2*)(pl + ((size_t)((unsigned)c < (unsigned)S.n ? c : row) << S.ksh));
+        }
+        const Dbl2 pr = *(const Dbl2*)(pl + ((size_t)row << S.ksh));
+        const int l = CLS ? rowb[row] : row - r0;
+        const unsigned m = CLS ? sm.tab.mask[l] : (unsigned)sm.csr.col[l];
+        double sum0 = 0.0, sum1 = 0.0;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            const double a = CLS ? sm.tab.val[l * kClassDiag + d] : sm.csr.val[d * kTileRows + l];
+            const bool on = (m >> d) & 1u;
+            const double t0 = a * xv[d].x, t1 = a * xv[d].y;
+            sum0 = sum0 + (on ? t0 : 0.0);
+            sum1 = sum1 + (on ? t1 : 0.0);
+        }
+        Dbl2 vi;
+        vi.x = sum0;
+        vi.y = sum1;
+        // read by the next kernel only
+        __builtin_nontemporal_store(vi, (Dbl2*)(vl + ((size_t)row << S.ksh)));
+        const double d0 = vi.x * pr.x;
+        acc = acc + d0;
+        const double d1 = vi.y * pr.y;
+        acc1 = acc1 + d1;
+    }
+}
+
 // ---------------------------------------------------------------- K1
 // v = A p ; partial of v.p per lane.  Folds the set-up partials first.
-__global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_bspmv(const BSys* __restrict__ sys,
+                                                  const BForm* __restrict__ forms,
                                                   const BBlk* __restrict__ tbl,
                                                   const double* __restrict__ p,
                                                   double* __restrict__ v, double* __restrict__ part,
@@ -290,7 +439,8 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
                                                   const BCtrl* __restrict__ cin,
                                                   BCtrl* __restrict__ cout, BPrm P)
 {
-    __shared__ CsrStage<double> sm;
+    __shared__ BK1Stage stage;
+    CsrStage<double>& sm = stage.csr;
     __shared__ double red[4 * 64];
     __shared__ double s1[kMaxRhs], s2[kMaxRhs], s3[kMaxRhs];
     __shared__ BCtrl lc[kMaxRhs];
@@ -298,7 +448,7 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
     const int b = blockIdx.x;  // hardware order: a block range has equal shares of every XCD
     const BBlk blk = tbl[b];
     if (blk.sys < 0) return;
-    const BSys S = sys[blk.sys];
+    const BSys S = load_sys(sys + blk.sys);
     read_lanes(cin, S, lc);
     if (lc[0].reduce == kBReduceSetup) {  // the same for every lane
         lane_partials(rpart, kpmax, S.b0, S.b1, S.kp, S.ksh, s1, red);
@@ -335,7 +485,25 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
     const double* ps = p + S.voff;
     double* vs = v + S.voff;
     double acc = 0.0;
-    if (S.kp == 1) {
+    const BForm& F = forms[blk.sys];
+    const double* fvals = as_global(F.vals);
+    const uint8_t* rowb = as_global(F.rowb);
+    if (F.kind == BForm::kClasses) stage.tab.load(fvals, as_global(F.cmask));
+    if (S.kp == 1 && F.kind == BForm::kDiagonals) {
+        const WideDiags<double, true> src{fvals, F.base, rowb};
+        auto edge = [&](const int (&r)[2], double (&sum)[2]) {
+            dia_rows<double, 2, 8, true>(S.n, F.nd, F.off, fvals, rowb, nullptr, r, XPlain<double>{ps}, sum);
+        };
+        acc = F.nd <= 7 ? b_wide<7>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1)
+                        : b_wide<8>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1);
+    } else if (S.kp == 1 && F.kind == BForm::kClasses) {
+        const WideClasses<double> src{rowb, &stage.tab};
+        auto edge = [&](const int (&r)[2], double (&sum)[2]) {
+            class_rows<double, 2>(S.n, F.nd, F.off, rowb, stage.tab, r, XPlain<double>{ps}, sum);
+        };
+        acc = F.nd <= 7 ? b_wide<7>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1)
+                        : b_wide<8>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1);
+    } else if (S.kp == 1) {
         // one right-hand side: the pipelined LDS tile of the single-system K1
         // (256 rows per tile, the next tile's loads in flight meanwhile)
         CsrTileStream<double> cs;
@@ -418,6 +586,30 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
             const int r0 = c * kTileRows;
             if (r0 >= S.n) break;  // uniform
             const int r1 = min(r0 + kTileRows, S.n);
+            if (F.kind == BForm::kClasses) {
+                if (on2) {
+                    if (F.nd <= 7) b_wide_rows<7, true>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                    else b_wide_rows<8, true>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                }
+                continue;
+            }
+            if (F.kind == BForm::kDiagonals) {
+                const int row = r0 + threadIdx.x;
+                const unsigned m = row < r1 ? rowb[row] : 0u;
+                double a[kClassDiag];
+#pragma unroll
+                for (int d = 0; d < kClassDiag; ++d) a[d] = (m >> d) & 1u ? fvals[F.base[d] + row] : 0.0;
+                __syncthreads();  // the previous chunk's stage is consumed
+#pragma unroll
+                for (int d = 0; d < kClassDiag; ++d) sm.val[d * kTileRows + threadIdx.x] = a[d];
+                sm.col[threadIdx.x] = (int)m;
+                __syncthreads();
+                if (on2) {
+                    if (F.nd <= 7) b_wide_rows<7, false>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                    else b_wide_rows<8, false>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                }
+                continue;
+            }
             const int e0 = S.xadj[r0];
             const int cnt = S.xadj[r1] - e0;
             const bool staged = cnt <= kStageCap;  // uniform across the block
@@ -554,7 +746,7 @@ __global__ __launch_bounds__(kBlock) void k_bspmv(const BSys* __restrict__ sys,
         return;
     }
     const double bs = lane_block_sum(acc, S.kp, red);
-    if (threadIdx.x < S.kp) part[(size_t)b * kpmax + threadIdx.x] = bs;
+    if (threadIdx.x < S.kp) part[(size_t)blk.slot * kpmax + threadIdx.x] = bs;
     write_lanes(cout, S, b == S.b0, lc);
 }
 
@@ -592,7 +784,7 @@ __global__ __launch_bounds__(kBlock) void k_bupdate_r(const BSys* __restrict__ s
     const int b = blockIdx.x;  // hardware order: a block range has equal shares of every XCD
     const BBlk blk = tbl[b];
     if (blk.sys < 0) return;
-    const BSys S = sys[blk.sys];
+    const BSys S = load_sys(sys + blk.sys);
     read_lanes(cin, S, lc);
     if (threadIdx.x == 0) {
         int a = 0;
@@ -691,7 +883,7 @@ __global__ __launch_bounds__(kBlock) void k_bupdate_xp(const BSys* __restrict__ 
     const int b = blockIdx.x;  // hardware order: a block range has equal shares of every XCD
     const BBlk blk = tbl[b];
     if (blk.sys < 0) return;
-    const BSys S = sys[blk.sys];
+    const BSys S = load_sys(sys + blk.sys);
     read_lanes(cin, S, lc);
     if (threadIdx.x == 0) {
         int a = 0;
@@ -817,6 +1009,8 @@ struct Batch {
     DevBuf<double> r, p, v, x, b, part1, part2, rpart;
     DevBuf<BCtrl> ctrl;  // 3 slots of `lanes` tokens
     std::vector<BSys> h_sys;
+    DevBuf<BForm> d_form;
+    std::vector<BForm> h_form;
     bool tuned = false;
     Tuning tune{0, 16, 0, 1};
     double tuned_ms_per_iter = 0.0;
@@ -852,7 +1046,7 @@ static int build_table(Batch& B, int G, int weight, const std::vector<char>& act
         W += w[s];
         ++nact;
     }
-    tbl.assign(G, BBlk{-1, 0, 0, 0, 0});
+    tbl.assign(G, BBlk{-1, 0, 0, 0, 0, 0});
     for (int s = 0; s < S; ++s) {
         if (k23)
             B.h_sys[s].c0 = B.h_sys[s].c1 = 0;
@@ -893,9 +1087,18 @@ static int build_table(Batch& B, int G, int weight, const std::vector<char>& act
         (k23 ? H.c0 : H.b0) = cur;
         (k23 ? H.c1 : H.b1) = cur + nb[s];
         const long long units = (((long long)H.n << H.ksh) + kBlock - 1) / kBlock;
+        // K1's ranges go to the blocks of one XCD after another (block b runs
+        // on XCD b mod 8), so that the rows a band away, which gather the same
+        // p and share a symmetric block's values, are mostly in one L2; the
+        // partials stay in range order
+        std::vector<int> at(nb[s]);
+        std::iota(at.begin(), at.end(), cur);
+        if (!k23)
+            std::stable_sort(at.begin(), at.end(), [](int a, int b) { return a % kXcds < b % kXcds; });
         for (int i = 0; i < nb[s]; ++i) {
-            BBlk& e = tbl[cur + i];
+            BBlk& e = tbl[at[i]];
             e.sys = s;
+            e.slot = cur + i;
             e.t0 = (int)((long long)H.ntiles * i / nb[s]);
             e.t1 = (int)((long long)H.ntiles * (i + 1) / nb[s]);
             e.u0 = units * i / nb[s];
@@ -916,10 +1119,40 @@ static int upload_table(Batch& B, const std::vector<BBlk>& tbl, const std::vecto
                            s));
     CEL_HIP(hipMemcpyAsync(B.d_sys.p, B.h_sys.data(), sizeof(BSys) * B.h_sys.size(),
                            hipMemcpyHostToDevice, s));
+    CEL_HIP(hipMemcpyAsync(B.d_form.p, B.h_form.data(), sizeof(BForm) * B.h_form.size(),
+                           hipMemcpyHostToDevice, s));
     // the copies read pageable host memory: finish them before the host
     // vectors change
     CEL_HIP(hipStreamSynchronize(s));
     return CEL_OK;
+}
+
+// The forms this solve's K1 reads the matrices in (its own CSR arrays / the
+// derived form, whole solves): 64 systems of 24^3..96^3 129.7 / 103.2 ms, 16
+// of 60^3..90^3 72.7 / 57.3, 4 of 100^3..110^3 64.0 / 50.6, 8 of 20^3..40^3
+// 4.00 / 3.74; 16 right-hand sides on 128^3 251 / 244, 11 on 91^3 73.0 /
+// 70.5.
+static void choose_forms(Batch& B, int iter_max)
+{
+    const size_t S = B.mats.size();
+    B.h_form.assign(S, BForm{});
+    derived_prepare_all(B.mats, iter_max);
+    for (size_t q = 0; q < S; ++q) {
+        const Mat& A = *B.mats[q];
+        const Derived& D = A.derived;
+        BForm& F = B.h_form[q];
+        const bool cls = D.kind == Derived::kClasses;
+        if (!cls && !(D.nd > 0 && D.vals.p && D.mask8.p)) continue;
+        F.kind = cls ? BForm::kClasses : BForm::kDiagonals;
+        F.nd = D.nd;
+        for (int d = 0; d < D.nd; ++d) F.off[d] = D.off[d];
+        F.omin = std::min(0, D.off[0]);
+        F.omax = std::max(0, D.off[D.nd - 1]);
+        F.vals = cls ? D.tab64.p : D.vals.p;
+        F.rowb = cls ? D.cls.p : D.mask8.p;
+        F.cmask = D.tabm.p;
+        F.arrays = dia_bases(A.n, D.nd, D.off, !cls && D.sym[Derived::kVals] == 1, F.base);
+    }
 }
 
 struct RunResult {
@@ -940,6 +1173,8 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     CEL_TRY(B.part2.alloc((size_t)2 * G2 * B.kpmax));
     CEL_TRY(B.rpart.alloc((size_t)3 * G * B.kpmax));
     CEL_TRY(B.ctrl.alloc((size_t)3 * B.lanes));
+    choose_forms(B, iter_cap);
+    CEL_TRY(B.d_form.alloc(B.h_form.size()));
     std::vector<char> active(S, 1);
     std::vector<BBlk> tbl, tbl2;
     CEL_TRY(build_table(B, G, T.weight, active, tbl, false));
@@ -974,7 +1209,7 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
                     : stream == kBStreamX ? k_bupdate_xp<kBStreamX>
                                           : k_bupdate_xp<kBStreamNone>;
     auto enqueue_iter = [&]() -> int {
-        hipLaunchKernelGGL(k_bspmv, dim3(G), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl.p, B.p.p, B.v.p,
+        hipLaunchKernelGGL(k_bspmv, dim3(G), dim3(kBlock), 0, s, B.d_sys.p, B.d_form.p, B.d_tbl.p, B.p.p, B.v.p,
                            B.part1.p, B.rpart.p, B.kpmax, G, C0, C1, P);
         hipLaunchKernelGGL(k2, dim3(G2), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl2.p, B.r.p,
                            B.v.p, B.part2.p, B.part1.p, B.kpmax, G2, C1, C2);
@@ -1381,7 +1616,11 @@ extern "C" int cel_gpu_batch_solve(cel_gpu_batch* h, const double* const* b, dou
             const Mat& A = *B.mats[q];
             // per iteration: matrix once for all lanes, p gather + v write,
             // K2 r,v,jac read + r write, K3 p,r,jac,x read + p,x write
-            bytes += 12.0 * A.nnz + 4.0 * (A.n + 1) + 8.0 * A.n * B.kp[q] * 10.0;
+            const BForm& F = B.h_form[q];
+            double m = 12.0 * A.nnz + 4.0 * (A.n + 1);
+            if (F.kind != BForm::kCsr) m = 1.0 * A.n;  // a byte per row, and the diagonals' arrays
+            if (F.kind == BForm::kDiagonals) m += 8.0 * F.arrays * A.n;
+            bytes += m + 8.0 * A.n * B.kp[q] * 10.0;
         }
         total->iter_bytes = bytes;
     }

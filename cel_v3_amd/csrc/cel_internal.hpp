@@ -310,10 +310,25 @@ int dia_prepare_f32(Mat& A);
 // *symmetric: the diagonal storage the solve runs on (its own or a derived
 // one) holds bit for bit the same value at (i, j) and (j, i).
 int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric);
+// The FP64 derived forms of a batch's matrices, smaller ones too.
+void derived_prepare_all(const std::vector<Mat*>& mats, int iter_max);
+// Where the wide walks find the values of nd <= kClassDiag diagonals: entry
+// (i, d) at base[d] + i of storage [nd][n].  Symmetric: those below the main
+// diagonal in the arrays above it, as entry (i, i + o), o < 0, is entry (i +
+// o, i) of the diagonal -o, so a product reads 4 of 7 arrays.  Returns the
+// number of arrays.
+int dia_bases(int n, int nd, const int* off, bool symmetric, long long* base);
 // The distinct offsets col - row of the local block, ascending, at most
 // `most` (<= 32) of them: *nd = most + 1 when there are more.  *ascending:
 // every row's columns strictly ascend (known only when *nd <= most).
 int dia_offsets(const Mat& A, int most, int* nd, int* off, bool* ascending);
+// dia_offsets of several matrices, with one synchronisation
+struct DiagonalSet {
+    int nd;
+    int off[32];
+    bool ascending;
+};
+int dia_offsets_all(const std::vector<Mat*>& mats, int most, std::vector<DiagonalSet>& out);
 // Diagonal-major values (v64, or v32 rounded to FP32) and row masks on at
 // most 8 diagonals; slots without an entry hold 0.
 int dia_fill(const Mat& A, int nd, const int* off, double* v64, float* v32, uint8_t* mask8);

@@ -9,6 +9,7 @@
 // without column indices and with x read contiguously per diagonal.  The
 // mask is one byte per row when there are at most 8 diagonals.
 #include <algorithm>
+#include <vector>
 
 #include "cel_internal.hpp"
 #include "spmv_device.hpp"
@@ -60,8 +61,9 @@ __device__ __forceinline__ bool offset_put(int* slot, int o, bool& added)
     return false;
 }
 
-__global__ void __launch_bounds__(kBlock) k_offset_clear(OffsetSet* g)
+__global__ void __launch_bounds__(kBlock) k_offset_clear(OffsetSet* sets)
 {
+    OffsetSet* g = sets + blockIdx.x;
     if (threadIdx.x < 2 * kMaxDiag) g->slot[threadIdx.x] = kNoOffset;
     if (threadIdx.x == 0) g->count = g->over = g->bad = 0;
 }
@@ -294,25 +296,42 @@ int launch_dia_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const 
     return CEL_OK;
 }
 
-int dia_offsets(const Mat& A, int most, int* nd, int* off, bool* ascending)
+int dia_offsets_all(const std::vector<Mat*>& mats, int most, std::vector<DiagonalSet>& out)
 {
+    const size_t k = mats.size();
+    out.assign(k, DiagonalSet{});
+    if (k == 0) return CEL_OK;
     hipStream_t st = rt().stream;
     DevBuf<OffsetSet> g;
-    CEL_TRY(g.alloc(1));
-    hipLaunchKernelGGL(k_offset_clear, dim3(1), dim3(kBlock), 0, st, g.p);
-    hipLaunchKernelGGL(k_offset_scan, dim3(grid_of(A.n)), dim3(kBlock), 0, st, A.n, A.xadj.p, A.cols.p, most, g.p);
+    CEL_TRY(g.alloc(k));
+    hipLaunchKernelGGL(k_offset_clear, dim3((unsigned)k), dim3(kBlock), 0, st, g.p);
+    for (size_t q = 0; q < k; ++q)
+        hipLaunchKernelGGL(k_offset_scan, dim3(grid_of(mats[q]->n)), dim3(kBlock), 0, st, mats[q]->n, mats[q]->xadj.p,
+                           mats[q]->cols.p, most, g.p + q);
     CEL_HIP(hipGetLastError());
-    OffsetSet h;
-    CEL_HIP(hipMemcpyAsync(&h, g.p, sizeof(h), hipMemcpyDeviceToHost, st));
+    std::vector<OffsetSet> h(k);
+    CEL_HIP(hipMemcpyAsync(h.data(), g.p, sizeof(OffsetSet) * k, hipMemcpyDeviceToHost, st));
     CEL_HIP(hipStreamSynchronize(st));
-    *ascending = !h.bad;
-    *nd = most + 1;
-    if (h.over || h.count > most) return CEL_OK;
-    int k = 0;
-    for (int v : h.slot)
-        if (v != kNoOffset) off[k++] = v;
-    std::sort(off, off + k);
-    *nd = k;
+    for (size_t q = 0; q < k; ++q) {
+        DiagonalSet& d = out[q];
+        d.ascending = !h[q].bad;
+        d.nd = most + 1;
+        if (h[q].over || h[q].count > most) continue;
+        d.nd = 0;
+        for (int v : h[q].slot)
+            if (v != kNoOffset) d.off[d.nd++] = v;
+        std::sort(d.off, d.off + d.nd);
+    }
+    return CEL_OK;
+}
+
+int dia_offsets(const Mat& A, int most, int* nd, int* off, bool* ascending)
+{
+    std::vector<DiagonalSet> d;
+    CEL_TRY(dia_offsets_all({const_cast<Mat*>(&A)}, most, d));
+    *ascending = d[0].ascending;
+    *nd = d[0].nd;
+    if (d[0].nd <= most) std::copy(d[0].off, d[0].off + d[0].nd, off);
     return CEL_OK;
 }
 

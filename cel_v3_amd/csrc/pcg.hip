@@ -1731,27 +1731,6 @@ int pcg_noalloc_setup(int device)
     return CEL_OK;
 }
 
-// Where the wide walk of a symmetric block finds the diagonals' values (V.nd
-// and V.doff are set): those below the main diagonal in the arrays above it,
-// as entry (i, i + o), o < 0, is entry (i + o, i) of the diagonal -o, so an
-// iteration reads 4 of 7 arrays.  Returns the number of arrays.
-static int dia_bases(MatView& V)
-{
-    int arrays = V.nd;
-    V.dwide = 1;
-    for (int d = 0; d < V.nd; ++d) {
-        V.dbase[d] = (long long)d * V.n;
-        if (V.doff[d] >= 0) continue;
-        for (int u = d + 1; u < V.nd; ++u)
-            if (V.doff[u] == -V.doff[d]) {
-                V.dbase[d] = (long long)u * V.n + V.doff[d];
-                --arrays;
-                break;
-            }
-    }
-    return arrays;
-}
-
 // Device pointers of one solve's work vectors, partial sums and token.
 struct WorkPtrs {
     double *r = nullptr, *p = nullptr, *v = nullptr, *part1 = nullptr, *part2 = nullptr,
@@ -2140,7 +2119,8 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         if (doff[d] == 0) V.dzero = d;
     }
     const bool sym = kfmt == CEL_FMT_DIA && symmetric;
-    const int arrays = sym ? dia_bases(V) : V.nd;
+    V.dwide = sym;
+    const int arrays = sym ? dia_bases(n, V.nd, V.doff, true, V.dbase) : V.nd;
     // (a symmetric block's values are read again a row, a line and a plane
     // later: 256^3 FP64 427 us per iteration marked as read once, 425 kept)
     const bool keep = sym || keep_matrix(A, kfmt, arrays, mixed);
