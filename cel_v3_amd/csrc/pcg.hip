@@ -724,6 +724,28 @@ __device__ __forceinline__ double k1_wide(const MatView& A, const VT* __restrict
     return acc;
 }
 
+// The tile stream of a step's CSR walk.  In FP64 it is opened (a tile's entries
+// to LDS) before the step's scalars are there: per iteration, after / before
+// them, FP64 20^3 11.2 / 10.7 us, 32^3 11.35 / 10.9, 64^3 15.1 / 14.6; in the
+// mixed form, whose registers it takes, 32^3 12.7 / 13.0, 64^3 14.4 / 14.6.
+template <typename VT>
+constexpr bool kOpenAhead = sizeof(VT) == 8;
+template <typename VT, int FMT, bool LONG, bool KEEP>
+struct StepStream {
+    __device__ __forceinline__ void open(const MatView&, typename StageOf<VT, FMT, LONG>::T&) {}
+};
+template <typename VT, bool LONG, bool KEEP>
+struct StepStream<VT, CEL_FMT_CSR, LONG, KEEP> {
+    typename CsrStreamOf<VT, LONG, KEEP>::Stream cs;
+    __device__ __forceinline__ void open(const MatView& A, typename CsrStreamOf<VT, LONG>::Stage& sm)
+    {
+        const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
+        const int t = (int)group_tile(0, ntiles);
+        if (t >= 0)  // uniform across the block
+            cs.open(A.n, t, (int)group_tile(1, ntiles), A.xadj, A.cols, csr_vals<VT>(A), sm);
+    }
+};
+
 // v = A d over the block's tiles, d the vector of the accessor X; returns the
 // thread's part of v.d.  STEP: X is XDirection, and d and the updated x of
 // every row are stored as well.  (Taking a step's scalars behind the first
@@ -731,6 +753,7 @@ __device__ __forceinline__ double k1_wide(const MatView& A, const VT* __restrict
 // 12.3 us per iteration.)  KEEP: keep_matrix().
 template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, bool KEEP, typename X>
 __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __restrict__ v,
+                                           StepStream<VT, FMT, LONG, KEEP>& first,
                                            typename StageOf<VT, FMT, LONG>::T& sm,
                                            typename WideStageOf<wide_form<FMT, HALO, STEP>>::T& wide,
                                            const StepRows<VT>& st, int walk = 0)
@@ -762,7 +785,11 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
         // record and read count 0.  Each loaded value is used once in the
         // step after it, in place: a copy of a register still being loaded
         // would wait for every load issued before it.
-        typename CsrStreamOf<VT, LONG, KEEP>::Stream cs;
+        typename CsrStreamOf<VT, LONG, KEEP>::Stream own;
+        auto& cs = [&]() -> auto& {
+            if constexpr (STEP && kOpenAhead<VT>) return first.cs;
+            else return own;
+        }();
         const VT* vals = csr_vals<VT>(A);
         const long long tfirst = group_tile(0, ntiles);
         const auto rrec = tile_rsrc(HALO ? A.hrec : nullptr, HALO ? A.hnq * 16 : 0);
@@ -779,7 +806,7 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
                 hf = A.hflag[fidx(tfirst)];
                 hq = A.hwq[fidx(tfirst) >> 6];
             }
-            cs.open(A.n, (int)tfirst, (int)group_tile(1, ntiles), A.xadj, A.cols, vals, sm);
+            if constexpr (!(STEP && kOpenAhead<VT>)) cs.open(A.n, (int)tfirst, (int)group_tile(1, ntiles), A.xadj, A.cols, vals, sm);
         }
         long long k = 0;
         for (long long t = tfirst; t >= 0; t = group_tile(++k, ntiles)) {
@@ -997,7 +1024,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves
             slot = gridDim.x % kXcds ? walk : (walk % kXcds) * (gridDim.x / kXcds) + walk / kXcds;
         }
     }
-    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, sm.tile, sm.wide, StepRows<VT>{}, walk);
+    StepStream<VT, FMT, LONG, KEEP> none;
+    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, none, sm.tile, sm.wide, StepRows<VT>{}, walk);
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[slot] = bs;
     write_ctrl(cout, c);
@@ -1027,7 +1055,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     __shared__ double fred[2 * kWaves];
     Ctrl c = read_ctrl(cin);
     // the partials' loads do not wait for the token
-    const double sz = strided_sum(part2, G2), sr = strided_sum(part2 + G2, G2);
+    const Parts<MIXED ? false : FMT == CEL_FMT_CSR> sz(part2, G2), sr(part2 + G2, G2);
+    StepStream<VT, FMT, false, true> first;
+    if constexpr (kOpenAhead<VT>) first.open(A, sm.tile);
     if (!c.run) {
         write_ctrl(cout, c);
         return;
@@ -1048,7 +1078,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         fold_pending(c, R.part, R.G, P, fred);
     } else {
         double rz, rr;
-        all_sum2(sz, sr, fred, rz, rr);
+        all_sum2(sz.sum(), sr.sum(), fred, rz, rr);
         next_scalars<MIXED>(c, rz, rr, P);
     }
     const VT sigma = VT(c.sigma), beta = VT(c.beta);
@@ -1073,7 +1103,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         return;
     }
     const double acc = k1_tiles<VT, FMT, false, false, true, true>(
-        A, XDirection<VT>{p, z, beta, pending}, v, sm.tile, sm.wide, StepRows<VT>{pout, x, sigma, !pending});
+        A, XDirection<VT>{p, z, beta, pending}, v, first, sm.tile, sm.wide, StepRows<VT>{pout, x, sigma, !pending});
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[logical_block()] = bs;
     write_ctrl(cout, c);
@@ -1131,7 +1161,13 @@ template <typename VT>
 struct JacOf<VT, true> {
     using Raw = unsigned;  // W class bytes
     const uint8_t* cls;
-    const VT* tab;
+    VT* tab;  // LDS
+    // the table to LDS; every thread of the block; it synchronises
+    __device__ __forceinline__ void table(const VT* __restrict__ jac) const
+    {
+        tab[threadIdx.x] = jac[threadIdx.x];  // kMaxClass == kBlock
+        __syncthreads();
+    }
     __device__ __forceinline__ Raw load(long long i) const
     {
         if constexpr (Vec<VT>::W == 2) return *reinterpret_cast<const uint16_t*>(cls + i);
@@ -1141,18 +1177,12 @@ struct JacOf<VT, true> {
     __device__ __forceinline__ VT at(long long i) const { return tab[cls[i]]; }
 };
 
-// (CLS) the table to LDS; every thread of the block; it synchronises
 template <typename VT, bool CLS>
 __device__ __forceinline__ JacOf<VT, CLS> jac_of(const VT* __restrict__ jac, const uint8_t* __restrict__ cls,
                                                  VT* lds)
 {
-    if constexpr (CLS) {
-        lds[threadIdx.x] = jac[threadIdx.x];  // kMaxClass == kBlock
-        __syncthreads();
-        return JacOf<VT, true>{cls, lds};
-    } else {
-        return JacOf<VT, false>{jac};
-    }
+    if constexpr (CLS) return JacOf<VT, true>{cls, lds};
+    else return JacOf<VT, false>{jac};
 }
 static_assert(kMaxClass == kBlock, "one table entry per thread");
 
@@ -1207,15 +1237,17 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
         if constexpr (ZOUT) end_slot(cout, c, progress);
         else write_ctrl(cout, c);
     };
-    const double sv = strided_sum(vpart, G1);  // (its loads do not wait for the token)
-    // a slot without a product: a replacement was requested (ru) or its
-    // residual is pending (reduce)
-    if (!c.run || c.ru || c.reduce != kReduceNone) {
-        done();
-        return;
-    }
+    // AHEAD: the block's first elements are loaded with the partials, before
+    // the token is looked at, and a step's at the end of the one before.
+    // Per iteration without / with it, FP64 32^3 11.9 / 11.6 us, JAD 61x47x73
+    // 15.5 / 15.2, DIA 128^3 50.9 / 50.3, 200^3 186.7 / 184.7; by classes 100^3
+    // 26.7 / 27.1, mixed 100^3 22.0 / 23.1 (the registers of 4 units).
+    const Parts<sizeof(VT) == 8> sv(vpart, G1);
     using V = typename Vec<VT>::T;
     constexpr int W = Vec<VT>::W;
+    __shared__ VT jlds[CLS ? kMaxClass : 1];
+    const JacOf<VT, CLS> J = jac_of<VT, CLS>(jac, cls, jlds);
+    constexpr bool AHEAD = sizeof(VT) == 8 && !CLS;
     const int lb = logical_block();
     const int G = gridDim.x;
     const long long unit = (long long)kBlock * W;
@@ -1223,7 +1255,27 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
     unit_range((n + unit - 1) / unit, G, lb, u0, u1);
     const long long lo = u0 * unit, hi = min(u1 * unit, n);
     long long i = lo + (long long)threadIdx.x * W;
-    const double vp = block_sum_all(sv, fred);
+    constexpr int kVecUnroll = kVecUnrollOf<VT>;
+    V vv[kVecUnroll], rv[kVecUnroll];
+    typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
+    // units i, i + unit, ... of the block, as far as they are whole vectors
+    auto load = [&]() {
+#pragma unroll
+        for (int u = 0; u < kVecUnroll; ++u) {
+            const long long at = i + u * unit < hi && i + u * unit + W <= n ? i + u * unit : 0;
+            vv[u] = ld_vec<STREAM == kStreamAll, V>(v + at);
+            rv[u] = ld_vec<STREAM == kStreamAll, V>(r + at);
+            jv[u] = J.load(at);
+        }
+    };
+    if (AHEAD && n >= W) load();  // uniform
+    // a slot without a product: a replacement was requested (ru) or its
+    // residual is pending (reduce)
+    if (!c.run || c.ru || c.reduce != kReduceNone) {
+        done();
+        return;
+    }
+    const double vp = block_sum_all(sv.sum(), fred);
     const double sigma = c.alpha / vp;
     if (!(vp > 0.0) || !isfinite(sigma)) {
         c.status = CEL_ERR_BREAKDOWN;
@@ -1232,71 +1284,54 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_r(long long n, VT* __rest
         return;
     }
     c.sigma = sigma;
-    __shared__ VT jlds[CLS ? kMaxClass : 1];
-    const auto J = jac_of<VT, CLS>(jac, cls, jlds);
+    if constexpr (CLS) J.table(jac);
+    if (!AHEAD && n >= W) load();
     const VT ms = VT(-sigma);
     double arz = 0.0, arr = 0.0;
-    constexpr int kVecUnroll = kVecUnrollOf<VT>;
+    auto element = [&](VT vj, VT& rj, VT jj, VT& zj) {
+        const VT t = ms * vj;
+        const VT ri = rj + t;
+        rj = ri;
+        const VT zi = ri * jj;
+        zj = zi;
+        const double rz = double(ri) * double(zi);
+        arz = arz + rz;
+        const double rr = double(ri) * double(ri);
+        arr = arr + rr;
+    };
+    auto vec = [&](int u, long long at) {
+        V zv{};
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            VT ri = lane<VT>(rv[u], k), zi;
+            element(lane<VT>(vv[u], k), ri, J.value(jv[u], k), zi);
+            set_lane<VT>(rv[u], k, ri);
+            if constexpr (ZOUT) set_lane<VT>(zv, k, zi);
+        }
+        *reinterpret_cast<V*>(r + at) = rv[u];
+        if constexpr (ZOUT) *reinterpret_cast<V*>(z + at) = zv;
+    };
     // kVecUnroll units per step while they are whole vectors (all their
     // loads in flight together), added to the partials in unit order
-    for (; i + (kVecUnroll - 1) * unit + W <= hi; i += kVecUnroll * unit) {
-        V vv[kVecUnroll], rv[kVecUnroll], zv[kVecUnroll];
-        typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
+    while (i + (kVecUnroll - 1) * unit + W <= hi) {
 #pragma unroll
-        for (int u = 0; u < kVecUnroll; ++u) {
-            vv[u] = ld_vec<STREAM == kStreamAll, V>(v + i + u * unit);
-            rv[u] = ld_vec<STREAM == kStreamAll, V>(r + i + u * unit);
-            jv[u] = J.load(i + u * unit);
-        }
-#pragma unroll
-        for (int u = 0; u < kVecUnroll; ++u) {
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                VT t = ms * lane<VT>(vv[u], k);
-                VT ri = lane<VT>(rv[u], k) + t;
-                set_lane<VT>(rv[u], k, ri);
-                VT zi = ri * J.value(jv[u], k);
-                if constexpr (ZOUT) set_lane<VT>(zv[u], k, zi);
-                double rz = double(ri) * double(zi);
-                arz = arz + rz;
-                double rr = double(ri) * double(ri);
-                arr = arr + rr;
-            }
-            *reinterpret_cast<V*>(r + i + u * unit) = rv[u];
-            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i + u * unit) = zv[u];
-        }
+        for (int u = 0; u < kVecUnroll; ++u) vec(u, i + u * unit);
+        i += kVecUnroll * unit;
+        load();
     }
-    for (; i < hi; i += unit) {
-        if (i + W <= n) {
-            const V vv = *reinterpret_cast<const V*>(v + i);
-            V rv = *reinterpret_cast<const V*>(r + i);
-            const auto jv = J.load(i);
-            V zv{};
 #pragma unroll
-            for (int k = 0; k < W; ++k) {
-                VT t = ms * lane<VT>(vv, k);
-                VT ri = lane<VT>(rv, k) + t;
-                set_lane<VT>(rv, k, ri);
-                VT zi = ri * J.value(jv, k);
-                if constexpr (ZOUT) set_lane<VT>(zv, k, zi);
-                double rz = double(ri) * double(zi);
-                arz = arz + rz;
-                double rr = double(ri) * double(ri);
-                arr = arr + rr;
-            }
-            *reinterpret_cast<V*>(r + i) = rv;
-            if constexpr (ZOUT) *reinterpret_cast<V*>(z + i) = zv;
-        } else {
-            for (long long j = i; j < hi; ++j) {
-                VT t = ms * v[j];
-                VT ri = r[j] + t;
-                r[j] = ri;
-                VT zi = ri * J.at(j);
-                if constexpr (ZOUT) z[j] = zi;
-                double rz = double(ri) * double(zi);
-                arz = arz + rz;
-                double rr = double(ri) * double(ri);
-                arr = arr + rr;
+    for (int u = 0; u < kVecUnroll; ++u) {
+        const long long at = i + u * unit;
+        if (at < hi) {
+            if (at + W <= n) {
+                vec(u, at);
+            } else {
+                for (long long j = at; j < hi; ++j) {
+                    VT rj = r[j], zj;
+                    element(v[j], rj, J.at(j), zj);
+                    r[j] = rj;
+                    if constexpr (ZOUT) z[j] = zj;
+                }
             }
         }
     }
@@ -1324,116 +1359,106 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_xp(long long n, VT* __res
 {
     __shared__ double red[2 * kWaves];
     Ctrl c = read_ctrl(cin);
-    const double sz = strided_sum(rpart, G2), sr = strided_sum(rpart + G2, G2);
-    if (!c.run || c.reduce != kReduceNone) {
-        end_slot(cout, c, progress);
-        return;
-    }
-    double rz, rr;
-    all_sum2(sz, sr, red, rz, rr);
-    const VT sigma = VT(c.sigma);
-    // scalars of the next iteration (they do not depend on the vectors)
-    next_scalars<MIXED>(c, rz, rr, P);
-    const VT beta = VT(c.beta);
-    // mixed, replacement iteration: the FP32 correction is folded into the
-    // FP64 solution here (x64 = x64 + e, e = 0) instead of in a kernel of
-    // its own; same arithmetic
-    const bool flush = MIXED && c.ru;
-    __shared__ VT jlds[CLS ? kMaxClass : 1];
-    const auto J = jac_of<VT, CLS>(jac, cls, jlds);
+    const Parts<!MIXED> sz(rpart, G2), sr(rpart + G2, G2);
     using V = typename Vec<VT>::T;
     constexpr int W = Vec<VT>::W;
+    __shared__ VT jlds[CLS ? kMaxClass : 1];
+    const JacOf<VT, CLS> J = jac_of<VT, CLS>(jac, cls, jlds);
+    constexpr bool AHEAD = sizeof(VT) == 8 && !CLS;
     const int lb = logical_block();
     const long long unit = (long long)kBlock * W;
     long long u0, u1;
     unit_range((n + unit - 1) / unit, gridDim.x, lb, u0, u1);
     const long long lo = u0 * unit, hi = min(u1 * unit, n);
-    constexpr int kVecUnroll = kVecUnrollOf<VT>;
     long long i = lo + (long long)threadIdx.x * W;
-    // kVecUnroll units per step while they are whole vectors
-    for (; i + (kVecUnroll - 1) * unit + W <= hi; i += kVecUnroll * unit) {
-        V pv[kVecUnroll], rv[kVecUnroll];
-        typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
-        VT xs[kVecUnroll][W];
+    constexpr int kVecUnroll = kVecUnrollOf<VT>;
+    V pv[kVecUnroll], rv[kVecUnroll];
+    typename JacOf<VT, CLS>::Raw jv[kVecUnroll];
+    VT xs[kVecUnroll][W];
+    // units i, i + unit, ... of the block, as far as they are whole vectors;
+    // the first ones before the token is looked at (as in K2)
+    auto load = [&]() {
 #pragma unroll
         for (int u = 0; u < kVecUnroll; ++u) {
-            pv[u] = *reinterpret_cast<const V*>(p + i + u * unit);
-            rv[u] = ld_vec<STREAM == kStreamAll, V>(r + i + u * unit);
-            jv[u] = J.load(i + u * unit);
+            const long long at = i + u * unit < hi && i + u * unit + W <= n ? i + u * unit : 0;
+            pv[u] = *reinterpret_cast<const V*>(p + at);
+            rv[u] = ld_vec<STREAM == kStreamAll, V>(r + at);
+            jv[u] = J.load(at);
 #pragma unroll
             for (int k = 0; k < W; ++k)
-                xs[u][k] = STREAM != kStreamNone ? __builtin_nontemporal_load(x + i + u * unit + k)
-                                                 : x[i + u * unit + k];
+                xs[u][k] = STREAM != kStreamNone ? __builtin_nontemporal_load(x + at + k) : x[at + k];
         }
-#pragma unroll
-        for (int u = 0; u < kVecUnroll; ++u) {
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                const VT pi = lane<VT>(pv[u], k);
-                VT t = VT(sigma * pi);
-                xs[u][k] = xs[u][k] + t;
-                VT zi = lane<VT>(rv[u], k) * J.value(jv[u], k);
-                VT bp = beta * pi;
-                set_lane<VT>(pv[u], k, bp + zi);
-            }
-            if (flush) {
-#pragma unroll
-                for (int k = 0; k < W; ++k) {
-                    double t = (double)xs[u][k];
-                    x64[i + u * unit + k] = x64[i + u * unit + k] + t;
-                    xs[u][k] = VT(0);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                if constexpr (STREAM != kStreamNone) __builtin_nontemporal_store(xs[u][k], x + i + u * unit + k);
-                else x[i + u * unit + k] = xs[u][k];
-            }
-            *reinterpret_cast<V*>(p + i + u * unit) = pv[u];
-        }
+    };
+    if (AHEAD && n >= W) load();  // uniform
+    if (!c.run || c.reduce != kReduceNone) {
+        end_slot(cout, c, progress);
+        return;
     }
-    for (; i < hi; i += unit) {
-        if (i + W <= n) {
-            V pv = *reinterpret_cast<const V*>(p + i);
-            const V rv = *reinterpret_cast<const V*>(r + i);
-            const auto jv = J.load(i);
-            VT xs[W];
+    double rz, rr;
+    all_sum2(sz.sum(), sr.sum(), red, rz, rr);
+    const VT sigma = VT(c.sigma);
+    // scalars of the next iteration (they do not depend on the vectors)
+    next_scalars<MIXED>(c, rz, rr, P);
+    const VT beta = VT(c.beta);
+    if constexpr (CLS) J.table(jac);
+    if (!AHEAD && n >= W) load();
+    // mixed, replacement iteration: the FP32 correction is folded into the
+    // FP64 solution here (x64 = x64 + e, e = 0) instead of in a kernel of
+    // its own; same arithmetic
+    const bool flush = MIXED && c.ru;
+    auto vec = [&](int u, long long at) {
 #pragma unroll
-            for (int k = 0; k < W; ++k) xs[k] = x[i + k];
+        for (int k = 0; k < W; ++k) {
+            const VT pi = lane<VT>(pv[u], k);
+            VT t = VT(sigma * pi);
+            xs[u][k] = xs[u][k] + t;
+            VT zi = lane<VT>(rv[u], k) * J.value(jv[u], k);
+            VT bp = beta * pi;
+            set_lane<VT>(pv[u], k, bp + zi);
+        }
+        if (flush) {
 #pragma unroll
             for (int k = 0; k < W; ++k) {
-                const VT pi = lane<VT>(pv, k);
-                VT t = VT(sigma * pi);
-                xs[k] = xs[k] + t;
-                VT zi = lane<VT>(rv, k) * J.value(jv, k);
-                VT bp = beta * pi;
-                set_lane<VT>(pv, k, bp + zi);
+                double t = (double)xs[u][k];
+                x64[at + k] = x64[at + k] + t;
+                xs[u][k] = VT(0);
             }
-            if (flush) {
+        }
 #pragma unroll
-                for (int k = 0; k < W; ++k) {
-                    double t = (double)xs[k];
-                    x64[i + k] = x64[i + k] + t;
-                    xs[k] = VT(0);
-                }
-            }
+        for (int k = 0; k < W; ++k) {
+            if constexpr (STREAM != kStreamNone) __builtin_nontemporal_store(xs[u][k], x + at + k);
+            else x[at + k] = xs[u][k];
+        }
+        *reinterpret_cast<V*>(p + at) = pv[u];
+    };
+    // kVecUnroll units per step while they are whole vectors
+    while (i + (kVecUnroll - 1) * unit + W <= hi) {
 #pragma unroll
-            for (int k = 0; k < W; ++k) x[i + k] = xs[k];
-            *reinterpret_cast<V*>(p + i) = pv;
-        } else {
-            for (long long j = i; j < hi; ++j) {
-                const VT pi = p[j];
-                VT t = VT(sigma * pi);
-                VT xj = x[j] + t;
-                if (flush) {
-                    double tt = (double)xj;
-                    x64[j] = x64[j] + tt;
-                    xj = VT(0);
+        for (int u = 0; u < kVecUnroll; ++u) vec(u, i + u * unit);
+        i += kVecUnroll * unit;
+        load();
+    }
+#pragma unroll
+    for (int u = 0; u < kVecUnroll; ++u) {
+        const long long at = i + u * unit;
+        if (at < hi) {
+            if (at + W <= n) {
+                vec(u, at);
+            } else {
+                for (long long j = at; j < hi; ++j) {
+                    const VT pi = p[j];
+                    VT t = VT(sigma * pi);
+                    VT xj = x[j] + t;
+                    if (flush) {
+                        double tt = (double)xj;
+                        x64[j] = x64[j] + tt;
+                        xj = VT(0);
+                    }
+                    x[j] = xj;
+                    VT zi = r[j] * J.at(j);
+                    VT bp = beta * pi;
+                    p[j] = bp + zi;
                 }
-                x[j] = xj;
-                VT zi = r[j] * J.at(j);
-                VT bp = beta * pi;
-                p[j] = bp + zi;
             }
         }
     }
