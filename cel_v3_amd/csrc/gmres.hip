@@ -324,6 +324,96 @@ __device__ __forceinline__ void column_done(int jj, int m, double folded, GmStat
     __syncthreads();
 }
 
+// column_done for the first columns (JJ <= kShort): the algebra in registers,
+// in every thread, its operands loaded side by side with the partials.  In
+// one thread over LDS each operand waited for the one before it, about 6 us
+// of a launch (GMRES(3), 48^3: the last column's kernel 10.1 -> 5.5 us, with
+// the loads ahead of it in k_last_small).
+constexpr int kShort = 4;
+template <int JJ>
+__device__ __forceinline__ void column_short(int m, double folded, GmState* st, Column& c, double* red)
+{
+    double h[JJ + 2], cs[JJ + 1], sn[JJ + 1], gam[JJ + 1], alp[JJ + 1], R[JJ + 1][JJ + 1];
+#pragma unroll
+    for (int i = 1; i <= JJ; ++i) h[i] = st->H[i * kM1 + JJ];
+#pragma unroll
+    for (int i = 1; i < JJ; ++i) {
+        cs[i] = st->cs[i];
+        sn[i] = st->sn[i];
+        gam[i] = st->gam[i];
+#pragma unroll
+        for (int k = i; k < JJ; ++k) R[i][k] = st->R[i * kM1 + k];
+    }
+    gam[JJ] = st->gin[JJ];
+    const double eps = st->eps;
+    const double s = sum256(folded, red);
+    h[JJ + 1] = sqrt(s);
+#pragma unroll
+    for (int i = 1; i < JJ; ++i) {  // both statements assign h(ii,jj) (:722-727)
+        double a = h[i] * cs[i];
+        double d = h[i + 1] * sn[i];
+        h[i] = a + d;
+        a = -h[i] * sn[i];
+        d = h[i + 1] * cs[i];
+        h[i] = a + d;
+    }
+    const double a = h[JJ] * h[JJ];
+    const double d = h[JJ + 1] * h[JJ + 1];
+    const double betta = sqrt(a + d);
+    const double sj = h[JJ + 1] / betta, cj = h[JJ] / betta;
+    const double gnext = -sj * gam[JJ];
+    gam[JJ] = cj * gam[JJ];
+    const bool conv = fabs(gnext) <= eps;
+    const int k = conv || JJ == m ? JJ : 0;
+    h[JJ] = betta;
+#pragma unroll
+    for (int i = 1; i <= JJ; ++i) R[i][JJ] = h[i];
+    if (k) {  // uniform
+#pragma unroll
+        for (int i = JJ; i >= 1; --i) {
+            double sum = 0.0;
+#pragma unroll
+            for (int kk = i + 1; kk <= JJ; ++kk) {
+                const double t = R[i][kk] * alp[kk];
+                sum = sum + t;
+            }
+            const double inv = 1.0 / R[i][i];
+            alp[i] = inv * (gam[i] - sum);
+        }
+    }
+    if (threadIdx.x == 0) {
+        c.k = k;
+        c.h[JJ + 1] = h[JJ + 1];
+        if (k) {
+#pragma unroll
+            for (int i = 1; i <= JJ; ++i) c.alp[i] = alp[i];
+        }
+        if (blockIdx.x == 0) {
+#pragma unroll
+            for (int i = 1; i <= JJ; ++i) st->R[i * kM1 + JJ] = h[i];
+            st->cs[JJ] = cj;
+            st->sn[JJ] = sj;
+            st->gin[JJ + 1] = gnext;
+            st->gam[JJ] = gam[JJ];
+            st->ncols = st->ncols + 1;
+            if (conv) st->halt = JJ;
+        }
+    }
+    __syncthreads();
+}
+
+// MOST: the last column that runs in registers (those of k_col hold its loads).
+template <int MOST>
+__device__ __forceinline__ void column_end(int jj, int m, double folded, GmState* st, Column& c, double* red)
+{
+    static_assert(MOST <= kShort, "a case each");
+    if (jj == 1) column_short<1>(m, folded, st, c, red);  // (jj is uniform)
+    else if (MOST >= 2 && jj == 2) column_short<2>(m, folded, st, c, red);
+    else if (MOST >= 3 && jj == 3) column_short<3>(m, folded, st, c, red);
+    else if (MOST >= 4 && jj == 4) column_short<4>(m, folded, st, c, red);
+    else column_done(jj, m, folded, st, c, red);
+}
+
 // x = x + a_1 z_1 + ... + a_k z_k, added in that order
 __device__ __forceinline__ double x_updated(double xi, const Column& c, const double* __restrict__ Z,
                                             long long n, long long i)
@@ -348,7 +438,7 @@ k_next(long long n, long long chunk, int jj, int m, const double* __restrict__ p
     const double f = fold_part(part, G);
     // (a flag of this column is this launch's own)
     if (st->stop || (st->halt && st->halt != jj)) return;
-    column_done(jj, m, f, st, c, red);
+    column_end<kShort>(jj, m, f, st, c, red);
     if (c.k > 0) {
         CHUNK_LOOP(i) x[i] = x_updated(x[i], c, Z, n, i);
         return;
@@ -480,7 +570,7 @@ k_col(GmMat A, long long chunk, int j, int m, int cycle, const double* __restric
         if (blockIdx.x == 0 && threadIdx.x == 0) st->gin[1] = beta;
     } else {
         if (st->halt && st->halt != j - 1) return;
-        column_done(j - 1, m, f, st, c, red + kWaves);
+        column_end<2>(j - 1, m, f, st, c, red + kWaves);
         if (c.k > 0) {
             CHUNK_LOOP(i) x[i] = x_updated(x[i], c, Z, n, i);
             return;
@@ -552,6 +642,218 @@ k_resid_small(GmMat A, long long chunk, const double* __restrict__ x, const doub
     if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
+// k_next of a small system's last column: the x update, on the blocks of its
+// other kernels, two rows per thread.
+__global__ void __launch_bounds__(kWide)
+k_last_small(long long n, long long chunk, int m, const double* __restrict__ part, int G,
+             const double* __restrict__ Z, double* __restrict__ x, GmState* st)
+{
+    __shared__ double red[kWaves];
+    __shared__ Column c;
+    const double f = fold_part(part, G);
+    CHUNK_BOUNDS
+    int r[2];
+    double xi[2], z[2][kShort];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const long long i = c0 + threadIdx.x + (long long)k * kWide;
+        r[k] = i < c1 ? (int)i : (int)n;
+        const int rc = r[k] < n ? r[k] : 0;
+        xi[k] = x[rc];
+#pragma unroll
+        for (int j = 0; j < kShort; ++j) z[k][j] = Z[(long long)(j < m ? j : 0) * n + rc];
+    }
+    if (st->stop || (st->halt && st->halt != m)) return;
+    column_end<kShort>(m, m, f, st, c, red);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        if (r[k] < n) {
+            double s = xi[k];
+#pragma unroll
+            for (int j = 0; j < kShort; ++j) {
+                if (j < c.k) {
+                    const double t = c.alp[j + 1] * z[k][j];
+                    s = s + t;
+                }
+            }
+            for (int j = kShort; j < c.k; ++j) {
+                const double t = c.alp[j + 1] * Z[(long long)j * n + r[k]];
+                s = s + t;
+            }
+            x[r[k]] = s;
+        }
+}
+
+// DIA rows of a small system's chunk with the vector's values in LDS.  The
+// gathers of 2,048 rows on one CU, and a quotient for each of them, are what
+// a column's launch consists of (54 blocks at 48^3); so a block forms each
+// value of its chunk once, kNear rows on either side with it, and a row
+// takes the inner diagonals from there and forms the two outer ones itself:
+// 3.1 values per row instead of 7.  All loads are issued before the scalars
+// are there.  k_col 12.1 -> 10.7 us, the first column's 10.1 -> 8.5; a cycle
+// of GMRES(3) with column_short and k_last_small 77.3 -> 67.4 us (CSR, without
+// the window, 93.6 -> 87.8), 16^3 69.8 -> 62.3, 80^3 97.6 -> 96.3.  The
+// Gram-Schmidt launches, 4.1 us each, are near an empty one's 3.  (512-row
+// chunks would fill the chip but group the sums anew, and the reference's
+// rotation answers rounding with other iteration counts.)  A rule on the
+// offsets (window()): all diagonals but the first and the last within kNear
+// of the main one.
+constexpr int kNear = 1024;
+struct Window {
+    double val[kWideRows + 2 * kNear];  // [kNear + i - c0]
+};
+template <typename X>
+struct WindowRows {
+    typename X::Raw own[2], first[2], last[2], side[2];
+    double a[2][kGather];
+    unsigned m[2];
+    int r[2], at[2];  // rows (n: none) and the rows beside the chunk
+
+    __device__ __forceinline__ void load(const GmMat& A, long long c0, long long c1, const X& x)
+    {
+        const auto rx = x.buf((unsigned)A.n * 8u);
+        const int far0 = A.off[0], far1 = A.off[A.nd - 1];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const long long i = c0 + threadIdx.x + (long long)k * kWide;
+            r[k] = i < c1 ? (int)i : A.n;
+            const int rc = r[k] < A.n ? r[k] : 0;
+            own[k] = x.load(rc);
+            // (an absent entry's column may lie outside [0, n): as dia_rows)
+            first[k] = x.load(rx, (int)((unsigned)(rc + far0) * 8u));
+            last[k] = x.load(rx, (int)((unsigned)(rc + far1) * 8u));
+            m[k] = A.mask8[rc];
+#pragma unroll
+            for (int d = 0; d < kGather; ++d) a[k][d] = d < A.nd ? A.dvals[(long long)d * A.n + rc] : 0.0;
+        }
+        // kNear = kWide rows before the chunk and after it
+        at[0] = (int)(c0 - kNear + threadIdx.x);
+        at[1] = (int)(c1 + threadIdx.x);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) side[k] = x.load(rx, (int)((unsigned)at[k] * 8u));
+    }
+    // every thread of the block; it synchronises
+    __device__ __forceinline__ void stage(const GmMat& A, long long c0, const X& x, Window& w) const
+    {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (r[k] < A.n) w.val[kNear + r[k] - c0] = x.value(own[k]);
+            w.val[kNear + at[k] - c0] = x.value(side[k]);
+        }
+        __syncthreads();
+    }
+    __device__ __forceinline__ double sum(int k, const GmMat& A, long long c0, const X& x, const Window& w) const
+    {
+        double s = 0.0;
+        const double* near = w.val + (kNear + r[k] - c0);
+#pragma unroll
+        for (int d = 0; d < kGather; ++d)
+            if (d < A.nd) {
+                const double z = d == 0 ? x.value(first[k]) : d == A.nd - 1 ? x.value(last[k]) : near[A.off[d]];
+                const double t = a[k][d] * z;
+                const double u = s + t;
+                s = (m[k] >> d) & 1u ? u : s;
+            }
+        return s;
+    }
+};
+static_assert(kNear == kWide, "one row beside the chunk per thread and side");
+
+// k_col and k_resid_small by the window
+template <bool FIRST>
+__global__ void __launch_bounds__(kWide)
+k_col_window(GmMat A, long long chunk, int j, int m, int cycle, const double* __restrict__ prev, int G,
+             const double* __restrict__ src, const double* __restrict__ jac, double* __restrict__ V,
+             double* __restrict__ Z, double* __restrict__ w, double* __restrict__ x,
+             double* __restrict__ part, GmState* st)
+{
+    __shared__ double red[2 * kWaves];
+    __shared__ double terms[kWideRows];
+    __shared__ Window win;
+    __shared__ Column c;
+    const long long n = A.n;
+    const double f = fold_part(prev, G);
+    using X = XKrylov<FIRST>;
+    CHUNK_BOUNDS
+    WindowRows<X> rows;
+    rows.load(A, c0, c1, X{src, jac, 1.0, Quotient(1.0)});
+    double v1[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        if constexpr (!FIRST) v1[k] = V[rows.r[k] < A.n ? rows.r[k] : 0];
+    double beta = 1.0;
+    if (st->stop) return;
+    if constexpr (FIRST) {
+        beta = residual_done(cycle, f, st, red + kWaves);
+        if (beta < 0.0) return;  // uniform
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->gin[1] = beta;
+    } else {
+        if (st->halt && st->halt != j - 1) return;
+        column_end<2>(j - 1, m, f, st, c, red + kWaves);
+        if (c.k > 0) {
+            for (long long i = c0 + threadIdx.x; i < c1; i += kWide) x[i] = x_updated(x[i], c, Z, n, i);
+            return;
+        }
+    }
+    const X kx{src, jac, 1.0 / beta, Quotient(FIRST ? 1.0 : c.h[j])};
+    double* v = V + (long long)(j - 1) * n;
+    double* z = Z + (long long)(j - 1) * n;
+    rows.stage(A, c0, kx, win);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int r = rows.r[k];
+        if (r < A.n) {
+            const double vi = kx.v(rows.own[k]), wi = 0.0 + rows.sum(k, A, c0, kx, win);
+            v[r] = vi;
+            z[r] = vi * rows.own[k].j;
+            w[r] = wi;
+            const double p = (FIRST ? vi : v1[k]) * wi;
+            terms[r - c0] = p;
+        }
+    }
+    __syncthreads();
+    double acc = 0.0;
+    if (threadIdx.x < kBlock)
+        for (int i = threadIdx.x; i < (int)(c1 - c0); i += kBlock) acc = acc + terms[i];
+    const double t = sum256(acc, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = t;
+}
+
+__global__ void __launch_bounds__(kWide)
+k_resid_window(GmMat A, long long chunk, const double* __restrict__ x, const double* __restrict__ b,
+               double* __restrict__ rr, double* __restrict__ part, const GmState* __restrict__ st)
+{
+    __shared__ double red[kWaves];
+    __shared__ double terms[kWideRows];
+    __shared__ Window win;
+    const long long n = A.n;
+    CHUNK_BOUNDS
+    const XPlain<double> X{x};
+    WindowRows<XPlain<double>> rows;
+    rows.load(A, c0, c1, X);
+    double bi[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) bi[k] = b[rows.r[k] < A.n ? rows.r[k] : 0];
+    if (st->stop) return;
+    rows.stage(A, c0, X, win);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int r = rows.r[k];
+        if (r < A.n) {
+            const double ri = bi[k] - (0.0 + rows.sum(k, A, c0, X, win));
+            rr[r] = ri;
+            const double p = ri * ri;
+            terms[r - c0] = p;
+        }
+    }
+    __syncthreads();
+    double acc = 0.0;
+    if (threadIdx.x < kBlock)
+        for (int i = threadIdx.x; i < (int)(c1 - c0); i += kBlock) acc = acc + terms[i];
+    const double t = sum256(acc, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = t;
+}
+
 struct Gmres {
     const Mat& A;
     int format;
@@ -577,6 +879,13 @@ struct Gmres {
     // than the launches).  Long rows gather too much at any size (30,011 mesh
     // rows of 11 entries 185 / 169).
     bool small() const { return format != CEL_FMT_JAD && n <= 600000 && !csr_long_rows(A); }
+    bool window() const
+    {
+        if (format != CEL_FMT_DIA || A.dia_nd > kGather) return false;
+        for (int d = 1; d + 1 < A.dia_nd; ++d)
+            if (A.dia_off[d] < -kNear || A.dia_off[d] > kNear) return false;
+        return true;
+    }
     GmMat mat() const
     {
         GmMat M{};
@@ -669,12 +978,13 @@ int gmres_solve(Mat& A, const double* b_in, double* x_out, const cel_gmres_param
     DevBuf<double> w2;
     if (small) CEL_TRY(w2.alloc(n));
     const GmMat GM = S.mat();
-    const bool dia = prm.format == CEL_FMT_DIA;
+    const bool dia = prm.format == CEL_FMT_DIA, win = S.window();
     // the same on a small system: k_col in place of k_scale_jac / k_next and
     // the product
     auto enqueue_small = [&]() -> int {
         auto resid = [&]() {
-            if (dia) k_resid_small<CEL_FMT_DIA><<<G, kWide, 0, st>>>(GM, ck, x, b, r.p, partA.p, gs);
+            if (win) k_resid_window<<<G, kWide, 0, st>>>(GM, ck, x, b, r.p, partA.p, gs);
+            else if (dia) k_resid_small<CEL_FMT_DIA><<<G, kWide, 0, st>>>(GM, ck, x, b, r.p, partA.p, gs);
             else k_resid_small<CEL_FMT_CSR><<<G, kWide, 0, st>>>(GM, ck, x, b, r.p, partA.p, gs);
         };
         auto col = [&](auto kernel, int j, int cycle, const double* prev, const double* src, double* out, double* part) {
@@ -684,8 +994,8 @@ int gmres_solve(Mat& A, const double* b_in, double* x_out, const cel_gmres_param
         for (int c = 0; c <= m; ++c) {
             double *cur = partA.p, *nxt = partB.p, *wi = w.p, *wo = w2.p;
             for (int jj = 1; jj <= m; ++jj) {
-                if (jj == 1) col(dia ? k_col<CEL_FMT_DIA, true> : k_col<CEL_FMT_CSR, true>, jj, c > 0, cur, r.p, wo, nxt);
-                else col(dia ? k_col<CEL_FMT_DIA, false> : k_col<CEL_FMT_CSR, false>, jj, 0, cur, wi, wo, nxt);
+                if (jj == 1) col(win ? k_col_window<true> : dia ? k_col<CEL_FMT_DIA, true> : k_col<CEL_FMT_CSR, true>, jj, c > 0, cur, r.p, wo, nxt);
+                else col(win ? k_col_window<false> : dia ? k_col<CEL_FMT_DIA, false> : k_col<CEL_FMT_CSR, false>, jj, 0, cur, wi, wo, nxt);
                 std::swap(cur, nxt);
                 std::swap(wi, wo);
                 for (int ii = 1; ii <= jj; ++ii) {
@@ -694,7 +1004,7 @@ int gmres_solve(Mat& A, const double* b_in, double* x_out, const cel_gmres_param
                     std::swap(cur, nxt);
                 }
             }
-            k_next<<<G, kThreads, 0, st>>>(n, ck, m, m, cur, G, wi, A.jac.p, V.p, Z.p, x, gs);
+            k_last_small<<<G, kWide, 0, st>>>(n, ck, m, cur, G, Z.p, x, gs);
             resid();
         }
         k_cycle_end<<<1, kThreads, 0, st>>>(partA.p, G, gs);
