@@ -1031,6 +1031,74 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves
     write_ctrl(cout, c);
 }
 
+// A group of CSR tiles of the step kernel, one row of each tile per thread,
+// every row read by its own thread: a block's chain is three round trips
+// (row bounds, entries, gathers) for all of its rows, without LDS and
+// barriers, and none of them waits for the step's scalars.  A lane's entries
+// lie 28 to 84 bytes from the next one's, so every load touches the lines of
+// all of a wave's rows, which pays as long as few blocks share the caches.
+// Per iteration, tiles in LDS / so: FP64 20^3 10.4 / 9.8 us, 32^3 10.5 / 9.95,
+// 40^3 11.8 / 11.2, 44^3 12.2 / 12.8, 64^3 14.4 / 15.0; mixed 20^3 12.1 / 11.3,
+// 32^3 11.8 / 10.9, 48^3 12.5 / 12.2, 52^3 13.6 / 14.1, 64^3 13.7 / 15.0; hence
+// the lines in step_kernel, 70,000 and 120,000 rows.
+template <typename VT>
+struct DirectGroup {
+    static constexpr int R = kTileGroup;
+    int r[R], lo[R], hi[R];
+    VT a[R][kGather], xo[R];
+    typename XDirection<VT>::Raw xv[R][kGather], own[R];
+
+    __device__ __forceinline__ void load(const MatView& A, long long q, const XDirection<VT>& d, const VT* x)
+    {
+        const VT* vals = csr_vals<VT>(A);
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const long long i = (R * q + k) * kTileRows + threadIdx.x;
+            r[k] = i < A.n ? (int)i : A.n;
+            const int rc = r[k] < A.n ? r[k] : 0;
+            lo[k] = A.xadj[rc];
+            hi[k] = A.xadj[rc + 1];
+        }
+        int c[R][kGather];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int i = 0; i < kGather; ++i) {
+                const int at = lo[k] + i < hi[k] ? lo[k] + i : 0;
+                c[k][i] = A.cols[at];
+                a[k][i] = vals[at];
+            }
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int rc = r[k] < A.n ? r[k] : 0;
+            own[k] = d.load(rc);
+            xo[k] = x[rc];
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int i = 0; i < kGather; ++i) xv[k][i] = d.load(c[k][i]);
+    }
+    // the row's sum in column order (rows of more than kGather entries read
+    // the others here)
+    __device__ __forceinline__ VT sum(int k, const MatView& A, const XDirection<VT>& d) const
+    {
+        VT s = VT(0);
+#pragma unroll
+        for (int i = 0; i < kGather; ++i) {
+            const VT prod = a[k][i] * d.value(xv[k][i]);
+            const VT t = s + prod;
+            s = lo[k] + i < hi[k] ? t : s;
+        }
+        const VT* vals = csr_vals<VT>(A);
+        for (int j = lo[k] + kGather; j < hi[k]; ++j) {
+            const VT prod = vals[j] * d.value(d.load(A.cols[j]));
+            s = s + prod;
+        }
+        return s;
+    }
+};
+
 // K3 and the next iteration's K1 in one launch, for small systems (rule at
 // step_form): beta and the loop decision from K2's partials, x += sigma p,
 // p_new = beta p + z, v = A p_new and the partials of v.p_new.  A block
@@ -1042,7 +1110,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves
 // (x64 += e, e = 0) is K3's, and the next launch forms the residual.  What
 // it saves is a launch and K3's second look at p; what it costs is a second
 // gather per entry.
-template <typename VT, int FMT>
+template <typename VT, int FMT, bool DIRECT = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(VT) == 4 ? 4 : 2, 8))) void k_pcg_step(
     MatView A, const VT* __restrict__ p, const VT* __restrict__ z, VT* __restrict__ pout,
     VT* __restrict__ x, double* __restrict__ x64, VT* __restrict__ v, double* __restrict__ part,
@@ -1057,7 +1125,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
     // the partials' loads do not wait for the token
     const Parts<MIXED ? false : FMT == CEL_FMT_CSR> sz(part2, G2), sr(part2 + G2, G2);
     StepStream<VT, FMT, false, true> first;
-    if constexpr (kOpenAhead<VT>) first.open(A, sm.tile);
+    if constexpr (!DIRECT && kOpenAhead<VT>) first.open(A, sm.tile);
+    DirectGroup<VT> grp;
+    const long long ngroups = ((long long)A.n + kTileGroup * kTileRows - 1) / (kTileGroup * kTileRows);
+    if constexpr (DIRECT) grp.load(A, blockIdx.x, XDirection<VT>{p, z, VT(0), false}, x);
     if (!c.run) {
         write_ctrl(cout, c);
         return;
@@ -1102,8 +1173,32 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
         write_ctrl(cout, c);
         return;
     }
-    const double acc = k1_tiles<VT, FMT, false, false, true, true>(
-        A, XDirection<VT>{p, z, beta, pending}, v, first, sm.tile, sm.wide, StepRows<VT>{pout, x, sigma, !pending});
+    double acc = 0.0;
+    const XDirection<VT> d{p, z, beta, pending};
+    if constexpr (DIRECT) {
+        for (long long q = blockIdx.x; q < ngroups; q += gridDim.x) {
+            if (q != blockIdx.x) grp.load(A, q, d, x);
+#pragma unroll
+            for (int k = 0; k < kTileGroup; ++k) {
+                const int row = grp.r[k];
+                if (row >= A.n) continue;
+                VT s = grp.sum(k, A, d);
+                s = A.coo ? s : VT(0) + s;
+                const VT dk = d.value(grp.own[k]);
+                v[row] = s;
+                pout[row] = dk;
+                if (!pending) {
+                    const VT t = sigma * grp.own[k].p;
+                    x[row] = grp.xo[k] + t;
+                }
+                const double prod = double(s) * double(dk);
+                acc = acc + prod;
+            }
+        }
+    } else {
+        acc = k1_tiles<VT, FMT, false, false, true, true>(A, d, v, first, sm.tile, sm.wide,
+                                                          StepRows<VT>{pout, x, sigma, !pending});
+    }
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[logical_block()] = bs;
     write_ctrl(cout, c);
@@ -1698,9 +1793,10 @@ using StepFn = void (*)(MatView, const VT*, const VT*, VT*, VT*, double*, VT*, d
                         const double*, int, const Ctrl*, Ctrl*, Prm);
 
 template <typename VT>
-static StepFn<VT> step_kernel(int fmt)
+static StepFn<VT> step_kernel(int fmt, int n)
 {
     if (fmt == CEL_FMT_JAD) return k_pcg_step<VT, CEL_FMT_JAD>;
+    if (fmt == CEL_FMT_CSR && n <= (sizeof(VT) == 8 ? 70000 : 120000)) return k_pcg_step<VT, CEL_FMT_CSR, true>;
     return fmt == CEL_FMT_DIA ? k_pcg_step<VT, CEL_FMT_DIA> : k_pcg_step<VT, CEL_FMT_CSR>;
 }
 
@@ -2235,7 +2331,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     auto enqueue_step = [&](long long slot) -> int {
         const int in = (int)(slot & 1), out = in ^ 1;
         if (!mixed) {
-            hipLaunchKernelGGL(step_kernel<double>(fmt), dim3(G1), dim3(kBlock), 0, s, V,
+            hipLaunchKernelGGL(step_kernel<double>(fmt, n), dim3(G1), dim3(kBlock), 0, s, V,
                                (const double*)pbuf[in], (const double*)zbuf, pbuf[out], dx, (double*)nullptr, w.v,
                                w.part1, R64, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
             hipLaunchKernelGGL((k_pcg_update_r<double, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v,
@@ -2243,7 +2339,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         } else {
             ResArgs<float> R = R32;
             R.p = pbuf32[out];  // a restart's direction
-            hipLaunchKernelGGL(step_kernel<float>(fmt), dim3(G1), dim3(kBlock), 0, s, V,
+            hipLaunchKernelGGL(step_kernel<float>(fmt, n), dim3(G1), dim3(kBlock), 0, s, V,
                                (const float*)pbuf32[in], (const float*)zbuf32, pbuf32[out], w.e32, dx, w.v32,
                                w.part1, R, (const double*)w.part2, Gv, (const Ctrl*)C0, C1, P);
             hipLaunchKernelGGL((k_pcg_update_r<float, true, false>), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,

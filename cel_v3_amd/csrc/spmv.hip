@@ -39,6 +39,43 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int* __restric
     }
 }
 
+// A small block: a row per thread, read by its own thread, its first kGather
+// entries and their x at once; three round trips and a store.
+template <typename VT>
+__global__ __launch_bounds__(kBlock) void k_csr_direct(int n, const int* __restrict__ xadj,
+                                                       const int* __restrict__ cols,
+                                                       const VT* __restrict__ vals,
+                                                       const VT* __restrict__ x, VT* __restrict__ y,
+                                                       int accumulate, int coo, const int* __restrict__ skip)
+{
+    const int row = blockIdx.x * kBlock + threadIdx.x;
+    if (row >= n || (skip && *skip)) return;
+    const int lo = xadj[row], hi = xadj[row + 1];
+    const VT y0 = accumulate ? y[row] : VT(0);
+    VT a[kGather], xv[kGather];
+    int c[kGather];
+#pragma unroll
+    for (int i = 0; i < kGather; ++i) {
+        const bool on = lo + i < hi;
+        c[i] = on ? cols[lo + i] : 0;
+        a[i] = on ? vals[lo + i] : VT(0);
+    }
+#pragma unroll
+    for (int i = 0; i < kGather; ++i) xv[i] = x[c[i]];
+    VT s = coo ? y0 : VT(0);  // COO adds the entries to y one by one
+#pragma unroll
+    for (int i = 0; i < kGather; ++i) {
+        const VT prod = a[i] * xv[i];
+        const VT t = s + prod;
+        s = lo + i < hi ? t : s;
+    }
+    for (int j = lo + kGather; j < hi; ++j) {
+        const VT prod = vals[j] * x[cols[j]];
+        s = s + prod;
+    }
+    y[row] = coo ? s : y0 + s;
+}
+
 // FP64 product fused with the next dot product (kFuseDot / kFuseResid,
 // cel_internal.hpp): block b walks the 256-row tiles of its row chunk
 // [b*chunk, b*chunk + chunk) with the same tile stream as k_csr_spmv (same
@@ -127,6 +164,17 @@ static int launch_csr_tiles(const Mat& A, const VT* vals, const VT* x, VT* y, in
                             int coo, const int* skip)
 {
     const bool init = coo && accumulate;
+    // Measured per call (cel_gpu_spmv, device pointers, 13 us of it the launch
+    // and the wait), tiles in LDS / a row per thread: FP64 20^3 15.9 / 13.5 us,
+    // 32^3 15.9 / 13.5, 48^3 16.6 / 15.0, 56^3 17.4 / 16.5, 64^3 17.5 / 18.5,
+    // 80^3 21.7 / 28.0; FP32 32^3 15.3 / 13.5, 56^3 16.5 / 14.9, 64^3 16.7 / 16.2,
+    // 80^3 18.2 / 21.2.
+    if (!csr_long_rows(A) && A.n <= (sizeof(VT) == 8 ? 200000 : 300000)) {
+        hipLaunchKernelGGL(k_csr_direct<VT>, dim3((A.n + kBlock - 1) / kBlock), dim3(kBlock), 0, rt().stream, A.n,
+                           A.xadj.p, A.cols.p, vals, x, y, accumulate, coo, skip);
+        CEL_HIP(hipGetLastError());
+        return CEL_OK;
+    }
     if (csr_long_rows(A))
         return init ? launch_csr_tiles_of<VT, true, true>(A, vals, x, y, accumulate, coo, skip)
                     : launch_csr_tiles_of<VT, false, true>(A, vals, x, y, accumulate, coo, skip);
