@@ -1162,7 +1162,9 @@ struct RunResult {
 };
 
 // One batched solve with tuning T from the current x (x0 already in B.x).
-static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int iter_cap,
+// form_iters: the iterations the choice of the matrices' forms reckons with (a
+// tuning sample is short, the solves it is for are not).
+static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int iter_cap, int form_iters,
                      RunResult& out)
 {
     hipStream_t s = rt().stream;
@@ -1173,7 +1175,7 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     CEL_TRY(B.part2.alloc((size_t)2 * G2 * B.kpmax));
     CEL_TRY(B.rpart.alloc((size_t)3 * G * B.kpmax));
     CEL_TRY(B.ctrl.alloc((size_t)3 * B.lanes));
-    choose_forms(B, iter_cap);
+    choose_forms(B, form_iters);
     CEL_TRY(B.d_form.alloc(B.h_form.size()));
     std::vector<char> active(S, 1);
     std::vector<BBlk> tbl, tbl2;
@@ -1535,7 +1537,7 @@ extern "C" int cel_gpu_batch_tune(cel_gpu_batch* h, const double* const* b, int 
         RunResult rr;
         // the sample is a whole number of chunks
         const int cap = std::max(T.chunk, (iters + T.chunk - 1) / T.chunk * T.chunk) - 1;
-        CEL_TRY(run_batch(B, T, prm, cap, rr));
+        CEL_TRY(run_batch(B, T, prm, cap, 1 << 20, rr));
         int it = 0;
         for (const BCtrl& c : rr.lanes) it = std::max(it, c.iter);
         const double per = rr.ms / std::max(1, it);
@@ -1564,7 +1566,7 @@ extern "C" int cel_gpu_batch_solve(cel_gpu_batch* h, const double* const* b, dou
     CEL_TRY(load_rhs(B, b, prm.memspace));
     CEL_TRY(init_x(B, x, prm));
     RunResult rr;
-    CEL_TRY(run_batch(B, B.tune, prm, prm.iter_max, rr));
+    CEL_TRY(run_batch(B, B.tune, prm, prm.iter_max, prm.iter_max, rr));
     hipStream_t s = rt().stream;
     DevBuf<double> tmp;
     for (size_t q = 0; q < B.mats.size(); ++q) {
