@@ -1343,45 +1343,6 @@ struct cel_gpu_batch {
     Batch b;
 };
 
-// Bandwidth max |col - row| of a square block (0-based rows and columns):
-// per-block maxima, the host takes the largest.
-__global__ __launch_bounds__(kBlock) void k_bandwidth(int n, const int* __restrict__ xadj,
-                                                      const int* __restrict__ cols,
-                                                      int* __restrict__ out)
-{
-    __shared__ int wm[kWaves];
-    int m = 0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long long)gridDim.x * blockDim.x)
-        for (int k = xadj[i]; k < xadj[i + 1]; ++k) m = max(m, abs(cols[k] - (int)i));
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int b = 0;
-        for (int w = 0; w < kWaves; ++w) b = max(b, wm[w]);
-        out[blockIdx.x] = b;
-    }
-}
-
-static int block_bandwidth(const Mat& A, int& bw)
-{
-    bw = 0;
-    if (A.n == 0) return CEL_OK;
-    constexpr int kG = 256;
-    DevBuf<int> part;
-    CEL_TRY(part.alloc(kG));
-    hipStream_t s = rt().stream;
-    hipLaunchKernelGGL(k_bandwidth, dim3(kG), dim3(kBlock), 0, s, A.n, A.xadj.p, A.cols.p, part.p);
-    CEL_HIP(hipGetLastError());
-    std::vector<int> h(kG);
-    CEL_HIP(hipMemcpyAsync(h.data(), part.p, sizeof(int) * kG, hipMemcpyDeviceToHost, s));
-    CEL_HIP(hipStreamSynchronize(s));
-    for (int v : h) bw = std::max(bw, v);
-    return CEL_OK;
-}
-
 extern "C" int cel_gpu_batch_create(cel_gpu_batch** out, int nsys, cel_gpu_mat* const* mats,
                                     const int* nrhs)
 {

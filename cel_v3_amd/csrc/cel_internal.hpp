@@ -226,6 +226,7 @@ struct Mat {
     std::vector<int> h_jad_begin;  // host copy (0-based starts, mmax+1)
 
     Derived derived;
+    int band = -1;  // largest |column - row| of the block (-1: not looked up)
 
     // halo (distributed block split of one rank)
     std::vector<HaloBlock> halo;
@@ -305,6 +306,8 @@ int launch_csr_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const 
 int launch_dia_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const double* x,
                           double* y, const double* aux, double* part, const int* skip);
 int dia_prepare_f32(Mat& A);
+// The largest |column - row| of a square block.
+int block_bandwidth(const Mat& A, int& bw);
 // The derived form (Derived::k*) a PCG solve of at most iter_max iterations
 // runs on, built on the first call that wants it; never an error.
 // *symmetric: the diagonal storage the solve runs on (its own or a derived

@@ -238,6 +238,7 @@ struct MatView {
     // row classes (rowclass.hip), with the diagonals above
     const uint8_t* cls;
     RowClasses ctab;
+    int band;         // window K1s: the largest |column - row|
     const int* walk;  // by K1 block, wide walks: the walk it takes (null: its own)
     // halo (FP64 only)
     const int *hrow_tile, *hrows, *hrowq, *hptr, *hcols;
@@ -968,6 +969,85 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
         }
     }
     return acc;
+}
+
+// The FP64 K1 of long rows in a narrow band: x of a tile group's columns in
+// LDS.  CsrLongStream is bound by its gathers (11 per row of a mesh, a line
+// of L2 each); 2 * band + 512 values loaded in order are a fraction of those
+// bytes, and the gathers then read LDS.  The rows, blocks and orders are the
+// K1's, so the partials are the same.  Two blocks per CU (kWindowCap).
+// Per iteration, from L2 / from LDS: 1,000,003 rows of 13 entries in a band of
+// 3500 76.7 / 55.9 us, of 1400 61.7 / 53.9, 2,000,003 rows in 1400 128.8 /
+// 104.9, 200,003 in 3420 25.4 / 21.7 (27 entries 40.2 / 30.6), 300,007 in 700
+// 29.6 / 27.8, 100,003 in 3420 19.5 / 18.5 and in 1000 17.7 / 18.0, 20,011 in
+// 700 16.8 / 17.1: hence kWindowRows.  Not in the mixed form, whose values are
+// half as wide (600,011 rows 38.6 / 38.0, 300,007 28.9 / 30.2).
+constexpr int kWindowCap = 7680;  // values: 60 KB beside the tile's stage, twice in 160 KB
+constexpr int kWindowRows = 120000;
+static bool window_fits(const Mat& A)
+{
+    return A.band >= 0 && 2LL * A.band + kTileGroup * kTileRows + 4 <= kWindowCap;
+}
+
+template <bool KEEP>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_pcg_window(
+    MatView A, const double* __restrict__ p, double* __restrict__ v, double* __restrict__ part, ResArgs<double> R,
+    const Ctrl* __restrict__ cin, Ctrl* __restrict__ cout, Prm P)
+{
+    __shared__ struct {
+        CsrLongStage<double> tile;
+        alignas(16) double win[kWindowCap];
+    } sm;
+    __shared__ double red[3 * kWaves];
+    __shared__ double fred[2 * kWaves];
+    Ctrl c = read_ctrl(cin);
+    if (c.reduce != kReduceNone) fold_pending(c, R.part, R.G, P, fred);
+    if (!c.run) {
+        write_ctrl(cout, c);
+        return;
+    }
+    const long long ntiles = (A.n + kTileRows - 1) / kTileRows;
+    const double* vals = A.vals;
+    CsrLongStream<double, KEEP> cs;
+    const long long tfirst = group_tile(0, ntiles);
+    if (tfirst >= 0) cs.open(A.n, (int)tfirst, (int)group_tile(1, ntiles), A.xadj, A.cols, vals, sm.tile);
+    double acc = 0.0;
+    XWindow<double> x{sm.win, 0, 0};
+    long long k = 0;
+    for (long long t = tfirst; t >= 0; t = group_tile(++k, ntiles)) {
+        if (k % kTileGroup == 0) {  // a new group: its columns
+            const int r0 = (int)t * kTileRows;
+            x.w0 = max(0, r0 - A.band) & ~1;
+            const int w1 = min(A.n, r0 + kTileGroup * kTileRows + A.band);
+            x.last = w1 - x.w0 - 1;
+            // (16 bytes per load; past w1 it returns 0)
+            const auto rx = tile_rsrc(p + x.w0, (w1 - x.w0) * 8);
+            __syncthreads();  // the group before is done with the window
+            constexpr int kAt = kWindowCap / 2 / kBlock;
+            U32x4 w[kAt];
+#pragma unroll
+            for (int i = 0; i < kAt; ++i)
+                w[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, 16 * (int)threadIdx.x, 16 * kBlock * i, 0);
+#pragma unroll
+            for (int i = 0; i < kAt; ++i)
+                reinterpret_cast<U32x4*>(sm.win)[threadIdx.x + kBlock * i] = w[i];
+            __syncthreads();
+        }
+        const int nxt = (int)group_tile(k + 1, ntiles);
+        const int aft = (int)group_tile(k + 2, ntiles);
+        const int row = (int)t * kTileRows + threadIdx.x;
+        double pr = 0.0;
+        double s = cs.template rows<double>(A.n, (int)t, nxt, aft, A.xadj, A.cols, vals, x, sm.tile, row, &pr);
+        s = A.coo ? s : 0.0 + s;
+        if (row < A.n) {
+            v[row] = s;
+            const double prod = s * pr;
+            acc = acc + prod;
+        }
+    }
+    const double bs = block_sum(acc, red);
+    if (threadIdx.x == 0) part[logical_block()] = bs;
+    write_ctrl(cout, c);
 }
 
 // LDS of a K1: its tile stage and that of a wide walk; in the mixed form the
@@ -2245,6 +2325,14 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     // (a symmetric block's values are read again a row, a line and a plane
     // later: 256^3 FP64 427 us per iteration marked as read once, 425 kept)
     const bool keep = sym || keep_matrix(A, kfmt, arrays, mixed);
+    // long rows in a narrow band: the band is looked up once per matrix
+    bool win = false;
+    if (kfmt == CEL_FMT_CSR && lr && !mixed && !halo && !noalloc && n >= kWindowRows &&
+        (A.band >= 0 || prm.iter_max >= 32)) {
+        if (A.band < 0) CEL_TRY(block_bandwidth(A, A.band));
+        win = window_fits(A);
+        V.band = A.band;
+    }
     if (use == Derived::kClasses || sym) CEL_TRY(wide_walk(V, *Wp, G1));
     if (halo) {
         V.hrow_tile = Wp->hrow_tile.p;
@@ -2366,7 +2454,9 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             CEL_HIP(hipEventRecord(ea, s));
         }
         if (!mixed) {
-            hipLaunchKernelGGL(k1_kernel<double>(kfmt, halo, lr, keep), dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
+            const auto k1 = !win ? k1_kernel<double>(kfmt, halo, lr, keep)
+                            : keep ? k_pcg_window<true> : k_pcg_window<false>;
+            hipLaunchKernelGGL(k1, dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
                                w.part1, R64, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL(k2_kernel<double>(bycls, stream), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r, w.v, vjac64,

@@ -158,6 +158,17 @@ struct XPlain {
     __device__ __forceinline__ Raw load(const Buf& b, int off) const { return buf_load<VT>(b.r, off); }
 };
 
+// x of the columns [w0, w0 + len) from a copy in LDS (an index outside reads
+// one of its ends: entries that a row does not have).
+template <typename VT>
+struct XWindow {
+    using Raw = VT;
+    const VT* win;
+    int w0, last;
+    __device__ __forceinline__ Raw load(int i) const { return win[min(max(i - w0, 0), last)]; }
+    __device__ __forceinline__ VT value(Raw r) const { return r; }
+};
+
 // beta p + z: the search direction of the next iteration, formed where it
 // is gathered (each product rounded before its add, as the update kernel
 // rounds them).  keep: the direction is p itself.
