@@ -1375,18 +1375,22 @@ constexpr int kVecUnrollOf = sizeof(VT) == 4 ? 4 : 2;
 // others: kStreamX: x, which only K3 touches; kStreamAll: also v and r where
 // they are read, so that what stays is what the next kernel reads (v from K1
 // to K2, r from K2 to K3, p from K3 to K1).  Measured per iteration with
-// none / x / all marked, Poisson cubes on row classes: FP64 192^3 (233 MB)
-// 125 / 127 / 130 us, 200^3 (264) 147.5 / 141 / 144, 216^3 (333) 181 / 175 /
-// 177, 232^3 (412) 236 / 214 / 214, 256^3 (554) 358 / 336 / 283, 320^3
-// (1081) 691 / 683 / 644; mixed 232^3 (212) 113 / 114 / 117, 256^3 (285)
-// 155 / 149 / 151, 288^3 (406) 231 / 213 / 209, 320^3 (557) 336 / 320 /
-// 284; variable coefficients FP64 176^3 (218) 146 / 147 / 149, 192^3 (283)
+// none / x / all marked, Poisson cubes on row classes: FP64 180^3 (192 MB)
+// 88.2 / 90.0 / 92.5 us, 200^3 (264) 124.9 / 116.2 / 119.8, 216^3 (333) 154.7
+// / 144.3 / 147.9, 232^3 (412) 205.6 / 181.5 / 177.1; mixed 232^3 (212) 97.7 /
+// 99.9 / 102.2, 256^3 (285) 138.8 / 126.8 / 129.4, 288^3 (406) 210.0 / 183.7 /
+// 180.7; general variable coefficients FP64 176^3 (218) 146 / 147 / 149, 192^3 (283)
 // 189 / 186 / 188, 216^3 (403) 285 / 267 / 264, 256^3 (671) 521 / 494 / 459.
+// The values of a symmetric block (`arrays` of them) are kept as well and
+// share the cache, so there the line is one on both together: 144^3 (215 MB)
+// 65.8 / 67.0 / 68.4 us, 160^3 (295) 98.2 / 91.6 / 90.9, 176^3 (392) 125.1 /
+// 122.9 / 122.0, 200^3 (576) 192.3 / 185.7 / 177.9, 230^3 (876) 311 / 295 / 279.
 enum StreamLevel { kStreamNone = 0, kStreamX = 1, kStreamAll = 2 };
-static int stream_level(long long n, bool mixed, bool cls)
+static int stream_level(long long n, bool mixed, bool cls, int arrays)
 {
     const double vb = mixed ? 4.0 : 8.0;
     const double bytes = ((cls ? 4.0 : 5.0) * vb + (cls ? 1.0 : 0.0)) * (double)n;
+    if (arrays) return bytes + arrays * vb * (double)n > 240e6 ? kStreamAll : kStreamNone;
     return bytes > 380e6 ? kStreamAll : bytes > 240e6 ? kStreamX : kStreamNone;
 }
 
@@ -2412,7 +2416,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     const double* vjac64 = bycls ? V.ctab.jac64 : jac64;
     const float* vjac32 = bycls ? V.ctab.jac32 : jac32;
     const uint8_t *vcls = bycls ? V.cls : nullptr, *nocls = nullptr;
-    const int stream = stream_level(n, mixed, bycls);
+    const int stream = stream_level(n, mixed, bycls, sym ? arrays : 0);
     // One slot of the two-kernel form: the step finishes the iteration before
     // (its vectors and scalars) and forms the next product, K2 updates r.
     // The direction alternates between two buffers by slot.
