@@ -716,7 +716,10 @@ def main():
             continue
         r = prof[pname]
         halo = "halo" in pname
-        name = (f"k_pcg_spmv<{vt},{fname[form]}" + (",halo>" if halo else ">") +
+        # a long solve of a block whose rows repeat runs on row classes, whatever
+        # the caller's form: x, v and a byte per row
+        classes = r["spmv_bytes"] == (1 + 2 * (4 if vt == "float" else 8)) * N ** 3
+        name = (f"k_pcg_spmv<{vt},{'classes' if classes else fname[form]}" + (",halo>" if halo else ">") +
                 (" (+6 halo faces, one-subdomain model)" if halo else " (v = A p fused with v.p)"))
         k1_ms, achieved = k1(r)
         res[key] = {"kernel": name, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
