@@ -374,8 +374,8 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric)
     // few iterations do not pay for the passes over the matrix.  Measured per
     // iteration, CSR arrays / classes / diagonal storage: 64^3 FP64 17.2 /
     // 17.0 / 17.1 us; 80^3 29.1 / 25.4 / 27.8, mixed 22.9 / 22.0 / 21.4;
-    // 100^3 39.6 / 30.0 / 36.4, mixed 31.8 / 24.3 / 28.4; 256^3 618 / 350 /
-    // 507, mixed 358 / 158 / 232.  Building takes 0.4 ms (100^3) to 1.3 ms
+    // 100^3 39.6 / 26.5 / 30.7, mixed 31.8 / 22.5 / 28.4; 256^3 618 / 240 /
+    // 411, mixed 358 / 127 / 232 (FP64 diagonals of 100^3 and 256^3 symmetric).  Building takes 0.4 ms (100^3) to 1.3 ms
     // (256^3), as much as 40 to 10 iterations save; a solve of such a block
     // to 1e-10 takes 300 to 800.
     if (A.n < kDerivedRows || (iter_max < 32 && !D.tried) || !A.jac.p || !A.jac32.p) return Derived::kNone;
