@@ -85,13 +85,22 @@ void* pool_alloc(size_t bytes, size_t* got, int* device)
         if (rt().stream) (void)hipStreamSynchronize(rt().stream);
         return p;
     }
-    if (hipMalloc(&p, want) == hipSuccess) return p;
+    return device_malloc(want);
+}
+
+void* device_malloc(size_t bytes)
+{
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
     (void)hipGetLastError();
-    {
+    int dev = 0;
+    if (hipGetDevice(&dev) == hipSuccess) {
+        Pool& P = pool();
         std::lock_guard<std::mutex> lock(P.mu);
         pool_drop(P, dev);
     }
-    if (hipMalloc(&p, want) == hipSuccess) return p;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
     return nullptr;
 }
 
@@ -159,7 +168,10 @@ extern "C" int cel_gpu_init(int device)
     CEL_HIP(hipSetDevice(device));
     hipDeviceProp_t prop;
     CEL_HIP(hipGetDeviceProperties(&prop, device));
-    if (R.stream) (void)hipStreamDestroy(R.stream);
+    if (R.stream) {
+        (void)hipStreamSynchronize(R.stream);  // kept blocks of that device may still be in use
+        (void)hipStreamDestroy(R.stream);
+    }
     // default priority stream, non-blocking w.r.t. the null stream
     CEL_HIP(hipStreamCreateWithFlags(&R.stream, hipStreamNonBlocking));
     R.device = device;
@@ -202,11 +214,8 @@ extern "C" int cel_gpu_malloc(void** ptr, size_t bytes)
 {
     CEL_TRY(ensure_init());
     if (!ptr) return fail(CEL_ERR_ARG, "null pointer");
-    if (hipMalloc(ptr, bytes ? bytes : 1) != hipSuccess) {
-        *ptr = nullptr;
-        return fail(CEL_ERR_OOM, "hipMalloc failed");
-    }
-    return CEL_OK;
+    *ptr = device_malloc(bytes ? bytes : 1);
+    return *ptr ? CEL_OK : fail(CEL_ERR_OOM, "hipMalloc failed");
 }
 
 extern "C" int cel_gpu_free(void* ptr)

@@ -51,12 +51,14 @@ int resident_grid(const void* kernel, long long work_items);
 // buffer of about its size instead of going back to the driver, whose
 // allocations and (synchronising) frees of large blocks cost 0.1-0.2 ms
 // each.  Kept blocks are bounded (kPoolBytes in all), go back when an
-// allocation fails and with cel_gpu_finalize.  A reused block may still be
+// allocation of the library fails (device_malloc: cel_gpu_malloc's too) and
+// with cel_gpu_finalize.  A reused block may still be
 // read by work on the library's stream, so that is waited for before it is
 // handed out; the lists are per device and locked.
 constexpr size_t kPoolBytes = size_t(2) << 30;
 void* pool_alloc(size_t bytes, size_t* got, int* device);  // null: no memory
 void pool_free(void* p, size_t bytes, int device);
+void* device_malloc(size_t bytes);  // hipMalloc; gives kept blocks back before it fails (null)
 void pool_release();
 
 // Device buffer owned by the library.

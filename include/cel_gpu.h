@@ -125,7 +125,14 @@ int cel_gpu_finalize(void);
 const char* cel_gpu_last_error(void);
 int cel_gpu_device_info(char* name, int name_len, int* num_cus);
 
-/* device memory for callers that keep inputs resident in HBM */
+/* device memory for callers that keep inputs resident in HBM.
+ *
+ * The library keeps up to 2 GiB of the device memory that its own objects
+ * (matrices, batches, solver workspaces) have freed, for the next object of
+ * about the same size.  It gives that memory back to the driver when one of
+ * its own allocations, cel_gpu_malloc among them, would otherwise fail, and
+ * in cel_gpu_finalize; allocators outside the library do not see it before.
+ * What cel_gpu_free releases goes to the driver at once. */
 int cel_gpu_malloc(void** ptr, size_t bytes);
 int cel_gpu_free(void* ptr);
 int cel_gpu_memcpy_h2d(void* dst, const void* src, size_t bytes);

@@ -1,0 +1,94 @@
+"""Decisions of the library's host code, without a GPU: the library runs in a
+child process over a stand-in for the HIP runtime (hoststub/hip_stub.cpp),
+where device memory has a budget and a kernel launch is a line of a log.
+No result is computed here; what is looked at is which calls succeed, which
+kernels they launch, and on how many blocks."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+STUB = os.path.join(HERE, "hoststub", "hip_stub.cpp")
+
+PRELUDE = """
+import ctypes as C, json, sys
+import numpy as np
+sys.path.insert(0, %r)
+import cel_v3_amd as cel
+S = C.CDLL(None)
+S.stub_log.restype = C.c_char_p
+S.stub_budget.argtypes = [C.c_size_t]
+S.stub_used.restype = S.stub_peak.restype = C.c_size_t
+cel.init(0)
+
+def box(nx, ny, nz):
+    '''7-point block, 0-based CSR arrays'''
+    n = nx * ny * nz
+    i = np.arange(n)
+    x, y, z = i %% nx, i // nx %% ny, i // (nx * ny)
+    cols = np.stack([i - nx * ny, i - nx, i - 1, i, i + 1, i + nx, i + nx * ny], 1)
+    on = np.stack([z > 0, y > 0, x > 0, i >= 0, x < nx - 1, y < ny - 1, z < nz - 1], 1)
+    xadj = np.concatenate([[0], np.cumsum(on.sum(1))])
+    vals = np.where(np.arange(7) == 3, 6.0, -1.0) * np.ones((n, 1))
+    return xadj, cols[on], vals[on]
+
+def matrix(*shape):
+    M = cel.Matrix.from_csr(*box(*shape), index_base=0)
+    M.set_jacobi()
+    return M
+
+def launches(name=None):
+    '''(kernel, blocks) since the log was cleared'''
+    out = [tuple(l.rsplit(" ", 1)) for l in S.stub_log().decode().splitlines() if " " in l]
+    return [(k, int(g)) for k, g in out if name is None or k.split("<")[0] == name]
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    import cel_v3_amd as cel
+
+    if not os.path.exists(cel.LIB_PATH) or shutil.which("g++") is None or not os.path.isdir("/opt/rocm/include/hip"):
+        pytest.skip("needs libcel_gpu.so, g++ and the HIP headers")
+    so = tmp_path_factory.mktemp("hoststub") / "libamdhip64.so.7"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", "-Wl,-soname,libamdhip64.so.7", STUB, "-o", str(so)], check=True)
+
+    def run(body):
+        """The JSON value that `body` assigns to `out`."""
+        code = PRELUDE % ROOT + body + "\nprint('OUT' + json.dumps(out))\n"
+        env = dict(os.environ, LD_PRELOAD=str(so))
+        r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return json.loads(r.stdout.split("OUT", 1)[1])
+
+    return run
+
+
+def test_kept_blocks_go_back_when_a_callers_allocation_fails(stub):
+    out = stub("""
+M = matrix(64, 64, 64)
+held = S.stub_used()
+del M
+kept = S.stub_used()
+S.stub_budget(kept + 1000)
+a = cel.DeviceArray(kept // 16)       # half of what is kept
+out = {"held": held, "kept": kept, "used": S.stub_used(), "got": kept // 16 * 8}
+""")
+    assert out["kept"] > 0.9 * out["held"]  # destroyed, and not with the driver
+    assert out["used"] == out["got"]
+
+
+@pytest.mark.parametrize("more", [0, 1])
+def test_an_allocation_that_cannot_be_had_is_still_refused(stub, more):
+    out = stub(f"""
+S.stub_budget(1 << 20)
+p = C.c_void_p(1)
+out = [cel.lib().cel_gpu_malloc(C.byref(p), C.c_size_t((1 << 20) + {more})), p.value]
+""")
+    assert (out[0] == 0 and out[1]) if not more else out == [-8, None]
