@@ -1175,8 +1175,10 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     CEL_TRY(B.part2.alloc((size_t)2 * G2 * B.kpmax));
     CEL_TRY(B.rpart.alloc((size_t)3 * G * B.kpmax));
     CEL_TRY(B.ctrl.alloc((size_t)3 * B.lanes));
+    CEL_TRY(B.d_form.alloc(S));
+    std::vector<DerivedUse> reading(S);
+    for (int q = 0; q < S; ++q) reading[q].begin(B.mats[q]->derived);
     choose_forms(B, form_iters);
-    CEL_TRY(B.d_form.alloc(B.h_form.size()));
     std::vector<char> active(S, 1);
     std::vector<BBlk> tbl, tbl2;
     CEL_TRY(build_table(B, G, T.weight, active, tbl, false));

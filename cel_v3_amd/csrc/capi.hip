@@ -57,7 +57,7 @@ void pool_drop(Pool& P, int device)
 }
 }  // namespace
 
-void* pool_alloc(size_t bytes, size_t* got, int* device)
+void* pool_alloc(size_t bytes, size_t* got, int* device, bool spare)
 {
     Pool& P = pool();
     int dev = 0;
@@ -85,22 +85,31 @@ void* pool_alloc(size_t bytes, size_t* got, int* device)
         if (rt().stream) (void)hipStreamSynchronize(rt().stream);
         return p;
     }
-    return device_malloc(want);
+    p = device_malloc(want, spare);
+    if (!p && want - bytes >= 512) {  // the last memory: only what is asked for
+        *got = (bytes + 511) / 512 * 512;
+        p = device_malloc(*got, spare);
+    }
+    return p;
 }
 
-void* device_malloc(size_t bytes)
+void* device_malloc(size_t bytes, bool spare)
 {
     void* p = nullptr;
     if (hipMalloc(&p, bytes) == hipSuccess) return p;
     (void)hipGetLastError();
     int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        Pool& P = pool();
-        std::lock_guard<std::mutex> lock(P.mu);
-        pool_drop(P, dev);
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    Pool& P = pool();
+    for (const bool forms : {false, true}) {
+        if (forms && (spare || !derived_give_back())) break;
+        {
+            std::lock_guard<std::mutex> lock(P.mu);
+            pool_drop(P, dev);
+        }
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
     }
-    if (hipMalloc(&p, bytes) == hipSuccess) return p;
-    (void)hipGetLastError();
     return nullptr;
 }
 
@@ -486,7 +495,7 @@ extern "C" int cel_gpu_mat_set_jacobi(cel_gpu_mat* A, int row_scaled)
     Mat& M = A->m;
     if (!M.has_diag) CEL_TRY(launch_extract_diag(M));
     M.has_diag = true;
-    M.derived.release();  // its row forms hold the Jacobi values
+    M.derived.drop();  // its row forms hold the Jacobi values
     CEL_TRY(launch_set_jacobi(M, row_scaled));
     M.has_jac = true;
     M.jac_row_scaled = row_scaled != 0;
@@ -502,7 +511,7 @@ extern "C" int cel_gpu_mat_scale_diagonal(cel_gpu_mat* A)
     CEL_TRY(launch_scale_rows(M));
     M.is_scaled = true;
     // derived copies are stale now
-    M.derived.release();
+    M.derived.drop();
     M.vals32.release();
     M.jad_mode = -1;
     M.jad_vals32.release();

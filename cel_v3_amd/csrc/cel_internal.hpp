@@ -56,9 +56,12 @@ int resident_grid(const void* kernel, long long work_items);
 // read by work on the library's stream, so that is waited for before it is
 // handed out; the lists are per device and locked.
 constexpr size_t kPoolBytes = size_t(2) << 30;
-void* pool_alloc(size_t bytes, size_t* got, int* device);  // null: no memory
+void* pool_alloc(size_t bytes, size_t* got, int* device, bool spare);  // null: no memory
 void pool_free(void* p, size_t bytes, int device);
-void* device_malloc(size_t bytes);  // hipMalloc; gives kept blocks back before it fails (null)
+// hipMalloc; before it fails (null) it gives the kept blocks back and, unless
+// the memory is only wanted where there is some to spare, the derived forms
+// that no solve is reading.
+void* device_malloc(size_t bytes, bool spare = false);
 void pool_release();
 
 // Device buffer owned by the library.
@@ -72,11 +75,11 @@ struct DevBuf {
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
-    int alloc(size_t count) {
+    int alloc(size_t count, bool spare = false) {
         if (count == n && p) return CEL_OK;
         release();
         if (count == 0) return CEL_OK;
-        p = static_cast<T*>(pool_alloc(count * sizeof(T), &bytes, &device));
+        p = static_cast<T*>(pool_alloc(count * sizeof(T), &bytes, &device, spare));
         if (!p) {
             return fail(CEL_ERR_OOM, "hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed");
         }
@@ -155,7 +158,9 @@ struct HaloBlock {
     std::vector<int> h_recv_perm;  // ascending local column ids (1-based)
 };
 
-// Derived forms of a block for long solves (rowclass.hip).
+// Derived forms of a block for long solves (rowclass.hip).  They only save
+// time: they are built in memory that is to spare, and those no solve is
+// reading go back when an allocation of the library fails.
 constexpr int kMaxClass = 256;   // row forms a byte tells apart
 constexpr int kClassDiag = 8;    // diagonals of a row form
 constexpr int kDerivedRows = 800000;
@@ -188,7 +193,24 @@ struct Derived {
         return RowClasses{tab64.p, tab64.p + kMaxClass * kClassDiag, tab32.p, tab32.p + kMaxClass * kClassDiag,
                           tabm.p};
     }
+    int users = 0;   // solves that read it (DerivedUse)
+    bool listed = false;  // among the forms derived_give_back looks at
+    Derived *before = nullptr, *after = nullptr;
+    ~Derived();
     void release();
+    void drop();     // release, for a handle that no solve is reading
+};
+bool derived_give_back();  // drops every form without users; false: there was none
+
+// Marks a handle's form as being read (or built) until it goes out of scope.
+struct DerivedUse {
+    Derived* d = nullptr;
+    DerivedUse() = default;
+    DerivedUse(const DerivedUse&) = delete;
+    DerivedUse& operator=(const DerivedUse&) = delete;
+    ~DerivedUse() { end(); }
+    void begin(Derived& D);
+    void end();
 };
 
 struct Mat {
@@ -311,7 +333,8 @@ int dia_prepare_f32(Mat& A);
 // The largest |column - row| of a square block.
 int block_bandwidth(const Mat& A, int& bw);
 // The derived form (Derived::k*) a PCG solve of at most iter_max iterations
-// runs on, built on the first call that wants it; never an error.
+// runs on, built on the first call that wants it; never an error.  The caller
+// holds a DerivedUse of A and has made its own allocations.
 // *symmetric: the diagonal storage the solve runs on (its own or a derived
 // one) holds bit for bit the same value at (i, j) and (j, i).
 int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric);

@@ -2135,34 +2135,10 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         if (Gv >= kXcds) Gv = Gv / kXcds * kXcds;
     }
 
-    // the form the K1s run on, and its residual's: the caller's, or a derived
-    // one with the same bits (its grids are the caller's form's)
-    int use = Derived::kNone;
-    bool symmetric = false;
-    if (!noalloc && !halo && !coo && fmt != CEL_FMT_JAD)
-        use = derived_prepare(A, fmt, mixed, prm.iter_max, &symmetric);
-    const int kfmt = use == Derived::kClasses ? kFmtClass : use == Derived::kDiagonals ? CEL_FMT_DIA : fmt;
-    const int kres = use == Derived::kClasses ? kFmtClass : rfmt;
-
     if (noalloc && ((size_t)G1 > kNoAllocMaxGrid || (size_t)Gr > kNoAllocMaxGrid ||
                     (size_t)Gv > kNoAllocMaxGrid))
         return fail(CEL_ERR_ARG, "the allocation-free solve holds at most " +
                                      std::to_string(kNoAllocMaxGrid) + " blocks per kernel");
-
-    // matrix data for the mixed inner operator (once per matrix)
-    if (mixed) {
-        if (fmt == CEL_FMT_DIA && kfmt == CEL_FMT_DIA) CEL_TRY(dia_prepare_f32(A));
-        // the DIA K1 reads dia_vals32 and the residual kernels the FP64 CSR
-        // values, so only a CSR solve needs the FP32 CSR copy
-        if (kfmt == CEL_FMT_CSR && !A.vals32.p) {
-            CEL_TRY(A.vals32.alloc(A.nnz > 0 ? A.nnz : 1));
-            CEL_TRY(launch_to_f32(A.vals.p, A.vals32.p, A.nnz));
-        }
-        if (fmt == CEL_FMT_JAD && !A.jad_vals32.p) {
-            CEL_TRY(A.jad_vals32.alloc(A.jad_nnz > 0 ? A.jad_nnz : 1));
-            CEL_TRY(launch_to_f32(A.jad_vals.p, A.jad_vals32.p, A.jad_nnz));
-        }
-    }
 
     // workspace: the matrix handle's buffers, or the scratch array
     const size_t nn = n > 0 ? n : 1;
@@ -2205,26 +2181,6 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         w.v32 = W.v32.p;
         w.e32 = W.e32.p;
     }
-    // two kernels per iteration on small systems; the halo blocks need a
-    // stored direction before the product, profiling a product of its own
-    const bool step = !noalloc && !halo && !prm.profile && use == Derived::kNone &&
-                      step_form(A, fmt, mixed);
-    double *pbuf[2] = {w.p, nullptr}, *zbuf = nullptr;
-    float *pbuf32[2] = {w.p32, nullptr}, *zbuf32 = nullptr;
-    if (step) {
-        Workspace& W = *Wp;
-        if (mixed) {
-            CEL_TRY(W.p2_32.alloc(nn));
-            CEL_TRY(W.z32.alloc(nn));
-            pbuf32[1] = W.p2_32.p;
-            zbuf32 = W.z32.p;
-        } else {
-            CEL_TRY(W.p2.alloc(nn));
-            CEL_TRY(W.z.alloc(nn));
-            pbuf[1] = W.p2.p;
-            zbuf = W.z.p;
-        }
-    }
     const double* db = b;
     double* dx = x;
     if (prm.memspace == CEL_MEM_HOST) {
@@ -2260,6 +2216,54 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         CEL_TRY(build_hrow_tile(A, W, ntiles));
     }
 
+    // the form the K1s run on, and its residual's: the caller's, or a derived
+    // one with the same bits (its grids are the caller's form's).  It is built
+    // in what the solve's own memory, above, has left.
+    int use = Derived::kNone;
+    bool symmetric = false;
+    DerivedUse reading;
+    if (!noalloc && !halo && !coo && fmt != CEL_FMT_JAD) {
+        reading.begin(A.derived);
+        use = derived_prepare(A, fmt, mixed, prm.iter_max, &symmetric);
+        if (use == Derived::kNone) reading.end();
+    }
+    const int kfmt = use == Derived::kClasses ? kFmtClass : use == Derived::kDiagonals ? CEL_FMT_DIA : fmt;
+    const int kres = use == Derived::kClasses ? kFmtClass : rfmt;
+
+    // matrix data for the mixed inner operator (once per matrix)
+    if (mixed) {
+        if (fmt == CEL_FMT_DIA && kfmt == CEL_FMT_DIA) CEL_TRY(dia_prepare_f32(A));
+        // the DIA K1 reads dia_vals32 and the residual kernels the FP64 CSR
+        // values, so only a CSR solve needs the FP32 CSR copy
+        if (kfmt == CEL_FMT_CSR && !A.vals32.p) {
+            CEL_TRY(A.vals32.alloc(A.nnz > 0 ? A.nnz : 1));
+            CEL_TRY(launch_to_f32(A.vals.p, A.vals32.p, A.nnz));
+        }
+        if (fmt == CEL_FMT_JAD && !A.jad_vals32.p) {
+            CEL_TRY(A.jad_vals32.alloc(A.jad_nnz > 0 ? A.jad_nnz : 1));
+            CEL_TRY(launch_to_f32(A.jad_vals.p, A.jad_vals32.p, A.jad_nnz));
+        }
+    }
+
+    // two kernels per iteration on small systems; the halo blocks need a
+    // stored direction before the product, profiling a product of its own
+    bool step = !noalloc && !halo && !prm.profile && use == Derived::kNone && step_form(A, fmt, mixed);
+    const std::string err = last_error();  // (what is tried and not had below is no error of the solve)
+    double *pbuf[2] = {w.p, nullptr}, *zbuf = nullptr;
+    float *pbuf32[2] = {w.p32, nullptr}, *zbuf32 = nullptr;
+    if (step) {
+        Workspace& W = *Wp;
+        if (mixed) {
+            step = W.p2_32.alloc(nn) == CEL_OK && W.z32.alloc(nn) == CEL_OK;
+            pbuf32[1] = W.p2_32.p;
+            zbuf32 = W.z32.p;
+        } else {
+            step = W.p2.alloc(nn) == CEL_OK && W.z.alloc(nn) == CEL_OK;
+            pbuf[1] = W.p2.p;
+            zbuf = W.z.p;
+        }
+        if (!step) set_error(err);  // no memory for them: three kernels
+    }
     Prm P{};
     P.tol = prm.tol;
     P.tol_mode = prm.tol_mode;
@@ -2333,11 +2337,14 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     bool win = false;
     if (kfmt == CEL_FMT_CSR && lr && !mixed && !halo && !noalloc && n >= kWindowRows &&
         (A.band >= 0 || prm.iter_max >= 32)) {
-        if (A.band < 0) CEL_TRY(block_bandwidth(A, A.band));
+        if (A.band < 0 && block_bandwidth(A, A.band) != CEL_OK) {  // without the window
+            A.band = -1;
+            set_error(err);
+        }
         win = window_fits(A);
         V.band = A.band;
     }
-    if (use == Derived::kClasses || sym) CEL_TRY(wide_walk(V, *Wp, G1));
+    if ((use == Derived::kClasses || sym) && wide_walk(V, *Wp, G1) != CEL_OK) set_error(err);  // each block its own walk
     if (halo) {
         V.hrow_tile = Wp->hrow_tile.p;
         V.hrows = A.halo_rows.p;

@@ -24,8 +24,10 @@
 // derived_prepare), belong to the handle, and are dropped when the values,
 // the Jacobi vector or the scaling change.  A matrix they do not fit costs
 // one pass that stops early; without memory for them the solve runs on the
-// CSR arrays.
+// CSR arrays.  The memory they take is returned when another allocation needs
+// it (device_malloc) and no solve is reading them.
 #include <algorithm>
+#include <mutex>
 #include <type_traits>
 
 #include "cel_internal.hpp"
@@ -293,10 +295,10 @@ int build_classes(Mat& A, const Offs& O, bool* ok)
     CEL_HIP(hipMemcpyAsync(h, &T.p->count, sizeof(h), hipMemcpyDeviceToHost, st));
     CEL_HIP(hipStreamSynchronize(st));
     if (h[1] || h[0] > kMaxClass) return CEL_OK;
-    CEL_TRY(D.cls.alloc((size_t)A.n));
-    CEL_TRY(D.tab64.alloc((size_t)kMaxClass * (kClassDiag + 1)));
-    CEL_TRY(D.tab32.alloc((size_t)kMaxClass * (kClassDiag + 1)));
-    CEL_TRY(D.tabm.alloc(kMaxClass));
+    CEL_TRY(D.cls.alloc((size_t)A.n, true));
+    CEL_TRY(D.tab64.alloc((size_t)kMaxClass * (kClassDiag + 1), true));
+    CEL_TRY(D.tab32.alloc((size_t)kMaxClass * (kClassDiag + 1), true));
+    CEL_TRY(D.tabm.alloc(kMaxClass, true));
     const RowClasses tab = D.classes();
     hipLaunchKernelGGL(k_class_table, dim3(1), dim3(kBlock), 0, st, h[0], T.p, A.xadj.p, A.cols.p, A.vals.p,
                        A.jac.p, A.jac32.p, O, tab);
@@ -346,6 +348,58 @@ int dia_bases(int n, int nd, const int* off, bool symmetric, long long* base)
             }
     }
     return arrays;
+}
+
+// The forms that a solve has looked at, as a list through them.
+static std::mutex forms_lock;
+static Derived* forms = nullptr;
+
+void DerivedUse::begin(Derived& D)
+{
+    end();
+    std::lock_guard<std::mutex> lock(forms_lock);
+    if (!D.listed) {
+        D.listed = true;
+        D.after = forms;
+        if (forms) forms->before = &D;
+        forms = &D;
+    }
+    ++D.users;
+    d = &D;
+}
+
+void DerivedUse::end()
+{
+    if (!d) return;
+    std::lock_guard<std::mutex> lock(forms_lock);
+    --d->users;
+    d = nullptr;
+}
+
+bool derived_give_back()
+{
+    std::lock_guard<std::mutex> lock(forms_lock);
+    bool any = false;
+    for (Derived* D = forms; D; D = D->after)
+        if (D->users == 0 && (D->cls.p || D->mask8.p || D->vals.p || D->vals32.p)) {
+            D->release();
+            any = true;
+        }
+    return any;
+}
+
+Derived::~Derived()
+{
+    std::lock_guard<std::mutex> lock(forms_lock);
+    if (!listed) return;
+    if (after) after->before = before;
+    (before ? before->after : forms) = after;
+}
+
+void Derived::drop()
+{
+    std::lock_guard<std::mutex> lock(forms_lock);
+    release();
 }
 
 void Derived::release()
@@ -411,8 +465,8 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric)
         const size_t cnt = (size_t)D.nd * (size_t)A.n;
         if (!tried) {
             tried = true;
-            rc = D.mask8.p ? CEL_OK : D.mask8.alloc((size_t)A.n);
-            if (rc == CEL_OK) rc = mixed ? D.vals32.alloc(cnt) : D.vals.alloc(cnt);
+            rc = D.mask8.p ? CEL_OK : D.mask8.alloc((size_t)A.n, true);
+            if (rc == CEL_OK) rc = mixed ? D.vals32.alloc(cnt, true) : D.vals.alloc(cnt, true);
             if (rc == CEL_OK)
                 rc = dia_fill(A, D.nd, D.off, mixed ? nullptr : D.vals.p, mixed ? D.vals32.p : nullptr, D.mask8.p);
             if (rc != CEL_OK) {
@@ -475,8 +529,8 @@ void derived_prepare_all(const std::vector<Mat*>& mats, int iter_max)
         Mat& A = *todo[q];
         Derived& D = A.derived;
         if (!sets[q].ascending || sets[q].nd > kClassDiag || (long long)sets[q].nd * A.n > 2LL * A.nnz) continue;
-        rc = D.mask8.alloc((size_t)A.n);
-        if (rc == CEL_OK) rc = D.vals.alloc((size_t)sets[q].nd * (size_t)A.n);
+        rc = D.mask8.alloc((size_t)A.n, true);
+        if (rc == CEL_OK) rc = D.vals.alloc((size_t)sets[q].nd * (size_t)A.n, true);
         if (rc == CEL_OK) rc = dia_fill(A, sets[q].nd, sets[q].off, D.vals.p, nullptr, D.mask8.p);
         if (rc != CEL_OK) break;
         Offs O{};

@@ -368,7 +368,13 @@ void cel_gpu_pcg_params_default(cel_pcg_params* p);
  * Requires cel_gpu_mat_set_jacobi.  With use_halo the halo blocks are
  * applied with a zero ghost region (one subdomain, no neighbours present)
  * and the send faces are packed every SpMV; FP64 only, in the CSR or the
- * DIA form, with fewer than 2^27 rows that have halo entries. */
+ * DIA form, with fewer than 2^27 rows that have halo entries.
+ * A solve of 800,000 rows or more in the CSR or DIA form may build another
+ * form of the block for its product (same bits), which stays with the handle
+ * until its values or its Jacobi vector change: 1 to 65 bytes a row, up to 32
+ * more once it has solved in both precisions (batches: from 20,000 rows on).
+ * It takes memory that is to spare, after the solve's own, and goes back when
+ * an allocation of the library would otherwise fail. */
 int cel_gpu_pcg_solve(cel_gpu_mat* A, const double* b, double* x, const cel_pcg_params* params,
                       cel_pcg_stats* stats, double* hist);
 

@@ -92,3 +92,56 @@ p = C.c_void_p(1)
 out = [cel.lib().cel_gpu_malloc(C.byref(p), C.c_size_t((1 << 20) + {more})), p.value]
 """)
     assert (out[0] == 0 and out[1]) if not more else out == [-8, None]
+
+
+# A block of 820,911 rows: its derived diagonal storage takes 47 MB in FP64, 24 MB
+# in FP32; a solve on the CSR arrays needs 42 MB in FP64 (r, p, v, b, x in
+# pieces of 2 MB), 57 MB mixed (r, p, v, e, b, x and the FP32 values).
+@pytest.mark.parametrize("prec,spare", [("FP64", 44), ("FP64", 60), ("MIXED", 57)])
+def test_a_solve_has_its_memory_before_a_derived_form_has(stub, prec, spare):
+    out = stub(f"""
+S.stub_classes_fit(0)
+M = matrix(97, 93, 91)
+S.stub_budget(S.stub_used() + {spare} * 1000000)
+S.stub_log_clear()
+r = M.pcg(np.ones(M.n), precision=cel.PREC_{prec}, iter_max=40)
+out = [k for k, _ in launches("k_pcg_spmv")]
+S.stub_budget(1 << 34)
+S.stub_log_clear()
+N = matrix(97, 93, 91)
+N.pcg(np.ones(N.n), precision=cel.PREC_{prec}, iter_max=40)
+out = [out, [k for k, _ in launches("k_pcg_spmv")]]
+""")
+    vt = "double" if prec == "FP64" else "float"
+    assert len(out[0]) >= 40 and {k.split(",")[0] + k.split(",")[1] for k in out[0]} == {f"k_pcg_spmv<{vt} 1"}  # CSR
+    assert {k.split(",")[0] + k.split(",")[1] for k in out[1]} == {f"k_pcg_spmv<{vt} 4"}  # diagonals, with memory
+
+
+def test_derived_forms_go_back_when_memory_is_short(stub):
+    out = stub("""
+S.stub_classes_fit(0)
+M = matrix(97, 93, 91)
+kw = dict(iter_max=40)
+M.pcg(np.ones(M.n), fmt=cel.FMT_COO, **kw)
+plain = S.stub_used()                      # matrix and workspace
+M.pcg(np.ones(M.n), **kw)
+form = S.stub_used() - plain
+S.stub_budget(S.stub_used() + 1000000)
+a = cel.DeviceArray(5000000)               # 40 MB, which only the form can give
+short = S.stub_used()
+S.stub_log_clear()
+M.pcg(np.ones(M.n), **kw)                  # on the CSR arrays
+csr = sorted({k for k, _ in launches("k_pcg_spmv")})
+a.free()
+S.stub_budget(1 << 34)
+B = cel.Batch([M, matrix(31, 30, 29)])     # a batch's forms likewise
+B.solve([np.ones(m.n) for m in B.mats], iter_max=40)
+S.stub_budget(S.stub_used())
+p = C.c_void_p()
+rc = cel.lib().cel_gpu_malloc(C.byref(p), C.c_size_t(3000000))
+out = {"form": form, "short": short - plain - 40000000, "csr": csr, "rc": rc}
+""")
+    assert out["form"] > 45e6
+    assert out["short"] <= 2e6
+    assert len(out["csr"]) == 1 and out["csr"][0].startswith("k_pcg_spmv<double, 1")
+    assert out["rc"] == 0
