@@ -35,7 +35,6 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
-#include <initializer_list>
 #include <thread>
 #include <vector>
 
@@ -1748,16 +1747,13 @@ static int build_hrow_tile(const Mat& A, Workspace& W, int ntiles)
     return CEL_OK;
 }
 
-// Resident blocks of several kernels at once: the smallest, so every
-// variant that feeds the same consumer uses the same grid (and therefore
-// the same partials and the same sums).
 // Blocks per CU of the vector kernels (K2, K3).  Measured on the 256^3
 // solve: larger grids of these kernels, and K1 grids larger than the
 // resident blocks, were slower -- every consumer block sums all producer
 // partials, so more blocks cost more reduction work.
 constexpr int kVecBlocksPerCu = 4;
 
-// Blocks per CU of the K1s (at most the resident blocks).  Measured on the
+// Blocks per CU of the K1s.  Measured on the
 // 256^3 block (mean K1 time over 100-iteration solves, three interleaved
 // repetitions on one box): FP32 4 per CU (CSR 206-223 us, DIA 121-127 us,
 // against 223-230 / 136-145 us with every resident block), FP64 2 per CU
@@ -1765,23 +1761,28 @@ constexpr int kVecBlocksPerCu = 4;
 constexpr int kK1BlocksPerCuF32 = 4;
 constexpr int kK1BlocksPerCuF64 = 2;
 
-static int common_grid(std::initializer_list<const void*> kernels, long long work)
+// Blocks per CU of the residual kernels: the set-up's and the replacement's
+// sums are grouped by them.  As many as were resident when it was measured.
+constexpr int kResBlocksPerCu = 6;
+constexpr int kResBlocksPerCuJad = 7;
+
+// At most per_cu blocks per CU, a multiple of the XCDs.  A constant, not the
+// occupancy of the kernel: every dot product is grouped by its grid, and a
+// register more would otherwise change the last bits of every solve.
+static int fixed_grid(int per_cu, long long work)
 {
-    int g = 1 << 30;
-    for (const void* k : kernels) g = std::min(g, resident_grid(k, work));
-    return g;
+    const long long g = std::max(1LL, std::min((long long)rt().num_cus * per_cu, work));
+    return (int)(g >= kXcds ? g / kXcds * kXcds : g);
 }
 
-// The K1 grid: at most kK1BlocksPerCu* blocks per CU, a multiple of the XCDs.
-static int k1_cap(int G1, bool mixed)
+// The K1s' grid: the CSR and DIA forms share it, with and without halo, so
+// that their partials, and the solves, stay bitwise equal.
+static int k1_grid(long long ntiles, bool mixed)
 {
-    const int cap = rt().num_cus * (mixed ? kK1BlocksPerCuF32 : kK1BlocksPerCuF64);
-    if (G1 > cap) G1 = cap >= kXcds ? cap / kXcds * kXcds : cap;
-    return G1;
+    return fixed_grid(mixed ? kK1BlocksPerCuF32 : kK1BlocksPerCuF64, ntiles);
 }
 
-// The K1 of a form, and the grid the FP64 K1s of the CSR and DIA forms
-// share (so that their partials, and the solves, stay bitwise equal).
+// The K1 of a form.
 template <typename VT>
 using K1Fn = void (*)(MatView, const VT*, VT*, double*, ResArgs<VT>, const Ctrl*, Ctrl*, Prm);
 
@@ -1831,17 +1832,6 @@ static bool keep_matrix(const Mat& A, int fmt, int nd, bool mixed)
                                           : (4.0 + vb) * (double)A.nnz + 4.0 * n;
     // the vectors: FP64 x, r, p, v, b, Jacobi; mixed r, p, v, e, Jacobi and x
     return m + (mixed ? 28.0 : 48.0) * n <= kKeepBytes;
-}
-
-static int k1_grid_f64(long long ntiles)
-{
-    int g = 1 << 30;
-    for (const bool halo : {false, true}) {
-        for (const bool lr : {false, true})
-            g = std::min(g, resident_grid((const void*)k1_kernel<double>(CEL_FMT_CSR, halo, lr), ntiles));
-        g = std::min(g, resident_grid((const void*)k1_kernel<double>(CEL_FMT_DIA, halo, false), ntiles));
-    }
-    return g;
 }
 
 template <typename VT>
@@ -1967,7 +1957,7 @@ int pcg_spmv_dot(Mat& A, int fmt, const double* x, const double* ghost, double* 
     if (dot) *dot = 0.0;
     if (n == 0) return CEL_OK;
     const int ntiles = (n + kTileRows - 1) / kTileRows;
-    const int G1 = k1_cap(k1_grid_f64(ntiles), false);
+    const int G1 = k1_grid(ntiles, false);
     Workspace& W = ws_of(A);
     CEL_TRY(W.part1.reserve((size_t)G1));
     CEL_TRY(W.ctrl.reserve(5));
@@ -2106,28 +2096,14 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     }
 
     const int ntiles = std::max(1, (n + kTileRows - 1) / kTileRows);
-    // grids: K1 variants that must agree (with and without halo) share one
-    // grid; the residual kernels share one; K2 and K3 share one.
-    int G1, Gr, Gv;
-    // the DIA K1 runs on the CSR K1's grid (the same rows per block, so the
-    // same partial sums); the residual kernels of a DIA solve use the CSR form
+    // grids: K1 variants that must agree share one grid, and so do the
+    // residual kernels, and K2 and K3
+    const int G1 = k1_grid(ntiles, mixed);
+    const int Gr = fixed_grid(fmt == CEL_FMT_JAD ? kResBlocksPerCuJad : kResBlocksPerCu, ntiles);
+    int Gv;
+    // the residual kernels of a DIA solve use the CSR form
     const int rfmt = fmt == CEL_FMT_DIA ? CEL_FMT_CSR : fmt;
     const bool lr = csr_long_rows(A);
-    if (!mixed) {
-        if (fmt == CEL_FMT_JAD) G1 = resident_grid((const void*)k1_kernel<double>(fmt, false, false), ntiles);
-        else G1 = k1_grid_f64(ntiles);
-        Gr = common_grid({(const void*)res_kernel<double>(rfmt, false, lr),
-                          (const void*)res_kernel<double>(rfmt, rfmt == CEL_FMT_CSR, lr)}, ntiles);
-    } else {
-        G1 = fmt == CEL_FMT_JAD
-                 ? resident_grid((const void*)k1_kernel<float>(fmt, false, false), ntiles)
-                 : common_grid({(const void*)k1_kernel<float>(CEL_FMT_CSR, false, false),
-                                (const void*)k1_kernel<float>(CEL_FMT_CSR, false, true),
-                                (const void*)k1_kernel<float>(CEL_FMT_DIA, false, false),
-                                (const void*)k1_kernel<float>(CEL_FMT_DIA, false, true)}, ntiles);
-        Gr = resident_grid((const void*)res_kernel<float>(rfmt, false, lr), ntiles);
-    }
-    G1 = k1_cap(G1, mixed);
     {
         const long long units = ((long long)n + 2 * kBlock - 1) / (2 * kBlock);
         Gv = (int)std::min<long long>((long long)rt().num_cus * kVecBlocksPerCu,

@@ -145,3 +145,21 @@ out = {"form": form, "short": short - plain - 40000000, "csr": csr, "rc": rc}
     assert out["short"] <= 2e6
     assert len(out["csr"]) == 1 and out["csr"][0].startswith("k_pcg_spmv<double, 1")
     assert out["rc"] == 0
+
+
+def test_solve_grids_do_not_depend_on_occupancy(stub):
+    out = stub("""
+M = matrix(80, 80, 80)
+M.to_dia()
+out = []
+for per_cu in (8, 5, 1):
+    S.stub_occupancy(per_cu)
+    S.stub_log_clear()
+    for prec in (cel.PREC_FP64, cel.PREC_MIXED):
+        for fmt in (cel.FMT_CSR, cel.FMT_COO, cel.FMT_DIA):
+            M.pcg(np.ones(M.n), fmt=fmt, precision=prec, iter_max=3)
+    out.append([l for l in launches() if l[0].startswith(("k_residual", "k_pcg"))])
+""")
+    assert out[0] == out[1] == out[2]
+    # the residual: 6 blocks per CU; 2,000 tiles of 256 rows
+    assert {g for k, g in out[0] if k.startswith("k_residual<")} == {1536}
