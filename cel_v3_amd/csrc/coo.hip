@@ -192,15 +192,14 @@ k_starts(long long nnz, const int* __restrict__ head, const int* __restrict__ ih
 
 // Groups of at most kSmall entries: the rank of entry j is #{k : col_k <
 // col_j} + #{k < j : col_k == col_j}, i.e. the stable order by column, and
-// entry j goes to slot rank.  A workgroup takes 256 consecutive groups; when
-// their entries fit (kTileCap) the columns go to LDS, with each entry's
-// group beside it, and every thread ranks up to 8 entries, which it holds in
-// registers (neighbouring lanes compare within the same group, so their LDS
-// reads coincide; a thread per group with the entries staged in and out
-// of 66 KB of LDS took 331 us for the 14.6M entries of a 128^3 block, 118 us
-// so).  Otherwise each thread works on its group in global memory.  Longer
-// groups are left in place here and listed for k_group_medium (order of the
-// list is free: groups are independent).
+// entry j goes to slot rank.  A workgroup takes 256 consecutive groups, as
+// many at a time as have kTileCap entries: the columns go to LDS, with each
+// entry's group beside it, and every thread ranks up to 8 entries, which it
+// holds in registers (neighbouring lanes compare within the same group, so
+// their LDS reads coincide; a thread per group with the entries staged in
+// and out of 66 KB of LDS took 331 us for the 14.6M entries of a 128^3 block,
+// 118 us so).  Longer groups are left in place here and listed for
+// k_group_medium (order of the list is free: groups are independent).
 constexpr int kTileCap = 2048;
 constexpr int kPerThread = kTileCap / kThreads;
 
@@ -219,19 +218,27 @@ k_group_small(int G, const int* __restrict__ starts, const uint32_t* __restrict_
         const int ng = (int)min((long long)kThreads, G - g0);
         for (int i = tid; i <= ng; i += kThreads) st[i] = starts[g0 + i];
         __syncthreads();
-        const int base = st[0];
-        const int E = st[ng] - base;
-        const int g = (int)g0 + tid;
-        int s = 0, L = 0;
         if (tid < ng) {
-            s = st[tid] - base;
-            L = st[tid + 1] - st[tid];
+            const int L = st[tid + 1] - st[tid];
             if (L > kSmall) {
-                longer[atomicAdd(nlonger, 1)] = g;
+                longer[atomicAdd(nlonger, 1)] = (int)g0 + tid;
                 atomicMax(maxlen, L);
             }
         }
-        if (E <= kTileCap) {
+        // groups [a, b) at a time, as many as fit (uniform across the block)
+        for (int a = 0, b; a < ng; a = b) {
+            b = ng;
+            if (st[ng] - st[a] > kTileCap) {
+                int over = ng;  // [a, over) does not fit; [a, b) does, or is one group
+                b = a + 1;
+                while (over - b > 1) {
+                    const int mid = (b + over) / 2;
+                    if (st[mid] - st[a] > kTileCap) over = mid;
+                    else b = mid;
+                }
+            }
+            const int base = st[a], E = st[b] - base;
+            if (E > kTileCap) continue;  // a longer group
             Pay q[kPerThread];
             uint32_t row[kPerThread];
 #pragma unroll
@@ -244,8 +251,11 @@ k_group_small(int G, const int* __restrict__ starts, const uint32_t* __restrict_
             }
             // a longer group's entries keep their places (k_group_medium
             // rewrites it later): groups of one entry each
-            for (int j = 0; j < L; ++j)
-                grp[s + j] = L <= kSmall ? (uint32_t)s | ((uint32_t)L << 16) : (uint32_t)(s + j) | (1u << 16);
+            if (tid >= a && tid < b) {
+                const int s = st[tid] - base, L = st[tid + 1] - st[tid];
+                for (int j = 0; j < L; ++j)
+                    grp[s + j] = L <= kSmall ? (uint32_t)s | ((uint32_t)L << 16) : (uint32_t)(s + j) | (1u << 16);
+            }
 #pragma unroll
             for (int k = 0; k < kPerThread; ++k) {
                 const int i = tid + k * kThreads;
@@ -268,22 +278,9 @@ k_group_small(int G, const int* __restrict__ starts, const uint32_t* __restrict_
                     vals[base + r] = pay_val(q[k]);
                 }
             }
-        } else if (tid < ng && L <= kSmall) {
-            const int gs = base + s;
-            for (int j = 0; j < L; ++j) {
-                const uint32_t cj = pay[gs + j].col;
-                int r = 0;
-                for (int k = 0; k < L; ++k) {
-                    const uint32_t ck = pay[gs + k].col;
-                    r += ck < cj || (ck == cj && k < j);
-                }
-                const Pay q = pay[gs + j];
-                rows[gs + r] = (int)rk[gs + j] + rbase;
-                cols[gs + r] = (int)cj + cbase;
-                vals[gs + r] = pay_val(q);
-            }
+            __syncthreads();  // the tile is reused by the next groups
         }
-        __syncthreads();  // st and the tiles are reused by the next round
+        __syncthreads();  // st is reused by the next round
     }
 }
 
