@@ -25,6 +25,7 @@ struct State {
     int classes_fit = 1;    // whether k_class_scan finds few enough forms
     int stop_after = 0;     // the slot a solve stops in (0: never)
     int slots = 0;
+    int waits = 0;          // stream synchronisations
     dim3 grid, block;
     size_t shmem = 0;
     hipStream_t stream = nullptr;
@@ -115,6 +116,7 @@ void stub_stop_after(int slots)
     S().stop_after = slots;
     S().slots = 0;
 }
+int stub_waits() { return S().waits; }
 const char* stub_log() { return S().log.c_str(); }
 void stub_log_clear() { S().log.clear(); }
 
@@ -254,7 +256,11 @@ hipError_t hipStreamDestroy(hipStream_t s)
     std::free(s);
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    ++S().waits;
+    return hipSuccess;
+}
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
 {

@@ -163,3 +163,17 @@ for per_cu in (8, 5, 1):
     assert out[0] == out[1] == out[2]
     # the residual: 6 blocks per CU; 2,000 tiles of 256 rows
     assert {g for k, g in out[0] if k.startswith("k_residual<")} == {1536}
+
+
+def test_one_wait_serves_all_kept_blocks(stub):
+    out = stub("""
+M = matrix(4, 5, 6)
+x = np.ones(M.n)
+out = []
+for _ in range(3):                      # two device buffers a call, kept from the one before
+    before = S.stub_waits()
+    M.spmv(x)
+    out.append(S.stub_waits() - before)
+""")
+    # the end of the call, and one before the first kept block is used again
+    assert out == [1, 2, 2]
