@@ -285,6 +285,8 @@ static int mat_from_host(Mat& M, int n, int ncols, const std::vector<int>& xadj0
     M.n = n;
     M.ncols = ncols;
     M.nnz = nnz;
+    M.longest = 0;
+    for (int i = 0; i < n; ++i) M.longest = std::max(M.longest, xadj0[i + 1] - xadj0[i]);
     CEL_TRY(upload(M.xadj, xadj0.data(), (size_t)n + 1));
     CEL_TRY(upload(M.cols, cols0.data(), (size_t)nnz));
     CEL_TRY(upload(M.vals, vals, (size_t)nnz));
@@ -395,6 +397,7 @@ static int gen7(cel_gpu_mat** A, int nx, int ny, int nz, const double* kappa, in
     Mat& M = h->m;
     M.n = M.ncols = (int)n;
     M.nnz = (int)nnz;
+    M.longest = 7;
     int rc = M.xadj.alloc((size_t)n + 1);
     if (rc == CEL_OK) rc = M.cols.alloc((size_t)nnz);
     if (rc == CEL_OK) rc = M.vals.alloc((size_t)nnz);

@@ -250,7 +250,8 @@ struct Mat {
     std::vector<int> h_jad_begin;  // host copy (0-based starts, mmax+1)
 
     Derived derived;
-    int band = -1;  // largest |column - row| of the block (-1: not looked up)
+    int band = -1;     // largest |column - row| of the block (-1: not looked up)
+    int longest = -1;  // most entries of a row (-1: not looked up)
 
     // halo (distributed block split of one rank)
     std::vector<HaloBlock> halo;
@@ -332,6 +333,8 @@ int launch_dia_spmv_fused(const Mat& A, int fuse, long long chunk, int G, const 
 int dia_prepare_f32(Mat& A);
 // The largest |column - row| of a square block.
 int block_bandwidth(const Mat& A, int& bw);
+// The most entries of a row.
+int block_longest(const Mat& A, int& longest);
 // The derived form (Derived::k*) a PCG solve of at most iter_max iterations
 // runs on, built on the first call that wants it; never an error.  The caller
 // holds a DerivedUse of A and has made its own allocations.

@@ -750,8 +750,8 @@ struct StepStream<VT, CEL_FMT_CSR, LONG, KEEP> {
 // thread's part of v.d.  STEP: X is XDirection, and d and the updated x of
 // every row are stored as well.  (Taking a step's scalars behind the first
 // tile's gathers instead of before them measured slower, 32^3 12.7 against
-// 12.3 us per iteration.)  KEEP: keep_matrix().
-template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, bool KEEP, typename X>
+// 12.3 us per iteration.)  KEEP: keep_matrix(); TAIL: deep_rows().
+template <typename VT, int FMT, bool HALO, bool LONG, bool STEP, bool KEEP, int TAIL, typename X>
 __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __restrict__ v,
                                            StepStream<VT, FMT, LONG, KEEP>& first,
                                            typename StageOf<VT, FMT, LONG>::T& sm,
@@ -785,7 +785,7 @@ __device__ __forceinline__ double k1_tiles(const MatView& A, const X& x, VT* __r
         // record and read count 0.  Each loaded value is used once in the
         // step after it, in place: a copy of a register still being loaded
         // would wait for every load issued before it.
-        typename CsrStreamOf<VT, LONG, KEEP>::Stream own;
+        typename CsrStreamOf<VT, LONG, KEEP, TAIL>::Stream own;
         auto& cs = [&]() -> auto& {
             if constexpr (STEP && kOpenAhead<VT>) return first.cs;
             else return own;
@@ -1069,7 +1069,7 @@ constexpr int k1_waves = sizeof(VT) == 8 && (FMT == kFmtClass || FMT == CEL_FMT_
 // K1: v = A p, per-block partial of v.p.  Mixed: a requested replacement
 // residual takes the place of the product (K2 and K3 then do nothing, and
 // the next K1 folds its partials).  LONG of a DIA K1: its residual's.
-template <typename VT, int FMT, bool HALO, bool LONG, bool KEEP = false>
+template <typename VT, int FMT, bool HALO, bool LONG, bool KEEP = false, int TAIL = 1>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves<VT, FMT>, 8))) void k_pcg_spmv(MatView A, const VT* __restrict__ p,
                                                      VT* __restrict__ v, double* __restrict__ part,
                                                      ResArgs<VT> R,
@@ -1104,7 +1104,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves
         }
     }
     StepStream<VT, FMT, LONG, KEEP> none;
-    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP>(A, XPlain<VT>{p}, v, none, sm.tile, sm.wide, StepRows<VT>{}, walk);
+    const double acc = k1_tiles<VT, FMT, HALO, LONG, false, KEEP, TAIL>(A, XPlain<VT>{p}, v, none, sm.tile, sm.wide, StepRows<VT>{}, walk);
     const double bs = block_sum(acc, red);
     if (threadIdx.x == 0) part[slot] = bs;
     write_ctrl(cout, c);
@@ -1275,7 +1275,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(V
             }
         }
     } else {
-        acc = k1_tiles<VT, FMT, false, false, true, true>(A, d, v, first, sm.tile, sm.wide,
+        acc = k1_tiles<VT, FMT, false, false, true, true, 1>(A, d, v, first, sm.tile, sm.wide,
                                                           StepRows<VT>{pout, x, sigma, !pending});
     }
     const double bs = block_sum(acc, red);
@@ -1787,10 +1787,13 @@ template <typename VT>
 using K1Fn = void (*)(MatView, const VT*, VT*, double*, ResArgs<VT>, const Ctrl*, Ctrl*, Prm);
 
 // keep: the same kernel with ordinary loads of the matrix (keep_matrix); it
-// runs on the other one's grid.
+// runs on the other one's grid.  deep: deep_rows().
 template <typename VT>
-static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr, bool keep = false)
+static K1Fn<VT> k1_kernel(int fmt, bool halo, bool lr, bool keep = false, bool deep = false)
 {
+    if (deep)
+        return keep ? k_pcg_spmv<VT, CEL_FMT_CSR, false, false, true, kGather>
+                    : k_pcg_spmv<VT, CEL_FMT_CSR, false, false, false, kGather>;
     if (keep && !halo && fmt != kFmtClass) {
         if (fmt == CEL_FMT_JAD) return k_pcg_spmv<VT, CEL_FMT_JAD, false, false, true>;
         if constexpr (sizeof(VT) == 4)
@@ -1886,6 +1889,19 @@ static bool step_form(const Mat& A, int fmt, bool mixed)
 {
     return A.n <= (mixed ? 1200000 : 300000) && !csr_long_rows(A) && !(fmt == CEL_FMT_JAD && A.jad_mmax > kGather);
 }
+
+// Whether a CSR solve runs on the K1 that loads the entries of long rows
+// kGather at a time (and never on k_pcg_step, whose second gather they pay
+// for one after another): matrices of short rows, most of them, and a few
+// that one thread sums for longer than an iteration otherwise takes.
+// Measured per iteration, rows of 5 entries and 30 longer ones, without / so:
+// FP64 20,011 rows, longest of 26 17.6 / 17.0 us, of 74 42.6 / 22.5, of 522 239
+// / 80; mixed 26 23.2 / 22.1, 522 228 / 107; FP64 600,011 rows 25 33.1 / 31.9,
+// 521 276 / 102.  Loading them so in the kernels of every matrix costs those
+// without long rows 2 to 6% (registers): FP64 32^3 11.3 / 11.7 us, mixed 40^3
+// 12.2 / 12.8.
+constexpr int kDeepRow = 24;
+static bool deep_rows(const Mat& A) { return A.longest > kDeepRow && !csr_long_rows(A); }
 
 // The set-up kernel of a solve in the CSR or JAD form.
 template <typename OUT_T>
@@ -2221,10 +2237,20 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         }
     }
 
+    const std::string err = last_error();  // (what is tried and not had below is no error of the solve)
+    // the longest row: known from the start for matrices from host arrays and
+    // of the generators, otherwise looked up once
+    bool deep = false;
+    if (kfmt == CEL_FMT_CSR && !lr && !halo && !noalloc) {
+        if (A.longest < 0 && block_longest(A, A.longest) != CEL_OK) {
+            A.longest = -1;
+            set_error(err);
+        }
+        deep = deep_rows(A);
+    }
     // two kernels per iteration on small systems; the halo blocks need a
     // stored direction before the product, profiling a product of its own
-    bool step = !noalloc && !halo && !prm.profile && use == Derived::kNone && step_form(A, fmt, mixed);
-    const std::string err = last_error();  // (what is tried and not had below is no error of the solve)
+    bool step = !noalloc && !halo && !prm.profile && use == Derived::kNone && !deep && step_form(A, fmt, mixed);
     double *pbuf[2] = {w.p, nullptr}, *zbuf = nullptr;
     float *pbuf32[2] = {w.p32, nullptr}, *zbuf32 = nullptr;
     if (step) {
@@ -2441,7 +2467,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             CEL_HIP(hipEventRecord(ea, s));
         }
         if (!mixed) {
-            const auto k1 = !win ? k1_kernel<double>(kfmt, halo, lr, keep)
+            const auto k1 = !win ? k1_kernel<double>(kfmt, halo, lr, keep, deep)
                             : keep ? k_pcg_window<true> : k_pcg_window<false>;
             hipLaunchKernelGGL(k1, dim3(G1), dim3(kBlock), 0, s, V, w.p, w.v,
                                w.part1, R64, C0, C1, P);
@@ -2451,7 +2477,7 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
             hipLaunchKernelGGL(k3_kernel<double>(bycls, stream), dim3(Gv), dim3(kBlock), 0, s, n_ll, dx, w.p, w.r,
                                vjac64, vcls, nullptr, w.part2, Gv, C2, C0, P, progress);
         } else {
-            hipLaunchKernelGGL(k1_kernel<float>(kfmt, false, lr, keep), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
+            hipLaunchKernelGGL(k1_kernel<float>(kfmt, false, lr, keep, deep), dim3(G1), dim3(kBlock), 0, s, V, w.p32, w.v32,
                                w.part1, R32, C0, C1, P);
             if (profile) CEL_HIP(hipEventRecord(eb, s));
             hipLaunchKernelGGL(k2_kernel<float>(bycls, stream), dim3(Gv), dim3(kBlock), 0, s, n_ll, w.r32, w.v32,

@@ -577,17 +577,22 @@ int launch_kappa_grad(int nx, int ny, int nz, const double* kappa, const double*
     return CEL_OK;
 }
 
-// Bandwidth max |col - row| of a square block (0-based rows and columns):
-// per-block maxima, the host takes the largest.
-__global__ __launch_bounds__(kBlock) void k_bandwidth(int n, const int* __restrict__ xadj,
-                                                      const int* __restrict__ cols,
-                                                      int* __restrict__ out)
+// Bandwidth max |col - row| of a square block (0-based rows and columns), or
+// (without columns) the most entries of a row: per-block maxima, the host
+// takes the largest.
+__global__ __launch_bounds__(kBlock) void k_row_max(int n, const int* __restrict__ xadj,
+                                                    const int* __restrict__ cols,
+                                                    int* __restrict__ out)
 {
     __shared__ int wm[kWaves];
     int m = 0;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long long)gridDim.x * blockDim.x)
-        for (int k = xadj[i]; k < xadj[i + 1]; ++k) m = max(m, abs(cols[k] - (int)i));
+         i += (long long)gridDim.x * blockDim.x) {
+        if (cols)
+            for (int k = xadj[i]; k < xadj[i + 1]; ++k) m = max(m, abs(cols[k] - (int)i));
+        else
+            m = max(m, xadj[i + 1] - xadj[i]);
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
     if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
@@ -599,7 +604,7 @@ __global__ __launch_bounds__(kBlock) void k_bandwidth(int n, const int* __restri
     }
 }
 
-int block_bandwidth(const Mat& A, int& bw)
+static int row_max(const Mat& A, const int* cols, int& bw)
 {
     bw = 0;
     if (A.n == 0) return CEL_OK;
@@ -607,7 +612,7 @@ int block_bandwidth(const Mat& A, int& bw)
     DevBuf<int> part;
     CEL_TRY(part.alloc(kG));
     hipStream_t s = rt().stream;
-    hipLaunchKernelGGL(k_bandwidth, dim3(kG), dim3(kBlock), 0, s, A.n, A.xadj.p, A.cols.p, part.p);
+    hipLaunchKernelGGL(k_row_max, dim3(kG), dim3(kBlock), 0, s, A.n, A.xadj.p, cols, part.p);
     CEL_HIP(hipGetLastError());
     std::vector<int> h(kG);
     CEL_HIP(hipMemcpyAsync(h.data(), part.p, sizeof(int) * kG, hipMemcpyDeviceToHost, s));
@@ -615,6 +620,9 @@ int block_bandwidth(const Mat& A, int& bw)
     for (int v : h) bw = std::max(bw, v);
     return CEL_OK;
 }
+
+int block_bandwidth(const Mat& A, int& bw) { return row_max(A, A.cols.p, bw); }
+int block_longest(const Mat& A, int& longest) { return row_max(A, nullptr, longest); }
 
 double spmv_bytes(const Mat& A, int format, int precision)
 {

@@ -79,21 +79,32 @@ struct CsrStage {
     int col[kStageCap];
 };
 
-// sum + sum_{start <= j < len} a[j] * x[c[j]] in j order, one entry at a
-// time: the path of rows longer than kGather and of tiles larger than the
-// stage.  Kept lean on purpose -- its registers would count against the
-// occupancy of the common path.  LDS or global a/c (NT: non-temporal
-// global loads).
-template <typename AT, typename VT, bool NT, typename X>
+// sum + sum_{start <= j < len} a[j] * x[c[j]] in j order: the path of rows
+// longer than kGather and of tiles larger than the stage.  B entries' loads
+// are in flight together (those past the row repeat its last one).  B = 1,
+// lean, in the kernels of any matrix: the registers of more count against
+// the common path (32^3 iteration 11.3 us, with 8 entries 11.7).  LDS or
+// global a/c.
+template <int B, typename AT, typename VT, typename X>
 __device__ __forceinline__ AT row_sum_from(AT sum, const VT* a, const int* c, int start, int len,
                                            const X& x)
 {
 #pragma unroll 1
-    for (int j = start; j < len; ++j) {
-        const int col = NT ? ld_stream(c + j) : c[j];
-        const VT av = NT ? ld_stream(a + j) : a[j];
-        AT prod = AT(av) * AT(x.value(x.load(col)));
-        sum = sum + prod;
+    for (int j = start; j < len; j += B) {
+        VT av[B];
+        typename X::Raw xv[B];
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            const int k = min(j + i, len - 1);
+            av[i] = a[k];
+            xv[i] = x.load(c[k]);
+        }
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+            const AT prod = AT(av[i]) * AT(x.value(xv[i]));
+            const AT t = sum + prod;
+            sum = j + i < len ? t : sum;
+        }
     }
     return sum;
 }
@@ -480,7 +491,7 @@ struct NoLoads {
 // as its entries, the tile's loads had to wait for the gathers issued before
 // them, which put one L2 round trip and one HBM round trip in series on
 // every step.)
-template <typename VT, bool KEEP = false>
+template <typename VT, bool KEEP = false, int TAIL = 1>
 struct CsrTileStream {
     static constexpr int EV = 16 / (int)sizeof(VT);  // values per 16-byte load
     VT v[kPer];
@@ -670,7 +681,7 @@ struct CsrTileStream {
         if (j0 < len) {
             const VT* av = staged ? (const VT*)(sm.val + l) : vals + b0 + l;
             const int* cv = staged ? (const int*)(sm.col + l) : cols + b0 + l;
-            sum = row_sum_from<AT, VT, false>(sum, av, cv, j0, len, x);
+            sum = row_sum_from<TAIL, AT, VT>(sum, av, cv, j0, len, x);
         }
         return sum;
     }
@@ -846,14 +857,14 @@ struct CsrLongStream {
     }
 };
 
-// The tile stream of a CSR kernel and its LDS stage.
-template <typename VT, bool LONG, bool KEEP = false>
+// The tile stream of a CSR kernel and its LDS stage.  TAIL: row_sum_from's B.
+template <typename VT, bool LONG, bool KEEP = false, int TAIL = 1>
 struct CsrStreamOf {
-    using Stream = CsrTileStream<VT, KEEP>;
+    using Stream = CsrTileStream<VT, KEEP, TAIL>;
     using Stage = CsrStage<VT>;
 };
-template <typename VT, bool KEEP>
-struct CsrStreamOf<VT, true, KEEP> {
+template <typename VT, bool KEEP, int TAIL>
+struct CsrStreamOf<VT, true, KEEP, TAIL> {
     using Stream = CsrLongStream<VT, KEEP>;
     using Stage = CsrLongStage<VT>;
 };

@@ -177,3 +177,23 @@ for _ in range(3):                      # two device buffers a call, kept from t
 """)
     # the end of the call, and one before the first kept block is used again
     assert out == [1, 2, 2]
+
+
+@pytest.mark.parametrize("longest,deep", [(8, False), (24, False), (25, True), (3000, True)])
+def test_matrices_with_a_few_long_rows(stub, longest, deep):
+    out = stub(f"""
+n = 30011
+count = np.full(n, 5)
+count[n // 2] = {longest}
+cols = np.concatenate([np.sort((i + np.arange(c) - c // 2) % n) for i, c in enumerate(count)])
+xadj = np.concatenate([[0], np.cumsum(count)])
+M = cel.Matrix.from_csr(xadj, cols, np.ones(cols.size), index_base=0)
+M.set_jacobi()
+out = []
+for prec in (cel.PREC_FP64, cel.PREC_MIXED):
+    S.stub_log_clear()
+    M.pcg(np.ones(n), precision=prec, iter_max=3)
+    out.append(sorted({{k for k, _ in launches() if k.startswith(("k_pcg_spmv", "k_pcg_step"))}}))
+""")
+    for vt, got in zip(("double", "float"), out):
+        assert got == [f"k_pcg_spmv<{vt}, 1, false, false, true, 8>" if deep else f"k_pcg_step<{vt}, 1, true>"]
