@@ -22,9 +22,10 @@
 // entry by entry against the matrix (the 64-bit keys only find candidates).
 // They are built on the first long solve of a matrix (rule at
 // derived_prepare), belong to the handle, and are dropped when the values,
-// the Jacobi vector or the scaling change.  A matrix they do not fit costs
-// one pass that stops early; without memory for them the solve runs on the
-// CSR arrays.  The memory they take is returned when another allocation needs
+// the Jacobi vector or the scaling change.  A matrix off the diagonals costs a
+// pass over its columns that stops early, one of too many forms that pass and
+// a look at 1,024 rows; without memory for them the solve runs on the CSR
+// arrays.  The memory they take is returned when another allocation needs
 // it (device_malloc) and no solve is reading them.
 #include <algorithm>
 #include <mutex>
@@ -55,6 +56,7 @@ struct Offs {
     int off[kClassDiag];
 };
 
+// The finaliser of SplitMix64 (Steele, Lea, Flood 2014).
 __device__ __forceinline__ unsigned long long mix(unsigned long long h)
 {
     h ^= h >> 30;
@@ -115,19 +117,25 @@ __global__ void __launch_bounds__(kBlock) k_keys_clear(KeyTable* T)
     if (threadIdx.x == 0) T->count = T->over = T->bad = 0;
 }
 
-// Classes of the rows: one thread per row puts its key into the table
-// unless the block has met it before.  Bound by one read of the matrix; it
-// stops as soon as there are too many classes.
+// Classes of the rows 0, step, 2 step, ...: one thread per row puts its key
+// into the table unless the block has met it before.  Bound by one read of
+// the matrix; it stops as soon as there are too many classes.  (Every
+// resident block has put rows into the table before the first of them can
+// see that: 254 us on 128^3, 814 us on 256^3.  Hence the sample, a row per
+// thread of a few blocks, ahead of the whole block: the first solve of a
+// matrix with variable coefficients takes 207 us more than the next one at
+// 857,000 rows, 351 us at 128^3, 403 and 589 us without.)
+constexpr int kSample = 1024;
 __global__ void __launch_bounds__(kBlock)
-k_class_scan(int n, const int* __restrict__ xadj, const int* __restrict__ cols,
+k_class_scan(int n, long long step, const int* __restrict__ xadj, const int* __restrict__ cols,
              const double* __restrict__ vals, const double* __restrict__ jac, Offs O, KeyTable* T)
 {
     __shared__ unsigned long long near_key[kNear];
     __shared__ int stop;
     for (int i = threadIdx.x; i < kNear; i += kBlock) near_key[i] = 0;
     __syncthreads();
-    for (long long i0 = (long long)blockIdx.x * kBlock; i0 < n; i0 += (long long)gridDim.x * kBlock) {
-        const long long i = i0 + threadIdx.x;
+    for (long long i0 = (long long)blockIdx.x * kBlock; i0 * step < n; i0 += (long long)gridDim.x * kBlock) {
+        const long long i = (i0 + threadIdx.x) * step;
         if (i < n) {
             RowForm f;
             if (!row_form(i, xadj, cols, vals, jac[i], O, f)) {
@@ -288,13 +296,17 @@ int build_classes(Mat& A, const Offs& O, bool* ok)
     DevBuf<KeyTable> T;
     CEL_TRY(T.alloc(1));
     hipLaunchKernelGGL(k_keys_clear, dim3(1), dim3(kBlock), 0, st, T.p);
-    hipLaunchKernelGGL(k_class_scan, dim3(grid_of(A.n)), dim3(kBlock), 0, st, A.n, A.xadj.p, A.cols.p, A.vals.p,
-                       A.jac.p, O, T.p);
-    CEL_HIP(hipGetLastError());
     int h[3];
-    CEL_HIP(hipMemcpyAsync(h, &T.p->count, sizeof(h), hipMemcpyDeviceToHost, st));
-    CEL_HIP(hipStreamSynchronize(st));
-    if (h[1] || h[0] > kMaxClass) return CEL_OK;
+    const long long sample = std::max(1LL, (long long)A.n / kSample);
+    for (const long long step : {sample, 1LL}) {
+        const long long rows = (A.n + step - 1) / step;
+        hipLaunchKernelGGL(k_class_scan, dim3(grid_of(rows)), dim3(kBlock), 0, st, A.n, step, A.xadj.p, A.cols.p,
+                           A.vals.p, A.jac.p, O, T.p);
+        CEL_HIP(hipGetLastError());
+        CEL_HIP(hipMemcpyAsync(h, &T.p->count, sizeof(h), hipMemcpyDeviceToHost, st));
+        CEL_HIP(hipStreamSynchronize(st));
+        if (h[1] || h[0] > kMaxClass) return CEL_OK;
+    }
     CEL_TRY(D.cls.alloc((size_t)A.n, true));
     CEL_TRY(D.tab64.alloc((size_t)kMaxClass * (kClassDiag + 1), true));
     CEL_TRY(D.tab32.alloc((size_t)kMaxClass * (kClassDiag + 1), true));
@@ -429,9 +441,14 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric)
     // iteration, CSR arrays / classes / diagonal storage: 64^3 FP64 17.2 /
     // 17.0 / 17.1 us; 80^3 29.1 / 25.4 / 27.8, mixed 22.9 / 22.0 / 21.4;
     // 100^3 39.6 / 26.5 / 30.7, mixed 31.8 / 22.5 / 28.4; 256^3 618 / 240 /
-    // 411, mixed 358 / 127 / 232 (FP64 diagonals of 100^3 and 256^3 symmetric).  Building takes 0.4 ms (100^3) to 1.3 ms
-    // (256^3), as much as 40 to 10 iterations save; a solve of such a block
-    // to 1e-10 takes 300 to 800.
+    // 411, mixed 358 / 127 / 232 (FP64 diagonals of 100^3 and 256^3
+    // symmetric).  Building (a first solve less the next one): classes 0.21 ms
+    // at 857,000 rows, 0.30 at 128^3, 0.8 at 200^3, 1.6 at 256^3, diagonals
+    // 0.21, 0.35, 1.1, 1.7: what 5 (256^3) to 25 iterations save, in the mixed
+    // form at 80^3 200.  (FP64 classes would pay there after 60.)  The
+    // solve's length is not known here, only iter_max: one that stops after
+    // 10 iterations has paid for more than it saved (128^3 Poisson FP64 0.93
+    // ms, the next one 0.60).
     if (A.n < kDerivedRows || (iter_max < 32 && !D.tried) || !A.jac.p || !A.jac32.p) return Derived::kNone;
     const std::string err = last_error();
     int rc = CEL_OK;

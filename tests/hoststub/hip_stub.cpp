@@ -89,7 +89,7 @@ void imitate(const std::string& k, void** a)
                 g->slot[g->count++] = cols[j] - i;
             }
     } else if (k == "k_class_scan") {
-        if (!S().classes_fit) arg<KeyTable*>(a, 6)->over = 1;
+        arg<KeyTable*>(a, 7)->over = !S().classes_fit;
     } else if (k.rfind("k_pcg_update_xp<", 0) == 0 || k.rfind("k_pcg_update_r<", 0) == 0) {
         int* progress = arg<int*>(a, k[13] == 'x' ? 12 : 11);
         if (!progress) return;

@@ -197,3 +197,17 @@ for prec in (cel.PREC_FP64, cel.PREC_MIXED):
 """)
     for vt, got in zip(("double", "float"), out):
         assert got == [f"k_pcg_spmv<{vt}, 1, false, false, true, 8>" if deep else f"k_pcg_step<{vt}, 1, true>"]
+
+
+def test_a_block_without_row_classes_is_not_scanned_whole(stub):
+    out = stub("""
+out = []
+for fit in (0, 1):
+    S.stub_classes_fit(fit)
+    M = matrix(97, 93, 91)
+    S.stub_log_clear()
+    M.pcg(np.ones(M.n), iter_max=40)
+    out.append([g for _, g in launches("k_class_scan")])
+""")
+    assert out[0] == [5]          # 1,025 rows, spread over the block
+    assert out[1] == [5, 3207]    # then all 820,911
