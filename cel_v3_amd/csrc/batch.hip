@@ -1127,16 +1127,15 @@ static int upload_table(Batch& B, const std::vector<BBlk>& tbl, const std::vecto
     return CEL_OK;
 }
 
-// The forms this solve's K1 reads the matrices in (its own CSR arrays / the
-// derived form, whole solves): 64 systems of 24^3..96^3 129.7 / 103.2 ms, 16
+// The forms the solve's K1 reads the matrices in: those that are built (its
+// own CSR arrays / the derived form, whole solves): 64 systems of 24^3..96^3 129.7 / 103.2 ms, 16
 // of 60^3..90^3 72.7 / 57.3, 4 of 100^3..110^3 64.0 / 50.6, 8 of 20^3..40^3
 // 4.00 / 3.74; 16 right-hand sides on 128^3 251 / 244, 11 on 91^3 73.0 /
 // 70.5.
-static void choose_forms(Batch& B, int iter_max)
+static void choose_forms(Batch& B)
 {
     const size_t S = B.mats.size();
     B.h_form.assign(S, BForm{});
-    derived_prepare_all(B.mats, iter_max);
     for (size_t q = 0; q < S; ++q) {
         const Mat& A = *B.mats[q];
         const Derived& D = A.derived;
@@ -1162,9 +1161,8 @@ struct RunResult {
 };
 
 // One batched solve with tuning T from the current x (x0 already in B.x).
-// form_iters: the iterations the choice of the matrices' forms reckons with (a
-// tuning sample is short, the solves it is for are not).
-static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int iter_cap, int form_iters,
+// sample: a tuning sample, on the forms that the solves it is for will find.
+static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int iter_cap, bool sample,
                      RunResult& out)
 {
     hipStream_t s = rt().stream;
@@ -1178,7 +1176,9 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     CEL_TRY(B.d_form.alloc(S));
     std::vector<DerivedUse> reading(S);
     for (int q = 0; q < S; ++q) reading[q].begin(B.mats[q]->derived);
-    choose_forms(B, form_iters);
+    derived_prepare_all(B.mats, sample ? 1 << 20 : prm.iter_max, sample);
+    choose_forms(B);
+    bool build = !sample;
     std::vector<char> active(S, 1);
     std::vector<BBlk> tbl, tbl2;
     CEL_TRY(build_table(B, G, T.weight, active, tbl, false));
@@ -1263,6 +1263,20 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
                     if (prev[B.lane0[q] + l].run) act[q] = 1;
             for (int q = 0; q < S; ++q) nrun += act[q];
             if (nrun == 0) break;
+            // the forms of small matrices that are not there yet, now that the
+            // solve goes on
+            if (build) {
+                build = false;
+                std::vector<Mat*> on;
+                for (int q = 0; q < S; ++q)
+                    if (act[q]) on.push_back(B.mats[q]);
+                if (derived_prepare_all(on, prm.iter_max, true)) {
+                    CEL_HIP(hipEventSynchronize(cev[k & 1]));  // the chunk in flight reads the table of forms
+                    choose_forms(B);
+                    rc = upload_table(B, tbl, tbl2, s);
+                    if (rc < 0) break;
+                }
+            }
             if (T.rebalance && act != active) {
                 // every lane of a dropped system has stored its final token
                 // in slot 0; the chunk in flight does not touch it again
@@ -1500,7 +1514,7 @@ extern "C" int cel_gpu_batch_tune(cel_gpu_batch* h, const double* const* b, int 
         RunResult rr;
         // the sample is a whole number of chunks
         const int cap = std::max(T.chunk, (iters + T.chunk - 1) / T.chunk * T.chunk) - 1;
-        CEL_TRY(run_batch(B, T, prm, cap, 1 << 20, rr));
+        CEL_TRY(run_batch(B, T, prm, cap, true, rr));
         int it = 0;
         for (const BCtrl& c : rr.lanes) it = std::max(it, c.iter);
         const double per = rr.ms / std::max(1, it);
@@ -1529,7 +1543,7 @@ extern "C" int cel_gpu_batch_solve(cel_gpu_batch* h, const double* const* b, dou
     CEL_TRY(load_rhs(B, b, prm.memspace));
     CEL_TRY(init_x(B, x, prm));
     RunResult rr;
-    CEL_TRY(run_batch(B, B.tune, prm, prm.iter_max, prm.iter_max, rr));
+    CEL_TRY(run_batch(B, B.tune, prm, prm.iter_max, false, rr));
     hipStream_t s = rt().stream;
     DevBuf<double> tmp;
     for (size_t q = 0; q < B.mats.size(); ++q) {

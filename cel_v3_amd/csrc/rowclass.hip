@@ -518,28 +518,41 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric)
 
 // The matrices of a batch are read by one K1 per iteration however small each
 // of them is, so those below kDerivedRows get diagonal storage too, built
-// with two synchronisations for all of them.  A matrix costs about 22 us;
-// the first solve saves that from about 10,000 rows on (2.2 ns a row in 200
-// iterations).
+// with two synchronisations for all of them.  One costs about 33 us of
+// kernels and its allocations, and saves 2.2 ns a row in 200 iterations.  So
+// the small ones (below kBatchAhead) are built when the solve is found to go
+// on after its first chunk; ahead of it they cost batches that stop there
+// more than they save.  First solves, without forms / built ahead / so, and
+// the later ones: 8 systems of 28^3..40^3 2 iterations 1.32 / 1.60 / 1.29 ms
+// (1.25), 162 iterations 5.2 / 4.6 / 4.8 (4.3); 2 of 28^3 and 30^3 123
+// iterations 2.50 / 2.47 / 2.54 (2.39).  Larger ones pay at once: 4 of
+// 60^3..70^3 2 iterations 3.0 without / 1.95, 272 iterations 15.6 / 11.1 (built
+// after the first chunk 11.7).
 constexpr int kBatchRows = 20000;
-void derived_prepare_all(const std::vector<Mat*>& mats, int iter_max)
+constexpr int kBatchAhead = 100000;
+bool derived_prepare_all(const std::vector<Mat*>& mats, int iter_max, bool small)
 {
+    bool any = false;
     const std::string err = last_error();
     std::vector<Mat*> todo;
     for (Mat* A : mats) {
         bool sym;
-        if (A->n >= kDerivedRows) (void)derived_prepare(*A, CEL_FMT_CSR, false, iter_max, &sym);
-        else if (A->n >= kBatchRows && iter_max >= 32 && !A->derived.tried64 && A->nnz > 0 && A->ncols == A->n) {
+        if (A->n >= kDerivedRows) {
+            any |= iter_max >= 32 && (!A->derived.tried || (A->derived.kind == Derived::kNone && !A->derived.tried64));
+            (void)derived_prepare(*A, CEL_FMT_CSR, false, iter_max, &sym);
+        } else if (A->n >= (small ? kBatchRows : kBatchAhead) && iter_max >= 32 && !A->derived.tried64 && A->nnz > 0 &&
+                   A->ncols == A->n) {
             A->derived.tried64 = true;  // (a matrix may be in the batch twice)
             todo.push_back(A);
         }
     }
+    if (todo.empty()) return any;
     std::vector<DiagonalSet> sets;
     int rc = dia_offsets_all(todo, kClassDiag, sets);
     hipStream_t st = rt().stream;
     DevBuf<int> bad;
-    if (rc == CEL_OK && !todo.empty()) rc = bad.alloc(todo.size());
-    if (rc == CEL_OK && !todo.empty() && hipMemsetAsync(bad.p, 0, sizeof(int) * todo.size(), st) != hipSuccess)
+    if (rc == CEL_OK) rc = bad.alloc(todo.size());
+    if (rc == CEL_OK && hipMemsetAsync(bad.p, 0, sizeof(int) * todo.size(), st) != hipSuccess)
         rc = CEL_ERR_HIP;
     std::vector<char> built(todo.size(), 0);
     for (size_t q = 0; q < todo.size() && rc == CEL_OK; ++q) {
@@ -558,7 +571,7 @@ void derived_prepare_all(const std::vector<Mat*>& mats, int iter_max)
         built[q] = 1;
     }
     std::vector<int> h(todo.size(), 1);
-    if (!todo.empty() && bad.p) {
+    if (bad.p) {
         const bool ok = hipGetLastError() == hipSuccess &&
                         hipMemcpyAsync(h.data(), bad.p, sizeof(int) * h.size(), hipMemcpyDeviceToHost, st) == hipSuccess &&
                         hipStreamSynchronize(st) == hipSuccess;
@@ -578,6 +591,7 @@ void derived_prepare_all(const std::vector<Mat*>& mats, int iter_max)
         set_error(err);
         (void)hipGetLastError();
     }
+    return true;
 }
 
 }  // namespace cel

@@ -211,3 +211,13 @@ for fit in (0, 1):
 """)
     assert out[0] == [5]          # 1,025 rows, spread over the block
     assert out[1] == [5, 3207]    # then all 820,911
+
+
+def test_a_batch_that_stops_early_builds_no_forms_of_small_matrices(stub):
+    out = stub("""
+B = cel.Batch([matrix(30, 31, 32), matrix(45, 46, 47)])
+S.stub_log_clear()
+B.solve([np.ones(m.n) for m in B.mats], iter_max=1000)   # (every lane is found stopped at the first look)
+out = [k for k, _ in launches() if "scan" in k or "fill<" in k]
+""")
+    assert out == []
