@@ -25,7 +25,8 @@
 // a kernel that needs a dot product sums the predecessor's per-block
 // partials itself, in every block, in the same fixed order.  All blocks
 // therefore hold bit-identical scalars, the sums do not depend on which
-// block finished first, and the host never waits inside the loop.  A
+// block finished first, and the device never waits for the host, which
+// stays a few iterations ahead by a progress word in its own memory.  A
 // stopped token is forwarded unchanged, so a captured chunk of iterations
 // can be replayed as a hipGraph and runs past convergence as no-ops.
 //
@@ -1699,10 +1700,14 @@ struct Workspace {
 
 // Waits until the solve's kernels have finished `upto` slots (1), or stopped
 // (0), or there is an error (< 0).  The word is in host memory, so looking
-// at it costs the stream nothing.
+// at it costs the stream nothing.  It looks without a pause for 100 us, the
+// slots of a small system (yielding from the first look on cost 32^3 0.25 us
+// per iteration of 11.2); after that it gives the core to any other thread
+// that wants it, every time round.
 static int wait_progress(hipStream_t s, const volatile int* progress, long long upto)
 {
-    auto last = std::chrono::steady_clock::now();
+    const auto begin = std::chrono::steady_clock::now();
+    auto last = begin;
     for (;;) {
         for (int k = 0; k < 512; ++k) {
             const int v = *progress;
@@ -1711,13 +1716,11 @@ static int wait_progress(hipStream_t s, const volatile int* progress, long long 
             __builtin_ia32_pause();
         }
         const auto now = std::chrono::steady_clock::now();
+        if (now - begin > std::chrono::microseconds(100)) std::this_thread::yield();
         if (now - last < std::chrono::milliseconds(1)) continue;
         last = now;
         const hipError_t e = hipStreamQuery(s);
-        if (e == hipErrorNotReady) {
-            std::this_thread::yield();
-            continue;
-        }
+        if (e == hipErrorNotReady) continue;
         if (e != hipSuccess) return fail(CEL_ERR_HIP, std::string("the solve's kernels: ") + hipGetErrorString(e));
         return *progress < 0 ? 0 : 1;  // everything enqueued has run
     }
@@ -2497,12 +2500,13 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     // iterations); replayed graphs go chunk by chunk, one chunk ahead.  The
     // allocation-free solve, which has no host memory, reads the token after
     // every chunk.
-    const int chunk = prm.check_every > 0 ? prm.check_every : 16;
-    const long long ahead = std::min(std::max(chunk, 2), 8);
+    const bool use_graph = prm.use_graph && !prm.profile && !noalloc;
+    long long chunk = prm.check_every > 0 ? prm.check_every : 16;
+    const long long ahead = std::min(std::max(chunk, 2LL), 8LL);
+    // a captured chunk of the two-kernel form starts at an even slot
+    if (use_graph && step && (chunk & 1)) chunk *= 2;
     int hrun_sync = 1;
 
-    // (a captured chunk of the two-kernel form starts at an even slot)
-    const bool use_graph = prm.use_graph && !prm.profile && !noalloc && !(step && (chunk & 1));
     int status = CEL_OK;
     // mixed: a replacement takes a slot, or two (the request of the two-kernel
     // form), and there is at most one per iteration

@@ -92,8 +92,14 @@ typedef struct {
     double ru_delta;   /* mixed: replace the FP32 residual by the FP64 one when it
                           has dropped by this factor (default 0.1) */
     int ru_restart;    /* mixed: 1 also restarts p (classic iterative refinement) */
-    int check_every;   /* iterations per host poll of the device state (default 16) */
-    int use_graph;     /* 1: replay one captured chunk of iterations as a hipGraph */
+    int check_every;   /* how far the host runs ahead of the device (default 16): with use_graph
+                          the iterations of the captured chunk (twice an odd number on small
+                          systems), one chunk ahead; in cel_gpu_pcg_solve_noalloc the iterations
+                          between two reads of the device state; otherwise 2 to 8 iterations
+                          (values above 8 mean 8).  The results do not depend on it.  Meanwhile
+                          the calling thread polls, and yields its core while an iteration takes
+                          long */
+    int use_graph;     /* 1: replay a captured chunk of iterations as a hipGraph */
     int profile;       /* 1: time every SpMV launch with HIP events (stats) */
     int alpha_stop;    /* 1 (reference): also stop when |alpha| <= 1.1 eps_mach, an absolute
                           test (cel_cgalg_module.f90:248); 0: only the norm test */

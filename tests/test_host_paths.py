@@ -221,3 +221,21 @@ B.solve([np.ones(m.n) for m in B.mats], iter_max=1000)   # (every lane is found 
 out = [k for k, _ in launches() if "scan" in k or "fill<" in k]
 """)
     assert out == []
+
+
+@pytest.mark.parametrize("prec", ["FP64", "MIXED"])
+@pytest.mark.parametrize("every", [1, 3, 4, 16, 17])
+def test_graph_solves_replay_a_graph(stub, every, prec):
+    out = stub(f"""
+M = matrix(12, 13, 14)
+S.stub_log_clear()
+M.pcg(np.ones(M.n), iter_max=99, use_graph=1, check_every={every}, precision=cel.PREC_{prec})
+log = S.stub_log().decode().splitlines()
+at = log.index("capture")
+end = log.index("graph")
+out = [sum("k_pcg_step" in l for l in log[at:end]), log.count("graph"),
+       sum("k_pcg_step" in l for l in log[:at] + log[end:])]
+""")
+    steps = every if every % 2 == 0 else 2 * every   # an even chunk of the two-kernel form
+    slots = 100 * (3 if prec == "MIXED" else 1)
+    assert out == [steps, slots // steps, slots % steps]
