@@ -2252,8 +2252,10 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
         deep = deep_rows(A);
     }
     // two kernels per iteration on small systems; the halo blocks need a
-    // stored direction before the product, profiling a product of its own
-    bool step = !noalloc && !halo && !prm.profile && use == Derived::kNone && !deep && step_form(A, fmt, mixed);
+    // stored direction before the product, profiling a product of its own (and
+    // symmetric diagonals the wide walk, which a step does not have)
+    bool step = !noalloc && !halo && !prm.profile && use == Derived::kNone && !symmetric && !deep &&
+                step_form(A, fmt, mixed);
     double *pbuf[2] = {w.p, nullptr}, *zbuf = nullptr;
     float *pbuf32[2] = {w.p32, nullptr}, *zbuf32 = nullptr;
     if (step) {

@@ -239,3 +239,19 @@ out = [sum("k_pcg_step" in l for l in log[at:end]), log.count("graph"),
     steps = every if every % 2 == 0 else 2 * every   # an even chunk of the two-kernel form
     slots = 100 * (3 if prec == "MIXED" else 1)
     assert out == [steps, slots // steps, slots % steps]
+
+
+@pytest.mark.parametrize("shape,symmetric", [((94, 93, 92), False), ((97, 96, 95), True), ((106, 105, 106), True)])
+def test_mixed_solves_in_the_callers_diagonal_storage(stub, shape, symmetric):
+    out = stub(f"""
+M = matrix(*{shape})
+M.to_dia()
+S.stub_classes_fit(0)
+S.stub_log_clear()
+r = M.pcg(np.ones(M.n), fmt=cel.FMT_DIA, precision=cel.PREC_MIXED, iter_max=40)
+ks = {{k.split("<")[0] for k, _ in launches()}}
+out = ["k_dia_symmetric" in ks, "k_pcg_step" in ks, "k_pcg_spmv" in ks, r["spmv_bytes"] / M.n]
+""")
+    # checked, two kernels, the wide walk, bytes a row (4 of 7 arrays, or all and the product's own)
+    assert out[:3] == [symmetric, not symmetric, symmetric]
+    assert out[3] == 25.0 if symmetric else out[3] >= 37.0
