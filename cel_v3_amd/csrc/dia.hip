@@ -117,6 +117,33 @@ k_offset_scan(int n, const int* __restrict__ xadj, const int* __restrict__ cols,
     }
 }
 
+// For the refusal of a block with too many diagonals: which offsets it has, as
+// bits (offset + n - 1), and whether a row's columns do not strictly ascend
+// (k_offset_scan stops before it has seen every row).
+__global__ void __launch_bounds__(kBlock)
+k_offset_bits(int n, const int* __restrict__ xadj, const int* __restrict__ cols, unsigned* bits, int* bad)
+{
+    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock) {
+        int prev = -1;
+        for (int j = xadj[i]; j < xadj[i + 1]; ++j) {
+            const int c = cols[j];
+            if (c <= prev) *(volatile int*)bad = 1;
+            prev = c;
+            const long long at = c - i + n - 1;
+            if (at < 0 || at >= 2LL * n - 1) continue;
+            const unsigned bit = 1u << (at & 31);
+            if (!(*(volatile unsigned*)&bits[at >> 5] & bit)) atomicOr(&bits[at >> 5], bit);
+        }
+    }
+}
+__global__ void __launch_bounds__(kBlock) k_count_bits(long long words, const unsigned* __restrict__ bits, int* sum)
+{
+    int c = 0;
+    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < words; i += (long long)gridDim.x * kBlock)
+        c += __popc(bits[i]);
+    if (c) atomicAdd(sum, c);
+}
+
 struct Offsets {
     int nd;
     int off[kMaxDiag];
@@ -335,6 +362,29 @@ int dia_offsets(const Mat& A, int most, int* nd, int* off, bool* ascending)
     return CEL_OK;
 }
 
+// The number of distinct offsets of a block, and whether every row's columns
+// strictly ascend.
+static int offset_count(const Mat& A, int* nd, bool* ascending)
+{
+    hipStream_t st = rt().stream;
+    const long long words = (2LL * A.n + 30) / 32;
+    DevBuf<unsigned> bits;
+    DevBuf<int> out;
+    CEL_TRY(bits.alloc((size_t)words));
+    CEL_TRY(out.alloc(2));
+    CEL_HIP(hipMemsetAsync(bits.p, 0, sizeof(unsigned) * (size_t)words, st));
+    CEL_HIP(hipMemsetAsync(out.p, 0, sizeof(int) * 2, st));
+    hipLaunchKernelGGL(k_offset_bits, dim3(grid_of(A.n)), dim3(kBlock), 0, st, A.n, A.xadj.p, A.cols.p, bits.p, out.p);
+    hipLaunchKernelGGL(k_count_bits, dim3(grid_of(words)), dim3(kBlock), 0, st, words, bits.p, out.p + 1);
+    CEL_HIP(hipGetLastError());
+    int h[2];
+    CEL_HIP(hipMemcpyAsync(h, out.p, sizeof(h), hipMemcpyDeviceToHost, st));
+    CEL_HIP(hipStreamSynchronize(st));
+    *ascending = !h[0];
+    *nd = h[1];
+    return CEL_OK;
+}
+
 int dia_fill(const Mat& A, int nd, const int* off, double* v64, float* v32, uint8_t* mask8)
 {
     Offsets O{};
@@ -387,9 +437,10 @@ extern "C" int cel_gpu_mat_to_dia(cel_gpu_mat* A)
     int nd = 0, hoff[kMaxDiag] = {};
     bool ascending = false;
     CEL_TRY(dia_offsets(M, kMaxDiag, &nd, hoff, &ascending));
+    if (nd > kMaxDiag) CEL_TRY(offset_count(M, &nd, &ascending));
     if (!ascending) return fail(CEL_ERR_BAD_MATRIX, "columns not strictly ascending in every row: no DIA form");
     if (nd > kMaxDiag)
-        return fail(CEL_ERR_BAD_MATRIX, "more diagonals than the DIA form holds (32)");
+        return fail(CEL_ERR_BAD_MATRIX, std::to_string(nd) + " diagonals: more than the DIA form holds (32)");
     if ((long long)nd * M.n > 2 * nnz)
         return fail(CEL_ERR_BAD_MATRIX, "DIA would store more than twice nnz slots");
     const size_t cnt = (size_t)nd * (size_t)M.n;
