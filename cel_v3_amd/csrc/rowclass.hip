@@ -504,10 +504,11 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric)
     // per iteration FP64 70^3 20.8 us either way, 80^3 23.4 without / 24.8
     // with the symmetric walk, 90^3 27.1 / 26.9, 100^3 33.1 / 30.7, 112^3 41.6
     // / 38.8, 128^3 58.3 / 51.8.  In the mixed form the other way is two
-    // kernels per iteration: 804,264 rows 21.0 / 21.5, 820,911 21.5 / 21.6,
+    // kernels per iteration (but for long rows): 804,264 rows 21.0 / 21.5, 820,911 21.5 / 21.6,
     // 100^3 23.2 / 21.0, 1,092,624 25.0 / 22.8, 1,179,780 25.9 / 24.8
     constexpr int kSymmetricMixed = 850000;
-    if (use == Derived::kNone && fmt == CEL_FMT_DIA && (!mixed || A.n >= kSymmetricMixed) && A.dia_nd > 0 && A.dia_nd <= kClassDiag && A.dia_mask8.p) {
+    const bool look = !mixed || A.n >= kSymmetricMixed || csr_long_rows(A);
+    if (use == Derived::kNone && fmt == CEL_FMT_DIA && look && A.dia_nd > 0 && A.dia_nd <= kClassDiag && A.dia_mask8.p) {
         signed char& y = D.sym[Derived::kOwnDia];  // (the FP32 copy of the values follows the FP64 ones)
         if (rc == CEL_OK) rc = dia_symmetric(A, A.dia_nd, A.dia_off, A.dia_vals.p, A.dia_mask8.p, &y);
         *symmetric = y == 1;
