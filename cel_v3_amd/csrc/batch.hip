@@ -1445,6 +1445,18 @@ extern "C" int cel_gpu_batch_info(const cel_gpu_batch* h, int* lanes, long long*
     return CEL_OK;
 }
 
+// For tests: the form each system's matrix had at the end of the last solve (0
+// CSR, 1 row classes, 2 diagonals) and the diagonals that were read.
+extern "C" int cel_gpu_internal_batch_forms(const cel_gpu_batch* h, int* kind, int* arrays)
+{
+    if (!h || !kind || !arrays) return fail(CEL_ERR_ARG, "null argument");
+    for (size_t q = 0; q < h->b.h_form.size(); ++q) {
+        kind[q] = h->b.h_form[q].kind;
+        arrays[q] = h->b.h_form[q].arrays;
+    }
+    return CEL_OK;
+}
+
 extern "C" int cel_gpu_batch_get_config(const cel_gpu_batch* h, int* grid, int* grid23, int* chunk,
                                         int* weight)
 {

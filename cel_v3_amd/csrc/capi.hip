@@ -1209,6 +1209,22 @@ extern "C" int cel_gpu_pcg_solve_noalloc(cel_gpu_mat* A, const double* b, double
     return rc;
 }
 
+// For tests: the path of the handle's last solve, as words.
+extern "C" int cel_gpu_internal_path(const cel_gpu_mat* A, char* out, int len)
+{
+    if (!A || !out || len < 1) return fail(CEL_ERR_ARG, "null argument");
+    const SolvePath& p = A->m.path;
+    std::string s = p.form;
+    const std::pair<bool, const char*> words[] = {{p.step, " step"}, {p.direct, " direct"}, {p.window, " window"},
+                                                  {p.wide, " wide"}, {p.deep, " deep"},     {p.keep, " keep"}};
+    for (const auto& w : words)
+        if (w.first) s += w.second;
+    if (p.stream) s += " stream" + std::to_string(p.stream);
+    std::strncpy(out, s.c_str(), (size_t)len - 1);
+    out[len - 1] = 0;
+    return CEL_OK;
+}
+
 // ------------------------------------------------------------------ adjoint
 extern "C" int cel_gpu_cg_adjoint(cel_gpu_mat* A, const double* x, const double* dLdx, double* dLdb,
                                   double* dLda, const cel_pcg_params* params, cel_pcg_stats* stats)

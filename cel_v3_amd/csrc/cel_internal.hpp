@@ -213,6 +213,19 @@ struct DerivedUse {
     void end();
 };
 
+// The kernels the last PCG or GMRES solve of a handle ran on: what
+// cel_gpu_internal_path reports, so that tests see which path they are on.
+struct SolvePath {
+    const char* form = "";  // the K1's matrix: csr, csr-long, dia, jad, classes; gmres
+    bool step = false;      // two kernels per iteration (GMRES: one launch per column)
+    bool direct = false;    // the step reads every row by its own thread
+    bool window = false;    // x of a band, or of a chunk, in LDS
+    bool wide = false;      // several rows per lane
+    bool deep = false;      // long rows several entries at a time
+    bool keep = false;      // the matrix loaded to stay in the cache
+    int stream = 0;         // vectors marked as read once: 0 none, 1 x, 2 all
+};
+
 struct Mat {
     int n = 0;          // local rows
     int ncols = 0;      // local columns (== n for a square local block)
@@ -252,6 +265,7 @@ struct Mat {
     Derived derived;
     int band = -1;     // largest |column - row| of the block (-1: not looked up)
     int longest = -1;  // most entries of a row (-1: not looked up)
+    SolvePath path;
 
     // halo (distributed block split of one rank)
     std::vector<HaloBlock> halo;

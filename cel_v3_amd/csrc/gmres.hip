@@ -979,6 +979,7 @@ int gmres_solve(Mat& A, const double* b_in, double* x_out, const cel_gmres_param
     if (small) CEL_TRY(w2.alloc(n));
     const GmMat GM = S.mat();
     const bool dia = prm.format == CEL_FMT_DIA, win = S.window();
+    A.path = SolvePath{"gmres", small, false, small && win};
     // the same on a small system: k_col in place of k_scale_jac / k_next and
     // the product
     auto enqueue_small = [&]() -> int {

@@ -1120,7 +1120,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(k1_waves
 // Per iteration, tiles in LDS / so: FP64 20^3 10.4 / 9.8 us, 32^3 10.5 / 9.95,
 // 40^3 11.8 / 11.2, 44^3 12.2 / 12.8, 64^3 14.4 / 15.0; mixed 20^3 12.1 / 11.3,
 // 32^3 11.8 / 10.9, 48^3 12.5 / 12.2, 52^3 13.6 / 14.1, 64^3 13.7 / 15.0; hence
-// the lines in step_kernel, 70,000 and 120,000 rows.
+// the lines in step_direct, 70,000 and 120,000 rows.
 template <typename VT>
 struct DirectGroup {
     static constexpr int R = kTileGroup;
@@ -1872,11 +1872,14 @@ template <typename VT>
 using StepFn = void (*)(MatView, const VT*, const VT*, VT*, VT*, double*, VT*, double*, ResArgs<VT>,
                         const double*, int, const Ctrl*, Ctrl*, Prm);
 
+// (lines: DirectGroup)
+static bool step_direct(int fmt, int n, bool mixed) { return fmt == CEL_FMT_CSR && n <= (mixed ? 120000 : 70000); }
+
 template <typename VT>
 static StepFn<VT> step_kernel(int fmt, int n)
 {
     if (fmt == CEL_FMT_JAD) return k_pcg_step<VT, CEL_FMT_JAD>;
-    if (fmt == CEL_FMT_CSR && n <= (sizeof(VT) == 8 ? 70000 : 120000)) return k_pcg_step<VT, CEL_FMT_CSR, true>;
+    if (step_direct(fmt, n, sizeof(VT) == 4)) return k_pcg_step<VT, CEL_FMT_CSR, true>;
     return fmt == CEL_FMT_DIA ? k_pcg_step<VT, CEL_FMT_DIA> : k_pcg_step<VT, CEL_FMT_CSR>;
 }
 
@@ -2431,6 +2434,12 @@ int pcg_solve(Mat& A, const double* b, double* x, const cel_pcg_params& prm, cel
     const float* vjac32 = bycls ? V.ctab.jac32 : jac32;
     const uint8_t *vcls = bycls ? V.cls : nullptr, *nocls = nullptr;
     const int stream = stream_level(n, mixed, bycls, sym ? arrays : 0);
+    A.path = SolvePath{bycls                    ? "classes"
+                       : kfmt == CEL_FMT_CSR ? (lr ? "csr-long" : "csr")
+                       : kfmt == CEL_FMT_DIA ? "dia"
+                                             : "jad",
+                       step, step && step_direct(fmt, n, mixed), win, bycls || sym, deep, step || (keep && !halo && !bycls),
+                       step ? 0 : stream};
     // One slot of the two-kernel form: the step finishes the iteration before
     // (its vectors and scalars) and forms the next product, K2 updates r.
     // The direction alternates between two buffers by slot.
