@@ -327,6 +327,10 @@ union BK1Stage {
     };
 };
 
+struct BCsrStage {
+    CsrStage<double> csr;
+};
+
 // v = A p of tiles [t0, t1) by classes or diagonals, one right-hand side: two
 // consecutive rows per lane, 16-byte loads, two tiles per step; the rows'
 // terms of v.p go through LDS to the threads that add them in the CSR walk,
@@ -429,7 +433,10 @@ __device__ __forceinline__ void b_wide_rows(const BSys& S, const BForm& F, const
 }
 
 // ---------------------------------------------------------------- K1
-// v = A p ; partial of v.p per lane.  Folds the set-up partials first.
+// v = A p ; partial of v.p per lane.  Folds the set-up partials first.  FORMS:
+// a matrix may be in another form than its CSR arrays (without: the walks of
+// those alone, 0.3 to 0.5 us of 20 an iteration less).
+template <bool FORMS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_bspmv(const BSys* __restrict__ sys,
                                                   const BForm* __restrict__ forms,
                                                   const BBlk* __restrict__ tbl,
@@ -439,7 +446,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                                                   const BCtrl* __restrict__ cin,
                                                   BCtrl* __restrict__ cout, BPrm P)
 {
-    __shared__ BK1Stage stage;
+    __shared__ std::conditional_t<FORMS, BK1Stage, BCsrStage> stage;
     CsrStage<double>& sm = stage.csr;
     __shared__ double red[4 * 64];
     __shared__ double s1[kMaxRhs], s2[kMaxRhs], s3[kMaxRhs];
@@ -449,6 +456,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     const BBlk blk = tbl[b];
     if (blk.sys < 0) return;
     const BSys S = load_sys(sys + blk.sys);
+    // (with the system, not behind its lanes: a round trip to memory of its own
+    // was 0.5 us of an iteration)
+    const BForm& F = forms[blk.sys];
+    const int kind = FORMS ? F.kind : (int)BForm::kCsr;
     read_lanes(cin, S, lc);
     if (lc[0].reduce == kBReduceSetup) {  // the same for every lane
         lane_partials(rpart, kpmax, S.b0, S.b1, S.kp, S.ksh, s1, red);
@@ -485,28 +496,35 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     const double* ps = p + S.voff;
     double* vs = v + S.voff;
     double acc = 0.0;
-    const BForm& F = forms[blk.sys];
-    const double* fvals = as_global(F.vals);
-    const uint8_t* rowb = as_global(F.rowb);
-    if (F.kind == BForm::kClasses) stage.tab.load(fvals, as_global(F.cmask));
-    if (S.kp == 1 && F.kind == BForm::kDiagonals) {
-        const WideDiags<double, true> src{fvals, F.base, rowb};
-        auto edge = [&](const int (&r)[2], double (&sum)[2]) {
-            dia_rows<double, 2, 8, true>(S.n, F.nd, F.off, fvals, rowb, nullptr, r, XPlain<double>{ps}, sum);
-        };
-        acc = F.nd <= 7 ? b_wide<7>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1)
-                        : b_wide<8>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1);
-    } else if (S.kp == 1 && F.kind == BForm::kClasses) {
-        const WideClasses<double> src{rowb, &stage.tab};
-        auto edge = [&](const int (&r)[2], double (&sum)[2]) {
-            class_rows<double, 2>(S.n, F.nd, F.off, rowb, stage.tab, r, XPlain<double>{ps}, sum);
-        };
-        acc = F.nd <= 7 ? b_wide<7>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1)
-                        : b_wide<8>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1);
-    } else if (S.kp == 1) {
+    const double* fvals = nullptr;
+    const uint8_t* rowb = nullptr;
+    bool walked = false;  // uniform
+    if constexpr (FORMS) {
+        fvals = as_global(F.vals);
+        rowb = as_global(F.rowb);
+        if (kind == BForm::kClasses) stage.tab.load(fvals, as_global(F.cmask));
+        if (S.kp == 1 && kind == BForm::kDiagonals) {
+            const WideDiags<double, true> src{fvals, F.base, rowb};
+            auto edge = [&](const int (&r)[2], double (&sum)[2]) {
+                dia_rows<double, 2, 8, true>(S.n, F.nd, F.off, fvals, rowb, nullptr, r, XPlain<double>{ps}, sum);
+            };
+            acc = F.nd <= 7 ? b_wide<7>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1)
+                            : b_wide<8>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1);
+            walked = true;
+        } else if (S.kp == 1 && kind == BForm::kClasses) {
+            const WideClasses<double> src{rowb, &stage.tab};
+            auto edge = [&](const int (&r)[2], double (&sum)[2]) {
+                class_rows<double, 2>(S.n, F.nd, F.off, rowb, stage.tab, r, XPlain<double>{ps}, sum);
+            };
+            acc = F.nd <= 7 ? b_wide<7>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1)
+                            : b_wide<8>(S.n, F, ps, vs, src, edge, stage.prod, blk.t0, blk.t1);
+            walked = true;
+        }
+    }
+    if (!walked && S.kp == 1) {
         // one right-hand side: the pipelined LDS tile of the single-system K1
         // (256 rows per tile, the next tile's loads in flight meanwhile)
-        CsrTileStream<double> cs;
+        CsrTileStream<double, false, kGather> cs;
         const int t0 = blk.t0, t1 = blk.t1;
         if (t0 < t1) {
             cs.start(S.n, t0, t0 + 1 < t1 ? t0 + 1 : -1, S.xadj, S.cols, S.vals, sm);
@@ -532,7 +550,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                 acc = acc + prod;
             }
         }
-    } else {
+    } else if (S.kp > 1) {
         // kp right-hand sides, two adjacent lanes per thread: the kp/2
         // threads of a row gather x[col][0..kp) contiguously, 16 bytes each
         // (one load instruction serves two lanes).  The block's steps go in
@@ -586,29 +604,31 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
             const int r0 = c * kTileRows;
             if (r0 >= S.n) break;  // uniform
             const int r1 = min(r0 + kTileRows, S.n);
-            if (F.kind == BForm::kClasses) {
-                if (on2) {
-                    if (F.nd <= 7) b_wide_rows<7, true>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
-                    else b_wide_rows<8, true>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+            if constexpr (FORMS) {
+                if (kind == BForm::kClasses) {
+                    if (on2) {
+                        if (F.nd <= 7) b_wide_rows<7, true>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                        else b_wide_rows<8, true>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                    }
+                    continue;
                 }
-                continue;
-            }
-            if (F.kind == BForm::kDiagonals) {
-                const int row = r0 + threadIdx.x;
-                const unsigned m = row < r1 ? rowb[row] : 0u;
-                double a[kClassDiag];
+                if (kind == BForm::kDiagonals) {
+                    const int row = r0 + threadIdx.x;
+                    const unsigned m = row < r1 ? rowb[row] : 0u;
+                    double a[kClassDiag];
 #pragma unroll
-                for (int d = 0; d < kClassDiag; ++d) a[d] = (m >> d) & 1u ? fvals[F.base[d] + row] : 0.0;
-                __syncthreads();  // the previous chunk's stage is consumed
+                    for (int d = 0; d < kClassDiag; ++d) a[d] = (m >> d) & 1u ? fvals[F.base[d] + row] : 0.0;
+                    __syncthreads();  // the previous chunk's stage is consumed
 #pragma unroll
-                for (int d = 0; d < kClassDiag; ++d) sm.val[d * kTileRows + threadIdx.x] = a[d];
-                sm.col[threadIdx.x] = (int)m;
-                __syncthreads();
-                if (on2) {
-                    if (F.nd <= 7) b_wide_rows<7, false>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
-                    else b_wide_rows<8, false>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                    for (int d = 0; d < kClassDiag; ++d) sm.val[d * kTileRows + threadIdx.x] = a[d];
+                    sm.col[threadIdx.x] = (int)m;
+                    __syncthreads();
+                    if (on2) {
+                        if (F.nd <= 7) b_wide_rows<7, false>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                        else b_wide_rows<8, false>(S, F, rowb, stage, r0, r1, pl, vl, acc, acc1);
+                    }
+                    continue;
                 }
-                continue;
             }
             const int e0 = S.xadj[r0];
             const int cnt = S.xadj[r1] - e0;
@@ -718,15 +738,26 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
                 const int row = r0 + st * R2 + my;
                 if (row < r1) {
                     const int lo = sx[row - r0], hi = sx[row - r0 + 1];
-                    double sum0 = 0.0, sum1 = 0.0;  // a chunk too large for the stage: entries from HBM
-                    for (int k = lo; k < hi; ++k) {
-                        const double a = ld_stream(S.vals + e0 + k);
-                        const Dbl2 xk =
-                            *(const Dbl2*)(pl + ((size_t)ld_stream(S.cols + e0 + k) << S.ksh));
-                        double prod0 = a * xk.x;
-                        double prod1 = a * xk.y;
-                        sum0 = sum0 + prod0;
-                        sum1 = sum1 + prod1;
+                    // a chunk too large for the stage: entries from HBM, the
+                    // loads of 8 together
+                    double sum0 = 0.0, sum1 = 0.0;
+                    for (int k0 = lo; k0 < hi; k0 += kGather) {
+                        double a[kGather];
+                        Dbl2 xk[kGather];
+#pragma unroll
+                        for (int i = 0; i < kGather; ++i) {
+                            const int k = e0 + min(k0 + i, hi - 1);
+                            a[i] = ld_stream(S.vals + k);
+                            xk[i] = *(const Dbl2*)(pl + ((size_t)ld_stream(S.cols + k) << S.ksh));
+                        }
+#pragma unroll
+                        for (int i = 0; i < kGather; ++i) {
+                            const double prod0 = a[i] * xk[i].x;
+                            const double prod1 = a[i] * xk[i].y;
+                            const double t0 = sum0 + prod0, t1 = sum1 + prod1;
+                            sum0 = k0 + i < hi ? t0 : sum0;
+                            sum1 = k0 + i < hi ? t1 : sum1;
+                        }
                     }
                     Dbl2 vi;
                     vi.x = 0.0 + sum0;
@@ -1018,7 +1049,7 @@ struct Batch {
 
 static int grid_max()
 {
-    int g = resident_grid((const void*)k_bspmv, 1 << 30);
+    int g = std::min(resident_grid((const void*)k_bspmv<true>, 1 << 30), resident_grid((const void*)k_bspmv<false>, 1 << 30));
     g = std::min(g, resident_grid((const void*)k_bresidual, 1 << 30));
     for (const void* k : {(const void*)k_bupdate_r<kBStreamNone>, (const void*)k_bupdate_r<kBStreamAll>,
                           (const void*)k_bupdate_xp<kBStreamNone>, (const void*)k_bupdate_xp<kBStreamX>,
@@ -1212,8 +1243,12 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     const auto k3 = stream == kBStreamAll ? k_bupdate_xp<kBStreamAll>
                     : stream == kBStreamX ? k_bupdate_xp<kBStreamX>
                                           : k_bupdate_xp<kBStreamNone>;
+    // (the graph is captured once: also where forms are only to be built)
+    bool forms = build && derived_wanted(B.mats, prm.iter_max);
+    for (const BForm& F : B.h_form) forms = forms || F.kind != BForm::kCsr;
+    const auto k1 = forms ? k_bspmv<true> : k_bspmv<false>;
     auto enqueue_iter = [&]() -> int {
-        hipLaunchKernelGGL(k_bspmv, dim3(G), dim3(kBlock), 0, s, B.d_sys.p, B.d_form.p, B.d_tbl.p, B.p.p, B.v.p,
+        hipLaunchKernelGGL(k1, dim3(G), dim3(kBlock), 0, s, B.d_sys.p, B.d_form.p, B.d_tbl.p, B.p.p, B.v.p,
                            B.part1.p, B.rpart.p, B.kpmax, G, C0, C1, P);
         hipLaunchKernelGGL(k2, dim3(G2), dim3(kBlock), 0, s, B.d_sys.p, B.d_tbl2.p, B.r.p,
                            B.v.p, B.part2.p, B.part1.p, B.kpmax, G2, C1, C2);

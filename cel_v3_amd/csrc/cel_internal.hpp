@@ -358,6 +358,8 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric);
 // The FP64 derived forms of a batch's matrices, also of those below
 // kDerivedRows (small: of the smallest, too).  false: there was nothing to try.
 bool derived_prepare_all(const std::vector<Mat*>& mats, int iter_max, bool small);
+// Whether it would try anything (small).
+bool derived_wanted(const std::vector<Mat*>& mats, int iter_max);
 // Where the wide walks find the values of nd <= kClassDiag diagonals: entry
 // (i, d) at base[d] + i of storage [nd][n].  Symmetric: those below the main
 // diagonal in the arrays above it, as entry (i, i + o), o < 0, is entry (i +

@@ -534,6 +534,25 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric)
 // after the first chunk 11.7).
 constexpr int kBatchRows = 20000;
 constexpr int kBatchAhead = 100000;
+// Whether derived_prepare_all would try the matrix: to be read by derived_prepare
+// (large), or in diagonal storage (from `least` rows on).
+static bool wanted_large(const Mat& A)
+{
+    const Derived& D = A.derived;
+    return A.n >= kDerivedRows && (!D.tried || (D.kind == Derived::kNone && D.nd > 0 && !D.tried64 &&
+                                                (long long)D.nd * A.n <= 2LL * A.nnz));
+}
+static bool wanted_small(const Mat& A, int least)
+{
+    return A.n < kDerivedRows && A.n >= least && !A.derived.tried64 && A.nnz > 0 && A.ncols == A.n;
+}
+bool derived_wanted(const std::vector<Mat*>& mats, int iter_max)
+{
+    return iter_max >= 32 && std::any_of(mats.begin(), mats.end(), [](const Mat* A) {
+               return wanted_large(*A) || wanted_small(*A, kBatchRows);
+           });
+}
+
 bool derived_prepare_all(const std::vector<Mat*>& mats, int iter_max, bool small)
 {
     bool any = false;
@@ -542,10 +561,9 @@ bool derived_prepare_all(const std::vector<Mat*>& mats, int iter_max, bool small
     for (Mat* A : mats) {
         bool sym;
         if (A->n >= kDerivedRows) {
-            any |= iter_max >= 32 && (!A->derived.tried || (A->derived.kind == Derived::kNone && !A->derived.tried64));
+            any |= iter_max >= 32 && wanted_large(*A);
             (void)derived_prepare(*A, CEL_FMT_CSR, false, iter_max, &sym);
-        } else if (A->n >= (small ? kBatchRows : kBatchAhead) && iter_max >= 32 && !A->derived.tried64 && A->nnz > 0 &&
-                   A->ncols == A->n) {
+        } else if (iter_max >= 32 && wanted_small(*A, small ? kBatchRows : kBatchAhead)) {
             A->derived.tried64 = true;  // (a matrix may be in the batch twice)
             todo.push_back(A);
         }
