@@ -1185,6 +1185,16 @@ static void choose_forms(Batch& B)
     }
 }
 
+// Iterations of a solve after which the derived forms that its matrices do not
+// have yet are built.  Ahead of it they cost batches that stop within a few
+// iterations more than they save; the first solve of one that goes on loses
+// little by a few iterations without.  First solves, without forms / built
+// ahead / after 4: 8 systems of 28^3..40^3, 2 iterations 1.34 / 1.63 / 1.08 ms,
+// 162 iterations 5.08 / 4.78 / 4.58; 4 of 60^3..70^3 3.0 / 2.0 / 1.5 and 15.2 /
+// 11.3 / 11.1; 2 of 28^3 and 30^3 0.72 / 0.85 / 0.56 and (123) 2.46 / 2.48 /
+// 2.57 (the next one 2.40); 64 of 24^3..96^3 352 iterations 258 / 189 / 186.
+constexpr int kFormsAfter = 4;
+
 struct RunResult {
     std::vector<BCtrl> lanes;
     float ms = 0.f;
@@ -1207,9 +1217,10 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     CEL_TRY(B.d_form.alloc(S));
     std::vector<DerivedUse> reading(S);
     for (int q = 0; q < S; ++q) reading[q].begin(B.mats[q]->derived);
-    derived_prepare_all(B.mats, sample ? 1 << 20 : prm.iter_max, sample);
+    if (sample) derived_prepare_all(B.mats, 1 << 20);
     choose_forms(B);
-    bool build = !sample;
+    // forms that are not there yet are built when the solve is found to go on
+    const bool build = !sample && derived_wanted(B.mats, prm.iter_max);
     std::vector<char> active(S, 1);
     std::vector<BBlk> tbl, tbl2;
     CEL_TRY(build_table(B, G, T.weight, active, tbl, false));
@@ -1243,8 +1254,7 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     const auto k3 = stream == kBStreamAll ? k_bupdate_xp<kBStreamAll>
                     : stream == kBStreamX ? k_bupdate_xp<kBStreamX>
                                           : k_bupdate_xp<kBStreamNone>;
-    // (the graph is captured once: also where forms are only to be built)
-    bool forms = build && derived_wanted(B.mats, prm.iter_max);
+    bool forms = build;  // (the graph is captured before they are)
     for (const BForm& F : B.h_form) forms = forms || F.kind != BForm::kCsr;
     const auto k1 = forms ? k_bspmv<true> : k_bspmv<false>;
     auto enqueue_iter = [&]() -> int {
@@ -1257,6 +1267,24 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
         CEL_HIP(hipGetLastError());
         return CEL_OK;
     };
+
+    BCtrl* hc = nullptr;
+    CEL_TRY(R.host_alloc(hc, 2 * (size_t)B.lanes));
+    const long long budget = (long long)iter_cap + 1;
+    long long enq = 0;
+    // the systems with running lanes, by the tokens at t
+    auto running = [&](const BCtrl* t, std::vector<char>& act) {
+        act.assign(S, 0);
+        for (int q = 0; q < S; ++q)
+            for (int l = 0; l < B.kp[q]; ++l)
+                if (t[B.lane0[q] + l].run) act[q] = 1;
+        return std::count(act.begin(), act.end(), 1) > 0;
+    };
+    std::vector<char> act;
+    if (build) {
+        for (; enq < kFormsAfter && enq < budget; ++enq) CEL_TRY(enqueue_iter());
+        CEL_HIP(hipMemcpyAsync(hc, C0, sizeof(BCtrl) * B.lanes, hipMemcpyDeviceToHost, s));
+    }
 
     // chunks of T.chunk iterations replayed from one captured graph; the
     // host checks the lanes one chunk behind and re-deals the blocks of
@@ -1273,16 +1301,26 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     CEL_HIP(hipGraphInstantiate(&R.exec, R.graph, nullptr, nullptr, 0));
     hipGraphExec_t gexec = R.exec;
 
-    BCtrl* hc = nullptr;
-    CEL_TRY(R.host_alloc(hc, 2 * (size_t)B.lanes));
+    bool more = true;
+    if (build) {
+        CEL_HIP(hipStreamSynchronize(s));
+        more = running(hc, act);
+        if (more) {
+            std::vector<Mat*> on;
+            for (int q = 0; q < S; ++q)
+                if (act[q]) on.push_back(B.mats[q]);
+            derived_prepare_all(on, prm.iter_max);
+            choose_forms(B);
+            CEL_TRY(upload_table(B, tbl, tbl2, s));
+        }
+    }
+
     hipEvent_t cev[2];
     CEL_TRY(R.event(cev[0], hipEventDisableTiming));
     CEL_TRY(R.event(cev[1], hipEventDisableTiming));
-    const long long budget = (long long)iter_cap + 1;
-    long long enq = 0;
     int k = 0;
     int rc = CEL_OK;
-    while (enq < budget) {
+    while (more && enq < budget) {
         CEL_HIP(hipGraphLaunch(gexec, s));
         enq += T.chunk;
         BCtrl* slot = hc + (size_t)(k & 1) * B.lanes;
@@ -1291,27 +1329,7 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
         if (k > 0) {
             CEL_HIP(hipEventSynchronize(cev[(k - 1) & 1]));
             const BCtrl* prev = hc + (size_t)((k - 1) & 1) * B.lanes;
-            std::vector<char> act(S, 0);
-            int nrun = 0;
-            for (int q = 0; q < S; ++q)
-                for (int l = 0; l < B.kp[q]; ++l)
-                    if (prev[B.lane0[q] + l].run) act[q] = 1;
-            for (int q = 0; q < S; ++q) nrun += act[q];
-            if (nrun == 0) break;
-            // the forms of small matrices that are not there yet, now that the
-            // solve goes on
-            if (build) {
-                build = false;
-                std::vector<Mat*> on;
-                for (int q = 0; q < S; ++q)
-                    if (act[q]) on.push_back(B.mats[q]);
-                if (derived_prepare_all(on, prm.iter_max, true)) {
-                    CEL_HIP(hipEventSynchronize(cev[k & 1]));  // the chunk in flight reads the table of forms
-                    choose_forms(B);
-                    rc = upload_table(B, tbl, tbl2, s);
-                    if (rc < 0) break;
-                }
-            }
+            if (!running(prev, act)) break;
             if (T.rebalance && act != active) {
                 // every lane of a dropped system has stored its final token
                 // in slot 0; the chunk in flight does not touch it again

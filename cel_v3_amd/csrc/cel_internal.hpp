@@ -355,10 +355,9 @@ int block_longest(const Mat& A, int& longest);
 // *symmetric: the diagonal storage the solve runs on (its own or a derived
 // one) holds bit for bit the same value at (i, j) and (j, i).
 int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric);
-// The FP64 derived forms of a batch's matrices, also of those below
-// kDerivedRows (small: of the smallest, too).  false: there was nothing to try.
-bool derived_prepare_all(const std::vector<Mat*>& mats, int iter_max, bool small);
-// Whether it would try anything (small).
+// The FP64 derived forms of a batch's matrices, smaller ones too.
+void derived_prepare_all(const std::vector<Mat*>& mats, int iter_max);
+// Whether it would try anything.
 bool derived_wanted(const std::vector<Mat*>& mats, int iter_max);
 // Where the wide walks find the values of nd <= kClassDiag diagonals: entry
 // (i, d) at base[d] + i of storage [nd][n].  Symmetric: those below the main

@@ -523,52 +523,42 @@ int derived_prepare(Mat& A, int fmt, bool mixed, int iter_max, bool* symmetric)
 // The matrices of a batch are read by one K1 per iteration however small each
 // of them is, so those below kDerivedRows get diagonal storage too, built
 // with two synchronisations for all of them.  One costs about 33 us of
-// kernels and its allocations, and saves 2.2 ns a row in 200 iterations.  So
-// the small ones (below kBatchAhead) are built when the solve is found to go
-// on after its first chunk; ahead of it they cost batches that stop there
-// more than they save.  First solves, without forms / built ahead / so, and
-// the later ones: 8 systems of 28^3..40^3 2 iterations 1.32 / 1.60 / 1.29 ms
-// (1.25), 162 iterations 5.2 / 4.6 / 4.8 (4.3); 2 of 28^3 and 30^3 123
-// iterations 2.50 / 2.47 / 2.54 (2.39).  Larger ones pay at once: 4 of
-// 60^3..70^3 2 iterations 3.0 without / 1.95, 272 iterations 15.6 / 11.1 (built
-// after the first chunk 11.7).
+// kernels and its allocations, and saves 2.2 ns a row in 200 iterations.
 constexpr int kBatchRows = 20000;
-constexpr int kBatchAhead = 100000;
-// Whether derived_prepare_all would try the matrix: to be read by derived_prepare
-// (large), or in diagonal storage (from `least` rows on).
+
+// Whether derived_prepare_all would try the matrix: as derived_prepare (large),
+// or in diagonal storage.
 static bool wanted_large(const Mat& A)
 {
     const Derived& D = A.derived;
     return A.n >= kDerivedRows && (!D.tried || (D.kind == Derived::kNone && D.nd > 0 && !D.tried64 &&
                                                 (long long)D.nd * A.n <= 2LL * A.nnz));
 }
-static bool wanted_small(const Mat& A, int least)
+static bool wanted_small(const Mat& A)
 {
-    return A.n < kDerivedRows && A.n >= least && !A.derived.tried64 && A.nnz > 0 && A.ncols == A.n;
+    return A.n < kDerivedRows && A.n >= kBatchRows && !A.derived.tried64 && A.nnz > 0 && A.ncols == A.n;
 }
 bool derived_wanted(const std::vector<Mat*>& mats, int iter_max)
 {
-    return iter_max >= 32 && std::any_of(mats.begin(), mats.end(), [](const Mat* A) {
-               return wanted_large(*A) || wanted_small(*A, kBatchRows);
-           });
+    return iter_max >= 32 && std::any_of(mats.begin(), mats.end(),
+                                         [](const Mat* A) { return wanted_large(*A) || wanted_small(*A); });
 }
 
-bool derived_prepare_all(const std::vector<Mat*>& mats, int iter_max, bool small)
+void derived_prepare_all(const std::vector<Mat*>& mats, int iter_max)
 {
-    bool any = false;
+    if (iter_max < 32) return;
     const std::string err = last_error();
     std::vector<Mat*> todo;
     for (Mat* A : mats) {
         bool sym;
-        if (A->n >= kDerivedRows) {
-            any |= iter_max >= 32 && wanted_large(*A);
+        if (wanted_large(*A)) {
             (void)derived_prepare(*A, CEL_FMT_CSR, false, iter_max, &sym);
-        } else if (iter_max >= 32 && wanted_small(*A, small ? kBatchRows : kBatchAhead)) {
+        } else if (wanted_small(*A)) {
             A->derived.tried64 = true;  // (a matrix may be in the batch twice)
             todo.push_back(A);
         }
     }
-    if (todo.empty()) return any;
+    if (todo.empty()) return;
     std::vector<DiagonalSet> sets;
     int rc = dia_offsets_all(todo, kClassDiag, sets);
     hipStream_t st = rt().stream;
@@ -613,7 +603,6 @@ bool derived_prepare_all(const std::vector<Mat*>& mats, int iter_max, bool small
         set_error(err);
         (void)hipGetLastError();
     }
-    return true;
 }
 
 }  // namespace cel

@@ -158,10 +158,9 @@ def test_batch_forms(gpu, scaled):
         assert gpu.lib().cel_gpu_internal_batch_forms(batch.h, kind, arrays) == 0
         return list(kind), [a for k, a in zip(kind, arrays) if k == 2]
 
-    # few iterations: none; a solve that stops in its first chunk: the large ones
+    # few iterations, or a solve that stops after a few: none
     assert forms(tol=1e-300, iter_max=31) == ([0] * 8, [])
-    small = [0, 0, 0, 0, 0, 0, 2, 1]
-    assert forms(tol=0.9, iter_max=1000) == (small, [7 if scaled else 4])
+    assert forms(tol=0.9, iter_max=1000) == ([0] * 8, [])
     full = ([0, 2, 2, 2, 2, 0, 2, 1], [7, 7, 5, 3, 7] if scaled else [4, 4, 3, 2, 4])
     assert forms(tol=1e-300, iter_max=40) == full
     assert forms(tol=0.9, iter_max=8) == full  # those that are there

@@ -213,9 +213,9 @@ for fit in (0, 1):
     assert out[1] == [5, 3207]    # then all 820,911
 
 
-def test_a_batch_that_stops_early_builds_no_forms_of_small_matrices(stub):
+def test_a_batch_that_stops_early_builds_no_forms(stub):
     out = stub("""
-B = cel.Batch([matrix(30, 31, 32), matrix(45, 46, 47)])
+B = cel.Batch([matrix(30, 31, 32), matrix(45, 46, 47), matrix(97, 93, 91)])
 S.stub_log_clear()
 B.solve([np.ones(m.n) for m in B.mats], iter_max=1000)   # (every lane is found stopped at the first look)
 out = [k for k, _ in launches() if "scan" in k or "fill<" in k]
