@@ -1281,8 +1281,9 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
         return std::count(act.begin(), act.end(), 1) > 0;
     };
     std::vector<char> act;
+    const int ahead = build ? std::min(kFormsAfter, T.chunk) : 0;
     if (build) {
-        for (; enq < kFormsAfter && enq < budget; ++enq) CEL_TRY(enqueue_iter());
+        for (int i = 0; i < ahead; ++i) CEL_TRY(enqueue_iter());
         CEL_HIP(hipMemcpyAsync(hc, C0, sizeof(BCtrl) * B.lanes, hipMemcpyDeviceToHost, s));
     }
 
@@ -1321,7 +1322,14 @@ static int run_batch(Batch& B, const Tuning& T, const cel_pcg_params& prm, int i
     int k = 0;
     int rc = CEL_OK;
     while (more && enq < budget) {
-        CEL_HIP(hipGraphLaunch(gexec, s));
+        if (k == 0 && ahead) {
+            // the rest of the first chunk: the blocks are re-dealt between the
+            // same iterations, and the sums grouped alike, in every solve
+            for (int i = ahead; i < T.chunk && rc >= 0; ++i) rc = enqueue_iter();
+            if (rc < 0) break;
+        } else {
+            CEL_HIP(hipGraphLaunch(gexec, s));
+        }
         enq += T.chunk;
         BCtrl* slot = hc + (size_t)(k & 1) * B.lanes;
         CEL_HIP(hipMemcpyAsync(slot, C0, sizeof(BCtrl) * B.lanes, hipMemcpyDeviceToHost, s));
