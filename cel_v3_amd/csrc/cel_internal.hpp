@@ -379,8 +379,6 @@ int dia_offsets_all(const std::vector<Mat*>& mats, int most, std::vector<Diagona
 // Diagonal-major values (v64, or v32 rounded to FP32) and row masks on at
 // most 8 diagonals; slots without an entry hold 0.
 int dia_fill(const Mat& A, int nd, const int* off, double* v64, float* v32, uint8_t* mask8);
-// Sets bit `bit` (= dia_nd) of the DIA row masks on the rows with halo
-// entries and clears it elsewhere; fails when the masks have no spare bit.
 int launch_halo_spmv(const Mat& A, const double* ghost, double* y);
 int launch_face_pack(const Mat& A, const double* x, double* sendbuf);
 int launch_extract_diag(Mat& A);
